@@ -99,9 +99,10 @@ constexpr int kRowsPerPass = kWave / kLanesPerRow;
 
 // Where element i of a query goes in LDS: the 8-byte pairs one lane of a quad
 // needs (pair a of every group of eight) lie next to each other, so that two
-// groups are one 16-byte read; two pairs of padding after each lane's run keep
-// the four runs on different banks.  `groups` = dp / 8.
-__host__ __device__ constexpr int query_run(int groups) { return groups + 2; }
+// groups are one 16-byte read; two pairs of padding after each lane's run (three
+// where the number of groups is odd: a run starts 16-byte aligned) keep the
+// four runs on different banks.  `groups` = dp / 8.
+__host__ __device__ constexpr int query_run(int groups) { return groups + 2 + (groups & 1); }
 __host__ __device__ constexpr int query_floats(int dp) { return 8 * query_run(dp >> 3); }
 __device__ __forceinline__ int query_slot(int i, int groups) {
     return 2 * (((i >> 1) & 3) * query_run(groups) + (i >> 3)) + (i & 1);
@@ -187,52 +188,99 @@ __host__ __device__ constexpr int row_pair_slot(int g, int a, int groups) {
 // at zero at `first`), in the host's order as above: the FMAs of a group
 // follow those of the group before it.  `row` is the row's start, `qrun` the
 // lane's run of the query in LDS (query_slot layout), `part` the lane's place
-// in its quad.  Eight blocks (16 groups) of loads are in flight at once.
-// Lane 0 of the quad returns the sum; every lane must call this.
+// in its quad.  Lane 0 of the quad returns the sum; every lane must call this.
+//
+// A row is read CHUNK blocks (2 CHUNK groups) at a time; what is left of a row
+// (and all of a row shorter than a chunk) is requested at once as well, in
+// pieces of 4, 2 and 1 blocks and the last group of an odd number.  A search
+// waits for its rows: taken one group after the other, each with its own trip
+// to memory, the rest (all of a 96-float row, every row with an odd number of
+// groups) made a whole wide-mode search of 3001 queries over a million
+// 96-float rows 2.66 ms, with the pieces 2.10 ms; two register sets, the next
+// chunk requested before this one is used, spilled (139 registers at H = 16).
 #ifndef PA_LONG_CHUNK
 #define PA_LONG_CHUNK 8
 #endif
+template <int CHUNK = PA_LONG_CHUNK>
 __device__ __forceinline__ float quad_square_dist_long(const float *row,
                                                        const float2 *qrun,
                                                        int groups, int first,
                                                        int part, bool active) {
+    static_assert((CHUNK & (CHUNK - 1)) == 0, "the rest is taken in halving pieces");
     float a0 = 0.f, a1 = 0.f;
     if (active) {
-        auto one_group = [&](int g) {
-            const float2 x = *reinterpret_cast<const float2 *>(
-                row + row_pair_slot(g, part, groups));
-            const float2 y = qrun[g];
+        const float4 *r4 = reinterpret_cast<const float4 *>(row) + part;
+        const float4 *q4 = reinterpret_cast<const float4 *>(qrun);
+        auto fetch = [&](float4 (&x)[CHUNK], int b) {
+#pragma unroll
+            for (int u = 0; u < CHUNK; ++u) x[u] = r4[4 * (b + u)];
+        };
+        auto use_block = [&](const float4 x, const float4 y) {
+            const float d0 = y.x - x.x, d1 = y.y - x.y;
+            a0 = fmaf(d0, d0, a0);
+            a1 = fmaf(d1, d1, a1);
+            const float d2 = y.z - x.z, d3 = y.w - x.w;
+            a0 = fmaf(d2, d2, a0);
+            a1 = fmaf(d3, d3, a1);
+        };
+        auto use = [&](const float4 (&x)[CHUNK], int b) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < CHUNK; ++u) {
+                use_block(x[u], q4[b + u]);
+                // not all of the query's reads at once: they take registers too
+                if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto use_group = [&](const float2 x, const float2 y) {
             const float d0 = y.x - x.x, d1 = y.y - x.y;
             a0 = fmaf(d0, d0, a0);
             a1 = fmaf(d1, d1, a1);
         };
-        int g = first;
-        // the query is read 16 bytes at a time: the run must start 16-byte
-        // aligned, which it does when the number of groups is even
-        if ((groups & 1) == 0) {
-            if (g & 1) one_group(g++);
-            constexpr int kChunk = PA_LONG_CHUNK;  // blocks per batch of loads
-            const float4 *r4 = reinterpret_cast<const float4 *>(row) + part;
-            const float4 *q4 = reinterpret_cast<const float4 *>(qrun);
-            for (; g + 2 * kChunk <= groups; g += 2 * kChunk) {
-                float4 x[kChunk];
+        // the blocks [b, blocks) left, fewer than CHUNK of them, and the last
+        // group of an odd number
+        const int blocks = groups >> 1;
+        float2 last;
+        auto fetch_rest = [&](float4 (&x)[CHUNK], int b) {
+            const int left = blocks - b;
 #pragma unroll
-                for (int u = 0; u < kChunk; ++u) x[u] = r4[4 * ((g >> 1) + u)];
-                __builtin_amdgcn_sched_barrier(0);
+            for (int piece = CHUNK / 2; piece >= 1; piece >>= 1) {
+                if (left & piece) {
+                    const int at = b + (left & ~(2 * piece - 1));
 #pragma unroll
-                for (int u = 0; u < kChunk; ++u) {
-                    const float4 y = q4[(g >> 1) + u];
-                    const float d0 = y.x - x[u].x, d1 = y.y - x[u].y;
-                    a0 = fmaf(d0, d0, a0);
-                    a1 = fmaf(d1, d1, a1);
-                    const float d2 = y.z - x[u].z, d3 = y.w - x[u].w;
-                    a0 = fmaf(d2, d2, a0);
-                    a1 = fmaf(d3, d3, a1);
+                    for (int u = 0; u < piece; ++u) x[CHUNK - 2 * piece + u] = r4[4 * (at + u)];
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
+            if (groups & 1)
+                last = *reinterpret_cast<const float2 *>(row + 8 * (groups - 1) + 2 * part);
+        };
+        auto use_rest = [&](const float4 (&x)[CHUNK], int b) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int left = blocks - b;
+#pragma unroll
+            for (int piece = CHUNK / 2; piece >= 1; piece >>= 1) {
+                if (left & piece) {
+                    const int at = b + (left & ~(2 * piece - 1));
+#pragma unroll
+                    for (int u = 0; u < piece; ++u)
+                        use_block(x[CHUNK - 2 * piece + u], q4[at + u]);
+                }
+            }
+            if (groups & 1) use_group(last, qrun[groups - 1]);
+        };
+        int b = first >> 1;
+        if ((first & 1) && b < blocks) {  // the second group of a block comes first
+            const float4 x = r4[4 * b];
+            use_group(make_float2(x.z, x.w), qrun[first]);
+            ++b;
         }
-        for (; g < groups; ++g) one_group(g);
+        float4 x[CHUNK];
+        for (; b + CHUNK <= blocks; b += CHUNK) {
+            fetch(x, b);
+            use(x, b);
+        }
+        fetch_rest(x, b);
+        use_rest(x, b);
     }
     return quad_reduce(a0, a1);
 }
@@ -270,7 +318,7 @@ __device__ __forceinline__ float quad_square_dist_rows(const float *row,
         }
         return quad_reduce(a0, a1);
     }
-    return quad_square_dist_long(row, qrun, groups, 0, part, active);
+    return quad_square_dist_long<>(row, qrun, groups, 0, part, active);
 }
 
 }  // namespace pa

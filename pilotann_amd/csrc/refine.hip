@@ -86,7 +86,7 @@ __device__ __forceinline__ void eval_rows_from(const float *__restrict__ storage
         const float *row = storage;
         if (active) row = storage + (size_t)cand_id[c] * (size_t)d;
         const float s =
-            quad_square_dist_long(row, qrun, groups, from >> 3, part, active);
+            quad_square_dist_long<>(row, qrun, groups, from >> 3, part, active);
         if (active && part == 0) cand_key[c] = s;
     }
 }
