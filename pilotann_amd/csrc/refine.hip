@@ -71,22 +71,24 @@ __global__ void reset_refine_counter(int *counter) { *counter = 0; }
 // rows listed in cand_id[0..n), written to cand_key: 16 rows per pass, four
 // lanes per row; the accumulators start at zero at `from`
 // (extension/inc/distance.h:31-55 called with an offset, traverse_cpu.cpp:56-59).
-// Rows are in the interleaved layout of pa_rows_prepare.
+// Rows are in the interleaved layout of pa_rows_prepare.  The WAVES wavefronts
+// of a workgroup take 16 rows each in turn.
+template <int WAVES, int CHUNK>
 __device__ __forceinline__ void eval_rows_from(const float *__restrict__ storage,
                                                const float *qv, const int *cand_id,
                                                float *cand_key, int n, int d,
-                                               int from, int lane) {
+                                               int from, int lane, int wave) {
     const int quad = lane >> 2, part = lane & 3;
     const int groups = d >> 3;
     const float2 *qrun =
         reinterpret_cast<const float2 *>(qv) + part * query_run(groups);
-    for (int base = 0; base < n; base += kRowsPerPass) {
+    for (int base = wave * kRowsPerPass; base < n; base += WAVES * kRowsPerPass) {
         const int c = base + quad;
         const bool active = c < n;
         const float *row = storage;
         if (active) row = storage + (size_t)cand_id[c] * (size_t)d;
-        const float s =
-            quad_square_dist_long<>(row, qrun, groups, from >> 3, part, active);
+        const float s = quad_square_dist_long<CHUNK>(row, qrun, groups, from >> 3,
+                                                     part, active);
         if (active && part == 0) cand_key[c] = s;
     }
 }
@@ -117,11 +119,22 @@ __global__ void interleave_rows(const float *__restrict__ src,
 #endif
 typedef Visited<PA_REFINE_SEEN_LOG2, PA_REFINE_SEEN_WAYS> RefineVisited;
 
-#define PA_REFINE_OCCUPANCY(H) \
-    __attribute__((amdgpu_waves_per_eu((H) <= 256 ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+constexpr int kHelped = 4;   // wavefronts of a query when there are few queries
+// blocks of a row read at once
+template <int WAVES>
+constexpr int kRefineChunk = WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
 
-template <int H>
-__global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(RefineArgs a) {
+#define PA_REFINE_OCCUPANCY(H, WAVES) \
+    __attribute__((amdgpu_waves_per_eu((H) <= 256 || ((WAVES) > 1 && (H) <= 512) ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+
+// WAVES = 1: the wavefront of a query reads its rows itself.  WAVES = 4: three
+// more wavefronts wait at a barrier and read rows with it.  A search with the
+// device to itself waits for its rows 58 % of the time (768 floats, H = 32):
+// 22 rows an expansion are two passes of 16, each of six trips to memory at 8
+// blocks a trip; with four wavefronts they are one pass of three trips at 16
+// blocks, which still fits the 128 registers that four wavefronts a SIMD have.
+template <int H, int WAVES>
+__global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void refine_kernel(RefineArgs a) {
     constexpr int S = (H + kWave - 1) / kWave;
     constexpr int kSortN = H <= kWave ? kWave : 1 << (floor_log2(H - 1) + 1);
     constexpr int kHeapCells =
@@ -130,13 +143,41 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
         uint32_t seen_table[RefineVisited::kWords];
         int cand_id[kWave];
         float cand_key[kWave];
+        int job_rows, job_from;  // WAVES > 1: rows to read, from which coordinate
         int2 heap[kHeapCells];   // open list tail; the sorts reuse it
         int res_key[Results<S>::kLdsKeys];  // result list: keys, unless in registers
                                             // (values: the slot's memory)
     };
     __shared__ __align__(16) Lds lds;
     extern __shared__ __align__(16) float qv[];  // the query, query_slot layout
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int d = a.d;
+    if constexpr (WAVES > 1) {
+        // a scalar: the two sides of this branch meet at the same barriers,
+        // two per job, and one when the queries are used up
+        const int wave = uni((int)(threadIdx.x / kWave));
+        if (wave > 0) {
+            for (;;) {
+                __syncthreads();
+                const int n = uni(lds.job_rows);
+                if (n < 0) return;
+                eval_rows_from<WAVES, kRefineChunk<WAVES>>(a.storage, qv, lds.cand_id,
+                                                          lds.cand_key, n, d,
+                                                          uni(lds.job_from), lane, wave);
+                __syncthreads();
+            }
+        }
+    }
+    // distances of the n rows in cand_id over the coordinates [from, d)
+    auto eval = [&](int n, int from) {
+        if constexpr (WAVES > 1) {
+            lds.job_rows = n, lds.job_from = from;
+            __syncthreads();
+        }
+        eval_rows_from<WAVES, kRefineChunk<WAVES>>(a.storage, qv, lds.cand_id,
+                                                  lds.cand_key, n, d, from, lane, 0);
+        if constexpr (WAVES > 1) __syncthreads();
+    };
     float *okey = reinterpret_cast<float *>(lds.heap);
     int *oval = reinterpret_cast<int *>(okey + kHeapCells);
     OpenList<H> open;
@@ -144,7 +185,6 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
     open.deep = nullptr;  // the whole list in registers and LDS
     int *cand_id = lds.cand_id;
     float *cand_key = lds.cand_key;
-    const int d = a.d;
     uint32_t *seen = a.seen + (size_t)blockIdx.x * (size_t)a.slot_stride;
     RefineVisited visited;
     visited.init(lds.seen_table, seen, a.n_nodes);
@@ -157,7 +197,13 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
         int q = 0;
         if (lane == 0) q = atomicAdd(a.work_counter, 1);
         q = uni(q);
-        if (q >= a.batch) break;
+        if (q >= a.batch) {
+            if constexpr (WAVES > 1) {
+                lds.job_rows = -1;
+                __syncthreads();
+            }
+            break;
+        }
 
         unsigned n_expand0 = 0, n_expand1 = 0, n_dist = 0, n_admit = 0, n_tail = 0, n_adj = 0;
 #ifdef PA_PHASE_TIMERS
@@ -213,8 +259,7 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
                     const int rank = lane_rank(mask);
                     if (u >= 0) cand_id[rank] = u;
                     wave_sync();
-                    eval_rows_from(a.storage, qv, cand_id, cand_key, n, d,
-                                   tail_from, lane);
+                    eval(n, tail_from);
                     n_tail += n;
                     wave_sync();
                     PA_TIMER(1);
@@ -261,7 +306,7 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
                 if (n == 0) continue;
                 if (fresh) cand_id[lane_rank(mask)] = v;
                 wave_sync();
-                eval_rows_from(a.storage, qv, cand_id, cand_key, n, d, 0, lane);
+                eval(n, 0);
                 n_dist += n;
                 wave_sync();
                 PA_TIMER(5);
@@ -369,20 +414,21 @@ __global__ __launch_bounds__(kWave) PA_REFINE_OCCUPANCY(H) void refine_kernel(Re
 
 typedef void (*RefineFn)(RefineArgs);
 
+template <int WAVES>
 RefineFn pick_kernel(int H) {
     switch (H) {
-        case 16: return refine_kernel<16>;
-        case 32: return refine_kernel<32>;
-        case 48: return refine_kernel<48>;
-        case 64: return refine_kernel<64>;
-        case 96: return refine_kernel<96>;
-        case 128: return refine_kernel<128>;
-        case 192: return refine_kernel<192>;
-        case 256: return refine_kernel<256>;
-        case 384: return refine_kernel<384>;
-        case 512: return refine_kernel<512>;
-        case 1024: return refine_kernel<1024>;
-        case 2048: return refine_kernel<2048>;
+        case 16: return refine_kernel<16, WAVES>;
+        case 32: return refine_kernel<32, WAVES>;
+        case 48: return refine_kernel<48, WAVES>;
+        case 64: return refine_kernel<64, WAVES>;
+        case 96: return refine_kernel<96, WAVES>;
+        case 128: return refine_kernel<128, WAVES>;
+        case 192: return refine_kernel<192, WAVES>;
+        case 256: return refine_kernel<256, WAVES>;
+        case 384: return refine_kernel<384, WAVES>;
+        case 512: return refine_kernel<512, WAVES>;
+        case 1024: return refine_kernel<1024, WAVES>;
+        case 2048: return refine_kernel<2048, WAVES>;
         default: return nullptr;
     }
 }
@@ -390,7 +436,7 @@ RefineFn pick_kernel(int H) {
 int round_up(int64_t x, int64_t m) { return (int)(((x + m - 1) / m) * m); }
 
 struct Plan {
-    int H, sort_n, lds_bytes, n_slots, words_per_slot, slot_stride;
+    int H, sort_n, lds_bytes, n_slots, words_per_slot, slot_stride, threads;
     size_t workspace_bytes;
     RefineFn fn;
 };
@@ -399,6 +445,31 @@ struct Plan {
 #define PA_REFINE_MAX_WAVES 20
 #endif
 constexpr int kMaxWavesPerCu = PA_REFINE_MAX_WAVES;
+
+// Workgroups of `fn` the current device holds at once.
+int residency(RefineFn fn, int threads, int lds_bytes, int *slots) {
+    int dev = 0, cus = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    // the residency of a (device, kernel, LDS size) never changes
+    static std::mutex mutex;
+    static std::map<std::tuple<int, const void *, int>, int> known;
+    std::lock_guard<std::mutex> guard(mutex);
+    const auto key = std::make_tuple(dev, reinterpret_cast<const void *>(fn), lds_bytes);
+    auto it = known.find(key);
+    if (it == known.end()) {
+        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e == hipSuccess)
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void *>(fn), threads, lds_bytes);
+        if (e != hipSuccess) return (int)e;
+        if (per_cu < 1) per_cu = 1;
+        if (per_cu > kMaxWavesPerCu) per_cu = kMaxWavesPerCu;
+        it = known.emplace(key, per_cu * cus).first;
+    }
+    *slots = it->second;
+    return PA_OK;
+}
 
 int make_plan(int64_t n_nodes, int64_t batch, int d, int ef_search, Plan *p) {
     if (n_nodes <= 0 || batch < 0) return PA_E_SHAPE;
@@ -409,35 +480,25 @@ int make_plan(int64_t n_nodes, int64_t batch, int d, int ef_search, Plan *p) {
     p->sort_n = kWave;
     while (p->sort_n < p->H) p->sort_n <<= 1;
     p->lds_bytes = query_floats(d) * 4;
-    p->fn = pick_kernel(p->H);
+    // Four wavefronts per query as long as every query has its workgroup at
+    // once (1024 queries at H <= 512).  Measured on 1M x 768, H = 32: 1 query
+    // 374 -> 286 us, 37 482 -> 322, 512 642 -> 447; beyond that the wavefronts
+    // that only read rows take the place of queries: 1536 910 -> 1100 us.
+    p->threads = kHelped * kWave;
+    p->fn = pick_kernel<kHelped>(p->H);
     if (!p->fn) return PA_E_EF;
-    int dev = 0, cus = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    {
-        static std::mutex mutex;
-        static std::map<std::tuple<int, const void *, int>, std::pair<int, int>> known;
-        std::lock_guard<std::mutex> guard(mutex);
-        const auto key = std::make_tuple(
-            dev, reinterpret_cast<const void *>(p->fn), p->lds_bytes);
-        auto it = known.find(key);
-        if (it == known.end()) {
-            e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-            if (e == hipSuccess)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void *>(p->fn), kWave,
-                    p->lds_bytes);
-            if (e != hipSuccess) return (int)e;
-            it = known.emplace(key, std::make_pair(cus, per_cu)).first;
-        }
-        cus = it->second.first, per_cu = it->second.second;
+    int slots = 0;
+    int rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
+    if (rc != PA_OK) return rc;
+    if (batch > slots) {
+        p->threads = kWave;
+        p->fn = pick_kernel<1>(p->H);
+        rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
+        if (rc != PA_OK) return rc;
     }
-    if (per_cu < 1) per_cu = 1;
-    if (per_cu > kMaxWavesPerCu) per_cu = kMaxWavesPerCu;
-    int64_t slots = (int64_t)per_cu * cus;
-    if (slots > batch) slots = batch;
+    if (slots > batch) slots = (int)batch;
     if (slots < 1) slots = 1;
-    p->n_slots = (int)slots;
+    p->n_slots = slots;
     p->words_per_slot = round_up((n_nodes + 31) / 32, kSlotAlignWords);
     // a slot: the visited slice, then the values of the result list
     p->slot_stride = p->words_per_slot + round_up(p->H, kWave);
@@ -522,6 +583,6 @@ extern "C" int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I,
 
     hipStream_t stream = (hipStream_t)stream_;
     reset_refine_counter<<<1, 1, 0, stream>>>(a.work_counter);
-    p.fn<<<p.n_slots, kWave, p.lds_bytes, stream>>>(a);
+    p.fn<<<p.n_slots, p.threads, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
 }
