@@ -145,8 +145,6 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
         float cand_key[kWave];
         int job_rows, job_from;  // WAVES > 1: rows to read, from which coordinate
         int2 heap[kHeapCells];   // open list tail; the sorts reuse it
-        int res_key[Results<S>::kLdsKeys];  // result list: keys, unless in registers
-                                            // (values: the slot's memory)
     };
     __shared__ __align__(16) Lds lds;
     extern __shared__ __align__(16) float qv[];  // the query, query_slot layout
@@ -236,14 +234,17 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
 
             PA_TIMER(0);
             open.reset(lane);
-            Results<S> res;
-            res.rk = lds.res_key;
-            res.rv = reinterpret_cast<int *>(seen + a.words_per_slot);
+            ResultKeys<S> res;
             res.init(H, lane);
+            ResultLog log;
+            log.entry = reinterpret_cast<int2 *>(seen + a.words_per_slot);
+            log.capacity = ResultLog::capacity_for(H);
+            log.n = 0;
             wave_sync();
 
             // traverse_cpu.cpp:42-79: complete the entries' distances, mark
             // the entries, push them on the open list in order
+            typename OpenList<H>::Leaf leaf = open.walk_to_large_leaf();
             for (int base = 0; base < n_ent; base += kWave) {
                 const int i = base + lane;
                 int u = -1;
@@ -270,25 +271,17 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     wave_sync();
                 }
                 if (u >= 0) visited.mark(u);
-                const int cnt = min(kWave, n_ent - base);
-                for (int j = 0; j < cnt; ++j) {
-                    const int uj = __builtin_amdgcn_readlane(u, j);
-                    if (uj < 0) continue;
-                    const float dj = __int_as_float(
-                        __builtin_amdgcn_readlane(__float_as_int(dist), j));
-                    open.template replace<true>(float_to_key(dj), uj, lane);
-                }
+                open.push_entries(leaf, __ballot(u >= 0), float_to_key(dist), u, lane);
                 PA_TIMER(2);
             }
 
-            // traverse_cpu.cpp:82-136
-            for (int step = 0; step < max_iter; ++step) {
-                int uk, u;
-                open.pop(lane, uk, u);
-                PA_TIMER(3);
-                if (u < 0 || uk >= res.worst) break;
-                n_expand0 += stage == 0, n_expand1 += stage != 0;
+            // traverse_cpu.cpp:82-136.  The next node's row of neighbour ids is
+            // requested as soon as the pop has shown which node is next, and
+            // again only if an insert put another one first: the request is
+            // on its way while this node's rows are read.
+            auto load_row = [&](int u) -> int {
                 int v = -1;
+                if (u < 0) return v;
                 if (stage == 0) {
                     const int64_t r = a.sub_mapping[u];
                     if (r >= 0 && lane < deg) {
@@ -298,10 +291,23 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 } else if (lane < deg) {
                     v = a.full_adj[(size_t)u * deg + lane];
                 }
+                return v;
+            };
+            int next = open.rl(open.Av, 1);
+            int next_row = load_row(next);
+            for (int step = 0; step < max_iter; ++step) {
+                int uk, u;
+                open.pop(lane, uk, u);
+                PA_TIMER(3);
+                if (u < 0 || uk >= res.worst) break;
+                n_expand0 += stage == 0, n_expand1 += stage != 0;
+                const int v = next_row;
                 n_adj += deg;
                 const bool fresh = v >= 0 && visited.mark(v);
                 const unsigned long long mask = __ballot(fresh);
                 const int n = __popcll(mask);
+                next = open.rl(open.Av, 1);
+                next_row = load_row(next);
                 PA_TIMER(4);
                 if (n == 0) continue;
                 if (fresh) cand_id[lane_rank(mask)] = v;
@@ -315,18 +321,34 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 wave_sync();
                 // heap_update, traverse_cpu.cpp:25-39, in adjacency order
                 unsigned long long todo = __ballot(dk < res.worst);
+                unsigned long long admitted = 0;
                 while (todo) {
                     const int j = __builtin_ctzll(todo);
                     todo &= todo - 1;
                     const int dj = __builtin_amdgcn_readlane(dk, j);
                     if (dj >= res.worst) continue;
                     const int vj = __builtin_amdgcn_readlane(id, j);
-                    int mine[S];
-                    res.begin_insert(dj, vj, lane, mine);
-                    const typename OpenList<H>::Leaf leaf = open.walk_to_large_leaf();
-                    res.finish_insert(lane, mine);
+                    if (OpenList<H>::kFusedTop) {
+                        // the result list's new maximum and the top of the
+                        // open list's walk in one instruction stream
+                        const typename OpenList<H>::Choice ch = open.template choices<true>();
+                        int first = res.replace_worst(dj, lane);
+                        const int j7 = OpenList<H>::top_levels_and_wave_max(ch, first);
+                        res.set_worst(first);
+                        leaf = open.walk_below(ch, 7, j7);
+                    } else {
+                        leaf = open.walk_to_large_leaf();
+                        res.insert(dj, lane);
+                    }
                     open.replace_leaf(leaf, dj, vj, lane);
-                    n_admit += 1;
+                    admitted |= 1ull << j;
+                }
+                if (admitted) {
+                    n_admit += __popcll(admitted);
+                    log.append(admitted, dk, id, lane);
+                    if (log.nearly_full()) log.cut(res.worst, lane);
+                    const int root = open.rl(open.Av, 1);
+                    if (root != next) next = root, next_row = load_row(root);
                 }
                 PA_TIMER(6);
             }
@@ -344,26 +366,50 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 }
                 const int dk = float_to_key(dist);
                 unsigned long long todo = __ballot(u >= 0 && dk < res.worst);
+                unsigned long long admitted = 0;
                 while (todo) {
                     const int j = __builtin_ctzll(todo);
                     todo &= todo - 1;
                     const int dj = __builtin_amdgcn_readlane(dk, j);
                     if (dj >= res.worst) continue;
-                    res.insert(dj, __builtin_amdgcn_readlane(u, j), lane);
+                    res.insert(dj, lane);
+                    admitted |= 1ull << j;
+                }
+                if (admitted) {
+                    log.append(admitted, dk, u, lane);
+                    if (log.nearly_full()) log.cut(res.worst, lane);
                 }
             }
 
             // traverse_cpu.cpp:150-162: best first; with more output slots
-            // than heap cells the surplus comes first, as (-1, -inf).  Sorted
-            // in the LDS the open list no longer needs.
+            // than heap cells the surplus comes first, as (-1, -inf).  The
+            // set is read back from the log, every entry below the maximum
+            // and of those at it as many as make H, and sorted in the LDS the
+            // open list no longer needs.
             wave_sync();
+            ResultLog::settle();
             for (int i = lane; i < a.sort_n; i += kWave)
                 okey[i] = INFINITY, oval[i] = -1;
             wave_sync();
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const int e = lane * S + s;
-                if (e < H) okey[e] = key_to_float(res.cell_key(lane, s)), oval[e] = res.rv[e];
+            int at_worst = 0;
+            for (int base = 0; base < log.n; base += kWave) {
+                const int i = base + lane;
+                at_worst += __popcll(__ballot(i < log.n && log.entry[i].x < res.worst));
+            }
+            int at_below = 0;
+            for (int base = 0; base < log.n; base += kWave) {
+                const int i = base + lane;
+                int2 e = make_int2(0x7fffffff, -1);
+                if (i < log.n) e = log.entry[i];
+                const bool below = i < log.n && e.x < res.worst;
+                const bool tie = i < log.n && e.x == res.worst;
+                const unsigned long long mb = __ballot(below), mt = __ballot(tie);
+                int place = -1;
+                if (below) place = at_below + lane_rank(mb);
+                if (tie) place = at_worst + lane_rank(mt);
+                if (place >= 0 && place < H) okey[place] = key_to_float(e.x), oval[place] = e.y;
+                at_below += __popcll(mb);
+                at_worst += __popcll(mt);
             }
             wave_sync();
             for (int size = 2; size <= a.sort_n; size <<= 1) {
@@ -500,8 +546,8 @@ int make_plan(int64_t n_nodes, int64_t batch, int d, int ef_search, Plan *p) {
     if (slots < 1) slots = 1;
     p->n_slots = slots;
     p->words_per_slot = round_up((n_nodes + 31) / 32, kSlotAlignWords);
-    // a slot: the visited slice, then the values of the result list
-    p->slot_stride = p->words_per_slot + round_up(p->H, kWave);
+    // a slot: the visited slice, then the log of admitted candidates
+    p->slot_stride = p->words_per_slot + 2 * ResultLog::capacity_for(p->H);
     p->workspace_bytes =
         kWorkCounterBytes + (size_t)p->n_slots * p->slot_stride * 4;
     return PA_OK;

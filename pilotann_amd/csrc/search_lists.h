@@ -463,105 +463,33 @@ struct OpenList {
             if (rise(L)) return;
         put(0, 1, k, v, lane);
     }
-    template <bool SPARSE = false>
-    __device__ __forceinline__ void replace(int k, int v, int lane) {
-        const Leaf leaf = walk_to_large_leaf();
-        replace_leaf<SPARSE>(leaf, k, v, lane);
+    // Pushes, in lane order, the entries (k, v) of the lanes in `who`, as one
+    // replace after the other would.  `leaf` is where the walk ends in the
+    // list as it stands: an entry not below its key changes nothing, so the
+    // walk is taken again only after an entry that got in, and everything
+    // that stays out is passed over by one comparison of all lanes.  Entries
+    // mostly come in ascending order; then nearly all of them stay out (the
+    // walk follows the larger child, not the free cells).
+    __device__ __forceinline__ void push_entries(Leaf &leaf, unsigned long long who,
+                                                 int k, int v, int lane) {
+        for (;;) {
+            const unsigned long long in = who & __ballot(k < leaf.key);
+            if (!in) return;
+            const int j = __builtin_ctzll(in);
+            who &= ~1ull << j;
+            replace_leaf<true>(leaf, rl(k, j), rl(v, j), lane);
+            leaf = walk_to_large_leaf();
+        }
     }
 };
 
-// ---- result list: the H smallest distances ------------------------------------
+// ---- result list: the H smallest distances, sorted keys per lane, entries in a log --
 //
 // The reference keeps them in a heap of negated keys whose root is the worst
 // kept (traverse_cpu.cpp:21-39): a candidate enters iff its distance is
 // strictly below that root, and replaces it.  Which array cell holds what has
-// no effect on the search; only the set and its maximum do.  Here the cells
-// are a flat LDS array, S per lane (lane l owns cells l*S .. l*S+S-1), of which
-// the registers keep only each lane's maximum, the wavefront's maximum and the
-// position of one cell that holds it: an insert is one store to that cell,
-// one read of every lane's own cells and a wavefront maximum.  Empty cells
-// hold +inf (so the maximum is +inf until H candidates came), cells beyond H
-// hold -inf and never win.  (Long lists keep the keys in registers instead.)
-
-template <int S>
-struct Results {
-    static constexpr int kInf = 0x7f800000;      // float_to_key(+inf)
-    static constexpr int kNegInf = (int)0x807fffff;  // float_to_key(-inf)
-    // Long lists (eight cells per lane and more) keep their keys in
-    // registers: that is lane-masked selects instead of LDS traffic per
-    // insert, and 4 KB of LDS less per wavefront at H = 1024, which is what
-    // bounds the residency there (measured 28.1 -> 23.3 ms per 10 000 queries
-    // at H = 1024; at H = 256 the LDS form is as fast or faster).
-    static constexpr bool kRegKeys = S >= 8;
-    static constexpr int kLdsKeys = kRegKeys ? 4 : S * kWave;
-    int key_reg[S];  // kRegKeys: the lane's cells
-    int *rk;      // !kRegKeys: LDS, float_to_key of the distance, kWave * S cells
-    int *rv;      // device memory: the values, same cells (written once per
-                  // insert, read at the end; every lane stores the same value
-                  // to a cell and so reads back its own store)
-    int lane_max;
-    int worst;    // uniform
-    int pos;      // uniform: a cell whose key is `worst`
-
-    __device__ __forceinline__ void init(int H, int lane) {
-        lane_max = kNegInf;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const int c = lane * S + s;
-            const int k = c < H ? kInf : kNegInf;
-            if (kRegKeys) key_reg[s] = k;
-            else rk[c] = k;
-            rv[c] = -1;
-            lane_max = max(lane_max, k);
-        }
-        worst = kInf;
-        pos = 0;
-    }
-    __device__ __forceinline__ int cell_key(int lane, int s) const {
-        return kRegKeys ? key_reg[s] : rk[lane * S + s];
-    }
-    // Caller has checked k < worst.  In two parts so that the caller can put
-    // independent work between the LDS traffic and its use.
-    __device__ __forceinline__ void begin_insert(int k, int v, int lane, int (&key)[S]) {
-        // Every lane stores the same pair to the same cell, so the lane that
-        // owns the cell reads back its own store: program order is enough.
-        rv[pos] = v;
-        if (kRegKeys) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                key_reg[s] = lane * S + s == pos ? k : key_reg[s];
-                key[s] = key_reg[s];
-            }
-        } else {
-            rk[pos] = k;
-#pragma unroll
-            for (int s = 0; s < S; ++s) key[s] = rk[lane * S + s];
-        }
-    }
-    __device__ __forceinline__ void finish_insert(int lane, const int (&key)[S]) {
-        int m = key[0];
-#pragma unroll
-        for (int s = 1; s < S; ++s) m = max(m, key[s]);
-        lane_max = m;
-        worst = wave_max_key(lane_max);
-        // the first lane that holds the new maximum, its first such cell
-        const int holder = __builtin_ctzll(__ballot(lane_max == worst));
-        int c = lane * S + S - 1;
-#pragma unroll
-        for (int s = S - 2; s >= 0; --s) c = key[s] == worst ? lane * S + s : c;
-        pos = __builtin_amdgcn_readlane(c, holder);
-    }
-    __device__ __forceinline__ void insert(int k, int v, int lane) {
-        int key[S];
-        begin_insert(k, v, lane, key);
-        finish_insert(lane, key);
-    }
-};
-
-// ---- result list of the traversal: sorted keys per lane, entries in a log -------
-//
-// The same set as Results<S> above, kept so that an insert touches no cell by
-// position.  Lane l owns S keys, largest first; the set's maximum is the
+// no effect on the search; only the set and its maximum do.  Here lane l owns
+// S keys, largest first; the set's maximum is the
 // largest first key, `holder` a lane that has it.  A candidate below the
 // maximum replaces it: in the holder lane the first key leaves and the new
 // key is sorted in, one v_med3_i32 per key (new[s] = the new key clamped
@@ -569,7 +497,10 @@ struct Results {
 // instructions with the largest integer for a key, which changes nothing.
 // Then a wavefront maximum over the first keys.  No key is ever looked up by
 // cell, so nothing depends on S but the S clamps: 22 instructions at S = 2,
-// 28 at S = 8, against 33 and 71 for the flat cells of Results<S>.
+// 28 at S = 8 (cells looked up by position: 33 and 71).  Measured in the
+// refine, with the entries pushed by push_entries and the next row requested
+// early: 10 000 queries over 1M x 96 at H = 96 2.48 -> 2.10 ms, one query 512
+// -> 451 us; 1M x 768 at H = 256, 37 queries 1.37 -> 1.14 ms.
 // Which node a key belongs to is not kept here: every admitted candidate is
 // also appended to a log in the wavefront's device memory (ResultLog), and
 // the final set is read back from the log by its keys.

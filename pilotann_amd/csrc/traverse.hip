@@ -202,6 +202,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         // is popped, and costs a step, like any other.
         const int64_t *eI = a.init_I + (size_t)q * a.n_init;
         const float *eD = a.init_D + (size_t)q * a.n_init;
+        typename Open::Leaf leaf = open.walk_to_large_leaf();
         for (int base = 0; base < a.n_init; base += kWave) {
             const int i = base + lane;
             int u = -1, row = -1;
@@ -216,15 +217,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                         atomicOr(&seen[row >> 5], 1u << (row & 31));
                 }
             }
-            const int cnt = min(kWave, a.n_init - base);
-            for (int j = 0; j < cnt; ++j) {
-                const int uj = __builtin_amdgcn_readlane(u, j);
-                if (uj < 0) continue;
-                const int rj = __builtin_amdgcn_readlane(row, j);
-                const float dj =
-                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), j));
-                open.template replace<true>(float_to_key(dj), rj >= 0 ? rj : -2 - (base + j), lane);
-            }
+            open.push_entries(leaf, __ballot(u >= 0), float_to_key(d),
+                              row >= 0 ? row : -2 - i, lane);
         }
 
         PA_TIMER(5);
@@ -301,7 +295,6 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                         const int dj = __builtin_amdgcn_readlane(d, j);
                         if (dj >= res.worst) continue;
                         const int vj = __builtin_amdgcn_readlane(id, j);
-                        typename Open::Leaf leaf;
                         if (Open::kFusedTop) {
                             // the result list's new maximum and the top of
                             // the open list's walk in one instruction stream
