@@ -321,6 +321,48 @@ __device__ __forceinline__ float quad_square_dist_rows(const float *row,
     return quad_square_dist_long<>(row, qrun, groups, 0, part, active);
 }
 
+// Two such rows at a time (DP8 even): the loads of both are in flight together
+// and a block of the query is read from LDS once for both.  `two`: this quad
+// has a second row.
+template <int DP8>
+__device__ __forceinline__ void quad_square_dist_two_rows(const float *row0,
+                                                          const float *row1,
+                                                          const float2 *qrun,
+                                                          int part, bool two,
+                                                          float &s0, float &s1) {
+    constexpr int kBlocks = DP8 / 2;
+    const float4 *r0 = reinterpret_cast<const float4 *>(row0) + part;
+    const float4 *r1 = reinterpret_cast<const float4 *>(row1) + part;
+    float4 x0[kBlocks], x1[kBlocks];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) x0[b] = r0[4 * b];
+    if (two) {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) x1[b] = r1[4 * b];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const float4 *q4 = reinterpret_cast<const float4 *>(qrun);
+    float a0 = 0.f, a1 = 0.f, c0 = 0.f, c1 = 0.f;
+    auto add = [](const float4 x, const float4 y, float &even, float &odd) {
+        const float d0 = y.x - x.x, d1 = y.y - x.y;
+        even = fmaf(d0, d0, even);
+        odd = fmaf(d1, d1, odd);
+        const float d2 = y.z - x.z, d3 = y.w - x.w;
+        even = fmaf(d2, d2, even);
+        odd = fmaf(d3, d3, odd);
+    };
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+        const float4 y = q4[b];
+        add(x0[b], y, a0, a1);
+        add(x1[b], y, c0, c1);
+        if ((b & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    s0 = quad_reduce(a0, a1);
+    s1 = quad_reduce(c0, c1);
+}
+
 }  // namespace pa
 
 #endif

@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 if (n > 0) {
                     if (fresh) cand_id[lane_rank(mask)] = v;
                     wave_sync();
-                    eval_rows<DP8>(a.storage, qv, cand_id, cand_key, n, dp, lane);
+                    eval_rows<DP8, (DP8 >= 16)>(a.storage, qv, cand_id, cand_key, n, dp, lane);
                     n_dist += n;
                     wave_sync();
                     PA_TIMER(3);

@@ -356,7 +356,7 @@ __global__ __launch_bounds__(kWave) void wide_kernel(WideArgs a) {
             }
             if (n == 0) continue;
             wave_sync();
-            eval_rows<DP8>(a.storage, qv, cand_id, cand_key, n, dp, lane);
+            eval_rows<DP8, true>(a.storage, qv, cand_id, cand_key, n, dp, lane);
             n_dist += n;
             wave_sync();
         }
