@@ -466,15 +466,25 @@ __global__ __launch_bounds__(256) void prune_kernel(
 }
 
 // Occlusion pruning straight from the rows: the same rule as prune_kernel,
-// with the candidate-to-candidate distances made on the spot.  A workgroup of
-// eight wavefronts takes one node: it gathers the rows of the node's k <= 256
-// candidates chunk by chunk into LDS (the transfers of knn_kernel, every lane
-// with the address of its own candidate's row), multiplies them with
-// themselves on the matrix cores — rows as two half-precision parts, x = hi +
-// lo, and hi.hi + hi.lo + lo.hi for the product, which is the float product to
-// about 22 bits — and reduces |a|^2 + |b|^2 - 2 a.b < dist(node, a) to one bit
-// per pair in LDS; then its first wavefront walks the candidates in order
-// against the bits of those kept so far.  The k x k table never leaves the CU.
+// with the candidate-to-candidate distances made on the spot.  Only a kept
+// candidate can block another one, and few are kept (a dozen or two of 240), so
+// the candidates are taken 64 at a time, closest first, and a block's rows are
+// multiplied with themselves (the lower triangle) and with the rows kept
+// before them: two fifths of the products of all pairs, and the blocks after
+// the m_keep-th kept candidate are never looked at.
+//
+// A workgroup of four wavefronts takes one node.  It gathers rows chunk by
+// chunk into LDS (the transfers of knn_kernel, every lane with the address of
+// its own row) and multiplies them on the matrix cores — rows as two
+// half-precision parts, x = hi + lo, and hi.hi + hi.lo + lo.hi for the product,
+// which is the float product to about 22 bits.  |a|^2 + |b|^2 - 2 a.b <
+// dist(node, a) is one bit per pair, and the first wavefront walks a block's
+// candidates from one that is kept to the next.  What bounds it is the
+// gathering of rows; one staging buffer, so that four workgroups share a
+// compute unit and each one's waits and serial walk hide behind the others'.
+// 120 000 nodes of 240 candidates of 768 floats, 48 to keep: 34.8 -> 15.0 ms
+// against all pairs on eight wavefronts with a double buffer, one workgroup
+// per compute unit; 20 011 nodes of 96 floats, 16 to keep: 2.67 -> 0.38 ms.
 constexpr int64_t kLaunchNodes = 1ll << 22;
 
 struct PruneRowsArgs {
@@ -489,167 +499,201 @@ struct PruneRowsArgs {
     float scale2;             // (scaled / unscaled) squared
 };
 
-__global__ __launch_bounds__(512, 2) void prune_rows_kernel(PruneRowsArgs a) {
-    constexpr int kRows = 256;                 // candidates of a node, padded
+__global__ __launch_bounds__(256, 4) void prune_rows_kernel(PruneRowsArgs a) {
+    constexpr int kMaxCand = 256;
+    constexpr int kBlock = 64;                 // candidates looked at together
+    constexpr int kSide = 32;                  // kept candidates multiplied with them at a time
+    constexpr int kRows = kBlock + kSide;      // rows staged
     constexpr int kRow = kChunk * 2;           // bytes of a staged row
     constexpr int kPart = kRows * kRow;        // one part (hi or lo) of a chunk
-    constexpr int kStage = 2 * kPart;
-    constexpr int kWords = kRows / 32;
-    __shared__ __align__(1024) unsigned char stage[2 * kStage];
-    __shared__ unsigned bits[kRows][kWords];   // bits[a][w]: bit b % 32 of word b / 32 says b blocks a
-    __shared__ float len2[kRows], reach[kRows];
-    __shared__ int valid_count;
+    __shared__ __align__(1024) unsigned char stage[2 * kPart];
+    __shared__ int64_t row_of[kMaxCand];       // candidate -> row
+    __shared__ float len2[kMaxCand], reach[kMaxCand];
+    __shared__ unsigned self_bits[kBlock][2];  // bit b of [a]: b of the block would block a of it
+    __shared__ unsigned side_bits[kBlock];     // not 0: a kept one of this pass blocks a
+    __shared__ int kept_at[kMaxCand];          // the candidates kept, in order
+    __shared__ int valid_count, kept_count;
     const int t = threadIdx.x;
-    const int lane = t & (kWave - 1), wave = t / kWave;
-    const int wr = wave % 2, wc = wave / 2;
+    const int lane = t & (kWave - 1), wave = uni(t / kWave);
     const int col = lane & 31, half = lane >> 5;
     const int64_t node = a.first + blockIdx.x;
     const int64_t *ids = a.cand + (size_t)node * a.k;
-    // a candidate: a row number inside the set, else -1 (nothing is read for it)
-    auto cand_at = [&](int i) -> int64_t {
-        const int64_t id = i < a.k ? ids[i] : -1;
-        return id < a.n_rows ? id : -1;
-    };
 
-    // the candidates' lengths and distances; what lies behind the list
-    // repeats the first candidate and can block nothing
-    if (t < kRows) {
-        const int64_t id = cand_at(t);
-        len2[t] = id >= 0 ? a.norm[id] : 0.f;
-        reach[t] = id >= 0 ? a.cand_dist[(size_t)node * a.k + t] * a.scale2 : -INFINITY;
-    }
+    // the candidates' rows, lengths and distances.  A candidate is a row
+    // number inside the set; what is none (what lies behind the list, too)
+    // repeats the first candidate's row and can be blocked by nothing
     if (t == 0) valid_count = 0;
     __syncthreads();
-    if (cand_at(t) >= 0) atomicAdd(&valid_count, 1);
-
-    // transfers: wavefront w brings rows 32 w .. 32 w + 31 of both parts, 8
-    // rows an instruction, lane l the piece that belongs at place l % 8 of row
-    // l / 8 (places as in knn_kernel)
-    const int bring_row = lane >> 3;
-    size_t from[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = 32 * wave + 8 * i + bring_row;
-        int64_t id = cand_at(row);
-        if (id < 0) id = cand_at(0) >= 0 ? cand_at(0) : 0;
-        from[i] = ((size_t)id * a.d) * 2 + 16u * ((lane & 7) ^ (((8 * i + bring_row) >> 1) & 7));
+    {
+        auto cand_at = [&](int i) -> int64_t {
+            const int64_t id = i < a.k ? ids[i] : -1;
+            return id < a.n_rows ? id : -1;
+        };
+        const int64_t first_id = cand_at(0);
+        const int64_t id = cand_at(t);
+        row_of[t] = id >= 0 ? id : first_id >= 0 ? first_id : 0;
+        len2[t] = id >= 0 ? a.norm[id] : 0.f;
+        reach[t] = id >= 0 ? a.cand_dist[(size_t)node * a.k + t] * a.scale2 : -INFINITY;
+        const unsigned long long valid = __ballot(id >= 0);
+        if (lane == 0) atomicAdd(&valid_count, (int)__popcll(valid));
     }
-    const unsigned bring_to =
-        (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)stage +
-        32 * wave * kRow;
+    __syncthreads();
+    const int k_valid = uni(valid_count);
+
+    // transfers: an instruction brings 8 rows, lane l the piece that belongs
+    // at place l % 8 of row l / 8 (places as in knn_kernel); wavefront w brings
+    // rows 24 w .. 24 w + 23 of both parts
+    constexpr int kBrings = kRows / 8 / 4;
+    const int bring_row = lane >> 3;
     const unsigned char *hi = reinterpret_cast<const unsigned char *>(a.hi);
     const unsigned char *lo = reinterpret_cast<const unsigned char *>(a.lo);
-#define PA_BRING_CHUNK(k0, buf)                                                          \
-    _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                      \
-        bring_rows(hi + from[i] + (size_t)(k0) * 2, bring_to + (buf) * kStage + 8 * i * kRow); \
-        bring_rows(lo + from[i] + (size_t)(k0) * 2,                                      \
-                   bring_to + (buf) * kStage + kPart + 8 * i * kRow);                    \
-    }
+    const unsigned bring_to =
+        (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)stage;
     const unsigned mix = (col >> 1) & 7;
     const unsigned swizzle = 16u * (half ^ (mix & 1)) + 32u * (mix >> 1);
-    const unsigned char *a_tile = stage + (wr * 128 + col) * kRow;
-    const unsigned char *b_tile = stage + (wc * 64 + col) * kRow;
+    // wavefront w multiplies rows 32 (w % 2) .. + 31 of the block: the first
+    // two with the block itself, the other two with the kept rows
+    const int m0 = 32 * (wave & 1);
+    const bool with_side = wave >= 2;
 
-    floatx16 acc[4][2];
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-
-    PA_BRING_CHUNK(0, 0)
-    bring_wait<0>();
-    __syncthreads();
-    int buf = 0;
-#pragma unroll 1
-    for (int k0 = 0; k0 < a.d; k0 += kChunk, buf ^= 1) {
-        if (k0 + kChunk < a.d) PA_BRING_CHUNK(k0 + kChunk, buf ^ 1)
-        const unsigned char *a_now = a_tile + buf * kStage, *b_now = b_tile + buf * kStage;
-#pragma unroll
-        for (int s = 0; s < kChunk / 16; ++s) {
-            const unsigned at = swizzle ^ (32u * s);
-            half8 av[4], bv[2];
-            // hi . hi
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-                av[m] = *reinterpret_cast<const half8 *>(a_now + m * 32 * kRow + at);
-#pragma unroll
-            for (int n = 0; n < 2; ++n)
-                bv[n] = *reinterpret_cast<const half8 *>(b_now + n * 32 * kRow + at);
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int n = 0; n < 2; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[m], bv[n], acc[m][n], 0, 0, 0);
-            // hi . lo
-#pragma unroll
-            for (int n = 0; n < 2; ++n)
-                bv[n] = *reinterpret_cast<const half8 *>(b_now + kPart + n * 32 * kRow + at);
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int n = 0; n < 2; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[m], bv[n], acc[m][n], 0, 0, 0);
-            // lo . hi
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-                av[m] = *reinterpret_cast<const half8 *>(a_now + kPart + m * 32 * kRow + at);
-#pragma unroll
-            for (int n = 0; n < 2; ++n)
-                bv[n] = *reinterpret_cast<const half8 *>(b_now + n * 32 * kRow + at);
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-#pragma unroll
-                for (int n = 0; n < 2; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[m], bv[n], acc[m][n], 0, 0, 0);
-        }
-        bring_wait<0>();
-        __syncthreads();
-    }
-#undef PA_BRING_CHUNK
-
-    // a lane's 16 results of an instruction tile are
-    // D[i = 8 * (r / 4) + 4 * (l / 32) + r % 4][j = l % 32]: one ballot is the
-    // word of 32 columns for two rows
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        const int b = (wc * 2 + n) * 32 + col;
-        const float len_b = len2[b];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = (wr * 4 + m) * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                const float pair = (len2[row] + len_b) - 2.f * acc[m][n][r];
-                const unsigned long long word = __ballot(pair < reach[row]);
-                if (col == 0)
-                    bits[row][wc * 2 + n] = half ? (unsigned)(word >> 32) : (unsigned)word;
-            }
-        }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-
-    // the walk: lane w < 8 holds word w of the kept set
-    int32_t *out = a.selected + (size_t)node * a.m_keep;
-    const int k_valid = valid_count;
-    unsigned kept = 0;
     int count = 0;
-    for (int j = 0; j < k_valid && count < a.m_keep; ++j) {
-        const unsigned hit = lane < kWords ? (bits[j][lane] & kept) : 0u;
-        if (!__ballot(hit != 0)) {
-            if (lane == (j >> 5)) kept |= 1u << (j & 31);
-            if (lane == 0) out[count] = j;
-            count += 1;
+    int32_t *out = a.selected + (size_t)node * a.m_keep;
+    unsigned long long kept_mask[kMaxCand / kBlock];   // for the filling
+#pragma unroll
+    for (int blk = 0; blk < kMaxCand / kBlock; ++blk) {
+        kept_mask[blk] = 0;
+        const int c0 = blk * kBlock;
+        if (c0 >= k_valid || count >= a.m_keep) continue;
+        unsigned long long blocked = 0;   // of the block's candidates, in the first wavefront
+        // passes over the kept ones, 32 a time; the first pass does the block itself
+        int side0 = 0;
+        do {
+            const int n_side = min(kSide, count - side0);   // <= 0: none yet
+            const bool self_pass = side0 == 0;
+            size_t from[kBrings];
+            bool wanted[kBrings];
+#pragma unroll
+            for (int i = 0; i < kBrings; ++i) {
+                const int r8 = (wave * kBrings + i) * 8;
+                wanted[i] = r8 < kBlock || r8 - kBlock < n_side;
+                const int r = r8 + bring_row;
+                int c = 0;
+                if (r < kBlock) c = c0 + r;
+                else if (r - kBlock < n_side) c = kept_at[side0 + r - kBlock];
+                from[i] = (size_t)row_of[c] * a.d * 2 + 16u * ((lane & 7) ^ ((r >> 1) & 7));
+            }
+            floatx16 acc[2];
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+            // tiles of this wavefront: the block's columns 0 .. m0 + 31, or
+            // the kept rows
+            const int n_tiles = with_side ? (n_side > 0 ? 1 : 0) : self_pass ? 1 + (wave & 1) : 0;
+            const unsigned char *a_tile = stage + (m0 + col) * kRow;
+            const unsigned char *b_tile = stage + ((with_side ? kBlock : 0) + col) * kRow;
+#pragma unroll 1
+            for (int k0 = 0; k0 < a.d; k0 += kChunk) {
+#pragma unroll
+                for (int i = 0; i < kBrings; ++i) {
+                    if (wanted[i]) {
+                        const unsigned to = bring_to + (wave * kBrings + i) * 8 * kRow;
+                        bring_rows(hi + from[i] + (size_t)k0 * 2, to);
+                        bring_rows(lo + from[i] + (size_t)k0 * 2, to + kPart);
+                    }
+                }
+                bring_wait<0>();
+                __syncthreads();
+                if (n_tiles > 0) {
+#pragma unroll
+                    for (int s = 0; s < kChunk / 16; ++s) {
+                        const unsigned at = swizzle ^ (32u * s);
+                        const half8 ah = *reinterpret_cast<const half8 *>(a_tile + at);
+                        const half8 al = *reinterpret_cast<const half8 *>(a_tile + kPart + at);
+                        const half8 bh = *reinterpret_cast<const half8 *>(b_tile + at);
+                        const half8 bl = *reinterpret_cast<const half8 *>(b_tile + kPart + at);
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[0], 0, 0, 0);
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[0], 0, 0, 0);
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[0], 0, 0, 0);
+                        if (n_tiles > 1) {
+                            const half8 ch = *reinterpret_cast<const half8 *>(b_tile + 32 * kRow + at);
+                            const half8 cl = *reinterpret_cast<const half8 *>(b_tile + 32 * kRow + kPart + at);
+                            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ch, acc[1], 0, 0, 0);
+                            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, cl, acc[1], 0, 0, 0);
+                            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ch, acc[1], 0, 0, 0);
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+
+            // a lane's 16 results of an instruction tile are
+            // D[i = 8 * (r / 4) + 4 * (l / 32) + r % 4][j = l % 32]: one ballot
+            // is the word of 32 columns for two rows
+            auto tile_bits = [&](const floatx16 &sums, float len_b, bool real, unsigned *to,
+                                 int pitch) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = m0 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const float pair = (len2[c0 + row] + len_b) - 2.f * sums[r];
+                    const unsigned long long word = __ballot(real && pair < reach[c0 + row]);
+                    if (col == 0)
+                        to[row * pitch] = half ? (unsigned)(word >> 32) : (unsigned)word;
+                }
+            };
+            if (with_side) {
+                if (n_tiles > 0) {
+                    const bool real = col < n_side;
+                    tile_bits(acc[0], real ? len2[kept_at[side0 + col]] : 0.f, real,
+                              side_bits, 1);
+                }
+            } else if (n_tiles > 0) {
+                tile_bits(acc[0], len2[c0 + col], true, &self_bits[0][0], 2);
+                if (n_tiles > 1) tile_bits(acc[1], len2[c0 + 32 + col], true, &self_bits[0][1], 2);
+            }
+            __syncthreads();
+            if (wave == 0 && n_side > 0) blocked |= __ballot(side_bits[lane] != 0);
+            side0 += kSide;
+        } while (side0 < count);
+
+        // the walk: lane l holds the bits of the block's candidate l, of which
+        // those of candidates before it count
+        if (wave == 0) {
+            const unsigned b0 = self_bits[lane][0], b1 = lane >= 32 ? self_bits[lane][1] : 0u;
+            const unsigned long long mine = ((unsigned long long)b1 << 32) | b0;
+            unsigned long long alive = ~blocked;
+            if (k_valid - c0 < kBlock) alive &= (1ull << (k_valid - c0)) - 1;
+            unsigned long long kept = 0;
+            int n = count;
+            while (alive && n < a.m_keep) {
+                const int j = __builtin_ctzll(alive);
+                kept |= 1ull << j;
+                alive &= ~1ull << j;                          // those after it
+                alive &= ~__ballot((mine >> j) & 1ull);       // that it does not block
+                n += 1;
+            }
+            if ((kept >> lane) & 1ull) {
+                const int place = count + lane_rank(kept);
+                kept_at[place] = c0 + lane;
+                out[place] = c0 + lane;
+            }
+            kept_mask[blk] = kept;
+            if (lane == 0) kept_count = n;
         }
+        __syncthreads();
+        count = uni(kept_count);
     }
+    if (wave != 0) return;
+    // the closest rejected ones
     if (a.fill) {
-        for (int j = 0; j < k_valid && count < a.m_keep; ++j) {
-            const unsigned word = __builtin_amdgcn_readlane(kept, j >> 5);
-            if ((word >> (j & 31)) & 1u) continue;
-            if (lane == 0) out[count] = j;
-            count += 1;
+#pragma unroll
+        for (int blk = 0; blk < kMaxCand / kBlock; ++blk) {
+            const int c = blk * kBlock + lane;
+            const bool rejected = c < k_valid && !((kept_mask[blk] >> lane) & 1ull);
+            const unsigned long long mask = __ballot(rejected);
+            const int place = count + lane_rank(mask);
+            if (rejected && place < a.m_keep) out[place] = c;
+            count += __popcll(mask);
         }
     }
     for (int i = count + lane; i < a.m_keep; i += kWave) out[i] = -1;
@@ -736,10 +780,10 @@ extern "C" int pa_graph_prune_rows(int32_t *selected, const void *rows_hi_f16,
     a.norm = norm, a.cand = cand, a.cand_dist = cand_dist, a.selected = selected;
     a.n = n, a.n_rows = n_rows, a.d = d, a.k = k, a.m_keep = m_keep, a.fill = fill;
     a.scale2 = scale2;
-    // a launch holds fewer than 2^32 work-items: at most 2^22 nodes of 512
+    // a launch holds fewer than 2^32 work-items: at most 2^22 nodes of 256
     for (a.first = 0; a.first < n; a.first += kLaunchNodes) {
         const int64_t count = n - a.first < kLaunchNodes ? n - a.first : kLaunchNodes;
-        prune_rows_kernel<<<(unsigned)count, 512, 0, (hipStream_t)stream_>>>(a);
+        prune_rows_kernel<<<(unsigned)count, 256, 0, (hipStream_t)stream_>>>(a);
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return (int)err;
     }
