@@ -88,6 +88,9 @@ struct OpenList {
         kDeepCells ? kDeepBase - kRegNodes
                    : (kSize + 2 > kRegNodes ? kSize + 2 - kRegNodes : 0);
     static constexpr int kInf = 0x7f800000;       // float_to_key(+inf)
+    static constexpr int kBelowAll = (int)0x80000000;
+    static constexpr int kRegLevels = kDepth < 7 ? kDepth : 7;
+    static constexpr int kLow = kDepth - kRegLevels;  // levels below the registers
     int Ak, Av, Bk, Bv, Ck, Cv, Dk, Dv;
     int2 *cells;  // node j in [256, kDeepBase) at [j - 256] as (key, value); 16-byte aligned
     int2 *deep;   // node j >= kDeepBase at [j - kDeepBase], device memory, 16-byte aligned
@@ -97,6 +100,17 @@ struct OpenList {
     __device__ __forceinline__ static int rl(int x, int l) {
         return __builtin_amdgcn_readlane(x, l);
     }
+    // the value of another lane of a bank (taken modulo 64)
+    __device__ __forceinline__ static int of_lane(int bank, int l) {
+        return __builtin_amdgcn_ds_bpermute(l << 2, bank);
+    }
+    // A path from the root is named by its node on level 7, or by the
+    // leftmost descendant there of the node it ends in: the path's node on
+    // level L is at7 >> (7 - L).  For bank A: 7 - the level of the lane's node
+    // (lane 0, which holds none: 1, where no path matches).
+    __device__ __forceinline__ static int above7(int lane) {
+        return lane ? __builtin_clz(lane) - 24 : 1;
+    }
     // storage class of a level: 0 bank A, 1 bank B, 2 banks C/D, 3 LDS,
     // 4 device memory
     __device__ __forceinline__ static constexpr int kind(int level) {
@@ -105,7 +119,8 @@ struct OpenList {
     }
 
     __device__ __forceinline__ void reset(int lane) {
-        Ak = Bk = Ck = Dk = kInf;
+        Ak = lane == 0 ? kBelowAll : kInf;  // lane 0 holds no node: the root's parent
+        Bk = Ck = Dk = kInf;
         Av = Bv = Cv = Dv = -1;
         for (int i = lane; i < kLdsCells; i += kWave) cells[i] = make_int2(kInf, -1);
         for (int i = lane; i < kDeepCells; i += kWave) deep[i] = make_int2(kInf, -1);
@@ -260,38 +275,44 @@ struct OpenList {
         out_k = rl(Ak, 1);
         out_v = rl(Av, 1);
         const Choice ch = choices<false>();
-        // Register levels in three passes, so that no read waits for a write
-        // of the same bank: the path (masks only), then every entry on it,
-        // then the stores.  Reading first is the same thing: a level's store
-        // goes to the cell above the one read.
-        constexpr int kRegLevels = kDepth < 7 ? kDepth : 7;
-        int node[kRegLevels + 1];
-        node[0] = 1;
-        bool cut = false;  // level kDepth has no node below node[kDepth - 1]
+        // The path through the register levels first (masks only); then every
+        // lane on it takes the entry of its child on the path, all levels at
+        // once: a lane gather from bank A (levels 0..4) and one from bank B
+        // (level 5), and bank B's children are in banks C/D of the same lane.
+        int j = 1;
+        bool cut = false;  // level kDepth has no node below j
 #pragma unroll
         for (int L = 1; L <= kRegLevels; ++L) {
-            if (L == kDepth && 2 * node[L - 1] > kSize) {
-                cut = true;
-                node[L] = node[L - 1];
-            } else {
-                node[L] = step_down(L, node[L - 1], ch);
+            if (L == kDepth && 2 * j > kSize) cut = true;
+            else j = step_down(L, j, ch);
+        }
+        {
+            const int level = cut ? kRegLevels - 1 : kRegLevels;  // of j
+            const int at7 = j << (7 - level);
+            const int sh = above7(lane);
+            const int child = at7 >> (sh - 1);
+            bool here = (at7 >> sh) == lane;
+            if (kDepth <= 6) here = here && lane < (1 << level);
+            int ck = of_lane(Ak, child), cv = of_lane(Av, child);
+            if (kDepth >= 6) {
+                const int bk = of_lane(Bk, child), bv = of_lane(Bv, child);
+                ck = lane >= 32 ? bk : ck;
+                cv = lane >= 32 ? bv : cv;
             }
-        }
-        int ck[kRegLevels + 1], cv[kRegLevels + 1];
-#pragma unroll
-        for (int L = 1; L <= kRegLevels; ++L) {
-            ck[L] = key_of(kind(L), node[L]);
-            cv[L] = val_of(kind(L), node[L]);
-        }
-#pragma unroll
-        for (int L = 1; L <= kRegLevels; ++L) {
-            if (L == kDepth && cut) {
-                put(kind(L - 1), node[L - 1], kInf, -1, lane);
-                return;
+            if (kDepth >= 7) {
+                bool hereB = lane == (at7 >> 1) - 64;
+                if (kDepth == 7) hereB = hereB && !cut;
+                const bool right = Dk < Ck;
+                Bk = hereB ? (right ? Dk : Ck) : Bk;
+                Bv = hereB ? (right ? Dv : Cv) : Bv;
             }
-            put(kind(L - 1), node[L - 1], ck[L], cv[L], lane);
+            Ak = here ? ck : Ak;
+            Av = here ? cv : Av;
         }
-        int j = node[kRegLevels];
+        if (cut) {
+            put(kind(kRegLevels - 1), j, kInf, -1, lane);
+            return;
+        }
         pending_j = 0;
 #pragma unroll
         for (int L = kRegLevels + 1; L <= kDepth; ++L) {
@@ -356,6 +377,8 @@ struct OpenList {
         int j;       // the leaf
         int key;     // its key
         bool bottom; // it is on level kDepth
+        // the entries of the path on levels 8 and down, as the walk read them
+        int low_key[kLow ? kLow : 1], low_val[kLow ? kLow : 1];
     };
     __device__ __forceinline__ Leaf walk_to_large_leaf() const {
         return walk_below(choices<true>(), 0, 1);
@@ -364,6 +387,7 @@ struct OpenList {
     // were taken elsewhere).
     __device__ __forceinline__ Leaf walk_below(const Choice &ch, const int DONE,
                                                int j) const {
+        Leaf leaf;
         bool bottom = true;  // the walk reached level kDepth
         int walked_key = 0;  // key of node j when its level is an LDS level
 #pragma unroll
@@ -377,14 +401,15 @@ struct OpenList {
                 j = (L == kDepth && 2 * j == kSize) ? 2 * j : step_down(L, j, ch);
             } else {
                 int ka, kb, va, vb;
-                pair(kind(L), false, 2 * j, ka, kb, va, vb);
+                pair(kind(L), true, 2 * j, ka, kb, va, vb);
                 if (L == kDepth) kb = 2 * j == kSize ? ka : kb;
                 walked_key = max(ka, kb);
+                leaf.low_key[L - 8] = walked_key;
+                leaf.low_val[L - 8] = walked_key != ka ? vb : va;
                 j = add_if_ne(2 * j, walked_key, ka);
             }
         }
         // the leaf's key: the walk has it already when the leaf is in LDS
-        Leaf leaf;
         leaf.j = j, leaf.bottom = bottom;
         if (bottom)
             leaf.key = kind(kDepth) >= 3 ? walked_key : key_of(kind(kDepth), j);
@@ -433,35 +458,63 @@ struct OpenList {
             : "scc");
         return j;
     }
-    // SPARSE: the heap is nearly empty (the entries of a query are pushed),
-    // so most ancestors of the leaf are (inf, -1), and so is everything below
-    // such an ancestor: moving it down would write (inf, -1) over (inf, -1)
-    // and is left out.
-    template <bool SPARSE = false>
+    // The new entry rises: along the path to the leaf, whose keys do not fall
+    // from the root down, every entry with a larger key moves one level down
+    // and the new one takes the place of the highest of them.  So a node of the
+    // path with a key above k gets its parent's entry if that is above k too,
+    // else the new one, which all lanes decide at once from the lists as they
+    // were: the parents of bank A are a lane gather away, those of bank B are
+    // in lanes 32..63 of bank A, those of banks C/D in the same lane of bank B,
+    // and the walk has read the levels below.
     __device__ __forceinline__ void replace_leaf(const Leaf &leaf, int k, int v,
                                                  int lane) {
         if (k >= leaf.key) return;
-        int j = leaf.j;
-        // one store per level: the parent's entry while it is larger than
-        // the new key, the new entry where the rise stops
-        auto rise = [&](const int L) -> bool {
-            const int up = j >> 1;
-            const int pk = key_of(kind(L - 1), up);
-            if (SPARSE && pk == kInf) {
-                j = up;
-                return false;
-            }
-            const int pv = val_of(kind(L - 1), up);
-            const bool stop = pk <= k;
-            put(kind(L), j, stop ? k : pk, stop ? v : pv, lane);
-            j = up;
-            return stop;
-        };
-        if (leaf.bottom && rise(kDepth)) return;
+        const int depth = leaf.bottom ? kDepth : kDepth - 1;   // of the leaf
+        // the path's end in the register levels, and its level
+        int j7 = leaf.j, level = depth;
+        if (kLow) {
+            j7 >>= depth - 7;
+            level = 7;
+            int pk = key_of(2, j7), pv = val_of(2, j7);
 #pragma unroll
-        for (int L = kDepth - 1; L >= 1; --L)
-            if (rise(L)) return;
-        put(0, 1, k, v, lane);
+            for (int L = 8; L <= kDepth; ++L) {
+                if (L == kDepth && !leaf.bottom) break;
+                const int own = leaf.low_key[L - 8];
+                const bool down = pk > k;
+                const int node = leaf.j >> (depth - L);
+                if (own > k) put(kind(L), node, down ? pk : k, down ? pv : v, lane);
+                pk = own, pv = leaf.low_val[L - 8];
+            }
+        }
+        const int at7 = j7 << (7 - level);
+        const int sh = above7(lane);
+        const int pAk = of_lane(Ak, lane >> 1), pAv = of_lane(Av, lane >> 1);
+        if (kDepth >= 6) {
+            const int pBk = of_lane(Ak, 32 + (lane >> 1)), pBv = of_lane(Av, 32 + (lane >> 1));
+            const int l6 = (at7 >> 1) - 64;
+            if (kDepth >= 7) {
+                const bool down = Bk > k;
+                const int nk = down ? Bk : k, nv = down ? Bv : v;
+                bool here = lane == l6;
+                if (kDepth == 7) here = here && level == 7;
+                const bool hereC = here && !(at7 & 1) && Ck > k;
+                const bool hereD = here && (at7 & 1) && Dk > k;
+                Ck = hereC ? nk : Ck;
+                Cv = hereC ? nv : Cv;
+                Dk = hereD ? nk : Dk;
+                Dv = hereD ? nv : Dv;
+            }
+            const bool down = pBk > k;
+            bool here = lane == l6 && Bk > k;
+            if (kDepth == 6) here = here && level == 6;
+            Bk = here ? (down ? pBk : k) : Bk;
+            Bv = here ? (down ? pBv : v) : Bv;
+        }
+        const bool down = pAk > k;
+        bool here = (at7 >> sh) == lane && Ak > k;
+        if (kDepth <= 5) here = here && lane < (2 << level);
+        Ak = here ? (down ? pAk : k) : Ak;
+        Av = here ? (down ? pAv : v) : Av;
     }
     // Pushes, in lane order, the entries (k, v) of the lanes in `who`, as one
     // replace after the other would.  `leaf` is where the walk ends in the
@@ -477,7 +530,7 @@ struct OpenList {
             if (!in) return;
             const int j = __builtin_ctzll(in);
             who &= ~1ull << j;
-            replace_leaf<true>(leaf, rl(k, j), rl(v, j), lane);
+            replace_leaf(leaf, rl(k, j), rl(v, j), lane);
             leaf = walk_to_large_leaf();
         }
     }
