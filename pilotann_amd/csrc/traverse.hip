@@ -77,17 +77,18 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 
 // Wavefronts per SIMD the register allocator must fit.  A budget a few
 // registers under what the code needs costs more (spills, serialised loads)
-// than the extra wavefront brings — measured: H = 256 with 128-float rows
-// needs 113 registers and is 4 % faster at four wavefronts (128) than squeezed
-// into the 96 of five, while three wavefronts are 11 % slower than four.  So
-// only a floor is given, under which no instance has to be squeezed (the
-// largest heaps are bounded by their LDS anyway), and the allocator's own
-// count decides the residency above it: 8 for the smallest instances, 4 for
-// H = 256 with 128-float rows.
+// than the extra wavefront brings, so only a floor is given, under which no
+// instance has to be squeezed (the largest heaps are bounded by their LDS
+// anyway), and the allocator's own count decides the residency above it: 8 for
+// the smallest instances, 3 for 128-float rows, whose two passes of loads in
+// flight take 64 registers.  Measured for those over a million rows, three
+// wavefronts (153 registers) against four (128, 22 spilled): one query, H =
+// 128, 524 -> 507 us, 5000 1.63 -> 1.51 ms, 10 000 2.80 -> 2.67 ms; with one
+// pass in flight four (99) take 2.75 and five (95) 2.74 ms.
 #ifdef PA_WAVES_PER_EU
 #define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
 #else
-#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (DP8 == 16 ? 3 : 4) : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
 #endif
 
 // The longest open list (4096 cells) keeps its last two levels in the
@@ -229,8 +230,11 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         // the pop (the atomics are in flight while the pop sifts).  If the
         // search ends at the next pop instead, the marks set for a node that
         // is never expanded are harmless: the slice is cleared per query.
-        // (Requesting that node's row of neighbour ids even earlier, before
-        // the inserts, for the most likely next root, measured the same.)
+        // That node's row of neighbour ids is requested still earlier, right
+        // after the pop, for the root the pop leaves, and again only if an
+        // insert put another node there: it travels while the rows are read
+        // (one query, lists of 4096 cells, 5.49 -> 5.28 ms; 10 000, lists of
+        // 768, 3.50 -> 3.47 ms; where the rows take the time it is the same).
         auto load_row = [&](int r) -> int {
             int row = -1;
             if (r >= 0 && lane < deg) row = a.adj[(size_t)r * deg + lane];
@@ -262,6 +266,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         for (int step = 0; step < a.max_iter; ++step) {
             int uk, u;
             open.pop(lane, uk, u);
+            const int likely = Open::rl(open.Av, 1);
+            const int likely_row = load_row(likely);
             PA_TIMER(0);
             if (u == -1 || uk >= res.worst) break;
             n_expand += 1;
@@ -319,7 +325,9 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 }
             }
             if (!popped) open.pop_finish(lane);
-            v = load_row(Open::rl(open.Av, 1));
+            v = likely_row;
+            const int root = Open::rl(open.Av, 1);
+            if (root != likely) v = load_row(root);
             before = test_and_set(v);
             PA_TIMER(1);
         }
