@@ -306,6 +306,22 @@ int pa_knn_rerank(float *dist, const float *rows, const int64_t *cand,
                   int64_t m, int64_t first, int64_t n, int d, int k, void *stream);
 
 /*
+ * pa_knn's lists ranked in one call (no counterpart in the reference's
+ * extension either): the lists of the n_seg segments are merged (in place,
+ * into the first segment's), the exact squared float32 distances of the `keep`
+ * best by score are made as pa_knn_rerank makes them, and out_id / out_dist
+ * [m * k] receive the k <= keep closest rows of 0 .. n, closest first, equal
+ * distances by row number; -1 / infinity where a list is shorter.  The row
+ * itself has distance infinity, like a row number out of range; with hide_inf
+ * such places receive -1.  `rows` [n * d], d % 4 == 0, d <= 2048; the queries
+ * are rows first .. first + m.  Device pointers; enqueued on `stream`.
+ */
+int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
+                int32_t *cand_id, int32_t *cand_count, const float *rows,
+                int64_t m, int64_t first, int64_t n, int d, int keep, int n_seg,
+                int k, int hide_inf, void *stream);
+
+/*
  * Occlusion pruning of candidate lists, the edge selection of the graph
  * builder (faiss' part in the reference, pilot_ann/utils/graphs.py:15-20,52-56;
  * no entry point of the reference's extension corresponds to it).  For each of

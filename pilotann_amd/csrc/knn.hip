@@ -101,16 +101,29 @@ __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int 
         u[i] = e < n ? ordered(score[e]) : 0xffffffffu;
         v[i] = e < n ? id[e] : -1;
     }
-    // the KEEP-th smallest, bit by bit from the top: `bound` stays the largest
-    // value with fewer than KEEP entries below it
-    unsigned bound = 0;
+    // The KEEP-th smallest, bit by bit from the highest one in which the
+    // entries differ: `bound` stays the largest value with fewer than KEEP
+    // entries below it, until a value with exactly KEEP below it is met, which
+    // a list of a few hundred scores has after about ten bits (of 32).
+    unsigned low = 0xffffffffu, high = 0;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+        low = min(low, u[i]);
+        high = lane + kWave * i < n ? max(high, u[i]) : high;
+    }
+    low = ~((unsigned)wave_max_key((int)(~low ^ 0x80000000u)) ^ 0x80000000u);
+    high = (unsigned)wave_max_key((int)(high ^ 0x80000000u)) ^ 0x80000000u;
+    const int top = low == high ? -1 : 31 - __builtin_clz(low ^ high);
+    unsigned bound = top < 0 ? low : low & ~((2u << top) - 1u);
+    bool parted = false;   // exactly KEEP entries lie below `bound`
 #pragma unroll 1
-    for (int bit = 31; bit >= 0; --bit) {
+    for (int bit = top; bit >= 0 && !parted; --bit) {
         const unsigned trial = bound | (1u << bit);
         int below = 0;
 #pragma unroll
         for (int i = 0; i < kPerLane; ++i) below += __popcll(__ballot(u[i] < trial));
-        if (below < KEEP) bound = trial;
+        if (below <= KEEP) bound = trial;
+        parted = below == KEEP;
     }
     int n_below = 0;
 #pragma unroll
@@ -132,6 +145,12 @@ __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int 
         }
         at_below += __popcll(mb);
         at_equal += __popcll(me);
+    }
+    if (parted) {
+        high = 0;
+#pragma unroll
+        for (int i = 0; i < kPerLane; ++i) high = u[i] < bound ? max(high, u[i]) : high;
+        bound = (unsigned)wave_max_key((int)(high ^ 0x80000000u)) ^ 0x80000000u;
     }
     return unordered(bound);
 }
@@ -368,17 +387,88 @@ __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kerne
         if (q0 + r < a.m) a.cand_count[(size_t)seg * a.m + q0 + r] = count[r];
 }
 
-// Exact squared distances from query row first + q to its candidates, the
-// float arithmetic of the search itself (differences, then squares, summed).
-// A wavefront per query, its row in LDS; 16 lanes per candidate, four
-// candidates at a time, every lane 16 bytes of the candidate's row per step.
-// A candidate that is -1, out of range or the query row itself gets infinity.
+// The lists that the segments of a launch left for a row become one, in the
+// place of the first segment's: the `KEEP` smallest of them all.  A wavefront
+// per row; what is below the limit so far is appended and the list cut as in
+// knn_kernel.
 constexpr int kRankWaves = 4;
+constexpr int kMaxRankDim = 2048;   // rows of a workgroup and their lists fit 64 KB of LDS
 
+template <int KEEP>
+__global__ __launch_bounds__(kWave * kRankWaves) void merge_kernel(
+    float *__restrict__ score, int32_t *__restrict__ id, int32_t *__restrict__ count,
+    int64_t m, int n_seg) {
+    constexpr int kCap = KEEP + kSlack + kMaxBN;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t row = (int64_t)blockIdx.x * kRankWaves + threadIdx.x / kWave;
+    if (row >= m) return;
+    float *my_score = score + (size_t)row * kCap;
+    int32_t *my_id = id + (size_t)row * kCap;
+    int n = uni(count[row]);
+    float limit = INFINITY;
+    // the wavefront's stores before its other lanes' loads of the list, and
+    // those before the next stores
+    auto settle = []() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    };
+    auto cut = [&]() {
+        settle();
+        limit = uni(cut_list<KEEP, kMaxBN>(my_score, my_id, n, lane));
+        n = KEEP;
+        settle();
+    };
+    for (int seg = 1; seg < n_seg; ++seg) {
+        const size_t at = (size_t)seg * m + row;
+        const int cnt = uni(count[at]);
+        for (int base = 0; base < cnt; base += kWave) {
+            const int i = base + lane;
+            const float x = i < cnt ? score[at * kCap + i] : INFINITY;
+            const bool in = i < cnt && x < limit;
+            const unsigned long long mask = __ballot(in);
+            if (in) {
+                my_score[n + lane_rank(mask)] = x;
+                my_id[n + lane_rank(mask)] = id[at * kCap + i];
+            }
+            n += __popcll(mask);
+            if (n > kCap - kWave) cut();
+        }
+        if (n > KEEP) cut();
+    }
+    if (lane == 0) count[row] = n;
+}
+
+// The exact squared distance between a row in LDS (`mine`) and row `row`, the
+// float arithmetic of the search itself (differences, then squares, summed),
+// by the 16 lanes of a team, `place` the lane's place in it, every lane 16
+// bytes of the row per step.  Every lane of the wavefront calls this.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float team_square_dist(const floatx4 *mine, const floatx4 *row, int d4,
+                                                  int place, bool ok) {
+    float sum = 0.f;
+    if (ok) {
+        for (int i = place; i < d4; i += 16) {
+            const floatx4 x = row[i], y = mine[i];
+            const float e0 = x[0] - y[0], e1 = x[1] - y[1], e2 = x[2] - y[2], e3 = x[3] - y[3];
+            sum = fmaf(e0, e0, sum);
+            sum = fmaf(e1, e1, sum);
+            sum = fmaf(e2, e2, sum);
+            sum = fmaf(e3, e3, sum);
+        }
+    }
+#pragma unroll
+    for (int step = 8; step >= 1; step >>= 1) sum += __shfl_xor(sum, step, 16);
+    return sum;
+}
+
+// Exact squared distances from query row first + q to its candidates.  A
+// wavefront per query, its row in LDS; 16 lanes per candidate, four candidates
+// at a time.  A candidate that is -1, out of range or the query row itself gets
+// infinity.
 __global__ __launch_bounds__(kWave * kRankWaves) void rerank_kernel(
     const float *__restrict__ rows, const int64_t *__restrict__ cand,
     float *__restrict__ out, int64_t m, int64_t first, int64_t n, int d, int k) {
-    typedef float floatx4 __attribute__((ext_vector_type(4)));
     extern __shared__ __align__(16) unsigned char rank_lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int64_t q = (int64_t)blockIdx.x * kRankWaves + wave;
@@ -395,21 +485,74 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rerank_kernel(
         const int j = j0 + team;
         const int64_t id = j < k ? cand[(size_t)q * k + j] : -1;
         const bool ok = id >= 0 && id < n && id != first + q;
-        float sum = 0.f;
-        if (ok) {
-            const floatx4 *row = reinterpret_cast<const floatx4 *>(rows + (size_t)id * d);
-            for (int i = place; i < d4; i += 16) {
-                const floatx4 x = row[i], y = mine[i];
-                const float e0 = x[0] - y[0], e1 = x[1] - y[1], e2 = x[2] - y[2], e3 = x[3] - y[3];
-                sum = fmaf(e0, e0, sum);
-                sum = fmaf(e1, e1, sum);
-                sum = fmaf(e2, e2, sum);
-                sum = fmaf(e3, e3, sum);
-            }
-        }
-#pragma unroll
-        for (int step = 8; step >= 1; step >>= 1) sum += __shfl_xor(sum, step, 16);
+        const float sum = team_square_dist(
+            mine, reinterpret_cast<const floatx4 *>(rows + (ok ? (size_t)id * d : 0)), d4, place, ok);
         if (place == 0 && j < k) out[(size_t)q * k + j] = ok ? sum : INFINITY;
+    }
+}
+
+// The ranking that follows knn_kernel in one pass: the distances of a row's
+// list, as rerank_kernel makes them, sorted in LDS (by distance, then by row
+// number), the k closest written out.  What bounds it is the gathering of the
+// candidates' rows; the sort of 256 entries (36 passes of two exchanges a
+// lane) hides behind other wavefronts' reads, where ranking in steps of torch
+// (ids widened, top-k, gather, masks) wrote and read the table several times.
+template <int KEEP>
+__global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
+    const float *__restrict__ rows, const int32_t *__restrict__ cand_id,
+    const int32_t *__restrict__ count, int64_t *__restrict__ out_id,
+    float *__restrict__ out_dist, int64_t m, int64_t first, int64_t n, int d, int k,
+    int hide_inf) {
+    constexpr int kCap = KEEP + kSlack + kMaxBN;
+    extern __shared__ __align__(16) unsigned char rank_lds[];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int64_t q = (int64_t)blockIdx.x * kRankWaves + wave;
+    const int d4 = d / 4;
+    // per wavefront: the row, then (distance, row number) of the candidates
+    unsigned long long *entry =
+        reinterpret_cast<unsigned long long *>(rank_lds) + wave * KEEP;
+    floatx4 *mine = reinterpret_cast<floatx4 *>(rank_lds + kRankWaves * KEEP * 8) + wave * d4;
+    if (q >= m) return;
+    const floatx4 *src = reinterpret_cast<const floatx4 *>(rows + (size_t)(first + q) * d);
+    for (int i = lane; i < d4; i += kWave) mine[i] = src[i];
+    for (int i = lane; i < KEEP; i += kWave) entry[i] = ~0ull;
+    wave_sync();
+    const int32_t *ids = cand_id + (size_t)q * kCap;
+    const int cnt = min(KEEP, uni(count[q]));
+    const int team = lane >> 4, place = lane & 15;
+    for (int j0 = 0; j0 < cnt; j0 += 4) {
+        const int j = j0 + team;
+        const int32_t id = j < cnt ? ids[j] : -1;
+        const bool ok = id >= 0 && id < n && id != first + q;
+        const float sum = team_square_dist(
+            mine, reinterpret_cast<const floatx4 *>(rows + (ok ? (size_t)id * d : 0)), d4, place, ok);
+        if (place == 0 && j < cnt)
+            entry[j] = ((unsigned long long)__float_as_uint(ok ? sum : INFINITY) << 32) |
+                       (unsigned)id;
+    }
+    wave_sync();
+#pragma unroll 1
+    for (int size = 2; size <= KEEP; size <<= 1) {
+#pragma unroll 1
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+#pragma unroll
+            for (int t0 = 0; t0 < KEEP / 2; t0 += kWave) {
+                const int t = t0 + lane;
+                const int i = ((t & ~(stride - 1)) << 1) | (t & (stride - 1));
+                if (KEEP / 2 >= kWave || t < KEEP / 2) {
+                    const unsigned long long x = entry[i], y = entry[i | stride];
+                    if ((x > y) == ((i & size) == 0) && x != y) entry[i] = y, entry[i | stride] = x;
+                }
+            }
+            wave_sync();
+        }
+    }
+    for (int i = lane; i < k; i += kWave) {
+        const unsigned long long e = entry[i];
+        const int32_t id = (int32_t)(unsigned)e;
+        const float dist = id < 0 ? INFINITY : __uint_as_float((unsigned)(e >> 32));
+        out_id[(size_t)q * k + i] = hide_inf && isinf(dist) ? -1 : (int64_t)id;
+        out_dist[(size_t)q * k + i] = dist;
     }
 }
 
@@ -760,6 +903,39 @@ extern "C" int pa_knn_rerank(float *dist, const float *rows, const int64_t *cand
     const unsigned lds = (unsigned)(kRankWaves * d * sizeof(float));
     rerank_kernel<<<(unsigned)((m + kRankWaves - 1) / kRankWaves), kWave * kRankWaves, lds,
                     (hipStream_t)stream_>>>(rows, cand, dist, m, first, n, d, k);
+    return (int)hipGetLastError();
+}
+
+extern "C" int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
+                           int32_t *cand_id, int32_t *cand_count, const float *rows, int64_t m,
+                           int64_t first, int64_t n, int d, int keep, int n_seg, int k,
+                           int hide_inf, void *stream_) {
+    if (m < 0 || n < 0 || first < 0 || first + m > n || n_seg < 1) return PA_E_SHAPE;
+    if (keep != 64 && keep != 128 && keep != 256 && keep != 512) return PA_E_SHAPE;
+    if (k < 1 || k > keep) return PA_E_SHAPE;
+    if (d <= 0 || d % 4 || d > kMaxRankDim) return PA_E_DIM;
+    // row numbers are 32 bits; work-items of a launch
+    if (n >= (1ll << 31) || m >= (1ll << 32) / kWave) return PA_E_RANGE;
+    if (m == 0) return PA_OK;
+    if (!out_id || !out_dist || !cand_score || !cand_id || !cand_count || !rows) return PA_E_NULL;
+    hipStream_t stream = (hipStream_t)stream_;
+    const unsigned blocks = (unsigned)((m + kRankWaves - 1) / kRankWaves);
+    const unsigned lds = (unsigned)(kRankWaves * (d * sizeof(float) + keep * 8));
+#define PA_RANK(KEEP_)                                                                        \
+    {                                                                                         \
+        if (n_seg > 1)                                                                        \
+            merge_kernel<KEEP_><<<blocks, kWave * kRankWaves, 0, stream>>>(                   \
+                cand_score, cand_id, cand_count, m, n_seg);                                   \
+        rank_kernel<KEEP_><<<blocks, kWave * kRankWaves, lds, stream>>>(                      \
+            rows, cand_id, cand_count, out_id, out_dist, m, first, n, d, k, hide_inf);        \
+    }
+    switch (keep) {
+        case 64: PA_RANK(64) break;
+        case 128: PA_RANK(128) break;
+        case 256: PA_RANK(256) break;
+        default: PA_RANK(512) break;
+    }
+#undef PA_RANK
     return (int)hipGetLastError();
 }
 

@@ -391,6 +391,33 @@ class HalfRows:
 _KNN_RESIDENT = 256
 
 
+def _knn_lists(query, base, keep: int, n_seg: int = None):
+    """``pa_knn``'s raw lists for :class:`HalfRows` ``query`` / ``base``:
+    ``(score, ids, count)`` of ``[n_seg, m, capacity]``, the same and
+    ``[n_seg, m]``."""
+    _require(query.d == base.d, 'query.size(-1) == base.size(-1)')
+    _require(query.half.device == base.half.device, 'query.device == base.device')
+    _require(base.n >= 1, 'base.size(0) >= 1')
+    m, n, device = query.n, base.n, base.half.device
+    tile = query.tile
+    blocks, tiles = -(-m // tile), -(-n // tile)
+    if n_seg is None:
+        # enough workgroups for one per compute unit
+        n_seg = max(1, min(tiles, _KNN_RESIDENT // max(blocks, 1)))
+    cap = int(_lib.lib().pa_knn_list_capacity(int(keep)))
+    _require(cap > 0, 'keep is 64, 128, 256 or 512')
+    score = torch.empty(n_seg, m, cap, dtype=torch.float32, device=device)
+    ids = torch.empty(n_seg, m, cap, dtype=torch.int32, device=device)
+    count = torch.empty(n_seg, m, dtype=torch.int32, device=device)
+    if m:
+        with torch.cuda.device(device):
+            _lib.check(_lib.lib().pa_knn(
+                _ptr(score), _ptr(ids), _ptr(count), _ptr(query.half), _ptr(base.half),
+                _ptr(base.norm), m, n, base.half.size(1), int(keep), n_seg, _stream()),
+                'pa_knn')
+    return score, ids, count
+
+
 def knn_candidates(query, base, keep: int, n_seg: int = None):
     """For every row of ``query`` the ``keep`` (64, 128, 256 or 512) rows of ``base``
     that are closest by half-precision products (``pa_knn``; the step the
@@ -403,27 +430,11 @@ def knn_candidates(query, base, keep: int, n_seg: int = None):
         base = HalfRows(base)
     if not isinstance(query, HalfRows):
         query = HalfRows(query, scale=base.scale)
-    _require(query.d == base.d, 'query.size(-1) == base.size(-1)')
-    _require(query.half.device == base.half.device, 'query.device == base.device')
-    _require(base.n >= 1, 'base.size(0) >= 1')
-    m, n, device = query.n, base.n, base.half.device
+    m, device = query.n, base.half.device
+    score, ids, count = _knn_lists(query, base, keep, n_seg)
     if m == 0:
         return torch.empty(0, keep, dtype=torch.long, device=device)
-    tile = query.tile
-    blocks, tiles = -(-m // tile), -(-n // tile)
-    if n_seg is None:
-        # enough workgroups for one per compute unit
-        n_seg = max(1, min(tiles, _KNN_RESIDENT // blocks))
-    cap = int(_lib.lib().pa_knn_list_capacity(int(keep)))
-    _require(cap > 0, 'keep is 64, 128, 256 or 512')
-    score = torch.empty(n_seg, m, cap, dtype=torch.float32, device=device)
-    ids = torch.empty(n_seg, m, cap, dtype=torch.int32, device=device)
-    count = torch.empty(n_seg, m, dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
-        _lib.check(_lib.lib().pa_knn(
-            _ptr(score), _ptr(ids), _ptr(count), _ptr(query.half), _ptr(base.half),
-            _ptr(base.norm), m, n, base.half.size(1), int(keep), n_seg, _stream()),
-            'pa_knn')
+    n_seg = score.size(0)
     score, ids = score[:, :, :keep], ids[:, :, :keep]
     valid = torch.arange(keep, device=device).view(1, 1, keep) < count.unsqueeze(-1)
     ids = torch.where(valid, ids.long(), torch.full_like(ids, -1, dtype=torch.long))
@@ -453,6 +464,33 @@ def knn_rerank(rows: torch.Tensor, cand: torch.Tensor, first: int = 0):
             _ptr(dist), _ptr(rows), _ptr(cand), m, int(first), n, d, k, _stream()),
             'pa_knn_rerank')
     return dist
+
+
+def knn_nearest(rows: torch.Tensor, query: HalfRows, base: HalfRows, keep: int, k: int,
+                first: int = 0, hide_inf: bool = False):
+    """The ``k`` closest rows of ``base`` for every row of ``query``, closest
+    first: ``pa_knn``'s ``keep`` candidates ranked by exact float32 distances
+    (``pa_knn_rank``).  ``rows`` ``[n, d]`` float32 holds the rows themselves,
+    those of ``query`` from ``first`` on, those of ``base`` from 0 on.  Returns
+    ``(ids, d2)`` ``[m, k]``: a list that is shorter ends in ``-1`` / infinity,
+    and the row itself has distance infinity (``-1`` with ``hide_inf``)."""
+    _check(rows, 'rows', 2, torch.float32, True)
+    _require(rows.device == base.half.device, 'rows.device == base.device')
+    _require(rows.size(1) == base.d, 'rows.size(-1) == base.d')
+    _require(base.n <= rows.size(0), 'base.n <= rows.size(0)')
+    _require(0 <= first and first + query.n <= rows.size(0),
+             'first + query.n <= rows.size(0)')
+    _require(1 <= k <= keep, '1 <= k <= keep')
+    m = query.n
+    score, ids, count = _knn_lists(query, base, keep)
+    out_i = torch.empty(m, k, dtype=torch.long, device=rows.device)
+    out_d = torch.empty(m, k, dtype=torch.float32, device=rows.device)
+    with torch.cuda.device(rows.device):
+        _lib.check(_lib.lib().pa_knn_rank(
+            _ptr(out_i), _ptr(out_d), _ptr(score), _ptr(ids), _ptr(count), _ptr(rows), m,
+            int(first), rows.size(0), rows.size(1), int(keep), score.size(0), int(k),
+            int(bool(hide_inf)), _stream()), 'pa_knn_rank')
+    return out_i, out_d
 
 
 def graph_prune(pair: torch.Tensor, cand_dist: torch.Tensor, m_keep: int, fill: bool):

@@ -76,22 +76,18 @@ def _knn_graph_device(x: torch.Tensor, k: int, rows_per_pass: int = None):
         rows_per_pass = max(256, min(8192, (1 << 29) // (keep * d)))
     for lo in range(0, n, pass_rows):
         hi = min(n, lo + pass_rows)
-        cand = kernels.knn_candidates(rows.rows(lo, hi), rows, keep)
         if fused:
-            # exact distances to the candidates by one kernel
-            d2 = kernels.knn_rerank(x, cand, lo)
-            top = torch.topk(d2, k, dim=-1, largest=False)
-            out_i[lo:hi] = torch.gather(cand, 1, top.indices)
-            out_d[lo:hi] = top.values
+            # exact distances to the candidates and their ranking by one kernel
+            out_i[lo:hi], out_d[lo:hi] = _rank_device(x, rows, rows, lo, hi, keep, k)
             if __debug__:
                 # a kernel that left a place unwritten must raise here, not
                 # fault in a later gather
                 assert int(out_i[lo:hi].max()) < n and int(out_i[lo:hi].min()) >= -1
-            del d2
             if progress is not None:
                 torch.cuda.synchronize(x.device)   # report what is done, not what is queued
                 progress(f'neighbour table: {hi} of {n} rows')
             continue
+        cand = kernels.knn_candidates(rows.rows(lo, hi), rows, keep)
         own = torch.arange(lo, hi, device=x.device).unsqueeze(-1)
         for a in range(0, hi - lo, rows_per_pass):
             b = min(hi - lo, a + rows_per_pass)
@@ -108,6 +104,21 @@ def _knn_graph_device(x: torch.Tensor, k: int, rows_per_pass: int = None):
     return out_i, out_d
 
 
+def _rank_device(x, rows, base, lo: int, hi: int, keep: int, k: int, hide_inf: bool = False):
+    """The ``k`` closest of ``base`` for rows ``lo .. hi`` of ``x`` by exact
+    float32 distances to ``pa_knn``'s ``keep`` candidates."""
+    from .. import kernels
+    part = rows.rows(lo, hi)
+    if x.size(1) <= 2048:       # what pa_knn_rank holds of a row
+        return kernels.knn_nearest(x, part, base, keep, k, lo, hide_inf)
+    cand = kernels.knn_candidates(part, base, keep)
+    top = torch.topk(kernels.knn_rerank(x, cand, lo), k, dim=-1, largest=False)
+    ids = torch.gather(cand, 1, top.indices)
+    if hide_inf:
+        ids = torch.where(torch.isinf(top.values), -1, ids)
+    return ids, top.values
+
+
 def _knn_rows_device(x, rows, lo: int, hi: int, n_base: int, k: int):
     """The ``k`` nearest of rows ``0 .. n_base`` of ``x`` for rows ``lo .. hi``
     (the row itself excluded), as :func:`_knn_graph_device` ranks them:
@@ -115,24 +126,14 @@ def _knn_rows_device(x, rows, lo: int, hi: int, n_base: int, k: int):
     (``kernels.HalfRows(x)``), exact float32 distances decide.  ``lo`` and
     ``n_base`` are multiples of the kernel's tile (or ``n_base`` is all of
     ``x``).  Places without a candidate hold ``-1`` / infinity."""
-    from .. import kernels
     keep = next(size for size in (64, 128, 256, 512) if k + 16 <= size)
     base = rows if n_base == rows.n else rows.rows(0, n_base)
-    cand = kernels.knn_candidates(rows.rows(lo, hi), base, keep)
-    d2 = kernels.knn_rerank(x, cand, lo)
-    top = torch.topk(d2, min(k, d2.size(1)), dim=-1, largest=False)
-    ids = torch.gather(cand, 1, top.indices)
+    ids, dist = _rank_device(x, rows, base, lo, hi, keep, k, hide_inf=True)
     if __debug__:
         # a kernel that left a place unwritten must raise here, not fault in
         # a later gather
         assert int(ids.max()) < n_base and int(ids.min()) >= -1
-    ids = torch.where(torch.isinf(top.values), torch.full_like(ids, -1), ids)
-    if ids.size(1) < k:
-        pad = k - ids.size(1)
-        ids = torch.cat([ids, ids.new_full((hi - lo, pad), -1)], 1)
-        dist = torch.cat([top.values, top.values.new_full((hi - lo, pad), float('inf'))], 1)
-        return ids, dist
-    return ids, top.values
+    return ids, dist
 
 
 def _knn_rows_host(x, lo: int, hi: int, n_base: int, k: int, chunk: int = 2048):
