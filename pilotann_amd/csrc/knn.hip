@@ -39,8 +39,11 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kChunk = 64;        // contraction elements staged at a time; a
                                   // row is a whole number of chunks
-constexpr int kSlack = 128;       // appended entries a list may hold beyond
-                                  // `keep` before it must be cut
+// Appended entries a list may hold beyond `keep` before it must be cut.  Lists
+// of 256 (a graph build's) take 384: half as many cuts as with 128, and a fifth
+// more entries let in by the limit of the last one (55 000 rows against 120 000
+// of 768 floats: 128 21.4, 256 15.2, 384 14.9, 512 15.4 ms).
+constexpr int slack(int keep) { return keep == 256 ? 384 : 128; }
 constexpr int kMaxBN = 256;       // the most base rows a tile has in any form
 constexpr int kRowPad = 256;      // rows the caller's arrays are padded to
 
@@ -87,19 +90,23 @@ __device__ __forceinline__ void bring_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LEFT) : "memory");
 }
 
-// The wavefront cuts one list of `n` entries (keep < n <= keep + kSlack + BN)
+// The wavefront cuts one list of `n` entries (keep < n <= keep + slack + BN)
 // to its `keep` smallest, which end up in its first `keep` places, and returns
 // the largest score kept.
 template <int KEEP, int BN>
 __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int lane) {
-    constexpr int kPerLane = (KEEP + kSlack + BN + kWave - 1) / kWave;
+    constexpr int kPerLane = (KEEP + slack(KEEP) + BN + kWave - 1) / kWave;
     unsigned u[kPerLane];
     int32_t v[kPerLane];
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
         const int e = lane + kWave * i;
-        u[i] = e < n ? ordered(score[e]) : 0xffffffffu;
-        v[i] = e < n ? id[e] : -1;
+        u[i] = 0x7fffffffu;   // no score: ordered() of it is the largest number
+        v[i] = -1;
+        if (kWave * i + kWave <= KEEP || e < n) {
+            u[i] = __float_as_uint(score[e]);
+            v[i] = id[e];
+        }
     }
     // The KEEP-th smallest, bit by bit from the highest one in which the
     // entries differ: `bound` stays the largest value with fewer than KEEP
@@ -108,8 +115,9 @@ __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int 
     unsigned low = 0xffffffffu, high = 0;
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
+        u[i] = ordered(__uint_as_float(u[i]));
         low = min(low, u[i]);
-        high = lane + kWave * i < n ? max(high, u[i]) : high;
+        high = u[i] != 0xffffffffu ? max(high, u[i]) : high;
     }
     low = ~((unsigned)wave_max_key((int)(~low ^ 0x80000000u)) ^ 0x80000000u);
     high = (unsigned)wave_max_key((int)(high ^ 0x80000000u)) ^ 0x80000000u;
@@ -133,7 +141,7 @@ __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int 
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
         const bool below = u[i] < bound;
-        const bool equal = u[i] == bound && lane + kWave * i < n;
+        const bool equal = u[i] == bound;
         const unsigned long long mb = __ballot(below), me = __ballot(equal);
         const int pb = at_below + lane_rank(mb), pe = at_equal + lane_rank(me);
         if (below) {
@@ -169,7 +177,15 @@ __device__ __forceinline__ float cut_list(float *score, int32_t *id, int n, int 
 // from memory straight into the other buffer (global_load_lds, 16 bytes a
 // lane; no registers and no LDS stores in between); one barrier per chunk; the
 // chunk after a tile's last is the first of the next tile.
-template <int KEEP, int WR, int WC, int WM, int WN>
+//
+// SHORT: the list starts empty and a walk of few tiles, in which most sums
+// pass, is all it sees: places for a wavefront's entries are drawn row by row
+// with one atomic instruction, where an atomic for every lane and sum waits for
+// each result and meets others on a few words.  In a long walk few sums pass
+// and that form's counting costs more than it saves.  Per launch over 768
+// floats: one tile a list 90 against 52 us, 2 tiles 385 against 315, 4 tiles
+// 940 against 820, 32 tiles the same, 469 tiles 14.9 against 16.6 ms.
+template <int KEEP, bool SHORT, int WR, int WC, int WM, int WN>
 __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kernel(KnnArgs a) {
     constexpr int kThreads = kWave * WR * WC;
     constexpr int BM = 32 * WR * WM, BN = 32 * WC * WN;
@@ -178,7 +194,7 @@ __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kerne
     static_assert(BN <= kMaxBN && kRowPad % BM == 0 && kRowPad % BN == 0, "tile sizes");
     static_assert(kOwnRows == 32 || kOwnRows == 64, "lists per wavefront");
     static_assert(BM % kStageRows == 0 && BN % kStageRows == 0, "staging steps");
-    constexpr int kCap = KEEP + kSlack + kMaxBN;  // entries a list can hold
+    constexpr int kCap = KEEP + slack(KEEP) + kMaxBN;  // entries a list can hold
     // a staging buffer: the chunk of the query tile, then that of the base
     // tile, rows of kRow bytes without padding.  LDS has 64 banks of four
     // bytes and serves a 16-byte read to 16 lanes at a time: 16 consecutive
@@ -327,23 +343,77 @@ __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kerne
             float lim[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) lim[r] = limit[row0 + 8 * (r >> 2) + (r & 3)];
+            if constexpr (SHORT) {
+                unsigned live = 0;   // bit r: some lane's sum r is above its limit
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float best = acc[m][0][r];
-                if constexpr (WN == 4) {
-                    best = larger(larger(best, acc[m][1][r], acc[m][2][r]), acc[m][3][r]);
-                } else {
+                for (int r = 0; r < 16; ++r) {
+                    float best = acc[m][0][r];
 #pragma unroll
                     for (int n = 1; n < WN; ++n) best = larger(best, acc[m][n][r]);
+                    live |= __ballot(best > lim[r]) ? 1u << r : 0u;
                 }
-                if (best > lim[r]) {  // rare after the first tiles
-                    const int row = row0 + 8 * (r >> 2) + (r & 3);
+                if (!live) continue;
+                // How many each of the 32 rows takes from this wavefront goes
+                // to lane r + 16 half, and all their places are drawn with
+                // one atomic instruction; then the entries are stored.
+                int taken = 0;
 #pragma unroll
-                    for (int n = 0; n < WN; ++n) {
-                        if (acc[m][n][r] > lim[r]) {
-                            const unsigned at = row * kCap + atomicAdd(&count[row], 1);
-                            my_score[at] = -2.f * acc[m][n][r];
-                            my_id[at] = c0 + 32 * n;
+                for (int r = 0; r < 16; ++r) {
+                    if ((live >> r) & 1) {
+                        int low = 0, high = 0;
+#pragma unroll
+                        for (int n = 0; n < WN; ++n) {
+                            const unsigned long long some = __ballot(acc[m][n][r] > lim[r]);
+                            low += __popc((unsigned)some);
+                            high += __popc((unsigned)(some >> 32));
+                        }
+                        taken = lane == r ? low : lane == 16 + r ? high : taken;
+                    }
+                }
+                int place = 0;
+                if (taken > 0)
+                    place = atomicAdd(&count[(wr * WM + m) * 32 + 4 * (lane >> 4) +
+                                             8 * ((lane & 15) >> 2) + (lane & 3)], taken);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    if ((live >> r) & 1) {
+                        const int low = __builtin_amdgcn_readlane(place, r);
+                        const int high = __builtin_amdgcn_readlane(place, 16 + r);
+                        const unsigned row = row0 + 8 * (r >> 2) + (r & 3);
+                        unsigned at = row * kCap + (half ? high : low);
+#pragma unroll
+                        for (int n = 0; n < WN; ++n) {
+                            const bool in = acc[m][n][r] > lim[r];
+                            const unsigned long long some = __ballot(in);
+                            const unsigned mine = half ? (unsigned)(some >> 32) : (unsigned)some;
+                            if (in) {
+                                const unsigned to = at + __popc(mine & ((1u << col) - 1u));
+                                my_score[to] = -2.f * acc[m][n][r];
+                                my_id[to] = c0 + 32 * n;
+                            }
+                            at += __popc(mine);
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float best = acc[m][0][r];
+                    if constexpr (WN == 4) {
+                        best = larger(larger(best, acc[m][1][r], acc[m][2][r]), acc[m][3][r]);
+                    } else {
+#pragma unroll
+                        for (int n = 1; n < WN; ++n) best = larger(best, acc[m][n][r]);
+                    }
+                    if (best > lim[r]) {  // rare after the first tiles
+                        const int row = row0 + 8 * (r >> 2) + (r & 3);
+#pragma unroll
+                        for (int n = 0; n < WN; ++n) {
+                            if (acc[m][n][r] > lim[r]) {
+                                const unsigned at = row * kCap + atomicAdd(&count[row], 1);
+                                my_score[at] = -2.f * acc[m][n][r];
+                                my_id[at] = c0 + 32 * n;
+                            }
                         }
                     }
                 }
@@ -355,7 +425,7 @@ __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kerne
         {
             const int row = wave * kOwnRows + lane % kOwnRows;
             unsigned long long todo =
-                __ballot(lane < kOwnRows && count[row] > KEEP + kSlack);
+                __ballot(lane < kOwnRows && count[row] > KEEP + slack(KEEP));
             while (todo) {
                 const int r = wave * kOwnRows + __builtin_ctzll(todo);
                 todo &= todo - 1;
@@ -398,7 +468,7 @@ template <int KEEP>
 __global__ __launch_bounds__(kWave * kRankWaves) void merge_kernel(
     float *__restrict__ score, int32_t *__restrict__ id, int32_t *__restrict__ count,
     int64_t m, int n_seg) {
-    constexpr int kCap = KEEP + kSlack + kMaxBN;
+    constexpr int kCap = KEEP + slack(KEEP) + kMaxBN;
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t row = (int64_t)blockIdx.x * kRankWaves + threadIdx.x / kWave;
     if (row >= m) return;
@@ -503,7 +573,7 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     const int32_t *__restrict__ count, int64_t *__restrict__ out_id,
     float *__restrict__ out_dist, int64_t m, int64_t first, int64_t n, int d, int k,
     int hide_inf) {
-    constexpr int kCap = KEEP + kSlack + kMaxBN;
+    constexpr int kCap = KEEP + slack(KEEP) + kMaxBN;
     extern __shared__ __align__(16) unsigned char rank_lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int64_t q = (int64_t)blockIdx.x * kRankWaves + wave;
@@ -848,17 +918,24 @@ __global__ __launch_bounds__(256, 4) void prune_rows_kernel(PruneRowsArgs a) {
 constexpr int kWR = 2, kWC = 4, kWM = 4, kWN = 2;
 constexpr int kBM = 32 * kWR * kWM;
 
+constexpr int kShortWalk = 32;   // tiles
+
 template <int KEEP>
 int launch_knn(const KnnArgs &a, hipStream_t stream) {
+    constexpr int kBN = 32 * kWC * kWN;
     const dim3 grid((unsigned)((a.m + kBM - 1) / kBM), (unsigned)a.n_seg);
-    knn_kernel<KEEP, kWR, kWC, kWM, kWN><<<grid, 64 * kWR * kWC, 0, stream>>>(a);
+    const int64_t tiles = (a.n + kBN - 1) / kBN;   // dealt to the segments
+    if ((tiles + a.n_seg - 1) / a.n_seg <= kShortWalk)
+        knn_kernel<KEEP, true, kWR, kWC, kWM, kWN><<<grid, 64 * kWR * kWC, 0, stream>>>(a);
+    else
+        knn_kernel<KEEP, false, kWR, kWC, kWM, kWN><<<grid, 64 * kWR * kWC, 0, stream>>>(a);
     return (int)hipGetLastError();
 }
 
 }  // namespace
 
 extern "C" int64_t pa_knn_list_capacity(int keep) {
-    return keep == 64 || keep == 128 || keep == 256 || keep == 512 ? keep + kSlack + kMaxBN : 0;
+    return keep == 64 || keep == 128 || keep == 256 || keep == 512 ? keep + slack(keep) + kMaxBN : 0;
 }
 
 extern "C" int pa_knn_tile_rows(void) { return kRowPad; }
