@@ -23,8 +23,10 @@
 namespace {
 
 constexpr float kInf = std::numeric_limits<float>::infinity();
-constexpr int kTile = 4;       // rows per batched distance, traverse_cpu.cpp:8
+constexpr int kTile = 8;       // rows per batched distance (traverse_cpu.cpp:8: four)
 constexpr int kRefineSteps = 2;  // traverse_cpu.cpp:9
+constexpr int kStretch = 64;   // neighbours looked at together
+constexpr int kRowLines = 8;   // cache lines of a row requested ahead
 
 // ---- distance ---------------------------------------------------------------
 
@@ -36,37 +38,44 @@ inline float lanes_sum(__m256 acc) {
     return r;
 }
 
-// distance.h:31-55; [from, d) of one row.
-inline float square_dist(const float *q, const float *row, int d, int from = 0) {
-    __m256 acc = _mm256_setzero_ps();
-    for (int o = from; o < d; o += 8) {
-        const __m256 t = _mm256_sub_ps(_mm256_loadu_ps(q + o), _mm256_loadu_ps(row + o));
-        acc = _mm256_fmadd_ps(t, t, acc);
-    }
-    return lanes_sum(acc);
-}
-
-// distance.h:73-111; four rows share each load of the query.
-inline void square_dist4(float *out, const float *q, const float *storage,
-                         const int64_t *rows, int d) {
-    __m256 acc[kTile];
-    const float *p[kTile];
-    for (int i = 0; i < kTile; ++i) {
+// distance.h:31-55,73-111; [from, d) of T rows, which share each load of the
+// query and whose chains of FMAs run side by side.
+template <int T>
+inline void square_dist_rows(float *out, const float *q, const float *storage,
+                             const int64_t *rows, int d, int from) {
+    __m256 acc[T];
+    const float *p[T];
+    for (int i = 0; i < T; ++i) {
         acc[i] = _mm256_setzero_ps();
         p[i] = storage + rows[i] * (int64_t)d;
     }
-    for (int o = 0; o < d; o += 8) {
+    for (int o = from; o < d; o += 8) {
         const __m256 qq = _mm256_loadu_ps(q + o);
-        for (int i = 0; i < kTile; ++i) {
+        for (int i = 0; i < T; ++i) {
             const __m256 t = _mm256_sub_ps(qq, _mm256_loadu_ps(p[i] + o));
             acc[i] = _mm256_fmadd_ps(t, t, acc[i]);
         }
     }
-    for (int i = 0; i < kTile; ++i) out[i] = lanes_sum(acc[i]);
+    for (int i = 0; i < T; ++i) out[i] = lanes_sum(acc[i]);
+}
+inline void square_dists(float *out, const float *q, const float *storage,
+                         const int64_t *rows, int n, int d, int from = 0) {
+    int i = 0;
+    for (; i + kTile <= n; i += kTile)
+        square_dist_rows<kTile>(out + i, q, storage, rows + i, d, from);
+    if (kTile > 4 && i + 4 <= n) square_dist_rows<4>(out + i, q, storage, rows + i, d, from), i += 4;
+    if (i + 2 <= n) square_dist_rows<2>(out + i, q, storage, rows + i, d, from), i += 2;
+    if (i < n) square_dist_rows<1>(out + i, q, storage, rows + i, d, from);
 }
 
 inline void prefetch(const void *p) {
     _mm_prefetch(reinterpret_cast<const char *>(p), _MM_HINT_T1);
+}
+// the first lines of a row of d floats; the hardware's own prefetch of
+// ascending addresses takes over from there
+inline void prefetch_row(const float *row, int d) {
+    const int lines = d >> 4 < kRowLines ? (d + 15) >> 4 : kRowLines;
+    for (int i = 0; i < lines; ++i) prefetch(row + 16 * i);
 }
 
 // ---- heaps: heapq.cuh ---------------------------------------------------------
@@ -106,15 +115,19 @@ struct HeapView {
         key[0] = k, val[0] = v;
         sink_root();
     }
-    // heapq.cuh:47-77
-    void replace(float k, int64_t v) {
+    // heapq.cuh:47-77: the leaf a replacement would take ...
+    int large_leaf() const {
         int at = 0;
         for (;;) {
             int c = 2 * at + 1;
-            if (c >= size) break;
+            if (c >= size) return at;
             if (c + 1 < size && key[c + 1] > key[c]) ++c;
             at = c;
         }
+    }
+    void replace(float k, int64_t v) { replace_leaf(large_leaf(), k, v); }
+    // ... and the new entry's rise from there
+    void replace_leaf(int at, float k, int64_t v) {
         if (k >= key[at]) return;
         while (at > 0) {
             const int up = (at - 1) / 2;
@@ -163,21 +176,34 @@ void search_one(int64_t *out_I, float *out_D, int32_t *seen, int32_t marker,
                 int max_iter, HeapView result, HeapView open) {
     // :42-62 the entries' distances cover [0, d_principle); add the rest
     if (d_principle < d_model) {
-        for (int i = 0; i < n_init; ++i)
-            if (init_I[i] >= 0) prefetch(storage + init_I[i] * (int64_t)d_model + d_principle);
-        for (int i = 0; i < n_init; ++i)
-            if (init_I[i] >= 0)
-                init_D[i] += square_dist(q, storage + init_I[i] * (int64_t)d_model,
-                                         d_model, d_principle);
+        for (int base = 0; base < n_init; base += kStretch) {
+            const int end = n_init - base < kStretch ? n_init : base + kStretch;
+            int n = 0, place[kStretch];
+            int64_t v[kStretch];
+            float rest[kStretch];
+            for (int i = base; i < end; ++i) {
+                if (init_I[i] < 0) continue;
+                place[n] = i, v[n++] = init_I[i];
+                prefetch_row(storage + init_I[i] * (int64_t)d_model + d_principle,
+                             d_model - d_principle);
+            }
+            square_dists(rest, q, storage, v, n, d_model, d_principle);
+            for (int i = 0; i < n; ++i) init_D[place[i]] += rest[i];
+        }
     }
     // :65-79
     result.fill(-kInf);
     open.fill(kInf);
+    // an entry that stays out changes nothing: the walk is taken again only
+    // after one that got in
+    int leaf = open.large_leaf();
     for (int i = 0; i < n_init; ++i) {
         const int64_t u = init_I[i];
         if (u < 0) continue;
         seen[u] = marker;
-        open.replace(init_D[i], u);
+        if (init_D[i] >= open.key[leaf]) continue;
+        open.replace_leaf(leaf, init_D[i], u);
+        leaf = open.large_leaf();
     }
     auto admit = [&](const float *d, const int64_t *v, int n) {  // :25-39
         for (int i = 0; i < n; ++i) {
@@ -193,27 +219,34 @@ void search_one(int64_t *out_I, float *out_D, int32_t *seen, int32_t marker,
         int64_t u;
         open.pop(&uk, &u);
         if (u < 0 || uk >= -result.key[0]) break;
-        const int64_t lo = indptr[u], hi = indptr[u + 1];
-        for (int64_t e = lo; e < hi; ++e)
-            if (indices[e] >= 0) prefetch(&seen[indices[e]]);
-        int n = 0;
-        float d[kTile];
-        int64_t v[kTile];
-        for (int64_t e = lo; e < hi; ++e) {
-            const int64_t w = indices[e];
-            if (w < 0) break;
-            if (seen[w] == -1 || seen[w] == marker) continue;
-            seen[w] = marker;
-            v[n++] = w;
-            prefetch(storage + w * (int64_t)d_model);
-            if (n == kTile) {
-                square_dist4(d, q, storage, v, d_model);
-                admit(d, v, n);
-                n = 0;
+        const int64_t hi = indptr[u + 1];
+        for (int64_t e = indptr[u]; e < hi;) {
+            // a stretch of the row: which of its nodes are new, and all their
+            // rows requested, before the first distance is made
+            const int64_t end = hi - e < kStretch ? hi : e + kStretch;
+            for (int64_t i = e; i < end; ++i)
+                if (indices[i] >= 0) prefetch(&seen[indices[i]]);
+            int n = 0;
+            int64_t v[kStretch];
+            for (; e < end; ++e) {
+                const int64_t w = indices[e];
+                if (w < 0) {
+                    e = hi;
+                    break;
+                }
+                if (seen[w] == -1 || seen[w] == marker) continue;
+                seen[w] = marker;
+                v[n++] = w;
+                prefetch_row(storage + w * (int64_t)d_model, d_model);
             }
+            if (open.val[0] >= 0) {   // most likely the next to be expanded
+                const int64_t *row = indices + indptr[open.val[0]];
+                prefetch(row), prefetch(row + 8), prefetch(row + 16), prefetch(row + 24);
+            }
+            float d[kStretch];
+            square_dists(d, q, storage, v, n, d_model);
+            admit(d, v, n);
         }
-        for (int i = 0; i < n; ++i) d[i] = square_dist(q, storage + v[i] * (int64_t)d_model, d_model);
-        admit(d, v, n);
     }
     // :138-148
     for (int i = 0; i < n_init; ++i)
@@ -362,8 +395,8 @@ extern "C" int pa_bitmask_put(int32_t *marks, int64_t n, const int64_t *keys,
 }
 
 // square_dist_cpu, ops_cpu.cpp:53-85: squared L2 distance of the query to the
-// rows nodelist[i] of storage, four rows at a time while more than four are
-// left, then one by one (both forms add in the same order).
+// rows nodelist[i] of storage (how many rows are taken together does not change
+// the order a row's sum is added in).
 extern "C" int pa_square_dist(float *out, const float *query,
                               const float *storage, const int64_t *nodelist,
                               int64_t n_nodes, int64_t n_storage, int d_model) {
@@ -373,10 +406,8 @@ extern "C" int pa_square_dist(float *out, const float *query,
     if (!out || !query || !storage || !nodelist) return PA_E_NULL;
     for (int64_t i = 0; i < n_nodes; ++i)
         if (nodelist[i] < 0 || nodelist[i] >= n_storage) return PA_E_RANGE;
-    int64_t at = 0;
-    for (; at + kTile < n_nodes; at += kTile)
-        square_dist4(out + at, query, storage, nodelist + at, d_model);
-    for (; at < n_nodes; ++at)
-        out[at] = square_dist(query, storage + nodelist[at] * (int64_t)d_model, d_model);
+    for (int64_t at = 0; at < n_nodes; at += kStretch)
+        square_dists(out + at, query, storage, nodelist + at,
+                     (int)(n_nodes - at < kStretch ? n_nodes - at : kStretch), d_model);
     return PA_OK;
 }
