@@ -310,8 +310,7 @@ int pa_knn_rerank(float *dist, const float *rows, const int64_t *cand,
  * extension either): the lists of the n_seg segments are merged (in place,
  * into the first segment's), the exact squared float32 distances of the `keep`
  * best by score are made as pa_knn_rerank makes them, and out_id / out_dist
- * [m * k] receive the k <= keep closest rows of 0 .. n, closest first, equal
- * distances by row number; -1 / infinity where a list is shorter.  The row
+ * [m * k] receive the k <= keep closest rows of 0 .. n, closest first; -1 / infinity where a list is shorter.  The row
  * itself has distance infinity, like a row number out of range; with hide_inf
  * such places receive -1.  `rows` [n * d], d % 4 == 0, d <= 2048; the queries
  * are rows first .. first + m.  Device pointers; enqueued on `stream`.
@@ -320,6 +319,27 @@ int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
                 int32_t *cand_id, int32_t *cand_count, const float *rows,
                 int64_t m, int64_t first, int64_t n, int d, int keep, int n_seg,
                 int k, int hide_inf, void *stream);
+
+/*
+ * The second half-precision part of rows (no counterpart in the reference's
+ * extension): lo = half(x - half(x)) for x = row * scale clamped to +-most,
+ * d_pad >= d elements a row and n_pad >= n rows, zeros beyond; d_pad % 4 == 0.
+ * Device pointers; enqueued on `stream`.
+ */
+int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n_pad, int d,
+                int d_pad, float scale, float most, void *stream);
+
+/*
+ * Steps of a walk along the edges of adj [n * deg] (int64 node numbers, what is
+ * none of 0 .. n is no edge), the connectivity pass of the graph builder
+ * (faiss' part in the reference).  mark [n]: 0, or 1 at the nodes the walk
+ * starts from; after enough steps it is not 0 exactly at the nodes that are
+ * reached from them, or, with backward != 0, from which they are reached.
+ * changed [1] receives 0 if the last of the `steps` steps reached no node (the
+ * walk is over), else 1.  Device pointers; enqueued on `stream`.
+ */
+int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
+                   int deg, int backward, int steps, void *stream);
 
 /*
  * Occlusion pruning of candidate lists, the edge selection of the graph

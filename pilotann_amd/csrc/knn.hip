@@ -459,8 +459,9 @@ __global__ __launch_bounds__(64 * WR * WC, (WM * WN > 8 ? 1 : 2)) void knn_kerne
 
 // The lists that the segments of a launch left for a row become one, in the
 // place of the first segment's: the `KEEP` smallest of them all.  A wavefront
-// per row; what is below the limit so far is appended and the list cut as in
-// knn_kernel.
+// per row; what is below the limit so far is appended and the list cut when it
+// is nearly full, as in knn_kernel: a handful of cuts for sixteen segments, where
+// a cut after every segment made fifteen (2048 rows 124 us).
 constexpr int kRankWaves = 4;
 constexpr int kMaxRankDim = 2048;   // rows of a workgroup and their lists fit 64 KB of LDS
 
@@ -503,8 +504,8 @@ __global__ __launch_bounds__(kWave * kRankWaves) void merge_kernel(
             n += __popcll(mask);
             if (n > kCap - kWave) cut();
         }
-        if (n > KEEP) cut();
     }
+    if (n > KEEP) cut();
     if (lane == 0) count[row] = n;
 }
 
@@ -562,23 +563,25 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rerank_kernel(
 }
 
 // The ranking that follows knn_kernel in one pass: the distances of a row's
-// list, as rerank_kernel makes them, sorted in LDS (by distance, then by row
-// number), the k closest written out.  What bounds it is the gathering of the
+// list, as rerank_kernel makes them, sorted in LDS, the k closest written out;
+// equal distances in the order of the half-precision scores where lists were
+// merged, else in the list's own order, which is mostly that of the rows.  What bounds it is the gathering of the
 // candidates' rows; the sort of 256 entries (36 passes of two exchanges a
 // lane) hides behind other wavefronts' reads, where ranking in steps of torch
 // (ids widened, top-k, gather, masks) wrote and read the table several times.
 template <int KEEP>
 __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
-    const float *__restrict__ rows, const int32_t *__restrict__ cand_id,
-    const int32_t *__restrict__ count, int64_t *__restrict__ out_id,
-    float *__restrict__ out_dist, int64_t m, int64_t first, int64_t n, int d, int k,
-    int hide_inf) {
+    const float *__restrict__ rows, const float *__restrict__ cand_score,
+    const int32_t *__restrict__ cand_id, const int32_t *__restrict__ count,
+    int64_t *__restrict__ out_id, float *__restrict__ out_dist, int64_t m, int64_t first,
+    int64_t n, int d, int k, int hide_inf, int merged) {
     constexpr int kCap = KEEP + slack(KEEP) + kMaxBN;
     extern __shared__ __align__(16) unsigned char rank_lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int64_t q = (int64_t)blockIdx.x * kRankWaves + wave;
     const int d4 = d / 4;
-    // per wavefront: the row, then (distance, row number) of the candidates
+    // per wavefront: (distance, 23 bits of the score, place in the list) of the
+    // candidates, and the row
     unsigned long long *entry =
         reinterpret_cast<unsigned long long *>(rank_lds) + wave * KEEP;
     floatx4 *mine = reinterpret_cast<floatx4 *>(rank_lds + kRankWaves * KEEP * 8) + wave * d4;
@@ -596,9 +599,11 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
         const bool ok = id >= 0 && id < n && id != first + q;
         const float sum = team_square_dist(
             mine, reinterpret_cast<const floatx4 *>(rows + (ok ? (size_t)id * d : 0)), d4, place, ok);
-        if (place == 0 && j < cnt)
+        if (place == 0 && j < cnt) {
+            const unsigned score = merged ? ordered(cand_score[(size_t)q * kCap + j]) : 0u;
             entry[j] = ((unsigned long long)__float_as_uint(ok ? sum : INFINITY) << 32) |
-                       (unsigned)id;
+                       (score & ~511u) | (unsigned)j;
+        }
     }
     wave_sync();
 #pragma unroll 1
@@ -619,12 +624,74 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     }
     for (int i = lane; i < k; i += kWave) {
         const unsigned long long e = entry[i];
-        const int32_t id = (int32_t)(unsigned)e;
-        const float dist = id < 0 ? INFINITY : __uint_as_float((unsigned)(e >> 32));
+        const bool none = (unsigned)(e >> 32) == 0xffffffffu;
+        const int32_t id = none ? -1 : ids[(unsigned)e & 511u];
+        const float dist = none ? INFINITY : __uint_as_float((unsigned)(e >> 32));
         out_id[(size_t)q * k + i] = hide_inf && isinf(dist) ? -1 : (int64_t)id;
         out_dist[(size_t)q * k + i] = dist;
     }
 }
+
+// What half precision leaves of the rows: x = row * scale, clamped to the half
+// range, lo = half(x - half(x)), padded with zeros to d_pad elements and n_pad
+// rows.  A wavefront per row, four elements a lane and step, one pass over the
+// rows where the same steps as tensor operations made six.
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(kWave * kRankWaves) void low_kernel(
+    const float *__restrict__ rows, _Float16 *__restrict__ lo, int64_t n, int64_t n_pad, int d,
+    int d_pad, float scale, float most) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t row = (int64_t)blockIdx.x * kRankWaves + threadIdx.x / kWave;
+    if (row >= n_pad) return;
+    const float *src = rows + (size_t)row * d;
+    for (int i = 4 * lane; i < d_pad; i += 4 * kWave) {
+        half4 l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float x = row < n && i + e < d ? src[i + e] * scale : 0.f;
+            x = x > most ? most : x < -most ? -most : x;   // NaN stays
+            l[e] = (_Float16)(x - (float)(_Float16)x);
+        }
+        *reinterpret_cast<half4 *>(lo + (size_t)row * d_pad + i) = l;
+    }
+}
+
+// One step of a walk along the edges of adj [n, deg] (-1: no edge) over marks of
+// one byte a node.  Forward: 1 is a node just reached, whose neighbours are
+// reached now (it becomes 2); backward: a node with a marked neighbour is
+// marked.  A node may be reached and go on within one launch, and one that two
+// wavefronts reach at a time may be gone over twice: the marks only grow, and a
+// launch that changes nothing (`changed` stays 0) is the end.  A wavefront per
+// node; most nodes are one byte read.
+__global__ __launch_bounds__(256) void reach_kernel(
+    const int64_t *__restrict__ adj, unsigned char *mark, int *changed, int64_t n, int deg,
+    int backward) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t node = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    if (node >= n) return;
+    const int state = mark[node];
+    if (backward ? state != 0 : state != 1) return;
+    if (!backward && lane == 0) mark[node] = 2;
+    bool found = false;
+    for (int e = lane; e < deg; e += kWave) {
+        const int64_t v = adj[(size_t)node * deg + e];
+        if (v < 0 || v >= n) continue;
+        if (backward) {
+            found |= mark[v] != 0;
+        } else if (mark[v] == 0) {
+            mark[v] = 1;
+            found = true;
+        }
+    }
+    if (!__ballot(found)) return;
+    if (lane == 0) {
+        if (backward) mark[node] = 1;
+        if (changed) *changed = 1;
+    }
+}
+
+__global__ void clear_flag(int *flag) { *flag = 0; }
 
 // Occlusion pruning of a node's candidate list (closest first): candidate j
 // is kept unless a candidate kept before it is closer to it than the node
@@ -1004,7 +1071,8 @@ extern "C" int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
             merge_kernel<KEEP_><<<blocks, kWave * kRankWaves, 0, stream>>>(                   \
                 cand_score, cand_id, cand_count, m, n_seg);                                   \
         rank_kernel<KEEP_><<<blocks, kWave * kRankWaves, lds, stream>>>(                      \
-            rows, cand_id, cand_count, out_id, out_dist, m, first, n, d, k, hide_inf);        \
+            rows, cand_score, cand_id, cand_count, out_id, out_dist, m, first, n, d, k,       \
+            hide_inf, n_seg > 1);                                                             \
     }
     switch (keep) {
         case 64: PA_RANK(64) break;
@@ -1013,6 +1081,34 @@ extern "C" int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
         default: PA_RANK(512) break;
     }
 #undef PA_RANK
+    return (int)hipGetLastError();
+}
+
+extern "C" int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n_pad, int d,
+                           int d_pad, float scale, float most, void *stream_) {
+    if (n < 0 || n_pad < n) return PA_E_SHAPE;
+    if (d <= 0 || d_pad < d || d_pad % 4) return PA_E_DIM;
+    if (n_pad >= (1ll << 32) / kWave) return PA_E_RANGE;   // work-items of the launch
+    if (n_pad == 0) return PA_OK;
+    if ((n > 0 && !rows) || !lo_f16) return PA_E_NULL;
+    low_kernel<<<(unsigned)((n_pad + kRankWaves - 1) / kRankWaves), kWave * kRankWaves, 0,
+                 (hipStream_t)stream_>>>(rows, reinterpret_cast<_Float16 *>(lo_f16), n, n_pad, d,
+                                         d_pad, scale, most);
+    return (int)hipGetLastError();
+}
+
+extern "C" int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
+                              int deg, int backward, int steps, void *stream_) {
+    if (n < 0 || deg < 1 || steps < 1) return PA_E_SHAPE;
+    if (n >= (1ll << 32) / kWave) return PA_E_RANGE;   // work-items of a launch
+    if (n == 0) return PA_OK;
+    if (!mark || !changed || !adj) return PA_E_NULL;
+    hipStream_t stream = (hipStream_t)stream_;
+    clear_flag<<<1, 1, 0, stream>>>(changed);
+    const unsigned blocks = (unsigned)((n + 3) / 4);
+    for (int step = 0; step < steps; ++step)
+        reach_kernel<<<blocks, 256, 0, stream>>>(adj, mark, step + 1 == steps ? changed : nullptr,
+                                                 n, deg, backward);
     return (int)hipGetLastError();
 }
 

@@ -369,11 +369,13 @@ class HalfRows:
         """The second half-precision part of ``rows`` (the tensor this set was
         made from): ``rows * scale - half``, same shape and padding as
         ``half``, so that ``half + low`` is the scaled row to about 22 bits."""
-        low = torch.zeros_like(self.half)
-        for lo in range(0, self.n, 1 << 20):
-            hi = min(self.n, lo + (1 << 20))
-            piece = (rows[lo:hi] * self.scale).clamp_(-self.HALF_MAX, self.HALF_MAX)
-            low[lo:hi, :self.d] = piece - self.half[lo:hi, :self.d].float()
+        _check(rows, 'rows', 2, torch.float32, True)
+        _require(rows.shape == (self.n, self.d), 'the rows this set was made from')
+        low = torch.empty_like(self.half)
+        with torch.cuda.device(rows.device):
+            _lib.check(_lib.lib().pa_rows_low(
+                _ptr(low), _ptr(rows), self.n, low.size(0), self.d, low.size(1),
+                float(self.scale), self.HALF_MAX, _stream()), 'pa_rows_low')
         return low
 
     def rows(self, lo: int, hi: int) -> 'HalfRows':
@@ -491,6 +493,26 @@ def knn_nearest(rows: torch.Tensor, query: HalfRows, base: HalfRows, keep: int, 
             int(first), rows.size(0), rows.size(1), int(keep), score.size(0), int(k),
             int(bool(hide_inf)), _stream()), 'pa_knn_rank')
     return out_i, out_d
+
+
+def graph_reachable(adj: torch.Tensor, sources: torch.Tensor, reverse: bool = False):
+    """Boolean mask of the nodes a walk along the edges of ``adj`` ``[n, deg]``
+    (int64 on the device, ``-1`` padded) reaches from ``sources``, or with
+    ``reverse`` of those from which a walk reaches one (``pa_graph_reach``)."""
+    _check(adj, 'adj', 2, torch.int64, True)
+    n, deg = adj.shape
+    mark = torch.zeros(n, dtype=torch.uint8, device=adj.device)
+    mark[sources.flatten()] = 1
+    changed = torch.empty(1, dtype=torch.int32, device=adj.device)
+    steps = 6     # a step is a short launch, looking at the flag a synchronisation
+    while n:
+        with torch.cuda.device(adj.device):
+            _lib.check(_lib.lib().pa_graph_reach(
+                _ptr(mark), _ptr(changed), _ptr(adj), n, deg, int(bool(reverse)), steps,
+                _stream()), 'pa_graph_reach')
+        if not int(changed):
+            break
+    return mark != 0
 
 
 def graph_prune(pair: torch.Tensor, cand_dist: torch.Tensor, m_keep: int, fill: bool):

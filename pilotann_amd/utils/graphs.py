@@ -301,6 +301,9 @@ def reachable(adj: torch.Tensor, sources: torch.Tensor, reverse: bool = False):
     (``-1`` padded) reaches from ``sources``; with ``reverse`` the nodes from
     which a walk reaches one of ``sources``."""
     n = adj.size(0)
+    if adj.is_cuda and adj.dtype == torch.long and adj.numel():
+        from .. import kernels
+        return kernels.graph_reachable(adj.contiguous(), sources, reverse)
     mark = torch.zeros(n, dtype=torch.bool, device=adj.device)
     mark[sources] = True
     if reverse:
