@@ -113,7 +113,10 @@ constexpr int deep_from(int H) {
     return H == 2048 ? PA_DEEP_2048 : H == 1024 ? PA_DEEP_1024 : H == 512 ? PA_DEEP_512 : 0;
 }
 
-template <int H, int DP8>
+// NEAR: the visited bits of a query are in LDS (behind the query where that is
+// dynamic too), without a table in front of them: for launches whose queries
+// all run at once with so much LDS each (make_plan).
+template <int H, int DP8, bool NEAR>
 __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(TraverseArgs a) {
     // One static block, in this order: the compiler then knows every LDS
     // address, and a heap cell [j - 256] is the scalar j * 8 plus a positive
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     // where LDS does not bound the residency the smaller table only costs).
     constexpr int kSeenLog2 =
         H >= 1024 && kSeenCacheLog2 > 0 ? kSeenCacheLog2 - 1 : kSeenCacheLog2;
-    constexpr int kSeen = 1 << kSeenLog2;
+    constexpr int kSeen = NEAR ? 4 : 1 << kSeenLog2;
     struct Lds {
         uint32_t seen_cache[kSeen];
         int cand_id[kWave];
@@ -142,7 +145,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         int2 heap[kHeapCells];  // open list tail; the final sort reuses it
     };
     __shared__ __align__(16) Lds lds;
-    extern __shared__ __align__(16) float query_any_length[];  // DP8 == 0 only
+    // the query if its length is not known here, then NEAR's visited bits
+    extern __shared__ __align__(16) float query_any_length[];
     const int lane = threadIdx.x;
     float *okey = reinterpret_cast<float *>(lds.heap);
     int *oval = reinterpret_cast<int *>(okey + kHeapCells);
@@ -156,6 +160,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     const bool use_cache = a.n_storage <= (0xffff << kSeenLog2);
     const int deg = a.deg;
     uint32_t *seen = a.seen + (size_t)blockIdx.x * (size_t)a.slot_stride;
+    uint32_t *near_bits =
+        reinterpret_cast<uint32_t *>(query_any_length + (DP8 ? 0 : query_floats(dp)));
     // after the visited slice: the log of admitted candidates, then the
     // levels of the open list kept in device memory
     ResultLog log;
@@ -181,7 +187,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
 #endif
         for (int rep = 0; rep < PA_CLEAR_REPS; ++rep)
             for (int w = lane * 4; w < a.words_per_slot; w += kWave * 4)
-                *reinterpret_cast<uint4 *>(seen + w) = make_uint4(0, 0, 0, 0);
+                *reinterpret_cast<uint4 *>((NEAR ? near_bits : seen) + w) =
+                    make_uint4(0, 0, 0, 0);
         for (int i = lane; i < dp; i += kWave)
             qv[query_slot(i, dp >> 3)] = a.query[(size_t)q * dp + i];
         for (int i = lane; i < kSeen; i += kWave) seen_cache[i] = 0xffffffffu;
@@ -214,8 +221,12 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 if (g >= 0 && g < a.n_nodes) {
                     u = (int)g;
                     row = (int)a.mapping[g];
-                    if (row >= 0)
-                        atomicOr(&seen[row >> 5], 1u << (row & 31));
+                    if (row >= 0) {
+                        if constexpr (NEAR)
+                            atomicOr(&near_bits[row >> 5], 1u << (row & 31));
+                        else
+                            atomicOr(&seen[row >> 5], 1u << (row & 31));
+                    }
                 }
             }
             open.push_entries(leaf, __ballot(u >= 0), float_to_key(d),
@@ -250,6 +261,10 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         // bitmask, which is exact.
         auto test_and_set = [&](int v) -> uint32_t {
             uint32_t before = 0xffffffffu;
+            if constexpr (NEAR) {
+                if (v >= 0) before = atomicOr(&near_bits[v >> 5], 1u << (v & 31));
+                return before;
+            }
             if (v >= 0) {
                 const int cell = v & (kSeen - 1);
                 const uint32_t tag = (uint32_t)v >> kSeenLog2;
@@ -629,32 +644,75 @@ int next_pow2(int x) {
 
 typedef void (*TraverseFn)(TraverseArgs);
 
-template <int H>
+// more than five wavefronts per SIMD have measured slower on every instance
+// that fits them (the SIMDs' issue slots are the bound)
+#ifndef PA_MAX_WAVES_PER_CU
+#define PA_MAX_WAVES_PER_CU 20
+#endif
+constexpr int kMaxWavesPerCu = PA_MAX_WAVES_PER_CU;
+constexpr int kStaticLds = 20 << 10;   // no instance has more static LDS
+
+template <int H, bool NEAR>
 TraverseFn pick_dp(int dp) {
     switch (dp) {
-        case 32: return traverse_kernel<H, 4>;
-        case 64: return traverse_kernel<H, 8>;
-        case 128: return traverse_kernel<H, 16>;
-        default: return traverse_kernel<H, 0>;
+        case 32: return traverse_kernel<H, 4, NEAR>;
+        case 64: return traverse_kernel<H, 8, NEAR>;
+        case 128: return traverse_kernel<H, 16, NEAR>;
+        default: return traverse_kernel<H, 0, NEAR>;
     }
 }
 
+template <bool NEAR>
 TraverseFn pick_kernel(int H, int dp) {
     switch (H) {
-        case 16: return pick_dp<16>(dp);
-        case 32: return pick_dp<32>(dp);
-        case 48: return pick_dp<48>(dp);
-        case 64: return pick_dp<64>(dp);
-        case 96: return pick_dp<96>(dp);
-        case 128: return pick_dp<128>(dp);
-        case 192: return pick_dp<192>(dp);
-        case 256: return pick_dp<256>(dp);
-        case 384: return pick_dp<384>(dp);
-        case 512: return pick_dp<512>(dp);
-        case 1024: return pick_dp<1024>(dp);
-        case 2048: return pick_dp<2048>(dp);
+        case 16: return pick_dp<16, NEAR>(dp);
+        case 32: return pick_dp<32, NEAR>(dp);
+        case 48: return pick_dp<48, NEAR>(dp);
+        case 64: return pick_dp<64, NEAR>(dp);
+        case 96: return pick_dp<96, NEAR>(dp);
+        case 128: return pick_dp<128, NEAR>(dp);
+        case 192: return pick_dp<192, NEAR>(dp);
+        case 256: return pick_dp<256, NEAR>(dp);
+        case 384: return pick_dp<384, NEAR>(dp);
+        case 512: return pick_dp<512, NEAR>(dp);
+        case 1024: return pick_dp<1024, NEAR>(dp);
+        case 2048: return pick_dp<2048, NEAR>(dp);
         default: return nullptr;
     }
+}
+
+// Wavefronts (workgroups of one) of `fn` the current device holds at once, and
+// in *max_lds what LDS it gives one workgroup.
+int residency(TraverseFn fn, int lds_bytes, int64_t *slots, int *max_lds) {
+    struct Known {
+        int cus, per_cu, max_lds;
+    };
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    // the residency of a (device, kernel, LDS size) never changes
+    static std::mutex mutex;
+    static std::map<std::tuple<int, const void *, int>, Known> known;
+    std::lock_guard<std::mutex> guard(mutex);
+    const auto key = std::make_tuple(dev, reinterpret_cast<const void *>(fn), lds_bytes);
+    auto it = known.find(key);
+    if (it == known.end()) {
+        Known k = {0, 0, 0};
+        e = hipDeviceGetAttribute(&k.cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e == hipSuccess)
+            e = hipDeviceGetAttribute(&k.max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+        if (e == hipSuccess)
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &k.per_cu, reinterpret_cast<const void *>(fn), kWave, lds_bytes);
+        if (e != hipSuccess) return (int)e;
+        // sizes of NEAR follow the index: a few stay
+        if (known.size() > 4096) known.clear();
+        it = known.emplace(key, k).first;
+    }
+    *slots = (int64_t)it->second.per_cu * it->second.cus;
+    *max_lds = it->second.max_lds;
+    if (it->second.per_cu > kMaxWavesPerCu) *slots = (int64_t)kMaxWavesPerCu * it->second.cus;
+    return PA_OK;
 }
 
 struct Plan {
@@ -676,38 +734,12 @@ int make_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, Plan *p) {
 #ifdef PA_EXTRA_LDS  // tuning builds: lower the residency without touching code
     p->lds_bytes += PA_EXTRA_LDS;
 #endif
-    p->fn = pick_kernel(p->H, dp);
+    p->fn = pick_kernel<false>(p->H, dp);
     if (!p->fn) return PA_E_EF;
-    int dev = 0, cus = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    {
-        // the residency of a (device, kernel, LDS size) never changes
-        static std::mutex mutex;
-        static std::map<std::tuple<int, const void *, int>, std::pair<int, int>> known;
-        std::lock_guard<std::mutex> guard(mutex);
-        const auto key = std::make_tuple(
-            dev, reinterpret_cast<const void *>(p->fn), p->lds_bytes);
-        auto it = known.find(key);
-        if (it == known.end()) {
-            e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-            if (e == hipSuccess)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void *>(p->fn), kWave,
-                    p->lds_bytes);
-            if (e != hipSuccess) return (int)e;
-            it = known.emplace(key, std::make_pair(cus, per_cu)).first;
-        }
-        cus = it->second.first, per_cu = it->second.second;
-    }
-    if (per_cu < 1) per_cu = 1;
-    // more than five wavefronts per SIMD have measured slower on every
-    // instance that fits them (the SIMDs' issue slots are the bound)
-#ifndef PA_MAX_WAVES_PER_CU
-#define PA_MAX_WAVES_PER_CU 20
-#endif
-    if (per_cu > PA_MAX_WAVES_PER_CU) per_cu = PA_MAX_WAVES_PER_CU;
-    int64_t slots = (int64_t)per_cu * cus;
+    int64_t slots = 0;
+    int max_lds = 0;
+    const int rc = residency(p->fn, p->lds_bytes, &slots, &max_lds);
+    if (rc != PA_OK) return rc;
     if (slots < 1) slots = 1;
     if (slots > batch) slots = batch;
     if (slots < 1) slots = 1;
@@ -719,6 +751,21 @@ int make_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, Plan *p) {
                      round_up(2 * open_list_deep_cells(p->H, deep_from(p->H)), kWave);
     p->workspace_bytes =
         kWorkCounterBytes + (size_t)p->n_slots * p->slot_stride * 4;
+    // The visited bits in LDS as long as every query still has its wavefront at
+    // once: a test there is one LDS operation where it was a table look-up and
+    // a trip to L2 or beyond for the atomic.  (One word of table: a build for
+    // tests of the paths behind it.)  Measured with 250 000 rows (31 KB, 1024
+    // queries fit): 128-float rows, H = 128, one query 502 -> 478 us, 37 565 ->
+    // 520, 1024 710 -> 640; 64-float rows, H = 384, 37 queries 1.04 -> 0.99 ms;
+    // 500 000 rows, H = 1024, 512 queries 3.88 -> 3.63 ms.
+    const int64_t near_lds = p->lds_bytes + (int64_t)p->words_per_slot * 4;
+    if (kSeenCacheLog2 > 0 && near_lds + kStaticLds <= max_lds) {
+        const TraverseFn near_fn = pick_kernel<true>(p->H, dp);
+        int64_t near_slots = 0;
+        const int near_rc = residency(near_fn, (int)near_lds, &near_slots, &max_lds);
+        if (near_rc != PA_OK) return near_rc;
+        if (batch <= near_slots) p->fn = near_fn, p->lds_bytes = (int)near_lds;
+    }
     return PA_OK;
 }
 
