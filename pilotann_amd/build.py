@@ -4,6 +4,7 @@ source tree, where the ctypes loader looks for it."""
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -46,22 +47,19 @@ def build(verbose: bool = False, output: str = LIB,
     loader uses).  ``extra_hip_flags`` are added to the device compiles, e.g.
     ``-DPA_PHASE_TIMERS`` for the tuning build ``PHASE_LIB``."""
     include = os.path.join(ROOT, 'include')
-    objects = []
-    for name in HIP_SOURCES:
-        src = os.path.join(CSRC, name)
-        if not os.path.exists(src):
-            continue
-        obj = os.path.join(CSRC, name + '.o')
-        _run(['hipcc', *HIP_FLAGS, *extra_hip_flags, '-I', include, '-c', src,
-              '-o', obj], verbose)
-        objects.append(obj)
-    for name in CXX_SOURCES:
-        src = os.path.join(CSRC, name)
-        if not os.path.exists(src):
-            continue
-        obj = os.path.join(CSRC, name + '.o')
-        _run(['g++', *CXX_FLAGS, '-I', include, '-c', src, '-o', obj], verbose)
-        objects.append(obj)
+    compiles = []
+    for compiler, flags, names in (
+            ('hipcc', [*HIP_FLAGS, *extra_hip_flags], HIP_SOURCES),
+            ('g++', CXX_FLAGS, CXX_SOURCES)):
+        for name in names:
+            src = os.path.join(CSRC, name)
+            if os.path.exists(src):
+                compiles.append([compiler, *flags, '-I', include, '-c', src,
+                                 '-o', os.path.join(CSRC, name + '.o')])
+    # side by side: the traversal's instances take a minute by themselves
+    with ThreadPoolExecutor(max_workers=min(4, os.cpu_count() or 1)) as pool:
+        list(pool.map(lambda cmd: _run(cmd, verbose), compiles))
+    objects = [cmd[-1] for cmd in compiles]
     _run(['hipcc', '--offload-arch=gfx950', '-shared', '-fPIC', '-o', output,
           *objects, '-lgomp', '-lpthread'], verbose)
     for obj in objects:
