@@ -69,7 +69,7 @@ def _knn_graph_device(x: torch.Tensor, k: int, rows_per_pass: int = None):
     rows = kernels.HalfRows(x)
     out_i = torch.empty(n, k, dtype=torch.long, device=x.device)
     out_d = torch.empty(n, k, dtype=torch.float32, device=x.device)
-    # candidate lists of a pass: 2 * (keep + 384) * 4 bytes a row
+    # candidate lists of a pass: 8 * pa_knn_list_capacity(keep) bytes a row
     pass_rows = 1 << 21
     fused = d % 4 == 0 and d <= 4096 and rows_per_pass is None
     if rows_per_pass is None:
@@ -186,7 +186,7 @@ def insertion_order_candidates(x: torch.Tensor, pool: int, first: int = 1024):
     lo, hi = 0, min(n, first)
     while lo < n:
         # at most 2^21 rows a pass: the candidate lists of a pass are
-        # 2 * (keep + 384) * 4 bytes a row
+        # 8 * pa_knn_list_capacity(keep) bytes a row
         for a in range(lo, hi, 1 << 21):
             b = min(hi, a + (1 << 21))
             if device_path and hi > 128:
