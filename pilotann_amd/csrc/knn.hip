@@ -632,6 +632,11 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     }
 }
 
+// Nodes or rows of a launch of the kernels with a wavefront or a workgroup for
+// each: a launch holds fewer than 2^32 work-items, and 2^22 workgroups of 256
+// are 2^30.
+constexpr int64_t kLaunchNodes = 1ll << 22;
+
 // What half precision leaves of the rows: x = row * scale, clamped to the half
 // range, lo = half(x - half(x)), padded with zeros to d_pad elements and n_pad
 // rows.  A wavefront per row, four elements a lane and step, one pass over the
@@ -639,10 +644,10 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(kWave * kRankWaves) void low_kernel(
-    const float *__restrict__ rows, _Float16 *__restrict__ lo, int64_t n, int64_t n_pad, int d,
-    int d_pad, float scale, float most) {
+    const float *__restrict__ rows, _Float16 *__restrict__ lo, int64_t first, int64_t n,
+    int64_t n_pad, int d, int d_pad, float scale, float most) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t row = (int64_t)blockIdx.x * kRankWaves + threadIdx.x / kWave;
+    const int64_t row = first + (int64_t)blockIdx.x * kRankWaves + threadIdx.x / kWave;
     if (row >= n_pad) return;
     const float *src = rows + (size_t)row * d;
     for (int i = 4 * lane; i < d_pad; i += 4 * kWave) {
@@ -765,8 +770,6 @@ __global__ __launch_bounds__(256) void prune_kernel(
 // 120 000 nodes of 240 candidates of 768 floats, 48 to keep: 34.8 -> 15.0 ms
 // against all pairs on eight wavefronts with a double buffer, one workgroup
 // per compute unit; 20 011 nodes of 96 floats, 16 to keep: 2.67 -> 0.38 ms.
-constexpr int64_t kLaunchNodes = 1ll << 22;
-
 struct PruneRowsArgs {
     const _Float16 *hi, *lo;
     const float *norm;        // squared lengths of the scaled rows
@@ -1088,13 +1091,17 @@ extern "C" int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n
                            int d_pad, float scale, float most, void *stream_) {
     if (n < 0 || n_pad < n) return PA_E_SHAPE;
     if (d <= 0 || d_pad < d || d_pad % 4) return PA_E_DIM;
-    if (n_pad >= (1ll << 32) / kWave) return PA_E_RANGE;   // work-items of the launch
     if (n_pad == 0) return PA_OK;
     if ((n > 0 && !rows) || !lo_f16) return PA_E_NULL;
-    low_kernel<<<(unsigned)((n_pad + kRankWaves - 1) / kRankWaves), kWave * kRankWaves, 0,
-                 (hipStream_t)stream_>>>(rows, reinterpret_cast<_Float16 *>(lo_f16), n, n_pad, d,
-                                         d_pad, scale, most);
-    return (int)hipGetLastError();
+    for (int64_t first = 0; first < n_pad; first += kLaunchNodes) {
+        const int64_t count = n_pad - first < kLaunchNodes ? n_pad - first : kLaunchNodes;
+        low_kernel<<<(unsigned)((count + kRankWaves - 1) / kRankWaves), kWave * kRankWaves, 0,
+                     (hipStream_t)stream_>>>(rows, reinterpret_cast<_Float16 *>(lo_f16), first, n,
+                                             n_pad, d, d_pad, scale, most);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return (int)err;
+    }
+    return PA_OK;
 }
 
 extern "C" int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
