@@ -667,13 +667,14 @@ __global__ __launch_bounds__(kWave * kRankWaves) void low_kernel(
 // reached now (it becomes 2); backward: a node with a marked neighbour is
 // marked.  A node may be reached and go on within one launch, and one that two
 // wavefronts reach at a time may be gone over twice: the marks only grow, and a
-// launch that changes nothing (`changed` stays 0) is the end.  A wavefront per
+// step that changes nothing (`changed` stays 0) is the end.  A wavefront per
 // node; most nodes are one byte read.
 __global__ __launch_bounds__(256) void reach_kernel(
-    const int64_t *__restrict__ adj, unsigned char *mark, int *changed, int64_t n, int deg,
-    int backward) {
+    const int64_t *__restrict__ adj, unsigned char *mark, int *changed, int64_t first, int64_t n,
+    int deg, int backward) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t node = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const int64_t node =
+        first + (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
     if (node >= n) return;
     const int state = mark[node];
     if (backward ? state != 0 : state != 1) return;
@@ -1107,15 +1108,17 @@ extern "C" int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n
 extern "C" int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
                               int deg, int backward, int steps, void *stream_) {
     if (n < 0 || deg < 1 || steps < 1) return PA_E_SHAPE;
-    if (n >= (1ll << 32) / kWave) return PA_E_RANGE;   // work-items of a launch
     if (n == 0) return PA_OK;
     if (!mark || !changed || !adj) return PA_E_NULL;
     hipStream_t stream = (hipStream_t)stream_;
     clear_flag<<<1, 1, 0, stream>>>(changed);
-    const unsigned blocks = (unsigned)((n + 3) / 4);
-    for (int step = 0; step < steps; ++step)
-        reach_kernel<<<blocks, 256, 0, stream>>>(adj, mark, step + 1 == steps ? changed : nullptr,
-                                                 n, deg, backward);
+    for (int step = 0; step < steps; ++step) {
+        for (int64_t first = 0; first < n; first += kLaunchNodes) {
+            const int64_t count = n - first < kLaunchNodes ? n - first : kLaunchNodes;
+            reach_kernel<<<(unsigned)((count + 3) / 4), 256, 0, stream>>>(
+                adj, mark, step + 1 == steps ? changed : nullptr, first, n, deg, backward);
+        }
+    }
     return (int)hipGetLastError();
 }
 
