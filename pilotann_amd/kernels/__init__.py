@@ -369,13 +369,21 @@ class HalfRows:
         """The second half-precision part of ``rows`` (the tensor this set was
         made from): ``rows * scale - half``, same shape and padding as
         ``half``, so that ``half + low`` is the scaled row to about 22 bits."""
-        _check(rows, 'rows', 2, torch.float32, True)
-        _require(rows.shape == (self.n, self.d), 'the rows this set was made from')
+        _require(rows.dim() == 2 and rows.size(0) >= self.n and rows.size(1) == self.d,
+                 'the rows this set was made from')
+        _require(rows.device == self.half.device, 'rows.device == half.device')
+        rows = rows[:self.n]
         low = torch.empty_like(self.half)
-        with torch.cuda.device(rows.device):
-            _lib.check(_lib.lib().pa_rows_low(
-                _ptr(low), _ptr(rows), self.n, low.size(0), self.d, low.size(1),
-                float(self.scale), self.HALF_MAX, _stream()), 'pa_rows_low')
+        # strided rows go in pieces: no second copy of a large set
+        plain = rows.dtype == torch.float32 and rows.is_contiguous()
+        step = max(self.n, 1) if plain else 1 << 20
+        for lo in range(0, max(self.n, 1), step):
+            piece = rows[lo:lo + step].float().contiguous()
+            part = low[lo:] if lo + step >= self.n else low[lo:lo + step]
+            with torch.cuda.device(rows.device):
+                _lib.check(_lib.lib().pa_rows_low(
+                    _ptr(part), _ptr(piece), piece.size(0), part.size(0), self.d,
+                    low.size(1), float(self.scale), self.HALF_MAX, _stream()), 'pa_rows_low')
         return low
 
     def rows(self, lo: int, hi: int) -> 'HalfRows':
