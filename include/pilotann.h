@@ -331,14 +331,16 @@ int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n_pad, int d
 
 /*
  * Steps of a walk along the edges of adj [n * deg] (int64 node numbers, what is
- * none of 0 .. n is no edge), the connectivity pass of the graph builder
+ * negative is no edge), the connectivity pass of the graph builder
  * (faiss' part in the reference).  mark [n]: 0, or 1 at the nodes the walk
  * starts from; after enough steps it is not 0 exactly at the nodes that are
  * reached from them, or, with backward != 0, from which they are reached.
- * changed [1] receives 0 if the last of the `steps` steps reached no node (the
- * walk is over), else 1.  Device pointers; enqueued on `stream`.
+ * status [1] receives bit 0 unless the last of the `steps` steps reached no node
+ * (the walk is over), and bit 1 if a row that the walk looked at (forward: of a
+ * node it reached, backward: any) holds a number of n or more, which is no edge
+ * either.  Device pointers; enqueued on `stream`.
  */
-int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
+int pa_graph_reach(unsigned char *mark, int *status, const int64_t *adj, int64_t n,
                    int deg, int backward, int steps, void *stream);
 
 /*

@@ -662,26 +662,29 @@ __global__ __launch_bounds__(kWave * kRankWaves) void low_kernel(
     }
 }
 
-// One step of a walk along the edges of adj [n, deg] (-1: no edge) over marks of
-// one byte a node.  Forward: 1 is a node just reached, whose neighbours are
-// reached now (it becomes 2); backward: a node with a marked neighbour is
-// marked.  A node may be reached and go on within one launch, and one that two
-// wavefronts reach at a time may be gone over twice: the marks only grow, and a
-// step that changes nothing (`changed` stays 0) is the end.  A wavefront per
-// node; most nodes are one byte read.
+// One step of a walk along the edges of adj [n, deg] (negative: no edge) over
+// marks of one byte a node.  Forward: 1 is a node just reached, whose neighbours
+// are reached now (it becomes 2); backward: a node with a marked neighbour is
+// marked (2; 1 is a node the walk starts from, whose row is only looked at for
+// its numbers).  A node may be reached and go on within one launch, and one
+// that two wavefronts reach at a time may be gone over twice: the marks only
+// grow, and a step that changes nothing (bit 0 of `status` stays 0 in the
+// `last` one) is the end.  A number that is no node's is no edge and sets bit
+// 1.  A wavefront per node; most nodes are one byte read.
 __global__ __launch_bounds__(256) void reach_kernel(
-    const int64_t *__restrict__ adj, unsigned char *mark, int *changed, int64_t first, int64_t n,
-    int deg, int backward) {
+    const int64_t *__restrict__ adj, unsigned char *mark, int *status, int64_t first, int64_t n,
+    int deg, int backward, int last) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t node =
         first + (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
     if (node >= n) return;
     const int state = mark[node];
-    if (backward ? state != 0 : state != 1) return;
-    if (!backward && lane == 0) mark[node] = 2;
-    bool found = false;
+    if (backward ? state == 2 : state != 1) return;
+    if (state == 1 && lane == 0) mark[node] = 2;
+    bool found = false, beyond = false;
     for (int e = lane; e < deg; e += kWave) {
         const int64_t v = adj[(size_t)node * deg + e];
+        beyond |= v >= n;
         if (v < 0 || v >= n) continue;
         if (backward) {
             found |= mark[v] != 0;
@@ -690,11 +693,13 @@ __global__ __launch_bounds__(256) void reach_kernel(
             found = true;
         }
     }
-    if (!__ballot(found)) return;
-    if (lane == 0) {
-        if (backward) mark[node] = 1;
-        if (changed) *changed = 1;
-    }
+    const bool grown = __ballot(found) && !(backward && state == 1);
+    const int bits = (__ballot(beyond) ? 2 : 0) | (grown && last ? 1 : 0);
+    if (lane != 0) return;
+    if (backward && grown) mark[node] = 2;
+    // one wavefront's word is enough: most find the bit set
+    if (bits & ~__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicOr(status, bits);
 }
 
 __global__ void clear_flag(int *flag) { *flag = 0; }
@@ -1105,18 +1110,18 @@ extern "C" int pa_rows_low(void *lo_f16, const float *rows, int64_t n, int64_t n
     return PA_OK;
 }
 
-extern "C" int pa_graph_reach(unsigned char *mark, int *changed, const int64_t *adj, int64_t n,
+extern "C" int pa_graph_reach(unsigned char *mark, int *status, const int64_t *adj, int64_t n,
                               int deg, int backward, int steps, void *stream_) {
     if (n < 0 || deg < 1 || steps < 1) return PA_E_SHAPE;
     if (n == 0) return PA_OK;
-    if (!mark || !changed || !adj) return PA_E_NULL;
+    if (!mark || !status || !adj) return PA_E_NULL;
     hipStream_t stream = (hipStream_t)stream_;
-    clear_flag<<<1, 1, 0, stream>>>(changed);
+    clear_flag<<<1, 1, 0, stream>>>(status);
     for (int step = 0; step < steps; ++step) {
         for (int64_t first = 0; first < n; first += kLaunchNodes) {
             const int64_t count = n - first < kLaunchNodes ? n - first : kLaunchNodes;
             reach_kernel<<<(unsigned)((count + 3) / 4), 256, 0, stream>>>(
-                adj, mark, step + 1 == steps ? changed : nullptr, first, n, deg, backward);
+                adj, mark, status, first, n, deg, backward, step + 1 == steps);
         }
     }
     return (int)hipGetLastError();

@@ -506,19 +506,23 @@ def knn_nearest(rows: torch.Tensor, query: HalfRows, base: HalfRows, keep: int, 
 def graph_reachable(adj: torch.Tensor, sources: torch.Tensor, reverse: bool = False):
     """Boolean mask of the nodes a walk along the edges of ``adj`` ``[n, deg]``
     (int64 on the device, ``-1`` padded) reaches from ``sources``, or with
-    ``reverse`` of those from which a walk reaches one (``pa_graph_reach``)."""
+    ``reverse`` of those from which a walk reaches one (``pa_graph_reach``).
+    Raises where a row the walk looks at names a node that is not there."""
     _check(adj, 'adj', 2, torch.int64, True)
     n, deg = adj.shape
     mark = torch.zeros(n, dtype=torch.uint8, device=adj.device)
     mark[sources.flatten()] = 1
-    changed = torch.empty(1, dtype=torch.int32, device=adj.device)
+    status = torch.empty(1, dtype=torch.int32, device=adj.device)
     steps = 6     # a step is a short launch, looking at the flag a synchronisation
     while n:
         with torch.cuda.device(adj.device):
             _lib.check(_lib.lib().pa_graph_reach(
-                _ptr(mark), _ptr(changed), _ptr(adj), n, deg, int(bool(reverse)), steps,
+                _ptr(mark), _ptr(status), _ptr(adj), n, deg, int(bool(reverse)), steps,
                 _stream()), 'pa_graph_reach')
-        if not int(changed):
+        state = int(status)
+        if state & 2:
+            raise IndexError(f'an edge leads to a node that is not one of {n}')
+        if not state:
             break
     return mark != 0
 
