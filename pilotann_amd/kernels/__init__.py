@@ -401,13 +401,17 @@ class HalfRows:
 _KNN_RESIDENT = 256
 
 
+def _check_sets(query, base):
+    _require(query.d == base.d, 'query.size(-1) == base.size(-1)')
+    _require(query.half.device == base.half.device, 'query.device == base.device')
+    _require(base.n >= 1, 'base.size(0) >= 1')
+
+
 def _knn_lists(query, base, keep: int, n_seg: int = None):
     """``pa_knn``'s raw lists for :class:`HalfRows` ``query`` / ``base``:
     ``(score, ids, count)`` of ``[n_seg, m, capacity]``, the same and
     ``[n_seg, m]``."""
-    _require(query.d == base.d, 'query.size(-1) == base.size(-1)')
-    _require(query.half.device == base.half.device, 'query.device == base.device')
-    _require(base.n >= 1, 'base.size(0) >= 1')
+    _check_sets(query, base)
     m, n, device = query.n, base.n, base.half.device
     tile = query.tile
     blocks, tiles = -(-m // tile), -(-n // tile)
@@ -441,9 +445,10 @@ def knn_candidates(query, base, keep: int, n_seg: int = None):
     if not isinstance(query, HalfRows):
         query = HalfRows(query, scale=base.scale)
     m, device = query.n, base.half.device
-    score, ids, count = _knn_lists(query, base, keep, n_seg)
-    if m == 0:
+    if m == 0:      # whatever `keep` is
+        _check_sets(query, base)
         return torch.empty(0, keep, dtype=torch.long, device=device)
+    score, ids, count = _knn_lists(query, base, keep, n_seg)
     n_seg = score.size(0)
     score, ids = score[:, :, :keep], ids[:, :, :keep]
     valid = torch.arange(keep, device=device).view(1, 1, keep) < count.unsqueeze(-1)
