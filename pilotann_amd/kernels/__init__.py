@@ -450,11 +450,15 @@ def knn_candidates(query, base, keep: int, n_seg: int = None):
         return torch.empty(0, keep, dtype=torch.long, device=device)
     score, ids, count = _knn_lists(query, base, keep, n_seg)
     n_seg = score.size(0)
+    if n_seg == 1:
+        # the lists of many rows are large: what is not needed goes before
+        # the table is made
+        del score
+        valid = torch.arange(keep, device=device) < count[0].unsqueeze(-1)
+        return torch.where(valid, ids[0, :, :keep].long(), -1)
     score, ids = score[:, :, :keep], ids[:, :, :keep]
     valid = torch.arange(keep, device=device).view(1, 1, keep) < count.unsqueeze(-1)
-    ids = torch.where(valid, ids.long(), torch.full_like(ids, -1, dtype=torch.long))
-    if n_seg == 1:
-        return ids[0]
+    ids = torch.where(valid, ids.long(), -1)
     score = torch.where(valid, score, torch.full_like(score, float('inf')))
     score = score.permute(1, 0, 2).reshape(m, n_seg * keep)
     ids = ids.permute(1, 0, 2).reshape(m, n_seg * keep)
