@@ -310,9 +310,11 @@ int pa_knn_rerank(float *dist, const float *rows, const int64_t *cand,
  * extension either): the lists of the n_seg segments are merged (in place,
  * into the first segment's), the exact squared float32 distances of the `keep`
  * best by score are made as pa_knn_rerank makes them, and out_id / out_dist
- * [m * k] receive the k <= keep closest rows of 0 .. n, closest first; -1 / infinity where a list is shorter.  The row
- * itself has distance infinity, like a row number out of range; with hide_inf
- * such places receive -1.  `rows` [n * d], d % 4 == 0, d <= 2048; the queries
+ * [m * k] receive the k <= keep closest rows of 0 .. n, closest first (equal
+ * distances in the order of the scores where n_seg > 1, then in that of the row
+ * numbers); -1 / infinity where a list is shorter.  The row itself has distance
+ * infinity, like a row number out of range; with hide_inf such places receive
+ * -1.  `rows` [n * d], d % 4 == 0, d <= 2048; the queries
  * are rows first .. first + m.  Device pointers; enqueued on `stream`.
  */
 int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,

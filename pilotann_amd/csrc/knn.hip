@@ -565,10 +565,13 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rerank_kernel(
 // The ranking that follows knn_kernel in one pass: the distances of a row's
 // list, as rerank_kernel makes them, sorted in LDS, the k closest written out;
 // equal distances in the order of the half-precision scores where lists were
-// merged, else in the list's own order, which is mostly that of the rows.  What bounds it is the gathering of the
-// candidates' rows; the sort of 256 entries (36 passes of two exchanges a
-// lane) hides behind other wavefronts' reads, where ranking in steps of torch
-// (ids widened, top-k, gather, masks) wrote and read the table several times.
+// merged, and then in that of the rows: a candidate's place in its list is
+// where knn_kernel's wavefronts happened to put it, and two runs over the same
+// rows with equal ones among them would name them in different orders.  What
+// bounds it is the gathering of the candidates' rows; the sort of 256 entries
+// (36 passes of two exchanges a lane) hides behind other wavefronts' reads,
+// where ranking in steps of torch (ids widened, top-k, gather, masks) wrote and
+// read the table several times.
 template <int KEEP>
 __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     const float *__restrict__ rows, const float *__restrict__ cand_score,
@@ -576,6 +579,7 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     int64_t *__restrict__ out_id, float *__restrict__ out_dist, int64_t m, int64_t first,
     int64_t n, int d, int k, int hide_inf, int merged) {
     constexpr int kCap = KEEP + slack(KEEP) + kMaxBN;
+    constexpr unsigned kPlaces = 511;   // the bits of an entry that are its place in the list
     extern __shared__ __align__(16) unsigned char rank_lds[];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int64_t q = (int64_t)blockIdx.x * kRankWaves + wave;
@@ -602,7 +606,7 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
         if (place == 0 && j < cnt) {
             const unsigned score = merged ? ordered(cand_score[(size_t)q * kCap + j]) : 0u;
             entry[j] = ((unsigned long long)__float_as_uint(ok ? sum : INFINITY) << 32) |
-                       (score & ~511u) | (unsigned)j;
+                       (score & ~kPlaces) | (unsigned)j;
         }
     }
     wave_sync();
@@ -616,7 +620,10 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
                 const int i = ((t & ~(stride - 1)) << 1) | (t & (stride - 1));
                 if (KEEP / 2 >= kWave || t < KEEP / 2) {
                     const unsigned long long x = entry[i], y = entry[i | stride];
-                    if ((x > y) == ((i & size) == 0) && x != y) entry[i] = y, entry[i | stride] = x;
+                    bool after = x > y;
+                    if (x != y && (x ^ y) <= kPlaces && x != ~0ull && y != ~0ull)
+                        after = ids[x & kPlaces] > ids[y & kPlaces];
+                    if (after == ((i & size) == 0) && x != y) entry[i] = y, entry[i | stride] = x;
                 }
             }
             wave_sync();
@@ -625,7 +632,7 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     for (int i = lane; i < k; i += kWave) {
         const unsigned long long e = entry[i];
         const bool none = (unsigned)(e >> 32) == 0xffffffffu;
-        const int32_t id = none ? -1 : ids[(unsigned)e & 511u];
+        const int32_t id = none ? -1 : ids[(unsigned)e & kPlaces];
         const float dist = none ? INFINITY : __uint_as_float((unsigned)(e >> 32));
         out_id[(size_t)q * k + i] = hide_inf && isinf(dist) ? -1 : (int64_t)id;
         out_dist[(size_t)q * k + i] = dist;
