@@ -137,6 +137,34 @@ int pa_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
                 size_t workspace_bytes, uint64_t *counters, void *stream);
 
 /*
+ * pa_traverse for a launch that does not have the device to itself: `beside` is
+ * the number of queries of other launches that run at the same time (the other
+ * half of a batch on a second stream).  Same results, and the same plan: only
+ * the form of the kernel follows from it.  Visited bits in LDS (see
+ * pa_traverse_form) pay where the queries all run at once, which those of two
+ * launches that each fill the device do not: one waits for the other.  Measured
+ * for two launches on two streams, 250 000 rows of 128 floats, beam * ef = 512:
+ * 2 x 512 queries 2.21 ms in that form and 2.53 ms in the other, 2 x 640 2.69
+ * and 2.56, 2 x 1024 3.79 and 2.80 ms.  pa_traverse is this with beside = 0.
+ */
+int pa_traverse_beside(int64_t *out_I, float *out_D, const int32_t *adj,
+                       const int32_t *gid, const int64_t *mapping,
+                       const float *storage, const float *query,
+                       const int64_t *init_I, const float *init_D,
+                       int64_t batch, int64_t beside, int64_t n_nodes,
+                       int64_t n_storage, int dp, int n_init, int beam, int ef,
+                       int n_neighbors, void *workspace, size_t workspace_bytes,
+                       uint64_t *counters, void *stream);
+
+/*
+ * The form that such a launch takes: near_bits (out) is 1 where the visited bits
+ * of every query are in LDS, 0 where they are in the workspace behind a table in
+ * LDS.
+ */
+int pa_traverse_form(int64_t n_storage, int64_t batch, int64_t beside, int dp,
+                     int ef_total, int *near_bits);
+
+/*
  * pa_traverse for callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops and harnesses that forbid it).  No counterpart
  * in the reference.  Same arguments and same results as pa_traverse, without
@@ -483,6 +511,29 @@ int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
               int d_principle, int n_init, int n_buffers, int k, int ef_search,
               int sub_neighbors, int full_neighbors, void *workspace,
               size_t workspace_bytes, uint64_t *counters, void *stream);
+
+/*
+ * pa_refine for a launch that does not have the device to itself, as
+ * pa_traverse_beside is for the traversal: `beside` queries of other launches run
+ * at the same time.  Same results and the same plan; pa_refine is this with
+ * beside = 0.  Two launches on two streams, rows of 768 floats, ef_search = 128:
+ * 2 x 512 queries 1.12 ms with four wavefronts each and 1.50 ms with one, 2 x
+ * 1024 2.12 and 1.91 ms.
+ */
+int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
+                     const int64_t *init_I, float *init_D,
+                     const int32_t *sub_adj, const int32_t *sub_gid,
+                     const int64_t *sub_mapping, const int32_t *full_adj,
+                     const float *storage, const float *query, int64_t batch,
+                     int64_t beside, int64_t n_nodes, int d_model,
+                     int d_principle, int n_init, int n_buffers, int k,
+                     int ef_search, int sub_neighbors, int full_neighbors,
+                     void *workspace, size_t workspace_bytes,
+                     uint64_t *counters, void *stream);
+
+/* The form that such a launch takes: wavefronts (out), 1 or 4 per query. */
+int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, int d_model,
+                   int ef_search, int *wavefronts);
 
 #ifdef __cplusplus
 }

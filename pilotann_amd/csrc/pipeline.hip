@@ -138,12 +138,13 @@ extern "C" int pa_pipeline(
         }
         if (i < n_chunks && failure == PA_OK) {
             const int64_t lo = i * chunk_size;
-            rc = pa_traverse(s.dev_I, s.dev_D, adj, gid, mapping, storage_dev,
-                             query_dev + lo * (int64_t)d_principle,
-                             init_I + lo * n_init, init_D + lo * n_init,
-                             chunk_size, n_nodes, n_storage, d_principle, n_init,
-                             PA_BEAM_WIDTH, ef_search, n_neighbors, s.workspace,
-                             s.workspace_bytes, nullptr, s.stream);
+            // the other slot's chunk is on the device too
+            rc = pa_traverse_beside(
+                s.dev_I, s.dev_D, adj, gid, mapping, storage_dev,
+                query_dev + lo * (int64_t)d_principle, init_I + lo * n_init,
+                init_D + lo * n_init, chunk_size, n_chunks > 1 ? chunk_size : 0,
+                n_nodes, n_storage, d_principle, n_init, PA_BEAM_WIDTH, ef_search,
+                n_neighbors, s.workspace, s.workspace_bytes, nullptr, s.stream);
             hipError_t e = hipSuccess;
             if (rc == PA_OK)
                 e = hipMemcpyAsync(s.host_I, s.dev_I, cells * sizeof(int64_t),

@@ -523,8 +523,10 @@ int residency(RefineFn fn, int threads, int lds_bytes, int *slots) {
     return PA_OK;
 }
 
-int make_plan(int64_t n_nodes, int64_t batch, int d, int ef_search, Plan *p) {
-    if (n_nodes <= 0 || batch < 0) return PA_E_SHAPE;
+// `beside`: queries of other launches at the same time.  It decides about the
+// form alone: one wavefront per query never takes more slots than four.
+int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_search, Plan *p) {
+    if (n_nodes <= 0 || batch < 0 || beside < 0) return PA_E_SHAPE;
     if (n_nodes >= (1ll << 31)) return PA_E_RANGE;
     if (d <= 0 || d % 8) return PA_E_DIM;
     if (ef_search < 1 || ef_search > PA_MAX_EF_TOTAL) return PA_E_EF;
@@ -532,17 +534,18 @@ int make_plan(int64_t n_nodes, int64_t batch, int d, int ef_search, Plan *p) {
     p->sort_n = kWave;
     while (p->sort_n < p->H) p->sort_n <<= 1;
     p->lds_bytes = query_floats(d) * 4;
-    // Four wavefronts per query as long as every query has its workgroup at
-    // once (1024 queries at H <= 512).  Measured on 1M x 768, H = 32: 1 query
+    // Four wavefronts per query as long as every query, those of launches beside
+    // this one too, has its workgroup at once (1024 queries at H <= 512).  Measured on 1M x 768, H = 32: 1 query
     // 374 -> 286 us, 37 482 -> 322, 512 642 -> 447; beyond that the wavefronts
-    // that only read rows take the place of queries: 1536 910 -> 1100 us.
+    // that only read rows take the place of queries: 1536 910 -> 1100 us; two
+    // launches of 1024 at a time, H = 128, 2.12 ms with four, 1.91 with one.
     p->threads = kHelped * kWave;
     p->fn = pick_kernel<kHelped>(p->H);
     if (!p->fn) return PA_E_EF;
     int slots = 0;
     int rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
     if (rc != PA_OK) return rc;
-    if (batch > slots) {
+    if (batch > slots - beside) {
         p->threads = kWave;
         p->fn = pick_kernel<1>(p->H);
         rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
@@ -578,23 +581,31 @@ extern "C" int pa_refine_plan(int64_t n_nodes, int64_t batch, int d_model,
                               int ef_search, int *n_slots,
                               size_t *workspace_bytes) {
     Plan p;
-    const int rc = make_plan(n_nodes, batch, d_model, ef_search, &p);
+    const int rc = make_plan(n_nodes, batch, 0, d_model, ef_search, &p);
     if (rc != PA_OK) return rc;
     if (n_slots) *n_slots = p.n_slots;
     if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
     return PA_OK;
 }
 
-extern "C" int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I,
-                         float *buf_D, const int64_t *init_I, float *init_D,
-                         const int32_t *sub_adj, const int32_t *sub_gid,
-                         const int64_t *sub_mapping, const int32_t *full_adj,
-                         const float *storage, const float *query,
-                         int64_t batch, int64_t n_nodes, int d_model,
-                         int d_principle, int n_init, int n_buffers, int k,
-                         int ef_search, int sub_neighbors, int full_neighbors,
-                         void *workspace, size_t workspace_bytes,
-                         uint64_t *counters, void *stream_) {
+extern "C" int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, int d_model,
+                              int ef_search, int *wavefronts) {
+    Plan p;
+    const int rc = make_plan(n_nodes, batch, beside, d_model, ef_search, &p);
+    if (rc != PA_OK) return rc;
+    if (wavefronts) *wavefronts = p.threads / kWave;
+    return PA_OK;
+}
+
+extern "C" int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
+                                const int64_t *init_I, float *init_D, const int32_t *sub_adj,
+                                const int32_t *sub_gid, const int64_t *sub_mapping,
+                                const int32_t *full_adj, const float *storage,
+                                const float *query, int64_t batch, int64_t beside,
+                                int64_t n_nodes, int d_model, int d_principle, int n_init,
+                                int n_buffers, int k, int ef_search, int sub_neighbors,
+                                int full_neighbors, void *workspace, size_t workspace_bytes,
+                                uint64_t *counters, void *stream_) {
     if (batch < 0 || n_nodes <= 0 || n_init < 0 || n_buffers < 0 || k < 0)
         return PA_E_SHAPE;
     if (n_nodes >= (1ll << 31) || batch >= (1ll << 31)) return PA_E_RANGE;
@@ -604,7 +615,7 @@ extern "C" int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I,
     if (d_principle <= 0 || d_principle > d_model || d_principle % 8)
         return PA_E_DIM;
     Plan p;
-    const int rc = make_plan(n_nodes, batch, d_model, ef_search, &p);
+    const int rc = make_plan(n_nodes, batch, beside, d_model, ef_search, &p);
     if (rc != PA_OK) return rc;
     if (batch == 0) return PA_OK;
     if (!out_I || !out_D || !buf_I || !buf_D || !sub_adj || !sub_gid ||
@@ -637,4 +648,21 @@ extern "C" int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I,
     reset_refine_counter<<<1, 1, 0, stream>>>(a.work_counter);
     p.fn<<<p.n_slots, p.threads, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
+}
+
+extern "C" int pa_refine(int64_t *out_I, float *out_D, int64_t *buf_I,
+                         float *buf_D, const int64_t *init_I, float *init_D,
+                         const int32_t *sub_adj, const int32_t *sub_gid,
+                         const int64_t *sub_mapping, const int32_t *full_adj,
+                         const float *storage, const float *query,
+                         int64_t batch, int64_t n_nodes, int d_model,
+                         int d_principle, int n_init, int n_buffers, int k,
+                         int ef_search, int sub_neighbors, int full_neighbors,
+                         void *workspace, size_t workspace_bytes,
+                         uint64_t *counters, void *stream_) {
+    return pa_refine_beside(out_I, out_D, buf_I, buf_D, init_I, init_D, sub_adj, sub_gid,
+                            sub_mapping, full_adj, storage, query, batch, 0, n_nodes,
+                            d_model, d_principle, n_init, n_buffers, k, ef_search,
+                            sub_neighbors, full_neighbors, workspace, workspace_bytes,
+                            counters, stream_);
 }

@@ -719,10 +719,13 @@ struct Plan {
     int H, sort_n, lds_bytes, n_slots, words_per_slot, slot_stride;
     size_t workspace_bytes;
     TraverseFn fn;
+    bool near_bits;
 };
 
-int make_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, Plan *p) {
-    if (n_storage <= 0 || batch < 0) return PA_E_SHAPE;
+// `beside`: queries of other launches at the same time.  It decides about the
+// form alone; the workspace is the same.
+int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_total, Plan *p) {
+    if (n_storage <= 0 || batch < 0 || beside < 0) return PA_E_SHAPE;
     if (n_storage >= (1ll << 31)) return PA_E_RANGE;
     if (dp <= 0 || dp % 8) return PA_E_DIM;
     if (ef_total < 1 || ef_total > PA_MAX_EF_TOTAL) return PA_E_EF;
@@ -734,16 +737,15 @@ int make_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, Plan *p) {
 #ifdef PA_EXTRA_LDS  // tuning builds: lower the residency without touching code
     p->lds_bytes += PA_EXTRA_LDS;
 #endif
+    p->near_bits = false;
     p->fn = pick_kernel<false>(p->H, dp);
     if (!p->fn) return PA_E_EF;
     int64_t slots = 0;
     int max_lds = 0;
     const int rc = residency(p->fn, p->lds_bytes, &slots, &max_lds);
     if (rc != PA_OK) return rc;
-    if (slots < 1) slots = 1;
-    if (slots > batch) slots = batch;
-    if (slots < 1) slots = 1;
-    p->n_slots = (int)slots;
+    p->n_slots = (int)(slots < batch ? slots : batch);
+    if (p->n_slots < 1) p->n_slots = 1;
     p->words_per_slot = round_up((n_storage + 31) / 32, kSlotAlignWords);
     // a slot: the visited slice, the log of admitted candidates, the levels
     // of the open list that are kept in device memory (8 bytes an entry or cell)
@@ -751,20 +753,35 @@ int make_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, Plan *p) {
                      round_up(2 * open_list_deep_cells(p->H, deep_from(p->H)), kWave);
     p->workspace_bytes =
         kWorkCounterBytes + (size_t)p->n_slots * p->slot_stride * 4;
-    // The visited bits in LDS as long as every query still has its wavefront at
-    // once: a test there is one LDS operation where it was a table look-up and
-    // a trip to L2 or beyond for the atomic.  (One word of table: a build for
-    // tests of the paths behind it.)  Measured with 250 000 rows (31 KB, 1024
-    // queries fit): 128-float rows, H = 128, one query 502 -> 478 us, 37 565 ->
-    // 520, 1024 710 -> 640; 64-float rows, H = 384, 37 queries 1.04 -> 0.99 ms;
-    // 500 000 rows, H = 1024, 512 queries 3.88 -> 3.63 ms.
+    // The visited bits in LDS as long as every query, those of launches beside
+    // this one too, still has its wavefront at once: a test there is one LDS
+    // operation where it was a table look-up and a trip to L2 or beyond for the
+    // atomic.  (One word of table: a build for tests of the paths behind it.)
+    // Measured with 250 000 rows (31 KB, 1024 queries fit): 128-float rows, H =
+    // 128, one query 502 -> 478 us, 37 565 -> 520, 1024 710 -> 640; 64-float
+    // rows, H = 384, 37 queries 1.04 -> 0.99 ms; 500 000 rows, H = 1024, 512
+    // queries 3.88 -> 3.63 ms.
+    // Beside others, where only the other form has all queries at once, that
+    // one (whole searches in two halves; 100 000 rows of 64 floats, H = 512,
+    // 2 x 1500 queries 4.92 with near bits, 4.04 ms without; 75 000 rows of 40
+    // floats, H = 128, 2 x 2000 1.83 and 1.71 ms); where neither has, near bits
+    // if they leave three quarters of the queries at a time (the latter, 2 x
+    // 3000 queries, 3328 against 4096 at a time: 2.13 and 2.34 ms; 6250 rows,
+    // 2 x 5000, as many at a time: 2.03 and 2.14; the former, 2 x 2000, 2048
+    // against 3584: 5.63 and 5.56 ms).
     const int64_t near_lds = p->lds_bytes + (int64_t)p->words_per_slot * 4;
     if (kSeenCacheLog2 > 0 && near_lds + kStaticLds <= max_lds) {
         const TraverseFn near_fn = pick_kernel<true>(p->H, dp);
         int64_t near_slots = 0;
         const int near_rc = residency(near_fn, (int)near_lds, &near_slots, &max_lds);
         if (near_rc != PA_OK) return near_rc;
-        if (batch <= near_slots) p->fn = near_fn, p->lds_bytes = (int)near_lds;
+        const bool near_fits = batch <= near_slots - beside;
+        const bool far_fits = batch <= slots - beside;
+        if (near_fits ||
+            (!far_fits && batch <= near_slots && 4 * near_slots >= 3 * slots)) {
+            p->fn = near_fn, p->lds_bytes = (int)near_lds;
+            p->near_bits = true;
+        }
     }
     return PA_OK;
 }
@@ -834,10 +851,19 @@ extern "C" int pa_traverse_plan(int64_t n_storage, int64_t batch, int dp,
                                 int ef_total, int *n_slots,
                                 size_t *workspace_bytes) {
     Plan p;
-    const int rc = make_plan(n_storage, batch, dp, ef_total, &p);
+    const int rc = make_plan(n_storage, batch, 0, dp, ef_total, &p);
     if (rc != PA_OK) return rc;
     if (n_slots) *n_slots = p.n_slots;
     if (workspace_bytes) *workspace_bytes = p.workspace_bytes;
+    return PA_OK;
+}
+
+extern "C" int pa_traverse_form(int64_t n_storage, int64_t batch, int64_t beside, int dp,
+                                int ef_total, int *near_bits) {
+    Plan p;
+    const int rc = make_plan(n_storage, batch, beside, dp, ef_total, &p);
+    if (rc != PA_OK) return rc;
+    if (near_bits) *near_bits = p.near_bits;
     return PA_OK;
 }
 
@@ -853,8 +879,8 @@ int launch_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
                     const int32_t *gid, const int64_t *mapping,
                     const float *storage, const float *query,
                     const int64_t *init_I, const float *init_D, int64_t batch,
-                    int64_t n_nodes, int64_t n_storage, int dp, int n_init,
-                    int beam, int ef, int n_neighbors, void *workspace,
+                    int64_t beside, int64_t n_nodes, int64_t n_storage, int dp,
+                    int n_init, int beam, int ef, int n_neighbors, void *workspace,
                     size_t workspace_bytes, bool fit_slots, uint64_t *counters,
                     void *stream_) {
     if (batch < 0 || n_nodes <= 0 || n_init < 0 || beam < 1 || ef < 1)
@@ -863,7 +889,7 @@ int launch_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
     if (n_neighbors < 1 || n_neighbors > PA_MAX_NEIGHBORS) return PA_E_NEIGHBORS;
     if ((int64_t)beam * ef > PA_MAX_EF_TOTAL) return PA_E_EF;
     Plan p;
-    const int rc = make_plan(n_storage, batch, dp, beam * ef, &p);
+    const int rc = make_plan(n_storage, batch, beside, dp, beam * ef, &p);
     if (rc != PA_OK) return rc;
     if (batch == 0) return PA_OK;
     if (!out_I || !out_D || !adj || !gid || !mapping || !storage || !query ||
@@ -917,7 +943,21 @@ extern "C" int pa_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
                            size_t workspace_bytes, uint64_t *counters,
                            void *stream_) {
     return launch_traverse(out_I, out_D, adj, gid, mapping, storage, query,
-                           init_I, init_D, batch, n_nodes, n_storage, dp,
+                           init_I, init_D, batch, 0, n_nodes, n_storage, dp,
+                           n_init, beam, ef, n_neighbors, workspace,
+                           workspace_bytes, false, counters, stream_);
+}
+
+extern "C" int pa_traverse_beside(int64_t *out_I, float *out_D, const int32_t *adj,
+                                  const int32_t *gid, const int64_t *mapping,
+                                  const float *storage, const float *query,
+                                  const int64_t *init_I, const float *init_D,
+                                  int64_t batch, int64_t beside, int64_t n_nodes,
+                                  int64_t n_storage, int dp, int n_init, int beam, int ef,
+                                  int n_neighbors, void *workspace, size_t workspace_bytes,
+                                  uint64_t *counters, void *stream_) {
+    return launch_traverse(out_I, out_D, adj, gid, mapping, storage, query,
+                           init_I, init_D, batch, beside, n_nodes, n_storage, dp,
                            n_init, beam, ef, n_neighbors, workspace,
                            workspace_bytes, false, counters, stream_);
 }
@@ -937,7 +977,7 @@ extern "C" int pa_traverse_static(int64_t *out_I, float *out_D,
     // values are cleared by the search itself, per query: nothing of an
     // earlier call is read.
     return launch_traverse(out_I, out_D, adj, gid, mapping, storage, query,
-                           init_I, init_D, batch, n_nodes, n_storage, dp,
+                           init_I, init_D, batch, 0, n_nodes, n_storage, dp,
                            n_init, beam, ef, n_neighbors, ws,
                            PA_STATIC_SCRATCH_BYTES, true, counters, stream_);
 }

@@ -190,10 +190,13 @@ def traverse_cuda(output_I: torch.Tensor,
 
 
 def traverse_prepared(output_I, output_D, graph: PreparedGraph, storage,
-                      query, initial_I, initial_D, counters=None):
+                      query, initial_I, initial_D, counters=None, beside: int = 0):
     """:func:`traverse_cuda` on an already prepared graph (no checks beyond
     the C ABI's own).  ``storage``: plain rows (their device layout is made
-    once and cached) or :class:`PreparedRows`."""
+    once and cached) or :class:`PreparedRows`.  ``beside``: queries of other
+    launches that run at the same time on other streams, which the kernel's
+    form takes into account (``pa_traverse_beside``); the results are the
+    same."""
     lib = _lib.lib()
     storage = prepare_rows(storage).rows
     batch_size, d_model = query.shape
@@ -205,10 +208,10 @@ def traverse_prepared(output_I, output_D, graph: PreparedGraph, storage,
             graph.n_storage, batch_size, d_model, beam * ef_search, None,
             ctypes.byref(nbytes)), 'pa_traverse_plan')
         ws = _workspace(query.device, nbytes.value)
-        _lib.check(lib.pa_traverse(
+        _lib.check(lib.pa_traverse_beside(
             _ptr(output_I), _ptr(output_D), _ptr(graph.adj), _ptr(graph.gid),
             _ptr(graph.mapping), _ptr(storage), _ptr(query), _ptr(initial_I),
-            _ptr(initial_D), batch_size, graph.n_nodes, graph.n_storage,
+            _ptr(initial_D), batch_size, int(beside), graph.n_nodes, graph.n_storage,
             d_model, initial_I.size(-1), beam, ef_search, graph.n_neighbors,
             _ptr(ws), ws.numel(), _ptr(counters), _stream()), 'pa_traverse')
 
@@ -815,7 +818,7 @@ def traverse_refine_cuda(output_I: torch.Tensor,
                          query: torch.Tensor,
                          ef_search: int,
                          d_principle: int,
-                         counters: torch.Tensor = None):
+                         counters: torch.Tensor = None, beside: int = 0):
     """:func:`traverse_refine` on the device: the arguments of
     ``kernels.traverse_refine`` (``pilot_ann/kernels/__init__.py:78-94``) as
     device tensors, the two graphs in their prepared form (``subgraph`` from
@@ -823,7 +826,8 @@ def traverse_refine_cuda(output_I: torch.Tensor,
     :func:`prepare_full_graph`), the rows from :func:`prepare_rows`.  Same
     results as the host function;
     ``initial_D`` is completed in place, ``buffer_*`` may be ``initial_*``.
-    Enqueued on the current stream.  ``counters``: optional 6 int64."""
+    Enqueued on the current stream.  ``counters``: optional 6 int64.
+    ``beside`` as in :func:`traverse_prepared`."""
     _check(query, 'query', 2, torch.float32, True)
     if not isinstance(storage, PreparedRows):
         raise RuntimeError('storage must come from prepare_rows')
@@ -862,11 +866,11 @@ def traverse_refine_cuda(output_I: torch.Tensor,
             n_nodes, batch_size, d_model, int(ef_search), None,
             ctypes.byref(nbytes)), 'pa_refine_plan')
         ws = _workspace(query.device, nbytes.value)
-        _lib.check(lib.pa_refine(
+        _lib.check(lib.pa_refine_beside(
             _ptr(output_I), _ptr(output_D), _ptr(buffer_I), _ptr(buffer_D),
             _ptr(initial_I), _ptr(initial_D), _ptr(subgraph.adj),
             _ptr(subgraph.gid), _ptr(subgraph.mapping), _ptr(fullgraph.adj),
-            _ptr(storage.rows), _ptr(query), batch_size, n_nodes, d_model,
+            _ptr(storage.rows), _ptr(query), batch_size, int(beside), n_nodes, d_model,
             int(d_principle), initial_I.size(-1), buffer_I.size(-1),
             output_I.size(-1), int(ef_search), subgraph.n_neighbors,
             fullgraph.n_neighbors, _ptr(ws), ws.numel(), _ptr(counters),

@@ -299,17 +299,19 @@ class IndexStaged(nn.Module):
             self.mapping_cuda, self.storage_cuda.size(0), self.n_neighbors)
         full = self._full_prepared
 
-        traverse = (kernels.traverse_wide_prepared if traversal == 'wide'
-                    else kernels.traverse_prepared)
-
         def run(lo, hi):
-            traverse(cand_I[lo:hi], cand_D[lo:hi], sub, self.storage_cuda,
-                     query_cuda[lo:hi], EP_I[lo:hi], EP_D[lo:hi])
+            beside = batch - (hi - lo)      # queries of the other half
+            args = (cand_I[lo:hi], cand_D[lo:hi], sub, self.storage_cuda,
+                    query_cuda[lo:hi], EP_I[lo:hi], EP_D[lo:hi])
+            if traversal == 'wide':
+                kernels.traverse_wide_prepared(*args)
+            else:
+                kernels.traverse_prepared(*args, beside=beside)
             c_I, c_D = cand_I[lo:hi].flatten(1), cand_D[lo:hi].flatten(1)
             kernels.traverse_refine_cuda(
                 topk_I[lo:hi], topk_D[lo:hi], c_I, c_D, c_I, c_D, sub, full,
                 self.storage_full_cuda, query[lo:hi], ef_search,
-                self.d_principle)
+                self.d_principle, beside=beside)
 
         if batch < 2048:
             run(0, batch)
