@@ -512,8 +512,8 @@ int residency(RefineFn fn, int threads, int lds_bytes, int *slots) {
     if (it == known.end()) {
         e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess)
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void *>(fn), threads, lds_bytes);
+            e = workgroups_per_cu(reinterpret_cast<const void *>(fn), dev, threads, lds_bytes,
+                                  &per_cu);
         if (e != hipSuccess) return (int)e;
         if (per_cu < 1) per_cu = 1;
         if (per_cu > kMaxWavesPerCu) per_cu = kMaxWavesPerCu;

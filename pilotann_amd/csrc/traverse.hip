@@ -702,8 +702,8 @@ int residency(TraverseFn fn, int lds_bytes, int64_t *slots, int *max_lds) {
         if (e == hipSuccess)
             e = hipDeviceGetAttribute(&k.max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
         if (e == hipSuccess)
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &k.per_cu, reinterpret_cast<const void *>(fn), kWave, lds_bytes);
+            e = workgroups_per_cu(reinterpret_cast<const void *>(fn), dev, kWave, lds_bytes,
+                                  &k.per_cu);
         if (e != hipSuccess) return (int)e;
         // sizes of NEAR follow the index: a few stay
         if (known.size() > 4096) known.clear();
@@ -761,14 +761,15 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     // 128, one query 502 -> 478 us, 37 565 -> 520, 1024 710 -> 640; 64-float
     // rows, H = 384, 37 queries 1.04 -> 0.99 ms; 500 000 rows, H = 1024, 512
     // queries 3.88 -> 3.63 ms.
-    // Beside others, where only the other form has all queries at once, that
-    // one (whole searches in two halves; 100 000 rows of 64 floats, H = 512,
-    // 2 x 1500 queries 4.92 with near bits, 4.04 ms without; 75 000 rows of 40
-    // floats, H = 128, 2 x 2000 1.83 and 1.71 ms); where neither has, near bits
-    // if they leave three quarters of the queries at a time (the latter, 2 x
-    // 3000 queries, 3328 against 4096 at a time: 2.13 and 2.34 ms; 6250 rows,
-    // 2 x 5000, as many at a time: 2.03 and 2.14; the former, 2 x 2000, 2048
-    // against 3584: 5.63 and 5.56 ms).
+    // Where only the other form has all queries at once, that one (whole
+    // searches in two halves; 100 000 rows of 64 floats, H = 512, 2 x 1500
+    // queries 4.94 with near bits, 4.03 ms without; 75 000 rows of 40 floats, H
+    // = 128, 2 x 2000 1.83 and 1.69 ms).  Where neither has, near bits if they
+    // take no query's place, or up to a third of them and each launch runs at
+    // once (the latter, H = 256, 2 x 2500 queries, 2816 at a time against 4096:
+    // 3.41 and 3.53 ms; the former, 2 x 2000, 2048 against 3584: 5.63 and 5.56;
+    // 6250 rows of 64 floats, H = 1024, 2 x 2500, 2304 at a time in both: 9.9
+    // and 10.5 ms).
     const int64_t near_lds = p->lds_bytes + (int64_t)p->words_per_slot * 4;
     if (kSeenCacheLog2 > 0 && near_lds + kStaticLds <= max_lds) {
         const TraverseFn near_fn = pick_kernel<true>(p->H, dp);
@@ -778,7 +779,8 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
         const bool near_fits = batch <= near_slots - beside;
         const bool far_fits = batch <= slots - beside;
         if (near_fits ||
-            (!far_fits && batch <= near_slots && 4 * near_slots >= 3 * slots)) {
+            (!far_fits && (near_slots >= slots ||
+                           (batch <= near_slots && 3 * near_slots >= 2 * slots)))) {
             p->fn = near_fn, p->lds_bytes = (int)near_lds;
             p->near_bits = true;
         }
