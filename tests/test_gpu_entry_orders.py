@@ -40,6 +40,15 @@ def test_entry_orders(order, ef, n_init, problem, device):
     oracle.traverse_cpu(ref_I, ref_D, I.numpy().copy(), D.numpy().copy(),
                         p.sub_indptr.numpy(), p.sub_indices.numpy(), p.x.numpy(),
                         p.query.numpy(), 4 * ef)
-    # entries at exactly the worst distance kept may be others of that distance
+    x, query = p.x.numpy(), p.query.numpy()
+
+    def at_that_distance(b, ids, dist):
+        # an entry that was named with that distance, or a row at it
+        named = I[b][D[b] == dist].tolist()
+        rows = oracle.square_dist(query[b].copy(), x, ids.copy())
+        for node, row in zip(ids.tolist(), rows):
+            assert node in named or (int(p.mapping[node]) >= 0 and row == dist)
+    # with rounded distances, entries at exactly the worst distance kept may be
+    # others of that distance
     assert_same_search(out_I.flatten(1).cpu(), out_D.flatten(1).cpu(), ref_I, ref_D,
-                       worst_tie=lambda row, ids, dist: None)
+                       worst_tie=at_that_distance if order == 'coarse' else None)

@@ -1,5 +1,7 @@
-"""The same queries in a launch small enough for the visited bits in LDS and in
-one that is not: the same rows, bit for bit."""
+"""The same queries in a small launch and in one of more queries than run at once,
+whose wavefronts take one query after the other on the same lists and bits: the
+same rows, bit for bit.  (Both have the visited bits in LDS where these are few,
+as here; test_gpu_full_launches.py compares the two forms.)"""
 import pytest
 import torch
 

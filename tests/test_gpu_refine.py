@@ -52,23 +52,32 @@ def run_both(p, dp, ef_search, k, cand_I, cand_D, device, n_buffers=None,
     sub = kernels.prepare_graph(p.sub_indptr.to(device), p.sub_indices.to(device),
                                 p.mapping.to(device), p.nodelist.numel(), p.deg)
     full = kernels.prepare_full_graph(p.indptr.to(device), p.indices.to(device))
-    init_I, init_D = cand_I.clone(), cand_D.clone()
-    if alias:
-        buf_I, buf_D = init_I, init_D
-    else:
-        buf_I = torch.empty(B, n_buffers, dtype=torch.long, device=device)
-        buf_D = torch.empty(B, n_buffers, dtype=torch.float, device=device)
-    out_I = torch.empty(B, k, dtype=torch.long, device=device)
-    out_D = torch.empty(B, k, dtype=torch.float, device=device)
-    counters = torch.zeros(6, dtype=torch.long, device=device)
-    kernels.traverse_refine_cuda(out_I, out_D, buf_I, buf_D, init_I, init_D,
-                                 sub, full, kernels.prepare_rows(p.x.to(device)),
-                                 p.query.to(device), ef_search, dp,
-                                 counters=counters)
-    torch.cuda.synchronize()
-    got = dict(out_I=out_I.cpu().numpy(), out_D=out_D.cpu().numpy(),
-               buf_I=buf_I.cpu().numpy(), buf_D=buf_D.cpu().numpy(),
-               init_D=init_D.cpu().numpy(), counters=counters.cpu().numpy())
+    rows = kernels.prepare_rows(p.x.to(device))
+
+    def on_device(beside):
+        init_I, init_D = cand_I.clone(), cand_D.clone()
+        if alias:
+            buf_I, buf_D = init_I, init_D
+        else:
+            buf_I = torch.empty(B, n_buffers, dtype=torch.long, device=device)
+            buf_D = torch.empty(B, n_buffers, dtype=torch.float, device=device)
+        out_I = torch.empty(B, k, dtype=torch.long, device=device)
+        out_D = torch.empty(B, k, dtype=torch.float, device=device)
+        counters = torch.zeros(6, dtype=torch.long, device=device)
+        kernels.traverse_refine_cuda(out_I, out_D, buf_I, buf_D, init_I, init_D,
+                                     sub, full, rows, p.query.to(device), ef_search, dp,
+                                     counters=counters, beside=beside)
+        torch.cuda.synchronize()
+        return dict(out_I=out_I.cpu().numpy(), out_D=out_D.cpu().numpy(),
+                    buf_I=buf_I.cpu().numpy(), buf_D=buf_D.cpu().numpy(),
+                    init_D=init_D.cpu().numpy(), counters=counters.cpu().numpy())
+
+    got = on_device(0)
+    # one wavefront per query, as a launch that fills the device has it, where
+    # the call above had four: the same in every bit
+    alone = on_device(1 << 40)
+    for name in got:
+        assert np.array_equal(got[name], alone[name]), name
     ref = dict(out_I=ref_I, out_D=ref_D, buf_I=ref_buf_I, buf_D=ref_buf_D,
                init_D=ref_init_D)
     return got, ref

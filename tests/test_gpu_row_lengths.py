@@ -1,7 +1,8 @@
-"""Row lengths at the edges of how a row is read (chunks of 16 groups of eight,
-the rest in pieces of 8, 4 and 2 groups, a last odd group; a tail that starts
-at an odd group): the traversal on reduced rows without a kernel of their own
-and the refine, bit for bit the oracle's."""
+"""Row lengths at the edges of how a row is read (chunks of 16 groups of eight in
+the traversal and in the refine with one wavefront per query, of 32 in the one
+with four; the rest in pieces of 16, 8, 4 and 2 groups, a last odd group; a tail
+that starts at an odd group): the traversal on reduced rows without a kernel of
+their own and both forms of the refine, bit for bit the oracle's."""
 import numpy as np
 import pytest
 import torch
@@ -17,6 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize('d,dp', [
     (8, 8), (16, 8), (24, 16), (40, 24), (56, 40), (96, 96), (104, 72),
     (120, 104), (136, 8), (200, 120), (248, 136), (256, 248), (264, 40),
+    (384, 136), (504, 248), (520, 8), (632, 104), (760, 392), (768, 40), (768, 128),
 ])
 def test_row_lengths(d, dp, device):
     print('row lengths', d, dp, flush=True)
