@@ -460,15 +460,49 @@ struct OpenList {
     }
     // The new entry rises: along the path to the leaf, whose keys do not fall
     // from the root down, every entry with a larger key moves one level down
-    // and the new one takes the place of the highest of them.  So a node of the
-    // path with a key above k gets its parent's entry if that is above k too,
-    // else the new one, which all lanes decide at once from the lists as they
-    // were: the parents of bank A are a lane gather away, those of bank B are
-    // in lanes 32..63 of bank A, those of banks C/D in the same lane of bank B,
-    // and the walk has read the levels below.
+    // and the new one takes the place of the highest of them.  In one of two
+    // forms, of which the second leaves the register levels alone where an
+    // entry does not get that far, as most of those of long lists do not:
+    //  * all levels at once: a node of the path with a key above k gets its
+    //    parent's entry if that is above k too, else the new one, which all
+    //    lanes decide together from the lists as they were: the parents of
+    //    bank A are a lane gather away, those of bank B are in lanes 32..63 of
+    //    bank A, those of banks C/D in the same lane of bank B, and the walk has
+    //    read the levels below;
+    //  * level by level from the leaf (kByLevel, lists of 1024 cells and more),
+    //    below the registers with what the walk has read, up to the level
+    //    where the entry stays.
+    // Measured, first form / second, over a million rows of 128 floats and 400 000
+    // of 64 floats, ms: 4096 cells 10 000 queries 42.0 / 38.4 and 28.8 / 25.5, one
+    // query 6.04 / 5.38 and 4.44 / 3.98; 2048 cells 10 000 queries 24.3 / 23.6 and
+    // 15.6 / 14.8; 1024 cells 10 000 queries 10.64 / 10.63 and 4.84 / 4.74, one
+    // query 1.69 / 1.64 and 0.91 / 0.92; 768 cells as close; 256 cells one query
+    // 0.283 / 0.292 and 512 cells 0.396 / 0.412.  (Parents read again from LDS on
+    // the way up, as before the first form: 4096 cells 39.8 and 27.7.)
+    static constexpr bool kByLevel = kDepth >= 10;
     __device__ __forceinline__ void replace_leaf(const Leaf &leaf, int k, int v,
                                                  int lane) {
         if (k >= leaf.key) return;
+        if constexpr (kByLevel) {
+            int j = leaf.j;
+            // one store per level: the parent's entry while it is larger than
+            // the new key, the new entry where the rise stops
+            auto rise = [&](const int L) -> bool {
+                const int up = j >> 1;
+                const int pk = L > 8 ? leaf.low_key[L - 9] : key_of(kind(L - 1), up);
+                const int pv = L > 8 ? leaf.low_val[L - 9] : val_of(kind(L - 1), up);
+                const bool stop = pk <= k;
+                put(kind(L), j, stop ? k : pk, stop ? v : pv, lane);
+                j = up;
+                return stop;
+            };
+            if (leaf.bottom && rise(kDepth)) return;
+#pragma unroll
+            for (int L = kDepth - 1; L >= 1; --L)
+                if (rise(L)) return;
+            put(0, 1, k, v, lane);
+            return;
+        }
         const int depth = leaf.bottom ? kDepth : kDepth - 1;   // of the leaf
         // the path's end in the register levels, and its level
         int j7 = leaf.j, level = depth;
