@@ -234,6 +234,13 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
 
             PA_TIMER(0);
             open.reset(lane);
+            // Which node a key of the result list belongs to: beside it in its
+            // lane where a lane has one key, else in the log.  Measured with
+            // the log for all lists / now, rows of 768 floats: H = 32 one query
+            // 251 / 245 us, 1024 612 / 600, 10 000 5.19 / 5.06 ms (5.15 before
+            // the log); H = 64 411 / 401, 797 / 759 and 6.31 / 6.18 ms.
+            constexpr bool kBeside = S == 1;
+            int held = -1;   // kBeside: the node of the lane's key
             ResultKeys<S> res;
             res.init(H, lane);
             ResultLog log;
@@ -334,6 +341,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     const int dj = __builtin_amdgcn_readlane(dk, j);
                     if (dj >= res.worst) continue;
                     const int vj = __builtin_amdgcn_readlane(id, j);
+                    if (kBeside) held = lane == res.holder ? vj : held;
                     if (OpenList<H>::kFusedTop) {
                         // the result list's new maximum and the top of the
                         // open list's walk in one instruction stream
@@ -351,8 +359,10 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 }
                 if (admitted) {
                     n_admit += __popcll(admitted);
-                    log.append(admitted, dk, id, lane);
-                    if (log.nearly_full()) log.cut(res.worst, lane);
+                    if (!kBeside) {
+                        log.append(admitted, dk, id, lane);
+                        if (log.nearly_full()) log.cut(res.worst, lane);
+                    }
                 }
                 const int root = open.rl(open.Av, 1);
                 if (!kEarly || root != next) next = root, next_row = load_row(root);
@@ -378,10 +388,12 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     todo &= todo - 1;
                     const int dj = __builtin_amdgcn_readlane(dk, j);
                     if (dj >= res.worst) continue;
+                    if (kBeside)
+                        held = lane == res.holder ? __builtin_amdgcn_readlane(u, j) : held;
                     res.insert(dj, lane);
                     admitted |= 1ull << j;
                 }
-                if (admitted) {
+                if (admitted && !kBeside) {
                     log.append(admitted, dk, u, lane);
                     if (log.nearly_full()) log.cut(res.worst, lane);
                 }
@@ -389,33 +401,37 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
 
             // traverse_cpu.cpp:150-162: best first; with more output slots
             // than heap cells the surplus comes first, as (-1, -inf).  The
-            // set is read back from the log, every entry below the maximum
-            // and of those at it as many as make H, and sorted in the LDS the
-            // open list no longer needs.
+            // set is sorted in the LDS the open list no longer needs; from the
+            // log it takes every entry below the maximum and of those at it
+            // as many as make H.
             wave_sync();
-            ResultLog::settle();
+            if (!kBeside) ResultLog::settle();
             for (int i = lane; i < a.sort_n; i += kWave)
                 okey[i] = INFINITY, oval[i] = -1;
             wave_sync();
-            int at_worst = 0;
-            for (int base = 0; base < log.n; base += kWave) {
-                const int i = base + lane;
-                at_worst += __popcll(__ballot(i < log.n && log.entry[i].x < res.worst));
-            }
-            int at_below = 0;
-            for (int base = 0; base < log.n; base += kWave) {
-                const int i = base + lane;
-                int2 e = make_int2(0x7fffffff, -1);
-                if (i < log.n) e = log.entry[i];
-                const bool below = i < log.n && e.x < res.worst;
-                const bool tie = i < log.n && e.x == res.worst;
-                const unsigned long long mb = __ballot(below), mt = __ballot(tie);
-                int place = -1;
-                if (below) place = at_below + lane_rank(mb);
-                if (tie) place = at_worst + lane_rank(mt);
-                if (place >= 0 && place < H) okey[place] = key_to_float(e.x), oval[place] = e.y;
-                at_below += __popcll(mb);
-                at_worst += __popcll(mt);
+            if (kBeside) {
+                if (lane < H) okey[lane] = key_to_float(res.key[0]), oval[lane] = held;
+            } else {
+                int at_worst = 0;
+                for (int base = 0; base < log.n; base += kWave) {
+                    const int i = base + lane;
+                    at_worst += __popcll(__ballot(i < log.n && log.entry[i].x < res.worst));
+                }
+                int at_below = 0;
+                for (int base = 0; base < log.n; base += kWave) {
+                    const int i = base + lane;
+                    int2 e = make_int2(0x7fffffff, -1);
+                    if (i < log.n) e = log.entry[i];
+                    const bool below = i < log.n && e.x < res.worst;
+                    const bool tie = i < log.n && e.x == res.worst;
+                    const unsigned long long mb = __ballot(below), mt = __ballot(tie);
+                    int place = -1;
+                    if (below) place = at_below + lane_rank(mb);
+                    if (tie) place = at_worst + lane_rank(mt);
+                    if (place >= 0 && place < H) okey[place] = key_to_float(e.x), oval[place] = e.y;
+                    at_below += __popcll(mb);
+                    at_worst += __popcll(mt);
+                }
             }
             wave_sync();
             for (int size = 2; size <= a.sort_n; size <<= 1) {
@@ -555,8 +571,10 @@ int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_sear
     if (slots < 1) slots = 1;
     p->n_slots = slots;
     p->words_per_slot = round_up((n_nodes + 31) / 32, kSlotAlignWords);
-    // a slot: the visited slice, then the log of admitted candidates
-    p->slot_stride = p->words_per_slot + 2 * ResultLog::capacity_for(p->H);
+    // a slot: the visited slice, then the log of admitted candidates (lists of
+    // more than one key a lane)
+    p->slot_stride =
+        p->words_per_slot + (p->H > kWave ? 2 * ResultLog::capacity_for(p->H) : 0);
     p->workspace_bytes =
         kWorkCounterBytes + (size_t)p->n_slots * p->slot_stride * 4;
     return PA_OK;
