@@ -23,7 +23,8 @@
 namespace {
 
 constexpr float kInf = std::numeric_limits<float>::infinity();
-constexpr int kTile = 8;       // rows per batched distance (traverse_cpu.cpp:8: four)
+constexpr int kTile = 8;       // long rows per batched distance (traverse_cpu.cpp:8: four)
+constexpr int kWideRow = 192;  // floats of a long row
 constexpr int kRefineSteps = 2;  // traverse_cpu.cpp:9
 constexpr int kStretch = 64;   // neighbours looked at together
 constexpr int kRowLines = 8;   // cache lines of a row requested ahead
@@ -58,12 +59,18 @@ inline void square_dist_rows(float *out, const float *q, const float *storage,
     }
     for (int i = 0; i < T; ++i) out[i] = lanes_sum(acc[i]);
 }
+// Eight rows at a time from kWideRow floats on, four below: eight chains of FMAs
+// and their pointers are more than there are registers, which a short row does
+// not make up for.  100 000 random rows, ms, four / eight: 32 floats 0.24 / 0.43,
+// 96 floats 2.36 / 2.75, 128 floats 3.19 / 3.30, 200 floats 4.16 / 3.95, 768
+// floats 11.4 / 10.2; whole searches on the host the same either way.
 inline void square_dists(float *out, const float *q, const float *storage,
                          const int64_t *rows, int n, int d, int from = 0) {
     int i = 0;
-    for (; i + kTile <= n; i += kTile)
-        square_dist_rows<kTile>(out + i, q, storage, rows + i, d, from);
-    if (kTile > 4 && i + 4 <= n) square_dist_rows<4>(out + i, q, storage, rows + i, d, from), i += 4;
+    if (d - from >= kWideRow)
+        for (; i + kTile <= n; i += kTile)
+            square_dist_rows<kTile>(out + i, q, storage, rows + i, d, from);
+    for (; i + 4 <= n; i += 4) square_dist_rows<4>(out + i, q, storage, rows + i, d, from);
     if (i + 2 <= n) square_dist_rows<2>(out + i, q, storage, rows + i, d, from), i += 2;
     if (i < n) square_dist_rows<1>(out + i, q, storage, rows + i, d, from);
 }
