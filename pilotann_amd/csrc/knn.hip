@@ -42,7 +42,10 @@ constexpr int kChunk = 64;        // contraction elements staged at a time; a
 // Appended entries a list may hold beyond `keep` before it must be cut.  Lists
 // of 256 (a graph build's) take 384: half as many cuts as with 128, and a fifth
 // more entries let in by the limit of the last one (55 000 rows against 120 000
-// of 768 floats: 128 21.4, 256 15.2, 384 14.9, 512 15.4 ms).
+// of 768 floats: 128 21.4, 256 15.2, 384 14.9, 512 15.4 ms).  The others, 128
+// and 384: of 64 13.4 and 13.6 ms there and 19.9 and 20.8 for 100 000 rows against
+// 300 000 of 96 floats, of 128 14.3 and 14.2, 22.8 and 22.5; lists of 512, 21.4 and
+// 19.1, 44.1 and 37.0, keep the shorter ones for their memory (1 KB a row each).
 constexpr int slack(int keep) { return keep == 256 ? 384 : 128; }
 constexpr int kMaxBN = 256;       // the most base rows a tile has in any form
 constexpr int kRowPad = 256;      // rows the caller's arrays are padded to

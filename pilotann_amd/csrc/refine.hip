@@ -8,10 +8,12 @@
 // dimension in place (:42-62); then on the full graph from what the first one
 // kept.  Here one wavefront runs both searches of a query, with the lists of
 // the subgraph traversal (search_lists.h): the same array heap cell for cell,
-// the same exact visited set (one bit per node in the wavefront's slice of a
-// pooled bitmask, kept across the two searches), the same eight-accumulator
-// distances bit for bit.  Rows are d_model floats; a quad of lanes streams a
-// row sixteen 32-byte groups at a time.
+// the same eight-accumulator distances bit for bit, an exact visited set (an LDS
+// table; a node that finds its bucket full has a bit in the wavefront's slice of
+// a pooled bitmask), kept across the two searches.  Rows are d_model floats; a
+// quad of lanes streams a row sixteen 32-byte groups at a time.  In launches
+// whose queries all run at once three more wavefronts read a query's rows with
+// the first, 32 groups at a time.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -132,7 +134,11 @@ constexpr int kRefineChunk = WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
 // device to itself waits for its rows 58 % of the time (768 floats, H = 32):
 // 22 rows an expansion are two passes of 16, each of six trips to memory at 8
 // blocks a trip; with four wavefronts they are one pass of three trips at 16
-// blocks, which still fits the 128 registers that four wavefronts a SIMD have.
+// blocks.  Up to H = 512 that is a few registers more than the 128 that four
+// wavefronts a SIMD have (14 - 27 spilled).  Measured at H = 32, 768 floats, 1 /
+// 512 / 1024 queries: 249 / 416 / 620 us so, 247 / 408 / 735 without a spill at
+// half the queries a compute unit (for which 1024 take two rounds), 269 / 449 /
+// 629 with 8 blocks a trip.
 template <int H, int WAVES>
 __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void refine_kernel(RefineArgs a) {
     constexpr int S = (H + kWave - 1) / kWave;

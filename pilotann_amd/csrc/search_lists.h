@@ -784,7 +784,11 @@ struct Visited {
 // over a million rows, lists of 128 cells, 128-float rows 2.78 -> 2.73 ms
 // (1024 queries 0.80 -> 0.745, one query 542 -> 526 us), 64-float rows 1.67 ->
 // 1.74 ms in the traversal, whose fifth wavefront per SIMD it takes, but 0.84
-// -> 0.80 ms per 3001 queries in the wide kernel, which reads more rows a step.
+// -> 0.80 ms per 3001 queries in the wide kernel, which reads more rows a step;
+// there 128-float rows gain too, although three wavefronts per SIMD are left of
+// five and six: pools of 32 to 512, one query 116 -> 100, 208 -> 182, 562 -> 481,
+// 1468 -> 1287 us, 10 000 1.58 -> 1.52, 2.78 -> 2.69, 4.97 -> 4.81, 10.9 -> 10.6
+// ms.
 template <int DP8, bool TWO>
 __device__ __forceinline__ void eval_rows(const float *__restrict__ storage,
                                           const float *qv, const int *cand_id,

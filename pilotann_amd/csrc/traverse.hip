@@ -9,11 +9,13 @@
 //     whole wavefront advances it in lock step (uniform control flow, walks
 //     unrolled by level, scalar integer compares);
 //   * the result list is the exact set of the H best distances seen so far —
-//     what the reference's result heap holds — as a flat LDS array of which
-//     the registers track the maximum and where it sits;
-//   * the visited set is exact: one bit per storage row in a per-wavefront
-//     slice of a pooled HBM bitmask (atomic OR), behind a small LDS table of
-//     rows already known to be marked;
+//     what the reference's result heap holds — as sorted keys in registers
+//     (ResultKeys) and a log of the admitted candidates in device memory, from
+//     which the set's nodes are read back at the end (ResultLog);
+//   * the visited set is exact: one bit per storage row, in LDS where the
+//     queries of a launch all run at once with so much of it (NEAR), else in a
+//     per-wavefront slice of a pooled HBM bitmask (atomic OR), behind a small
+//     LDS table of rows already known to be marked;
 //   * a distance is the reference's eight-accumulator FMA sum
 //     (extension/inc/distance.h:31-55) bit for bit: four lanes share a row,
 //     lane a of the quad owns accumulators 2a and 2a+1 and streams its 16
@@ -21,7 +23,8 @@
 //     pa_rows_prepare: the pairs of two groups of eight interleaved by lane).
 // Expansion of a node therefore costs one coalesced row of neighbour ids, an
 // atomic for each neighbour the LDS table does not know and one coalesced
-// 4*dp-byte row per unvisited neighbour, 16 rows in flight per pass.
+// 4*dp-byte row per unvisited neighbour, 16 rows in flight per pass (32 where
+// rows are 128 floats long).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
