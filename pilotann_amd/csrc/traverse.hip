@@ -83,15 +83,17 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 // than the extra wavefront brings, so only a floor is given, under which no
 // instance has to be squeezed (the largest heaps are bounded by their LDS
 // anyway), and the allocator's own count decides the residency above it: 8 for
-// the smallest instances, 3 for 128-float rows, whose two passes of loads in
-// flight take 64 registers.  Measured for those over a million rows, three
+// the smallest instances, 3 for 128-float rows with two passes of loads in flight
+// (TWO), which take 64 registers.  Measured for those over a million rows, three
 // wavefronts (153 registers) against four (128, 22 spilled): one query, H =
-// 128, 524 -> 507 us, 5000 1.63 -> 1.51 ms, 10 000 2.80 -> 2.67 ms; with one
-// pass in flight four (99) take 2.75 and five (95) 2.74 ms.
+// 128, 524 -> 507 us, 5000 1.63 -> 1.51 ms, 10 000 2.80 -> 2.67 ms.  With one pass,
+// which is for launches that fill the device, five (95, at most 4 spilled) against
+// four (99 - 103): 500 000 rows, H = 256, 10 000 queries 3.45 -> 3.23 ms, 40 000 11.2
+// -> 10.3 ms.
 #ifdef PA_WAVES_PER_EU
 #define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
 #else
-#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (DP8 == 16 ? 3 : 4) : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
 #endif
 
 // The longest open list (4096 cells) keeps its last two levels in the
@@ -118,8 +120,9 @@ constexpr int deep_from(int H) {
 
 // NEAR: the visited bits of a query are in LDS (behind the query where that is
 // dynamic too), without a table in front of them: for launches whose queries
-// all run at once with so much LDS each (make_plan).
-template <int H, int DP8, bool NEAR>
+// all run at once with so much LDS each (make_plan).  TWO: two passes of rows are
+// read at a time.
+template <int H, int DP8, bool NEAR, bool TWO>
 __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(TraverseArgs a) {
     // One static block, in this order: the compiler then knows every LDS
     // address, and a heap cell [j - 256] is the scalar j * 8 plus a positive
@@ -299,7 +302,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 if (n > 0) {
                     if (fresh) cand_id[lane_rank(mask)] = v;
                     wave_sync();
-                    eval_rows<DP8, (DP8 >= 16)>(a.storage, qv, cand_id, cand_key, n, dp, lane);
+                    eval_rows<DP8, TWO>(a.storage, qv, cand_id, cand_key, n, dp, lane);
                     n_dist += n;
                     wave_sync();
                     PA_TIMER(3);
@@ -654,32 +657,34 @@ typedef void (*TraverseFn)(TraverseArgs);
 #endif
 constexpr int kMaxWavesPerCu = PA_MAX_WAVES_PER_CU;
 constexpr int kStaticLds = 20 << 10;   // no instance has more static LDS
+constexpr int64_t kTwoRowsBytes = 160ll << 20;   // see make_plan
 
-template <int H, bool NEAR>
+template <int H, bool NEAR, bool TWO>
 TraverseFn pick_dp(int dp) {
+    if (TWO) return dp == 128 ? traverse_kernel<H, 16, NEAR, true> : nullptr;
     switch (dp) {
-        case 32: return traverse_kernel<H, 4, NEAR>;
-        case 64: return traverse_kernel<H, 8, NEAR>;
-        case 128: return traverse_kernel<H, 16, NEAR>;
-        default: return traverse_kernel<H, 0, NEAR>;
+        case 32: return traverse_kernel<H, 4, NEAR, false>;
+        case 64: return traverse_kernel<H, 8, NEAR, false>;
+        case 128: return NEAR ? nullptr : traverse_kernel<H, 16, false, false>;
+        default: return traverse_kernel<H, 0, NEAR, false>;
     }
 }
 
-template <bool NEAR>
+template <bool NEAR, bool TWO>
 TraverseFn pick_kernel(int H, int dp) {
     switch (H) {
-        case 16: return pick_dp<16, NEAR>(dp);
-        case 32: return pick_dp<32, NEAR>(dp);
-        case 48: return pick_dp<48, NEAR>(dp);
-        case 64: return pick_dp<64, NEAR>(dp);
-        case 96: return pick_dp<96, NEAR>(dp);
-        case 128: return pick_dp<128, NEAR>(dp);
-        case 192: return pick_dp<192, NEAR>(dp);
-        case 256: return pick_dp<256, NEAR>(dp);
-        case 384: return pick_dp<384, NEAR>(dp);
-        case 512: return pick_dp<512, NEAR>(dp);
-        case 1024: return pick_dp<1024, NEAR>(dp);
-        case 2048: return pick_dp<2048, NEAR>(dp);
+        case 16: return pick_dp<16, NEAR, TWO>(dp);
+        case 32: return pick_dp<32, NEAR, TWO>(dp);
+        case 48: return pick_dp<48, NEAR, TWO>(dp);
+        case 64: return pick_dp<64, NEAR, TWO>(dp);
+        case 96: return pick_dp<96, NEAR, TWO>(dp);
+        case 128: return pick_dp<128, NEAR, TWO>(dp);
+        case 192: return pick_dp<192, NEAR, TWO>(dp);
+        case 256: return pick_dp<256, NEAR, TWO>(dp);
+        case 384: return pick_dp<384, NEAR, TWO>(dp);
+        case 512: return pick_dp<512, NEAR, TWO>(dp);
+        case 1024: return pick_dp<1024, NEAR, TWO>(dp);
+        case 2048: return pick_dp<2048, NEAR, TWO>(dp);
         default: return nullptr;
     }
 }
@@ -741,12 +746,32 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     p->lds_bytes += PA_EXTRA_LDS;
 #endif
     p->near_bits = false;
-    p->fn = pick_kernel<false>(p->H, dp);
+    p->fn = dp == 128 ? pick_kernel<false, true>(p->H, dp) : pick_kernel<false, false>(p->H, dp);
     if (!p->fn) return PA_E_EF;
     int64_t slots = 0;
     int max_lds = 0;
     const int rc = residency(p->fn, p->lds_bytes, &slots, &max_lds);
     if (rc != PA_OK) return rc;
+    // 128-float rows: two passes of reads in flight per wavefront, or one and five
+    // wavefronts per SIMD instead of three.  Two where the queries all run at
+    // once; beyond that one, if it still has them all at once and two would leave
+    // most of a second round empty, where the rows do not stay in cache, or
+    // with lists of 4096 cells (eight instead of nine wavefronts).  Measured,
+    // two passes / one, ms: 250 000 rows, H = 128, 3500 queries 1.31 / 1.24, 5000
+    // 1.49 / 1.55, 10 000 2.65 / 2.72, 40 000 9.40 / 9.70; 350 000 rows, H = 192, 5000
+    // queries 1.94 / 1.81, 40 000 10.8 / 10.0; 500 000 rows, H = 256, 5000 2.25 / 1.96,
+    // 10 000 3.70 / 3.23, 40 000 12.7 / 10.3; 250 000 rows, H = 2048, 10 000 42.0 /
+    // 37.2.  One query, one pass: 10 % slower and more.
+    if (dp == 128 && batch > slots - beside) {
+        const TraverseFn one = pick_kernel<false, false>(p->H, dp);
+        int64_t one_slots = 0;
+        const int one_rc = residency(one, p->lds_bytes, &one_slots, &max_lds);
+        if (one_rc != PA_OK) return one_rc;
+        const bool short_round =
+            batch <= one_slots - beside && batch <= 4 * slots / 3 - beside;
+        if (short_round || n_storage * 512 > kTwoRowsBytes || p->H > 1024)
+            p->fn = one, slots = one_slots;
+    }
     p->n_slots = (int)(slots < batch ? slots : batch);
     if (p->n_slots < 1) p->n_slots = 1;
     p->words_per_slot = round_up((n_storage + 31) / 32, kSlotAlignWords);
@@ -775,7 +800,8 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     // and 10.5 ms).
     const int64_t near_lds = p->lds_bytes + (int64_t)p->words_per_slot * 4;
     if (kSeenCacheLog2 > 0 && near_lds + kStaticLds <= max_lds) {
-        const TraverseFn near_fn = pick_kernel<true>(p->H, dp);
+        const TraverseFn near_fn =
+            dp == 128 ? pick_kernel<true, true>(p->H, dp) : pick_kernel<true, false>(p->H, dp);
         int64_t near_slots = 0;
         const int near_rc = residency(near_fn, (int)near_lds, &near_slots, &max_lds);
         if (near_rc != PA_OK) return near_rc;

@@ -101,6 +101,34 @@ def test_both_forms(ef, dp, graph, device):
     assert near == far
 
 
+def slots(n_storage, batch, dp, ef_total):
+    n = ctypes.c_int(-1)
+    _lib.check(_lib.lib().pa_traverse_plan(n_storage, batch, dp, ef_total, ctypes.byref(n),
+                                           None), 'pa_traverse_plan')
+    return n.value
+
+
+@pytest.fixture(scope='module')
+def large_graph():
+    """Rows of 128 floats beyond what is read in two passes when the device is full."""
+    return RandomGraph(340_000, 330_000, 128, 17, n_query=8, n_init=40, seed=9)
+
+
+@pytest.mark.parametrize('ef', [3, 8, 12, 16, 24, 32, 48, 64, 96, 128, 256, 512])
+def test_rows_one_pass_at_a_time(ef, large_graph, graph, device):
+    print('one pass at a time', ef, flush=True)
+    many, few = 40_000, large_graph.query.size(0)
+    if ef <= 128:       # more wavefronts fit than with two passes
+        assert slots(330_000, many, 128, 4 * ef) > slots(100_000, many, 128, 4 * ef)
+    assert near_bits(330_000, few, 1 << 40, 128, 4 * ef) == 0
+    two, one = large_graph.check(128, ef, device, [0, 1 << 40])
+    assert two == one
+    # and where a little more than what two passes hold is on the device
+    B = graph.query.size(0)
+    assert near_bits(graph.n_rows, B, 3500 - B, 128, 4 * ef) == 0
+    graph.check(128, ef, device, [3500 - B])
+
+
 @pytest.mark.parametrize('n', [650_000, 1_140_000])
 @pytest.mark.parametrize('ef', [4, 48, 256, 512])
 def test_bits_beyond_64_kb(n, ef, device):
