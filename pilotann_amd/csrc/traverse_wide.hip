@@ -187,7 +187,8 @@ struct Pool {
     }
 };
 
-template <int S, int DP8>
+// TWO: two passes of rows are read at a time.
+template <int S, int DP8, bool TWO>
 __global__ __launch_bounds__(kWave) void wide_kernel(WideArgs a) {
     constexpr int kCand = kMaxWidth * kWave;
     struct Lds {
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(kWave) void wide_kernel(WideArgs a) {
             }
             if (n == 0) continue;
             wave_sync();
-            eval_rows<DP8, true>(a.storage, qv, cand_id, cand_key, n, dp, lane);
+            eval_rows<DP8, TWO>(a.storage, qv, cand_id, cand_key, n, dp, lane);
             n_dist += n;
             wave_sync();
         }
@@ -391,28 +392,34 @@ __global__ __launch_bounds__(kWave) void wide_kernel(WideArgs a) {
 
 typedef void (*WideFn)(WideArgs);
 
+// `full`: the launch has more queries than run at once
 template <int S>
-WideFn pick_wide_dp(int dp) {
+WideFn pick_wide_dp(int dp, bool full) {
     switch (dp) {
-        case 32: return wide_kernel<S, 4>;
-        case 64: return wide_kernel<S, 8>;
-        case 128: return wide_kernel<S, 16>;
-        default: return wide_kernel<S, 0>;
+        case 32: return wide_kernel<S, 4, true>;
+        case 64: return wide_kernel<S, 8, true>;
+        case 128:
+            // the pool of 1024 holds four wavefronts per SIMD, with two passes
+            // two: 10 000 queries over 500 000 rows 13.9 -> 16.0 ms, 3000 4.78
+            // -> 6.31, but 1000 3.92 -> 3.61 and one 2.40 -> 2.24
+            if (S == 16 && full) return wide_kernel<S, 16, S != 16>;
+            return wide_kernel<S, 16, true>;
+        default: return wide_kernel<S, 0, false>;
     }
 }
 
 // the pool holds the ladder size of the exact mode, rounded up to whole
 // registers
-WideFn pick_wide(int H, int dp) {
+WideFn pick_wide(int H, int dp, bool full) {
     switch ((H + kWave - 1) / kWave) {
-        case 1: return pick_wide_dp<1>(dp);
-        case 2: return pick_wide_dp<2>(dp);
-        case 3: return pick_wide_dp<3>(dp);
-        case 4: return pick_wide_dp<4>(dp);
-        case 6: return pick_wide_dp<6>(dp);
-        case 8: return pick_wide_dp<8>(dp);
-        case 16: return pick_wide_dp<16>(dp);
-        case 32: return pick_wide_dp<32>(dp);
+        case 1: return pick_wide_dp<1>(dp, full);
+        case 2: return pick_wide_dp<2>(dp, full);
+        case 3: return pick_wide_dp<3>(dp, full);
+        case 4: return pick_wide_dp<4>(dp, full);
+        case 6: return pick_wide_dp<6>(dp, full);
+        case 8: return pick_wide_dp<8>(dp, full);
+        case 16: return pick_wide_dp<16>(dp, full);
+        case 32: return pick_wide_dp<32>(dp, full);
         default: return nullptr;
     }
 }
@@ -423,40 +430,52 @@ struct WidePlan {
     WideFn fn;
 };
 
+#ifndef PA_WIDE_MAX_WAVES_PER_CU
+#define PA_WIDE_MAX_WAVES_PER_CU 20
+#endif
+
+// Wavefronts of `fn` the current device holds at once.
+int wide_residency(WideFn fn, int lds_bytes, int64_t *slots) {
+    int dev = 0, cus = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    static std::mutex mutex;
+    static std::map<std::tuple<int, const void *, int>, std::pair<int, int>> known;
+    std::lock_guard<std::mutex> guard(mutex);
+    const auto key = std::make_tuple(dev, reinterpret_cast<const void *>(fn), lds_bytes);
+    auto it = known.find(key);
+    if (it == known.end()) {
+        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e == hipSuccess)
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void *>(fn), kWave, lds_bytes);
+        if (e != hipSuccess) return (int)e;
+        it = known.emplace(key, std::make_pair(cus, per_cu)).first;
+    }
+    cus = it->second.first, per_cu = it->second.second;
+    if (per_cu < 1) per_cu = 1;
+    if (per_cu > PA_WIDE_MAX_WAVES_PER_CU) per_cu = PA_WIDE_MAX_WAVES_PER_CU;
+    *slots = (int64_t)per_cu * cus;
+    return PA_OK;
+}
+
 int make_wide_plan(int64_t n_storage, int64_t batch, int dp, int ef_total, WidePlan *p) {
     if (n_storage <= 0 || batch < 0) return PA_E_SHAPE;
     if (n_storage > (int64_t)kIdMask) return PA_E_RANGE;
     if (dp <= 0 || dp % 8) return PA_E_DIM;
     if (ef_total < 1 || ef_total > PA_MAX_EF_TOTAL) return PA_E_EF;
     const int H = pa_heap_size(ef_total);
-    p->fn = pick_wide(H, dp);
+    p->fn = pick_wide(H, dp, false);
     if (!p->fn) return PA_E_EF;
     p->lds_bytes = (dp == 32 || dp == 64 || dp == 128) ? 0 : query_floats(dp) * 4;
-    int dev = 0, cus = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    {
-        static std::mutex mutex;
-        static std::map<std::tuple<int, const void *, int>, std::pair<int, int>> known;
-        std::lock_guard<std::mutex> guard(mutex);
-        const auto key = std::make_tuple(dev, reinterpret_cast<const void *>(p->fn), p->lds_bytes);
-        auto it = known.find(key);
-        if (it == known.end()) {
-            e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-            if (e == hipSuccess)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void *>(p->fn), kWave, p->lds_bytes);
-            if (e != hipSuccess) return (int)e;
-            it = known.emplace(key, std::make_pair(cus, per_cu)).first;
-        }
-        cus = it->second.first, per_cu = it->second.second;
+    int64_t slots = 0;
+    int rc = wide_residency(p->fn, p->lds_bytes, &slots);
+    if (rc != PA_OK) return rc;
+    if (batch > slots && pick_wide(H, dp, true) != p->fn) {
+        p->fn = pick_wide(H, dp, true);
+        rc = wide_residency(p->fn, p->lds_bytes, &slots);
+        if (rc != PA_OK) return rc;
     }
-    if (per_cu < 1) per_cu = 1;
-#ifndef PA_WIDE_MAX_WAVES_PER_CU
-#define PA_WIDE_MAX_WAVES_PER_CU 20
-#endif
-    if (per_cu > PA_WIDE_MAX_WAVES_PER_CU) per_cu = PA_WIDE_MAX_WAVES_PER_CU;
-    int64_t slots = (int64_t)per_cu * cus;
     if (slots > batch) slots = batch;
     if (slots < 1) slots = 1;
     p->n_slots = (int)slots;
