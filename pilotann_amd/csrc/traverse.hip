@@ -769,7 +769,10 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
         if (one_rc != PA_OK) return one_rc;
         const bool short_round =
             batch <= one_slots - beside && batch <= 4 * slots / 3 - beside;
-        if (short_round || n_storage * 512 > kTwoRowsBytes || p->H > 1024)
+        // (where LDS holds no more of them than of the other form, as with lists
+        // of 2048 cells, two: 500 000 rows, 40 000 queries 72.2 / 74.2)
+        if (one_slots > slots &&
+            (short_round || n_storage * 512 > kTwoRowsBytes || p->H > 1024))
             p->fn = one, slots = one_slots;
     }
     p->n_slots = (int)(slots < batch ? slots : batch);
