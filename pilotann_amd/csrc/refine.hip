@@ -257,7 +257,6 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
 
             // traverse_cpu.cpp:42-79: complete the entries' distances, mark
             // the entries, push them on the open list in order
-            typename OpenList<H>::Leaf leaf = open.walk_to_large_leaf();
             for (int base = 0; base < n_ent; base += kWave) {
                 const int i = base + lane;
                 int u = -1;
@@ -284,7 +283,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     wave_sync();
                 }
                 if (u >= 0) visited.mark(u);
-                open.push_entries(leaf, __ballot(u >= 0), float_to_key(dist), u, lane);
+                open.push_entries(__ballot(u >= 0), list_key(dist), u, lane);
                 PA_TIMER(2);
             }
 
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 }
                 return v;
             };
-            int next = open.rl(open.Av, 1);
+            int next = open.root_val();
             int next_row = load_row(next);
             for (int step = 0; step < max_iter; ++step) {
                 int uk, u;
@@ -324,7 +323,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 const unsigned long long mask = __ballot(fresh);
                 const int n = __popcll(mask);
                 if (kEarly || n == 0) {
-                    next = open.rl(open.Av, 1);
+                    next = open.root_val();
                     next_row = load_row(next);
                 }
                 PA_TIMER(4);
@@ -335,7 +334,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 n_dist += n;
                 wave_sync();
                 PA_TIMER(5);
-                const int dk = float_to_key(lane < n ? cand_key[lane] : INFINITY);
+                const int dk = list_key(lane < n ? cand_key[lane] : INFINITY);
                 const int id = lane < n ? cand_id[lane] : -1;
                 wave_sync();
                 // heap_update, traverse_cpu.cpp:25-39, in adjacency order
@@ -343,25 +342,12 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 unsigned long long admitted = 0;
                 while (todo) {
                     const int j = __builtin_ctzll(todo);
-                    todo &= todo - 1;
                     const int dj = __builtin_amdgcn_readlane(dk, j);
-                    if (dj >= res.worst) continue;
                     const int vj = __builtin_amdgcn_readlane(id, j);
                     if (kBeside) held = lane == res.holder ? vj : held;
-                    if (OpenList<H>::kFusedTop) {
-                        // the result list's new maximum and the top of the
-                        // open list's walk in one instruction stream
-                        const typename OpenList<H>::Choice ch = open.template choices<true>();
-                        int first = res.replace_worst(dj, lane);
-                        const int j7 = OpenList<H>::top_levels_and_wave_max(ch, first);
-                        res.set_worst(first);
-                        leaf = open.walk_below(ch, 7, j7);
-                    } else {
-                        leaf = open.walk_to_large_leaf();
-                        res.insert(dj, lane);
-                    }
-                    open.replace_leaf(leaf, dj, vj, lane);
+                    open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
                     admitted |= 1ull << j;
+                    todo &= (todo - 1) & __ballot(dk < res.worst);
                 }
                 if (admitted) {
                     n_admit += __popcll(admitted);
@@ -370,7 +356,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                         if (log.nearly_full()) log.cut(res.worst, lane);
                     }
                 }
-                const int root = open.rl(open.Av, 1);
+                const int root = open.root_val();
                 if (!kEarly || root != next) next = root, next_row = load_row(root);
                 PA_TIMER(6);
             }
@@ -386,7 +372,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     dist = eD[i];
                     if (g >= 0 && g < a.n_nodes) u = (int)g;
                 }
-                const int dk = float_to_key(dist);
+                const int dk = list_key(dist);
                 unsigned long long todo = __ballot(u >= 0 && dk < res.worst);
                 unsigned long long admitted = 0;
                 while (todo) {

@@ -24,548 +24,492 @@ constexpr int kSeenCache = 1 << kSeenCacheLog2;  // LDS words remembering visite
 // of extension/inc/heapq.cuh:13-88.  Here node i of that array is node
 // j = i + 1 (children 2j and 2j + 1), level L holds j in [2^L, 2^(L+1)).
 //
-// Levels 0..7 live in registers, one node per lane: bank A levels 0..5 (node j
-// in lane j), bank B level 6 (lane j - 64), banks C and D the left and right
-// children of level 7 (lane (j - 128) / 2), so a sibling pair is always two
-// v_readlane of known registers.  Deeper nodes sit in LDS at [j - 256] as
-// (key, value), a sibling pair per aligned 16 bytes; with DEEP the levels
-// from DEEP on sit in device memory instead (the wavefront's own region, at
-// [j - 2^DEEP], same cells): a long list then takes less LDS, more
-// wavefronts fit a compute unit, and a walk pays one memory round trip per
-// such level.  Keys are kept as
-// order-preserving integers (float_to_key) so that every comparison of a walk
-// is a scalar integer compare.  All lanes run the same, uniform, control flow; the walks
-// are unrolled by level so that each level is a dozen instructions.  After
-// each operation the heap is, cell for cell, the reference's.  Every lane
-// stores the same values to the same LDS cells and reads the same cells, so a
-// lane only ever reads back its own stores and the walks need no fences.
+// Levels 0..8 live in registers.  Bank A holds levels 0..5, node j in lane j;
+// below that every lane has a subtree of its own: node 64 + lane (bank B), its
+// children (C and D), its grandchildren (E F under C, G I under D) and, in a
+// list of 512 cells, the one node of level 9 (J, lane 0).  Longer lists have
+// the levels from 9 on in LDS at [j - 512] as (key, value), a sibling pair per
+// aligned 16 bytes; with DEEP the levels from DEEP on sit in device memory
+// instead (the wavefront's own region, at [j - 2^DEEP], same cells): a long
+// list then takes less LDS, more wavefronts fit a compute unit, and a walk pays
+// one memory round trip per such level.  Keys are kept as order-preserving
+// integers (float_to_key).  After each operation the heap is, cell for cell,
+// the reference's.
+//
+// In the registers nothing is walked.  Which child of every node a path takes
+// is decided for all nodes at once (one comparison with the sibling), a node is
+// on the path if everything above it is taken too (one lane mask and two
+// vector instructions), and every node on the path takes its parent's or its
+// child's entry in the same instructions.  What bounds it is the chain of
+// dependent instructions: a vector one takes a wavefront 4 cycles, a scalar one
+// 8, a lane gather or an LDS read 50 - 60, a value that crosses from one unit to the
+// other 12 - 20.  Measured, one wavefront, cycles for a pop / for an insert with
+// the result list's, against paths walked on the scalar unit (three instructions
+// a level) with levels 8 and on in LDS: lists of 64 cells 416 / 537 -> 204 / 288,
+// of 256 584 / 602 -> 236 / 332, of 512 695 / 669 -> 296 / 388, of 2048 860 / 911 ->
+// 541 / 745.  In the searches: 100 000 rows of 32 floats, H = 256, 128 queries 495
+// -> 405 us; a million rows, 250 000 of 128 floats, H = 128, one query 302 -> 253
+// us; 10 000 queries, rows of 64 floats, H = 256 2.60 -> 2.26 ms; H = 1024,
+// 500 000 rows of 128 floats 19.7 -> 17.7 ms.
 __device__ __forceinline__ int float_to_key(float x) {
     const int b = __float_as_int(x);
     return b ^ ((b >> 31) & 0x7fffffff);
+}
+// The key an entry has in the lists: above 0x80000000, which stands for "below
+// every key".  (That is the image of one NaN, which so counts as the key after.)
+__device__ __forceinline__ int list_key(float x) {
+    return max(float_to_key(x), (int)0x80000001);
 }
 __device__ __forceinline__ float key_to_float(int k) {
     return __int_as_float(k ^ ((k >> 31) & 0x7fffffff));
 }
 
-// c + (a != b) on the scalar unit (the compiler routes the boolean of a
-// uniform compare through a vector register otherwise).
-__device__ __forceinline__ int add_if_ne(int c, int a, int b) {
+__device__ __forceinline__ int med3(int a, int b, int c) {
     int r;
-    asm("s_cmp_lg_u32 %1, %2\n\ts_addc_u32 %0, %3, 0"
-        : "=s"(r)
-        : "s"(a), "s"(b), "s"(c)
-        : "scc");
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 
 constexpr int floor_log2(int x) { return x <= 1 ? 0 : 1 + floor_log2(x >> 1); }
 
-// c + bit `idx` of a 64-bit lane mask, on the scalar unit.
-__device__ __forceinline__ int add_if_bit(int c, unsigned long long mask, int idx) {
-    int r;
-    asm("s_bitcmp1_b64 %1, %2\n\ts_addc_u32 %0, %3, 0"
-        : "=s"(r)
-        : "s"(mask), "s"(idx), "s"(c)
-        : "scc");
-    return r;
-}
-
 // Cells of an open list of 2H cells that sit in device memory when the levels
 // from `deep` on do (0: none do).
 constexpr int open_list_deep_cells(int H, int deep) {
-    return deep >= 8 && deep <= floor_log2(2 * H) ? 2 * H + 2 - (1 << deep) : 0;
+    return deep >= 10 && deep < floor_log2(2 * H) ? 2 * H - (1 << deep) : 0;
 }
 
 template <int H, int DEEP = 0>
 struct OpenList {
     static constexpr int kSize = 2 * H;           // cells of the reference heap
     static constexpr int kDepth = floor_log2(kSize);  // deepest level
-    static constexpr int kRegNodes = 256;
+    static constexpr int kRegNodes = 512;
+    static constexpr bool kLong = kSize > kRegNodes;  // levels 9 and on in LDS
+    // the deepest level has one node (J), or, in a list of 768 cells, every other
+    static constexpr bool kOneLast = kSize == 1 << kDepth;
+    static constexpr int kEnd = kOneLast ? kDepth - 1 : kDepth;  // last level below J
     static constexpr int kDeepCells = open_list_deep_cells(H, DEEP);
     static constexpr int kDeepFrom = kDeepCells ? DEEP : kDepth + 1;
     static constexpr int kDeepBase = 1 << kDeepFrom;  // first node in device memory
-    static constexpr int kLdsCells =
-        kDeepCells ? kDeepBase - kRegNodes
-                   : (kSize + 2 > kRegNodes ? kSize + 2 - kRegNodes : 0);
+    // (the pair after the last one is for the lanes off a path)
+    static constexpr int kNowhere = kDeepCells ? kDeepBase : kOneLast ? kSize : kSize + 2;
+    static constexpr int kLdsCells = !kLong ? 0 : kNowhere + 2 - kRegNodes;
+    // The last level of the shorter lists is not complete: the lane that has its
+    // last node, a left child without a sibling.
+    static constexpr int kLast = kDepth == 5   ? kSize
+                                 : kDepth == 6 ? kSize - 64
+                                 : kDepth == 7 ? (kSize - 128) / 2
+                                 : kDepth == 8 ? (kSize - 256) / 4
+                                               : kWave;
     static constexpr int kInf = 0x7f800000;       // float_to_key(+inf)
     static constexpr int kBelowAll = (int)0x80000000;
-    static constexpr int kRegLevels = kDepth < 7 ? kDepth : 7;
-    static constexpr int kLow = kDepth - kRegLevels;  // levels below the registers
-    int Ak, Av, Bk, Bv, Ck, Cv, Dk, Dv;
-    int2 *cells;  // node j in [256, kDeepBase) at [j - 256] as (key, value); 16-byte aligned
+    static constexpr int kAboveAll = 0x7fffffff;
+
+    struct Cell {
+        int k, v;
+    };
+    Cell A, B, C, D, E, F, G, I, J;
+    int2 *cells;  // node j in [512, kDeepBase) at [j - 512] as (key, value); 16-byte aligned
     int2 *deep;   // node j >= kDeepBase at [j - kDeepBase], device memory, 16-byte aligned
+    // Lane constants (reset()).  The lanes of bank A with the nodes from level 1
+    // down to this lane's node of bank A, and down to the parent of its node of
+    // bank B.
+    int wayA_lo, wayA_hi, wayB_lo, wayB_hi;
+    int left;             // 1 in a pair's left lane, else 0
+    int tieA, tieB;       // see path()
     int4 pending;   // pop(): the requested pair of level kDeepFrom, until pop_finish()
-    int pending_j;  // its parent, 0 = nothing pending (uniform)
+    int pending_j;  // its parent, 0: nothing pending
 
     __device__ __forceinline__ static int rl(int x, int l) {
         return __builtin_amdgcn_readlane(x, l);
     }
-    // the value of another lane of a bank (taken modulo 64)
-    __device__ __forceinline__ static int of_lane(int bank, int l) {
-        return __builtin_amdgcn_ds_bpermute(l << 2, bank);
+    __device__ __forceinline__ int root_key() const { return rl(A.k, 1); }
+    __device__ __forceinline__ int root_val() const { return rl(A.v, 1); }
+    // the entry of another lane of a bank, taken modulo 64, by the lane's number
+    // times four
+    __device__ __forceinline__ static Cell of_lane(const Cell &bank, int l4) {
+        return {__builtin_amdgcn_ds_bpermute(l4, bank.k),
+                __builtin_amdgcn_ds_bpermute(l4, bank.v)};
     }
-    // A path from the root is named by its node on level 7, or by the
-    // leftmost descendant there of the node it ends in: the path's node on
-    // level L is at7 >> (7 - L).  For bank A: 7 - the level of the lane's node
-    // (lane 0, which holds none: 1, where no path matches).
-    __device__ __forceinline__ static int above7(int lane) {
-        return lane ? __builtin_clz(lane) - 24 : 1;
+    // x, made anew where it is used: one instruction instead of a register that
+    // is held through the whole search
+    __device__ __forceinline__ static int here(int x) {
+        asm volatile("" : "+v"(x));
+        return x;
     }
-    // storage class of a level: 0 bank A, 1 bank B, 2 banks C/D, 3 LDS,
-    // 4 device memory
-    __device__ __forceinline__ static constexpr int kind(int level) {
-        return level <= 5 ? 0 : level == 6 ? 1 : level == 7 ? 2
-                                           : level < kDeepFrom ? 3 : 4;
+    __device__ __forceinline__ static Cell pick(bool first, const Cell &a, const Cell &b) {
+        return {first ? a.k : b.k, first ? a.v : b.v};
+    }
+    __device__ __forceinline__ static Cell none() { return {kInf, -1}; }
+
+    static constexpr int kToBelowAll = (int)0xff800000;  // kInf less this: kBelowAll
+    static constexpr int kNoWay = 0xc;   // both children of the root: no path has them
+    // For bank A, level 1 and down: the lanes of node j and of what is above it
+    // (lane 0, which holds no node: no way).
+    __device__ __forceinline__ static unsigned long long way_to(int j) {
+        unsigned long long way = j == 0 ? kNoWay : 0;
+        for (; j > 1; j >>= 1) way |= 1ull << j;
+        return way;
     }
 
     __device__ __forceinline__ void reset(int lane) {
-        Ak = lane == 0 ? kBelowAll : kInf;  // lane 0 holds no node: the root's parent
-        Bk = Ck = Dk = kInf;
-        Av = Bv = Cv = Dv = -1;
+        const unsigned long long way = way_to(lane), way5 = way_to(32 + (lane >> 1));
+        wayA_lo = (int)way, wayA_hi = (int)(way >> 32);
+        wayB_lo = (int)way5, wayB_hi = (int)(way5 >> 32);
+        left = 1 & ~lane;
+        tieA = tieB = left;
+        if (kDepth == 5 && lane == kLast) tieA = kToBelowAll;
+        if (kDepth == 5 && lane > kLast) wayA_lo = kNoWay;
+        if (kDepth == 6 && lane == kLast) tieB = kToBelowAll;
+        if (kDepth == 6 && lane > kLast) wayB_lo = kNoWay;
+        A = B = C = D = E = F = G = I = J = none();
+        if (lane == 0) A.k = kBelowAll;  // lane 0 of bank A holds no node: the root's parent
         for (int i = lane; i < kLdsCells; i += kWave) cells[i] = make_int2(kInf, -1);
         for (int i = lane; i < kDeepCells; i += kWave) deep[i] = make_int2(kInf, -1);
         pending_j = 0;
     }
 
-    // keys (and values) of the sibling pair (c, c + 1), c even, of a level.
-    // KIND and VALS are constants once the level loops are unrolled.
-    __device__ __forceinline__ void pair(const int KIND, const bool VALS, int c,
-                                         int &ka, int &kb, int &va,
-                                         int &vb) const {
-        if (KIND == 0) {
-            ka = rl(Ak, c), kb = rl(Ak, c + 1);
-            if (VALS) va = rl(Av, c), vb = rl(Av, c + 1);
-        } else if (KIND == 1) {
-            const int l = c - 64;
-            ka = rl(Bk, l), kb = rl(Bk, l + 1);
-            if (VALS) va = rl(Bv, l), vb = rl(Bv, l + 1);
-        } else if (KIND == 2) {
-            const int l = (c - 128) >> 1;
-            ka = rl(Ck, l), kb = rl(Dk, l);
-            if (VALS) va = rl(Cv, l), vb = rl(Dv, l);
-        } else {
-            // one 16-byte read: both children with their values
-            const int4 p = KIND == 3
-                ? *reinterpret_cast<const int4 *>(cells + (c - kRegNodes))
-                : *reinterpret_cast<const int4 *>(deep + (c - kDeepBase));
-            if (VALS) va = uni(p.y), vb = uni(p.w);
-            ka = uni(p.x), kb = uni(p.z);
+    // The path from the root that takes the larger child (left on ties) or the
+    // smaller one (left on ties), for all lanes at once and without walking it.
+    // Of a pair's two in banks A and B, the left one is taken if it is not below
+    // (above) the right one, which is one integer away from "above (below)"
+    // (`left`).  Cells that the reference's heap does not have hold (inf, -1).  A
+    // pop's path may run on into them; the large leaf's must not: in banks A
+    // and B their lanes have no way, and a node without a sibling is taken because
+    // its tie constant makes the sibling's infinity smaller than every key
+    // (further down: on()).
+    struct Path {
+        int offA, offB;     // 0: all above and, in bank A, the lane's node are taken
+        bool takenB;        // the lane's node of bank B is taken
+        bool right, rightC, rightD;   // of the children of B, C, D the right one is
+    };
+    __device__ __forceinline__ static int less(int a, int b) {   // modulo 2^32
+        return (int)((unsigned)a - (unsigned)b);
+    }
+    template <bool LARGER>
+    __device__ __forceinline__ Path path() const {
+        Path w;
+        const int sa = __builtin_amdgcn_mov_dpp(A.k, 0xB1, 0xF, 0xF, true);
+        const unsigned long long not_taken =
+            __ballot(LARGER ? A.k <= less(sa, tieA) : A.k >= sa + left);
+        const int lo = (int)not_taken, hi = (int)(not_taken >> 32);
+        w.offB = 0, w.takenB = w.right = w.rightC = w.rightD = false;
+        if (kDepth >= 6) {
+            const int sb = __builtin_amdgcn_mov_dpp(B.k, 0xB1, 0xF, 0xF, true);
+            w.takenB = LARGER ? B.k > less(sb, tieB) : B.k < sb + left;
         }
-    }
-    __device__ __forceinline__ int key_of(const int KIND, int j) const {
-        if (KIND == 0) return rl(Ak, j);
-        if (KIND == 1) return rl(Bk, j - 64);
-        if (KIND == 2) {
-            // both banks are read and one result is kept: two instructions
-            // more than a branch on the parity of j would need, no branch
-            const int l = (j - 128) >> 1;
-            const int left = rl(Ck, l), right = rl(Dk, l);
-            return (j & 1) ? right : left;
+        if (kDepth >= 7) w.right = LARGER ? D.k > C.k : D.k < C.k;
+        if (kDepth >= 8 && kLast > 0) {
+            w.rightC = LARGER ? F.k > E.k : F.k < E.k;
+            w.rightD = LARGER ? I.k > G.k : I.k < G.k;
         }
-        return uni(KIND == 3 ? cells[j - kRegNodes].x : deep[j - kDeepBase].x);
+        w.offA = (hi & wayA_hi) | (lo & wayA_lo);
+        if (kDepth >= 6) w.offB = (hi & wayB_hi) | (lo & wayB_lo);
+        return w;
     }
-    __device__ __forceinline__ int val_of(const int KIND, int j) const {
-        if (KIND == 0) return rl(Av, j);
-        if (KIND == 1) return rl(Bv, j - 64);
-        if (KIND == 2) {
-            const int l = (j - 128) >> 1;
-            const int left = rl(Cv, l), right = rl(Dv, l);
-            return (j & 1) ? right : left;
-        }
-        return uni(KIND == 3 ? cells[j - kRegNodes].y : deep[j - kDeepBase].y);
-    }
-    // lane l of a key bank and of its value bank := two uniform values
-    // (v_writelane takes one scalar register besides M0, which holds the lane)
-    __device__ __forceinline__ static void set_lane(int &kbank, int &vbank, int k,
-                                                    int v, int l) {
-        asm("s_mov_b32 m0, %4\n\t"
-            "s_nop 0\n\t"
-            "v_writelane_b32 %0, %2, m0\n\t"
-            "v_writelane_b32 %1, %3, m0"
-            : "+v"(kbank), "+v"(vbank)
-            : "s"(k), "s"(v), "s"(l)
-            : "m0");
-    }
-    __device__ __forceinline__ void put(const int KIND, int j, int k, int v,
-                                        int lane) {
-        if (KIND == 0) {
-            set_lane(Ak, Av, k, v, j);
-        } else if (KIND == 1) {
-            set_lane(Bk, Bv, k, v, j - 64);
-        } else if (KIND == 2) {
-            // lane-masked selects on both banks instead of a branch on the
-            // parity of j around two v_writelane
-            const int l = (j - 128) >> 1;
-            const bool here = lane == l;
-            const bool right = j & 1;
-            Ck = (here && !right) ? k : Ck;
-            Cv = (here && !right) ? v : Cv;
-            Dk = (here && right) ? k : Dk;
-            Dv = (here && right) ? v : Dv;
-        } else if (KIND == 3) {
-            // every lane stores the same pair to the same cell: one LDS
-            // write, and no divergent branch around it
-            cells[j - kRegNodes] = make_int2(k, v);
-        } else {
-            deep[j - kDeepBase] = make_int2(k, v);
-        }
-    }
-
-    // Which child a walk takes, for every sibling pair of the register levels
-    // at once: lane-parallel compares against the sibling (one DPP move per
-    // bank), read back as lane masks, so that a level of the walk is three
-    // scalar instructions and no register read.  LARGER selects the rule of
-    // heap_replace (strictly larger right child), else that of the sift of a
-    // pop (strictly smaller right child); left wins ties in both.  In banks A
-    // and B bit i of the mask tells about the pair whose right child sits in
-    // lane i; in banks C/D lane i holds both children.
-    struct Choice {
-        unsigned long long a, b, cd;
+    // `yes` for the cells on a path, `no` for the others.
+    struct Spread {
+        int A, B, C, D, E, F, G, I, J;
     };
     template <bool LARGER>
-    __device__ __forceinline__ Choice choices() const {
-        Choice ch;
-        const int sa = __builtin_amdgcn_update_dpp(Ak, Ak, 0xB1, 0xF, 0xF, false);
-        ch.a = __ballot(LARGER ? Ak > sa : Ak < sa);
-        ch.b = 0, ch.cd = 0;
-        if (kDepth >= 6) {
-            const int sb = __builtin_amdgcn_update_dpp(Bk, Bk, 0xB1, 0xF, 0xF, false);
-            ch.b = __ballot(LARGER ? Bk > sb : Bk < sb);
+    __device__ __forceinline__ static Spread on(const Path &w, int yes, int no, int lane) {
+        Spread t;
+        t.A = w.offA == 0 ? yes : no;
+        const int taken = w.takenB ? yes : no;
+        t.B = w.offB == 0 ? taken : no;
+        t.C = w.right ? no : t.B, t.D = w.right ? t.B : no;
+        if (LARGER && kDepth == 7) {
+            t.C = lane == kLast ? t.B : lane > kLast ? no : t.C;
+            t.D = lane >= kLast ? no : t.D;
         }
-        if (kDepth >= 7) ch.cd = __ballot(LARGER ? Dk > Ck : Dk < Ck);
-        return ch;
-    }
-    // the child of j the walk takes on register level L (1..7), L < kDepth
-    // or the pair is known to be complete: 2j + (bit of the pair in the
-    // level's mask), three scalar instructions.  s_bitcmp1_b64 looks at the
-    // low six bits of its index only, so node numbers serve as lane numbers
-    // (bank B holds node j in lane j - 64, banks C/D the children of node j
-    // in lane j - 64).
-    __device__ __forceinline__ int step_down(const int L, int j,
-                                             const Choice &ch) const {
-        int r;
-        if (kind(L) <= 1) {
-            // t = 2j + 1, the right child, whose lane holds the pair's bit
-            asm("s_lshl1_add_u32 %0, %1, 1\n\t"
-                "s_bitcmp1_b64 %2, %0\n\t"
-                "s_addc_u32 %0, %0, -1"
-                : "=&s"(r)
-                : "s"(j), "s"(kind(L) == 0 ? ch.a : ch.b)
-                : "scc");
+        if (kDepth == 8 && kLast == 0) {
+            t.E = lane == 0 ? t.C : no;
+            t.F = t.G = t.I = no;
         } else {
-            asm("s_lshl_b32 %0, %1, 1\n\t"
-                "s_bitcmp1_b64 %2, %1\n\t"
-                "s_addc_u32 %0, %0, 0"
-                : "=&s"(r)
-                : "s"(j), "s"(ch.cd)
-                : "scc");
+            int c = t.C, d = t.D;
+            bool rightC = w.rightC;
+            if (LARGER && kDepth == 8) {
+                c = lane <= kLast ? c : no, d = lane < kLast ? d : no;
+                rightC = rightC && lane != kLast;
+            }
+            t.E = rightC ? no : c, t.F = rightC ? c : no;
+            t.G = w.rightD ? no : d, t.I = w.rightD ? d : no;
         }
-        return r;
+        t.J = lane == 0 ? t.E : no;
+        return t;
+    }
+    // Long lists: the lane's node on level 8 that a path through its subtree
+    // takes, and its entry.
+    __device__ __forceinline__ static int node8(const Path &w, int lane) {
+        const int under_d = w.rightD ? 3 : 2, under_c = w.rightC ? 1 : 0;
+        return 256 + 4 * lane + (w.right ? under_d : under_c);
+    }
+    __device__ __forceinline__ Cell at8(const Path &w) const {
+        return pick(w.right, pick(w.rightD, I, G), pick(w.rightC, F, E));
     }
 
+    // ---- levels below the registers: 3 LDS, 4 device memory.  A cell is only ever
+    // read and written by the lane that has the subtree it is in; lanes off a path
+    // read and write the pair kNowhere in LDS and nothing in device memory.
+
+    __device__ __forceinline__ static constexpr int kind(int level) {
+        return level < kDeepFrom ? 3 : 4;
+    }
+    // the sibling pair (c, c + 1), c even: one 16-byte read
+    __device__ __forceinline__ int4 pair(const int KIND, int c, bool on) const {
+        if (KIND == 3)
+            return *reinterpret_cast<const int4 *>(cells + ((on ? c : kNowhere) - kRegNodes));
+        int4 p = make_int4(kInf, -1, kInf, -1);
+        if (on) p = *reinterpret_cast<const int4 *>(deep + (c - kDeepBase));
+        return p;
+    }
+    __device__ __forceinline__ void put(const int KIND, int j, int k, int v, bool on) {
+        if (KIND == 3) cells[(on ? j : kNowhere) - kRegNodes] = make_int2(k, v);
+        else if (on) deep[j - kDeepBase] = make_int2(k, v);
+    }
+
+    // ---- pop
+
+    // The smaller of every sibling pair of a bank (left on ties), in the left
+    // lane of the pair.
+    __device__ __forceinline__ static Cell smaller_of_pair(const Cell &c) {
+        const Cell s = {__builtin_amdgcn_mov_dpp(c.k, 0xB1, 0xF, 0xF, true),
+                        __builtin_amdgcn_mov_dpp(c.v, 0xB1, 0xF, 0xF, true)};
+        return {min(c.k, s.k), s.k < c.k ? s.v : c.v};
+    }
     // heapq.cuh:37-45 with the sift of :13-29: the root leaves, (inf, -1)
     // sinks along the smaller child (left on ties).  The reference stops when
     // that child is (inf, -1) too; going on to the bottom instead only copies
     // (inf, -1) over (inf, -1) — every infinite cell carries -1 — so the
-    // final state is the same and the walk is straight-line code.  Levels
-    // 1..kDepth-1 are complete; on level kDepth only nodes up to kSize exist
-    // and node kSize has no sibling (its absent sibling's cell holds +inf and
-    // is never the smaller one).
+    // final state is the same.  Every node on the path takes the entry of its
+    // smaller child, the last one (inf, -1): the smaller children of bank A are
+    // a lane gather away (of bank A, of bank B for level 5), the others in the
+    // lane itself.
     __device__ __forceinline__ void pop(int lane, int &out_k, int &out_v) {
-        out_k = rl(Ak, 1);
-        out_v = rl(Av, 1);
-        const Choice ch = choices<false>();
-        // The path through the register levels first (masks only); then every
-        // lane on it takes the entry of its child on the path, all levels at
-        // once: a lane gather from bank A (levels 0..4) and one from bank B
-        // (level 5), and bank B's children are in banks C/D of the same lane.
-        int j = 1;
-        bool cut = false;  // level kDepth has no node below j
-#pragma unroll
-        for (int L = 1; L <= kRegLevels; ++L) {
-            if (L == kDepth && 2 * j > kSize) cut = true;
-            else j = step_down(L, j, ch);
+        out_k = root_key();
+        out_v = root_val();
+        const int left4 = here(lane) << 3;   // the left child's lane
+        const Cell underA = of_lane(smaller_of_pair(A), left4);
+        const Cell under5 = kDepth >= 6 ? of_lane(smaller_of_pair(B), left4) : none();
+        __builtin_amdgcn_sched_barrier(0);   // they travel while the path is found
+        const Path w = path<false>();
+        Cell under8 = none();
+        // long lists: the node on level 9 that is to be filled, and whether this
+        // lane has it
+        int j = 0;
+        bool mine = false;
+        if (kLong) {
+            j = 2 * node8(w, lane);
+            mine = w.takenB && w.offB == 0;
+            if (kDepth == 9) mine = mine && j <= kSize;
+            const int4 p = pair(kind(9), j, mine);
+            // node kSize has no sibling
+            const bool right = p.z < p.x && !(kDepth == 9 && j == kSize);
+            under8 = {right ? p.z : p.x, right ? p.w : p.y};
+            if (kDepth == 9) under8 = pick(mine, under8, none());
+            j += right;
         }
-        {
-            const int level = cut ? kRegLevels - 1 : kRegLevels;  // of j
-            const int at7 = j << (7 - level);
-            const int sh = above7(lane);
-            const int child = at7 >> (sh - 1);
-            bool here = (at7 >> sh) == lane;
-            if (kDepth <= 6) here = here && lane < (1 << level);
-            int ck = of_lane(Ak, child), cv = of_lane(Av, child);
-            if (kDepth >= 6) {
-                const int bk = of_lane(Bk, child), bv = of_lane(Bv, child);
-                ck = lane >= 32 ? bk : ck;
-                cv = lane >= 32 ? bv : cv;
-            }
-            if (kDepth >= 7) {
-                bool hereB = lane == (at7 >> 1) - 64;
-                if (kDepth == 7) hereB = hereB && !cut;
-                const bool right = Dk < Ck;
-                Bk = hereB ? (right ? Dk : Ck) : Bk;
-                Bv = hereB ? (right ? Dv : Cv) : Bv;
-            }
-            Ak = here ? ck : Ak;
-            Av = here ? cv : Av;
+        const Spread t = on<false>(w, 0, 1, lane);
+        const Cell underB = kDepth >= 7 ? pick(w.right, D, C) : none();
+        const Cell underC = kDepth >= 8 ? pick(w.rightC, F, E) : none();
+        const Cell underD = kDepth >= 8 && kLast > 0 ? pick(w.rightD, I, G) : none();
+        A = pick(t.A == 0, pick(lane >= 32, under5, underA), A);
+        if (kDepth >= 6) B = pick(t.B == 0, underB, B);
+        if (kDepth >= 7) C = pick(t.C == 0, underC, C), D = pick(t.D == 0, underD, D);
+        if (kDepth >= 8) E = pick(t.E == 0, kSize == 512 ? J : under8, E);
+        if (kDepth >= 8 && kLast > 0) {
+            F = pick(t.F == 0, under8, F);
+            G = pick(t.G == 0, under8, G);
+            I = pick(t.I == 0, under8, I);
         }
-        if (cut) {
-            put(kind(kRegLevels - 1), j, kInf, -1, lane);
-            return;
-        }
+        if (kSize == 512) J = pick(t.J == 0, none(), J);
         pending_j = 0;
-#pragma unroll
-        for (int L = kRegLevels + 1; L <= kDepth; ++L) {
-            if (L == kDepth && 2 * j > kSize) {
-                put(kind(L - 1), j, kInf, -1, lane);
-                return;
-            }
-            if (kDeepCells && L == kDeepFrom) {
-                // the pair is requested; pop_finish() goes on from here
-                pending = *reinterpret_cast<const int4 *>(deep + (2 * j - kDeepBase));
-                pending_j = j;
-                return;
-            }
-            int ka, kb, va, vb;
-            pair(kind(L), true, 2 * j, ka, kb, va, vb);
-            if (L == kDepth) kb = 2 * j == kSize ? ka : kb;
-            const int k = min(ka, kb);
-            const int v = k != ka ? vb : va;
-            const int c = add_if_ne(2 * j, k, ka);
-            put(kind(L - 1), j, k, v, lane);
-            j = c;
-        }
-        put(kind(kDepth), j, kInf, -1, lane);
+        if (kLong) pop_below(j, mine, false);
     }
-    // The levels of a pop that sit in device memory.  pop() only requests the
-    // first pair it needs from there; the caller puts the work that does not
-    // touch the list (the root is in registers) between the two, and calls
-    // this before the next walk or pop.  Nothing to do without such levels.
-    __device__ __forceinline__ void pop_finish(int lane) {
-        if (!kDeepCells) return;
-        int j = pending_j;
-        if (j == 0) return;
-        pending_j = 0;
+    // The levels from 10 on: cell j, on level 9, has given its entry away.  With
+    // levels in device memory pop() only requests the first pair it needs from
+    // there; the caller puts the work that does not touch the list (the root is
+    // in registers) between pop() and pop_finish(), which comes before the next
+    // insert or pop.
+    __device__ __forceinline__ void pop_below(int j, bool mine, const bool FINISH) {
 #pragma unroll
-        for (int L = kDeepFrom; L <= kDepth; ++L) {
-            if (L == kDepth && 2 * j > kSize) {
-                put(kind(L - 1), j, kInf, -1, lane);
-                return;
-            }
-            int ka, kb, va, vb;
-            if (L == kDeepFrom) {
-                ka = uni(pending.x), va = uni(pending.y);
-                kb = uni(pending.z), vb = uni(pending.w);
+        for (int L = FINISH ? kDeepFrom : 10; L <= kEnd; ++L) {
+            int4 p;
+            if (kDeepCells && L == kDeepFrom) {
+                if (!FINISH) {
+                    pending = pair(4, 2 * j, mine);
+                    pending_j = mine ? j : 0;
+                    return;
+                }
+                p = pending;
             } else {
-                pair(kind(L), true, 2 * j, ka, kb, va, vb);
+                p = pair(kind(L), 2 * j, mine);
             }
-            if (L == kDepth) kb = 2 * j == kSize ? ka : kb;
-            const int k = min(ka, kb);
-            const int v = k != ka ? vb : va;
-            const int c = add_if_ne(2 * j, k, ka);
-            put(kind(L - 1), j, k, v, lane);
-            j = c;
+            const bool right = p.z < p.x;
+            put(kind(L - 1), j, right ? p.z : p.x, right ? p.w : p.y, mine);
+            j = 2 * j + right;
         }
-        put(kind(kDepth), j, kInf, -1, lane);
+        const bool above = kOneLast && 2 * j == kSize;   // (a node of lane 0's)
+        put(kind(kEnd), j, above ? J.k : kInf, above ? J.v : -1, mine);
+        if (kOneLast) J = pick(above && mine, none(), J);
+    }
+    __device__ __forceinline__ void pop_finish() {
+        if (!kDeepCells || !__ballot(pending_j != 0)) return;
+        const int j = pending_j;
+        pending_j = 0;
+        pop_below(j, j != 0, true);
     }
 
+    // ---- insert
+    //
     // heapq.cuh:47-77: walk to a leaf through the larger child (left on
     // ties), overwrite it when the new key is strictly smaller, let the new
-    // entry rise.  In two parts so that the caller can put independent work
-    // between them: the walk is straight-line code, the rise branches.
-    struct Leaf {
-        int j;       // the leaf
-        int key;     // its key
-        bool bottom; // it is on level kDepth
-        // the entries of the path on levels 8 and down, as the walk read them
-        int low_key[kLow ? kLow : 1], low_val[kLow ? kLow : 1];
+    // entry rise: along the path, whose keys do not fall from the root down,
+    // every entry with a larger key moves one level down and the new one takes
+    // the place of the highest of them.  A new key that is not below the leaf's
+    // is not below any key of the path, and nothing moves.
+
+    // The parents' entries of bank A's and bank B's nodes.
+    struct Parents {
+        Cell A, B;
     };
-    __device__ __forceinline__ Leaf walk_to_large_leaf() const {
-        return walk_below(choices<true>(), 0, 1);
+    __device__ __forceinline__ Parents parents(int lane) const {
+        Parents up;
+        const int above4 = here(lane) << 1;   // (bits 0 and 1 don't count)
+        up.A = of_lane(A, above4);
+        up.B = kDepth >= 6 ? of_lane(A, above4 + 128) : none();
+        return up;
     }
-    // The walk from node j on level DONE down to a leaf (the levels above
-    // were taken elsewhere).
-    __device__ __forceinline__ Leaf walk_below(const Choice &ch, const int DONE,
-                                               int j) const {
-        Leaf leaf;
-        bool bottom = true;  // the walk reached level kDepth
-        int walked_key = 0;  // key of node j when its level is an LDS level
-#pragma unroll
-        for (int L = DONE + 1; L <= kDepth; ++L) {
-            if (L == kDepth && 2 * j > kSize) {
-                bottom = false;
-                break;
-            }
-            if (kind(L) <= 2) {
-                // node kSize has no sibling: the left child it is
-                j = (L == kDepth && 2 * j == kSize) ? 2 * j : step_down(L, j, ch);
-            } else {
-                int ka, kb, va, vb;
-                pair(kind(L), true, 2 * j, ka, kb, va, vb);
-                if (L == kDepth) kb = 2 * j == kSize ? ka : kb;
-                walked_key = max(ka, kb);
-                leaf.low_key[L - 8] = walked_key;
-                leaf.low_val[L - 8] = walked_key != ka ? vb : va;
-                j = add_if_ne(2 * j, walked_key, ka);
-            }
-        }
-        // the leaf's key: the walk has it already when the leaf is in LDS
-        leaf.j = j, leaf.bottom = bottom;
-        if (bottom)
-            leaf.key = kind(kDepth) >= 3 ? walked_key : key_of(kind(kDepth), j);
-        else
-            leaf.key = kind(kDepth - 1) >= 3 ? walked_key : key_of(kind(kDepth - 1), j);
-        return leaf;
+    // The registers.  A node on the path takes the median of its parent's key,
+    // its own and the new one, and the value that goes with that; a node off the
+    // path does the same with the largest key for the new one, which changes
+    // nothing (a parent's key is never above its child's).
+    __device__ __forceinline__ static void take(Cell &c, const Cell &up, int key, int moved) {
+        const bool moves = c.k > key;
+        c.k = med3(up.k, key, c.k);
+        c.v = moves ? moved : c.v;
     }
-    // The seven register levels of that walk (lists of 256 cells and more,
-    // where they are complete) together with a wavefront maximum of `x`,
-    // which comes back in lane 63: the six v_max_i32_dpp of the maximum each
-    // need two wait states after the one before, and the three scalar
-    // instructions of a level fill them, where apart they would be s_nop.
-    // Returns the node on level 7.
-    static constexpr bool kFusedTop = kDepth >= 8;
-    __device__ __forceinline__ static int top_levels_and_wave_max(const Choice &ch,
-                                                                  int &x) {
-        int j, t;
-        asm("s_bitcmp1_b64 %[a], 3\n\t"
-            "s_addc_u32 %[j], 2, 0\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "s_lshl1_add_u32 %[j], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[a], %[j]\n\t"
-            "s_addc_u32 %[j], %[j], -1\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-            "s_lshl1_add_u32 %[j], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[a], %[j]\n\t"
-            "s_addc_u32 %[j], %[j], -1\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-            "s_lshl1_add_u32 %[j], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[a], %[j]\n\t"
-            "s_addc_u32 %[j], %[j], -1\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] row_mirror row_mask:0xf bank_mask:0xf\n\t"
-            "s_lshl1_add_u32 %[j], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[a], %[j]\n\t"
-            "s_addc_u32 %[j], %[j], -1\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-            "s_lshl1_add_u32 %[j], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[b], %[j]\n\t"
-            "s_addc_u32 %[j], %[j], -1\n\t"
-            "v_max_i32_dpp %[x], %[x], %[x] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-            "s_lshl_b32 %[t], %[j], 1\n\t"
-            "s_bitcmp1_b64 %[cd], %[j]\n\t"
-            "s_addc_u32 %[j], %[t], 0"
-            : [j] "=&s"(j), [x] "+v"(x), [t] "=&s"(t)
-            : [a] "s"(ch.a), [b] "s"(ch.b), [cd] "s"(ch.cd)
-            : "scc");
-        return j;
+    __device__ __forceinline__ void shift(const Path &w, const Parents &up, int k, int v,
+                                          int lane) {
+        const Spread t = on<true>(w, k, kAboveAll, lane);
+        // what a node that changes takes: its parent's value or the new one
+        const int toA = up.A.k > k ? up.A.v : v, toB = up.B.k > k ? up.B.v : v;
+        const int toC = B.k > k ? B.v : v;
+        if (kDepth >= 8) {
+            const int toE = C.k > k ? C.v : v;
+            if (kSize == 512) take(J, E, t.J, E.k > k ? E.v : v);
+            take(E, C, t.E, toE);
+            if (kLast > 0) {
+                const int toG = D.k > k ? D.v : v;
+                take(F, C, t.F, toE);
+                take(G, D, t.G, toG), take(I, D, t.I, toG);
+            }
+        }
+        if (kDepth >= 7) take(C, B, t.C, toC), take(D, B, t.D, toC);
+        if (kDepth >= 6) take(B, up.B, t.B, toB);
+        take(A, up.A, t.A, toA);
     }
-    // The new entry rises: along the path to the leaf, whose keys do not fall
-    // from the root down, every entry with a larger key moves one level down
-    // and the new one takes the place of the highest of them.  In one of two
-    // forms, of which the second leaves the register levels alone where an
-    // entry does not get that far, as most of those of long lists do not:
-    //  * all levels at once: a node of the path with a key above k gets its
-    //    parent's entry if that is above k too, else the new one, which all
-    //    lanes decide together from the lists as they were: the parents of
-    //    bank A are a lane gather away, those of bank B are in lanes 32..63 of
-    //    bank A, those of banks C/D in the same lane of bank B, and the walk has
-    //    read the levels below;
-    //  * level by level from the leaf (kByLevel, lists of 1024 cells and more),
-    //    below the registers with what the walk has read, up to the level
-    //    where the entry stays.
-    // Measured, first form / second, over a million rows of 128 floats and 400 000
-    // of 64 floats, ms: 4096 cells 10 000 queries 42.0 / 38.4 and 28.8 / 25.5, one
-    // query 6.04 / 5.38 and 4.44 / 3.98; 2048 cells 10 000 queries 24.3 / 23.6 and
-    // 15.6 / 14.8; 1024 cells 10 000 queries 10.64 / 10.63 and 4.84 / 4.74, one
-    // query 1.69 / 1.64 and 0.91 / 0.92; 768 cells as close; 256 cells one query
-    // 0.283 / 0.292 and 512 cells 0.396 / 0.412.  (Parents read again from LDS on
-    // the way up, as before the first form: 4096 cells 39.8 and 27.7.)
-    static constexpr bool kByLevel = kDepth >= 10;
-    __device__ __forceinline__ void replace_leaf(const Leaf &leaf, int k, int v,
-                                                 int lane) {
-        if (k >= leaf.key) return;
-        if constexpr (kByLevel) {
-            int j = leaf.j;
-            // one store per level: the parent's entry while it is larger than
-            // the new key, the new entry where the rise stops
-            auto rise = [&](const int L) -> bool {
-                const int up = j >> 1;
-                const int pk = L > 8 ? leaf.low_key[L - 9] : key_of(kind(L - 1), up);
-                const int pv = L > 8 ? leaf.low_val[L - 9] : val_of(kind(L - 1), up);
-                const bool stop = pk <= k;
-                put(kind(L), j, stop ? k : pk, stop ? v : pv, lane);
-                j = up;
-                return stop;
-            };
-            if (leaf.bottom && rise(kDepth)) return;
+
+    // Long lists: the path below level 8, in the lane whose subtree it is in.
+    struct Low {
+        bool mine;
+        int j;        // the path's node on level kEnd
+        bool bottom;  // list of 768 cells: it has one there
+        static constexpr int kLow = kLong ? kEnd - 7 : 1;
+        Cell at[kLow];   // its entries of levels 8 .. kEnd
+    };
+    // `beside` is work of the caller's that does not touch the list, placed where
+    // the first pair travels.
+    template <class WORK>
+    __device__ __forceinline__ Low walk(const Path &w, int lane, const WORK &beside) const {
+        Low low;
+        int j = node8(w, lane);
+        low.mine = w.takenB && w.offB == 0;
+        low.bottom = low.mine && (kDepth > 9 || 2 * j <= kSize);
+        low.at[0] = at8(w);
 #pragma unroll
-            for (int L = kDepth - 1; L >= 1; --L)
-                if (rise(L)) return;
-            put(0, 1, k, v, lane);
-            return;
+        for (int L = 9; L <= kEnd; ++L) {
+            const int4 p = pair(kind(L), 2 * j, low.bottom);
+            if (L == 9) {
+                __builtin_amdgcn_sched_barrier(0);
+                beside();
+            }
+            const bool right = p.z > p.x && !(kDepth == 9 && 2 * j == kSize);
+            low.at[L - 8] = {right ? p.z : p.x, right ? p.w : p.y};
+            j = 2 * j + right;
         }
-        const int depth = leaf.bottom ? kDepth : kDepth - 1;   // of the leaf
-        // the path's end in the register levels, and its level
-        int j7 = leaf.j, level = depth;
-        if (kLow) {
-            j7 >>= depth - 7;
-            level = 7;
-            int pk = key_of(2, j7), pv = val_of(2, j7);
+        low.j = j;
+        return low;
+    }
+    // The new entry rises from a long list's leaf.  Below the registers every
+    // entry of the path is written back, moved or not, which needs no branch
+    // (in device memory: only where it moves); most entries stay there, and the
+    // registers are left alone.
+    __device__ __forceinline__ void rise(const Path &w, const Low &low, int k, int v, int lane) {
+        if (kOneLast) {
+            Cell last = J;
+            const Cell &up = low.at[kEnd - 8];
+            take(last, up, k, up.k > k ? up.v : v);
+            J = pick(low.mine && 2 * low.j == kSize, last, J);
+        }
 #pragma unroll
-            for (int L = 8; L <= kDepth; ++L) {
-                if (L == kDepth && !leaf.bottom) break;
-                const int own = leaf.low_key[L - 8];
-                const bool down = pk > k;
-                const int node = leaf.j >> (depth - L);
-                if (own > k) put(kind(L), node, down ? pk : k, down ? pv : v, lane);
-                pk = own, pv = leaf.low_val[L - 8];
-            }
+        for (int L = kEnd; L >= 9; --L) {
+            const Cell &own = low.at[L - 8], &up = low.at[L - 9];
+            const bool moves = own.k > k, down = up.k > k;
+            put(kind(L), low.j >> (kEnd - L), min(own.k, max(up.k, k)),
+                moves ? down ? up.v : v : own.v, low.bottom && (kind(L) == 3 || moves));
         }
-        const int at7 = j7 << (7 - level);
-        const int sh = above7(lane);
-        const int pAk = of_lane(Ak, lane >> 1), pAv = of_lane(Av, lane >> 1);
-        if (kDepth >= 6) {
-            const int pBk = of_lane(Ak, 32 + (lane >> 1)), pBv = of_lane(Av, 32 + (lane >> 1));
-            const int l6 = (at7 >> 1) - 64;
-            if (kDepth >= 7) {
-                const bool down = Bk > k;
-                const int nk = down ? Bk : k, nv = down ? Bv : v;
-                bool here = lane == l6;
-                if (kDepth == 7) here = here && level == 7;
-                const bool hereC = here && !(at7 & 1) && Ck > k;
-                const bool hereD = here && (at7 & 1) && Dk > k;
-                Ck = hereC ? nk : Ck;
-                Cv = hereC ? nv : Cv;
-                Dk = hereD ? nk : Dk;
-                Dv = hereD ? nv : Dv;
-            }
-            const bool down = pBk > k;
-            bool here = lane == l6 && Bk > k;
-            if (kDepth == 6) here = here && level == 6;
-            Bk = here ? (down ? pBk : k) : Bk;
-            Bv = here ? (down ? pBv : v) : Bv;
+        if (__ballot(low.mine && low.at[0].k > k)) shift(w, parents(lane), k, v, lane);
+    }
+    // The key of the leaf, for push_entries().
+    __device__ __forceinline__ int leaf_key(const Path &w, const Low &low, int lane) const {
+        int x = kBelowAll;
+        if (kLong) {
+            x = low.bottom ? low.at[kEnd - 8].k : low.at[0].k;
+            if (kOneLast) x = 2 * low.j == kSize ? J.k : x;
+            x = low.mine ? x : kBelowAll;
+        } else {
+            // the largest key of the path
+            const Spread t = on<true>(w, kAboveAll, kBelowAll, lane);
+            x = min(A.k, t.A);
+            if (kDepth >= 6) x = max(x, min(B.k, t.B));
+            if (kDepth >= 7) x = max(x, max(min(C.k, t.C), min(D.k, t.D)));
+            if (kDepth >= 8) x = max(x, min(E.k, t.E));
+            if (kDepth >= 8 && kLast > 0)
+                x = max(max(x, min(F.k, t.F)), max(min(G.k, t.G), min(I.k, t.I)));
+            if (kSize == 512) x = max(x, min(J.k, t.J));
         }
-        const bool down = pAk > k;
-        bool here = (at7 >> sh) == lane && Ak > k;
-        if (kDepth <= 5) here = here && lane < (2 << level);
-        Ak = here ? (down ? pAk : k) : Ak;
-        Av = here ? (down ? pAv : v) : Av;
+        return wave_max_key(x);
+    }
+    template <class WORK>
+    __device__ __forceinline__ void insert(int k, int v, int lane, const WORK &beside) {
+        if constexpr (kLong) {
+            const Path w = path<true>();
+            rise(w, walk(w, lane, beside), k, v, lane);
+        } else {
+            const Parents up = parents(lane);
+            __builtin_amdgcn_sched_barrier(0);
+            const Path w = path<true>();
+            beside();
+            shift(w, up, k, v, lane);
+        }
     }
     // Pushes, in lane order, the entries (k, v) of the lanes in `who`, as one
-    // replace after the other would.  `leaf` is where the walk ends in the
-    // list as it stands: an entry not below its key changes nothing, so the
-    // walk is taken again only after an entry that got in, and everything
-    // that stays out is passed over by one comparison of all lanes.  Entries
-    // mostly come in ascending order; then nearly all of them stay out (the
-    // walk follows the larger child, not the free cells).
-    __device__ __forceinline__ void push_entries(Leaf &leaf, unsigned long long who,
-                                                 int k, int v, int lane) {
-        for (;;) {
-            const unsigned long long in = who & __ballot(k < leaf.key);
+    // insert after the other would.  An entry not below the leaf's key changes
+    // nothing, so the leaf is looked for again only after an entry that got
+    // in, and everything that stays out is passed over by one comparison of all
+    // lanes.  Entries mostly come in ascending order; then nearly all of them stay
+    // out (the path follows the larger child, not the free cells).
+    __device__ __forceinline__ void push_entries(unsigned long long who, int k, int v, int lane) {
+        while (who) {
+            const Path w = path<true>();
+            Low low = {};
+            if constexpr (kLong) low = walk(w, lane, [] {});
+            const unsigned long long in = who & __ballot(k < leaf_key(w, low, lane));
             if (!in) return;
             const int j = __builtin_ctzll(in);
             who &= ~1ull << j;
-            replace_leaf(leaf, rl(k, j), rl(v, j), lane);
-            leaf = walk_to_large_leaf();
+            if constexpr (kLong) rise(w, low, rl(k, j), rl(v, j), lane);
+            else shift(w, parents(lane), rl(k, j), rl(v, j), lane);
         }
     }
 };
@@ -606,11 +550,6 @@ struct ResultKeys {
         for (int s = 0; s < S; ++s) key[s] = lane * S + s < H ? kInf : kNegInf;
         worst = kInf;
         holder = 0;
-    }
-    __device__ __forceinline__ static int med3(int a, int b, int c) {
-        int r;
-        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-        return r;
     }
     // Caller has checked k < worst.  In two parts for a caller that computes
     // the wavefront maximum of the first keys itself (`reduced`: any register

@@ -4,10 +4,9 @@
 // for step, what the reference's host search does for that query
 // (extension/traverse_cpu.cpp:12-163):
 //   * the open list is the same array heap, with the same sift rules
-//     (extension/inc/heapq.cuh:13-88): its top eight levels sit in registers
-//     (one node per lane, read with v_readlane), the rest in LDS, and the
-//     whole wavefront advances it in lock step (uniform control flow, walks
-//     unrolled by level, scalar integer compares);
+//     (extension/inc/heapq.cuh:13-88): its top nine levels sit in registers,
+//     where a pop or an insert changes a whole path at once, the rest in LDS
+//     (search_lists.h);
 //   * the result list is the exact set of the H best distances seen so far —
 //     what the reference's result heap holds — as sorted keys in registers
 //     (ResultKeys) and a log of the admitted candidates in device memory, from
@@ -87,36 +86,26 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 // (TWO), which take 64 registers.  Measured for those over a million rows, three
 // wavefronts (153 registers) against four (128, 22 spilled): one query, H =
 // 128, 524 -> 507 us, 5000 1.63 -> 1.51 ms, 10 000 2.80 -> 2.67 ms.  With one pass,
-// which is for launches that fill the device, five (95, at most 4 spilled) against
-// four (99 - 103): 500 000 rows, H = 256, 10 000 queries 3.45 -> 3.23 ms, 40 000 11.2
-// -> 10.3 ms.
+// which is for launches that fill the device, five (96, up to 15 spilled) against
+// four (103 - 115): 500 000 rows, H = 256, 10 000 queries 3.22 -> 3.10 ms, the other
+// sizes within 1 % (64-float rows at H = 256, 103 registers: four 2.24, five 2.27
+// ms, so no floor there).  H = 512 and 1024 with two passes need 172 - 183 and are
+// held to three wavefronts (168, up to 17 spilled), which LDS then allows.
 #ifdef PA_WAVES_PER_EU
 #define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
 #else
-#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 512 ? 3 : (H) <= 1024 ? (TWO ? 3 : 2) : 1, 8)))
 #endif
 
-// The longest open list (4096 cells) keeps its last two levels in the
-// wavefront's region of device memory instead of LDS (search_lists.h): first
-// level kept there, 0 = the whole list in registers and LDS.  Measured on
-// 10 000 queries over 500 000 rows of 128 floats: lists of 4096 cells run in
+// The longest open list (4096 cells) keeps level 11 in the wavefront's region of
+// device memory instead of LDS (search_lists.h): first level kept there, 0 = the
+// whole list in registers and LDS.  Measured, with one LDS level more, on 10 000 queries over 500 000 rows of 128 floats: lists of 4096 cells run in
 // 50.0 instead of 69.7 ms with level 11 on in device memory (7 instead of 4
 // wavefronts per compute unit) and in 60.4 ms with level 10 on; lists of 2048
 // cells take 23.1 ms with level 10 on in device memory against 23.4 ms
 // without (11 instead of 8 wavefronts, each as much slower) and 29.6 ms with
 // level 9 on, so they stay in LDS.
-#ifndef PA_DEEP_512
-#define PA_DEEP_512 0
-#endif
-#ifndef PA_DEEP_1024
-#define PA_DEEP_1024 0
-#endif
-#ifndef PA_DEEP_2048
-#define PA_DEEP_2048 11
-#endif
-constexpr int deep_from(int H) {
-    return H == 2048 ? PA_DEEP_2048 : H == 1024 ? PA_DEEP_1024 : H == 512 ? PA_DEEP_512 : 0;
-}
+constexpr int deep_from(int H) { return H == 2048 ? 11 : 0; }
 
 // NEAR: the visited bits of a query are in LDS (behind the query where that is
 // dynamic too), without a table in front of them: for launches whose queries
@@ -125,15 +114,18 @@ constexpr int deep_from(int H) {
 template <int H, int DP8, bool NEAR, bool TWO>
 __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(TraverseArgs a) {
     // One static block, in this order: the compiler then knows every LDS
-    // address, and a heap cell [j - 256] is the scalar j * 8 plus a positive
-    // constant that fits the instruction's offset field.
+    // address, and a heap cell [j - 512] is j * 8 plus a constant that fits the
+    // instruction's offset field.
     using Open = OpenList<H, deep_from(H)>;
     constexpr int S = (H + kWave - 1) / kWave;
     // cells of the final sort: all of them, and those sorted in LDS at once
     constexpr int kSortAll = H <= kWave ? kWave : 1 << (floor_log2(H - 1) + 1);
     constexpr int kSortLds = kSortAll > 1024 ? 1024 : kSortAll;
-    constexpr int kHeapCells =
-        Open::kLdsCells > kSortLds ? Open::kLdsCells : kSortLds;
+    // (NEAR: room for the levels from 8 on, and distances of their own: the size
+    // for which its lines in make_plan were measured)
+    constexpr int kNearCells = !NEAR ? 0 : H == 2048 ? 1792 : 2 * H > 254 ? 2 * H - 254 : 0;
+    constexpr int kListCells = Open::kLdsCells > kNearCells ? Open::kLdsCells : kNearCells;
+    constexpr int kHeapCells = kListCells > kSortLds ? kListCells : kSortLds;
     // The table of recently marked rows in front of the bitmask: half the
     // size for the long lists, whose residency is bound by LDS (lists of 2048
     // and 4096 cells: 9 instead of 8 wavefronts per compute unit, 5 % faster
@@ -145,8 +137,8 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     constexpr int kSeen = NEAR ? 4 : 1 << kSeenLog2;
     struct Lds {
         uint32_t seen_cache[kSeen];
-        int cand_id[kWave];
-        float cand_key[kWave];
+        int cand_id[kWave];   // a step's new rows, and then their distances
+        float near_key[NEAR ? kWave : 4];
         float query[DP8 ? query_floats(8 * DP8) : 4];
         int2 heap[kHeapCells];  // open list tail; the final sort reuses it
     };
@@ -159,7 +151,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     Open open;
     open.cells = lds.heap;
     int *cand_id = lds.cand_id;
-    float *cand_key = lds.cand_key;
+    float *cand_key = NEAR ? lds.near_key : reinterpret_cast<float *>(lds.cand_id);
     float *qv = DP8 ? lds.query : query_any_length;
     const int dp = DP8 ? DP8 * 8 : a.dp;
     uint32_t *seen_cache = lds.seen_cache;
@@ -216,7 +208,6 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         // is popped, and costs a step, like any other.
         const int64_t *eI = a.init_I + (size_t)q * a.n_init;
         const float *eD = a.init_D + (size_t)q * a.n_init;
-        typename Open::Leaf leaf = open.walk_to_large_leaf();
         for (int base = 0; base < a.n_init; base += kWave) {
             const int i = base + lane;
             int u = -1, row = -1;
@@ -235,7 +226,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                     }
                 }
             }
-            open.push_entries(leaf, __ballot(u >= 0), float_to_key(d),
+            open.push_entries(__ballot(u >= 0), list_key(d),
                               row >= 0 ? row : -2 - i, lane);
         }
 
@@ -282,12 +273,12 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
             }
             return before;
         };
-        int v = load_row(Open::rl(open.Av, 1));
+        int v = load_row(open.root_val());
         uint32_t before = test_and_set(v);
         for (int step = 0; step < a.max_iter; ++step) {
             int uk, u;
             open.pop(lane, uk, u);
-            const int likely = Open::rl(open.Av, 1);
+            const int likely = open.root_val();
             const int likely_row = load_row(likely);
             PA_TIMER(0);
             if (u == -1 || uk >= res.worst) break;
@@ -302,40 +293,28 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 if (n > 0) {
                     if (fresh) cand_id[lane_rank(mask)] = v;
                     wave_sync();
+                    const int id = lane < n ? cand_id[lane] : -1;
+                    wave_sync();
                     eval_rows<DP8, TWO>(a.storage, qv, cand_id, cand_key, n, dp, lane);
                     n_dist += n;
                     wave_sync();
                     PA_TIMER(3);
                     // levels of the open list in device memory: their pair
                     // was requested by the pop and has arrived with the rows
-                    open.pop_finish(lane);
+                    open.pop_finish();
                     popped = true;
 
-                    const int d = float_to_key(lane < n ? cand_key[lane] : INFINITY);
-                    const int id = lane < n ? cand_id[lane] : -1;
+                    const int d = list_key(lane < n ? cand_key[lane] : INFINITY);
                     // heap_update, traverse_cpu.cpp:25-39, in adjacency order
                     unsigned long long todo = __ballot(d < res.worst);
                     unsigned long long admitted = 0;
                     while (todo) {
                         const int j = __builtin_ctzll(todo);
-                        todo &= todo - 1;
                         const int dj = __builtin_amdgcn_readlane(d, j);
-                        if (dj >= res.worst) continue;
                         const int vj = __builtin_amdgcn_readlane(id, j);
-                        if (Open::kFusedTop) {
-                            // the result list's new maximum and the top of
-                            // the open list's walk in one instruction stream
-                            const typename Open::Choice ch = open.template choices<true>();
-                            int first = res.replace_worst(dj, lane);
-                            const int j7 = Open::top_levels_and_wave_max(ch, first);
-                            res.set_worst(first);
-                            leaf = open.walk_below(ch, 7, j7);
-                        } else {
-                            leaf = open.walk_to_large_leaf();
-                            res.insert(dj, lane);
-                        }
-                        open.replace_leaf(leaf, dj, vj, lane);
+                        open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
                         admitted |= 1ull << j;
+                        todo &= (todo - 1) & __ballot(d < res.worst);
                     }
                     if (admitted) {
                         n_admit += __popcll(admitted);
@@ -345,9 +324,9 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                     PA_TIMER(4);
                 }
             }
-            if (!popped) open.pop_finish(lane);
+            if (!popped) open.pop_finish();
             v = likely_row;
-            const int root = Open::rl(open.Av, 1);
+            const int root = open.root_val();
             if (root != likely) v = load_row(root);
             before = test_and_set(v);
             PA_TIMER(1);
@@ -365,7 +344,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                 d = eD[i];
                 if (g >= 0 && g < a.n_nodes) u = (int)g;
             }
-            const int dk = float_to_key(d);
+            const int dk = list_key(d);
             unsigned long long todo = __ballot(u >= 0 && dk < res.worst);
             unsigned long long admitted = 0;
             while (todo) {
