@@ -761,6 +761,192 @@ __device__ __forceinline__ void eval_rows(const float *__restrict__ storage,
     }
 }
 
+// The same for the rows of lanes that `wanted` names, the distance of lane l's row
+// to dist[l] (LDS).
+template <int DP8, bool TWO>
+__device__ __forceinline__ void eval_lanes(const float *__restrict__ storage, const float *qv,
+                                           bool wanted, int id, float *dist, int dp, int lane) {
+    const unsigned long long mask = __ballot(wanted);
+    const int n = __popcll(mask);
+    if (n == 0) return;
+    // the wanted lanes first, in order, then the others: lane c gets row c's id
+    // and the lane that is from
+    const int to4 = (wanted ? lane_rank(mask) : n + lane_rank(~mask)) << 2;
+    const int row_id = __builtin_amdgcn_ds_permute(to4, id);
+    const int from = __builtin_amdgcn_ds_permute(to4, lane);
+    const int quad = lane >> 2, part = lane & 3;
+    const float2 *qq = reinterpret_cast<const float2 *>(qv) + part * query_run(dp >> 3);
+    auto of = [](int x, int c) { return __builtin_amdgcn_ds_bpermute(c << 2, x); };
+    int base = 0;
+    if constexpr (TWO && DP8 > 0 && DP8 % 2 == 0) {
+        for (; base + kRowsPerPass < n; base += 2 * kRowsPerPass) {
+            const int c = base + quad, c2 = c + kRowsPerPass;
+            const bool two = c2 < n;
+            const int id1 = of(row_id, c), id2 = of(row_id, c2);
+            const int at1 = of(from, c), at2 = of(from, c2);
+            const float *row = storage + (size_t)id1 * (size_t)dp;
+            const float *row2 = two ? storage + (size_t)id2 * (size_t)dp : row;
+            float s, s2;
+            quad_square_dist_two_rows<DP8>(row, row2, qq, part, two, s, s2);
+            if (part == 0) {
+                dist[at1] = s;
+                if (two) dist[at2] = s2;
+            }
+        }
+    }
+    for (; base < n; base += kRowsPerPass) {
+        const int c = base + quad;
+        const bool active = c < n;
+        const int id1 = of(row_id, c), at1 = of(from, c);
+        const float *row = active ? storage + (size_t)id1 * (size_t)dp : storage;
+        const float s = quad_square_dist_rows<DP8>(row, qq, dp >> 3, part, active);
+        if (active && part == 0) dist[at1] = s;
+    }
+}
+
+// ---- helpers ------------------------------------------------------------------
+//
+// A search with the device to itself waits for memory two thirds of its time: a
+// node's neighbour ids, then their rows.  More wavefronts of its workgroup do that
+// for nodes it is about to expand (the top of the open list: 92 % of the popped
+// nodes are its root after the pop before, 88 % were among its first seven three
+// steps before).  The search puts a node into a slot in LDS, a helper that is free
+// takes it from there and leaves the node's neighbours and their distances in the
+// slot.  A distance depends on the row and the query alone, so work for a node
+// that is not popped soon, or ever, costs time and nothing else.
+//
+// A slot has one writer at a time: the search while it is idle, else the helper
+// that claimed it.  LDS operations of a wavefront take effect in order.  A slot
+// that holds a node is always taken and finished, so every wait of the search
+// ends; a helper returns at kExit, which the search gives when all are idle.
+template <int HELPERS>
+struct LookAhead {
+    static constexpr int kIdle = -1, kTaken = -2, kExit = -3;   // else: the node to do
+    static constexpr int kSlots = HELPERS > 0 ? 8 : 1;
+    // Set in the open list's value of a node that has been put into a slot.
+    static constexpr int kAsked = 1 << 30;
+    static constexpr unsigned long long kTop = 0xfe;   // its first seven cells
+    struct Slots {
+        int job[kSlots];
+        int ids[kSlots][HELPERS > 0 ? kWave : 4];
+        float dist[kSlots][HELPERS > 0 ? kWave : 4];
+    };
+    Slots &slots;
+    int node;    // lane s: what slot s holds or will hold, until it is taken; -1
+    int ring;    // the slot used next (the one used longest ago)
+    unsigned long long idle;   // slots seen idle since they were last used
+
+    template <class T>
+    __device__ __forceinline__ static T get(const T &x) {
+        return __hip_atomic_load(&x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ static void put(int &x, int value) {
+        __hip_atomic_store(&x, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    // LDS operations before this come before those after it.
+    __device__ __forceinline__ static void in_order() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+
+    template <class WORK>
+    __device__ __forceinline__ static void help(Slots &slots, int lane, WORK &&work) {
+        for (;;) {
+            const int job = get(slots.job[lane & (kSlots - 1)]);
+            if (__ballot(job == kExit)) return;
+            const unsigned long long todo = __ballot(job >= 0);
+            if (!todo) {
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+            const int slot = __builtin_ctzll(todo) & (kSlots - 1);
+            const int node = __builtin_amdgcn_readlane(job, slot);
+            int was = node;
+            if (lane == 0) was = atomicCAS(&slots.job[slot], node, kTaken);
+            if (uni(was) != node) continue;   // another helper was first
+            in_order();
+            work(node, slots.ids[slot], slots.dist[slot]);
+            in_order();
+            if (lane == 0) put(slots.job[slot], kIdle);
+        }
+    }
+
+    __device__ __forceinline__ void look(int lane) {
+        idle = __ballot(get(slots.job[lane & (kSlots - 1)]) == kIdle);
+    }
+    __device__ __forceinline__ void begin(int lane) {
+        in_order();   // the query and the entries' marks are in LDS
+        node = -1, ring = 0;
+        look(lane);
+    }
+    // The next slot is idle.
+    __device__ __forceinline__ bool room() const { return (idle >> ring) & 1; }
+    // Puts `what` into it; returns the node it held that was not taken, or -1.
+    __device__ __forceinline__ int give(int what, int lane) {
+        const int old = __builtin_amdgcn_readlane(node, ring);
+        node = lane == ring ? what : node;
+        if (lane == ring) put(slots.job[lane], what);
+        idle &= ~(1ull << ring);
+        ring = (ring + 1) & (kSlots - 1);
+        return old;
+    }
+    // Puts the first node at the top of the open list (its bank A) that is in no
+    // slot into one.  One whose slot that was may be put into one again.
+    __device__ __forceinline__ void ask(int &top, int lane) {
+        const unsigned long long open =
+            __ballot((unsigned)top < (unsigned)kAsked) & kTop;
+        if (!open || !room()) return;
+        const int at = __builtin_ctzll(open);
+        const int old = give(__builtin_amdgcn_readlane(top, at), lane);
+        top = lane == at ? top | kAsked : top;
+        top = top == (old | kAsked) && old >= 0 ? old : top;
+    }
+    // What the slot of the node popped holds: its neighbours (by lane, -1: none)
+    // and the distances of those that were not marked yet when it was asked for.
+    // In two parts, with the pop between them: it is read at once, in the hope that
+    // the helper is done (`job`, read before the rest), and again if it was not.
+    struct Found {
+        int slot, job, id;
+        float dist;
+    };
+    __device__ __forceinline__ void read(Found &f, int lane) const {
+        f.job = get(slots.job[lane & (kSlots - 1)]);
+        asm volatile("" ::: "memory");
+        f.id = get(slots.ids[f.slot][lane]);
+        f.dist = get(slots.dist[f.slot][lane]);
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ Found find(int what, int lane) {
+        Found f;
+        unsigned long long has = __ballot(node == what);
+        if (!has) {
+            while (!room()) look(lane);
+            has = 1ull << ring;
+            give(what, lane);
+        }
+        f.slot = __builtin_ctzll(has) & (kSlots - 1);
+        node = node == what ? -1 : node;
+        read(f, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        return f;
+    }
+    __device__ __forceinline__ void take(Found &f, int lane) {
+        idle = __ballot(f.job == kIdle);
+        while (!((idle >> f.slot) & 1)) {
+            read(f, lane);
+            idle = __ballot(f.job == kIdle);
+        }
+        in_order();   // read before the slot is used again
+    }
+    // All slots are idle.
+    __device__ __forceinline__ void drain(int lane) {
+        do look(lane);
+        while (~idle);
+    }
+    __device__ __forceinline__ void end(int lane) const {
+        if (lane < kSlots) put(slots.job[lane], kExit);
+    }
+};
+
 }  // namespace pa
 
 #endif

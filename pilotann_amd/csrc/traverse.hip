@@ -92,9 +92,9 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 // ms, so no floor there).  H = 512 and 1024 with two passes need 172 - 183 and are
 // held to three wavefronts (168, up to 17 spilled), which LDS then allows.
 #ifdef PA_WAVES_PER_EU
-#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
+#define PA_OCCUPANCY(H, WAVES) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
 #else
-#define PA_OCCUPANCY(H) __attribute__((amdgpu_waves_per_eu((H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 512 ? 3 : (H) <= 1024 ? (TWO ? 3 : 2) : 1, 8)))
+#define PA_OCCUPANCY(H, WAVES) __attribute__((amdgpu_waves_per_eu((WAVES) > 1 && (H) <= 512 ? 4 : (H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 512 ? 3 : (H) <= 1024 ? (TWO ? 3 : 2) : 1, 8)))
 #endif
 
 // The longest open list (4096 cells) keeps level 11 in the wavefront's region of
@@ -111,12 +111,20 @@ constexpr int deep_from(int H) { return H == 2048 ? 11 : 0; }
 // dynamic too), without a table in front of them: for launches whose queries
 // all run at once with so much LDS each (make_plan).  TWO: two passes of rows are
 // read at a time.
-template <int H, int DP8, bool NEAR, bool TWO>
-__global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(TraverseArgs a) {
+//
+// WAVES > 1 (with NEAR): the wavefront of a query has WAVES - 1 helpers, which read
+// the neighbour ids and the rows of nodes it is about to expand and hand it the
+// distances (LookAhead).  What is left to it, and bounds it, is the list work:
+// 128-float rows, H = 128, one query, cycles an expansion 4600 -> 2900, of which the
+// 2.6 inserts 1130, the pop 310.  It needs no registers for rows: 116 in place of 153,
+// four wavefronts a SIMD.
+template <int H, int DP8, bool NEAR, bool TWO, int WAVES>
+__global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_kernel(TraverseArgs a) {
     // One static block, in this order: the compiler then knows every LDS
     // address, and a heap cell [j - 512] is j * 8 plus a constant that fits the
     // instruction's offset field.
     using Open = OpenList<H, deep_from(H)>;
+    using Helped = LookAhead<WAVES - 1>;
     constexpr int S = (H + kWave - 1) / kWave;
     // cells of the final sort: all of them, and those sorted in LDS at once
     constexpr int kSortAll = H <= kWave ? kWave : 1 << (floor_log2(H - 1) + 1);
@@ -137,15 +145,17 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     constexpr int kSeen = NEAR ? 4 : 1 << kSeenLog2;
     struct Lds {
         uint32_t seen_cache[kSeen];
-        int cand_id[kWave];   // a step's new rows, and then their distances
-        float near_key[NEAR ? kWave : 4];
+        // a step's new rows, and then their distances
+        int cand_id[WAVES > 1 ? 4 : kWave];
+        float near_key[NEAR && WAVES == 1 ? kWave : 4];
         float query[DP8 ? query_floats(8 * DP8) : 4];
         int2 heap[kHeapCells];  // open list tail; the final sort reuses it
     };
     __shared__ __align__(16) Lds lds;
+    __shared__ __align__(16) typename Helped::Slots slots;   // (WAVES > 1)
     // the query if its length is not known here, then NEAR's visited bits
     extern __shared__ __align__(16) float query_any_length[];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
     float *okey = reinterpret_cast<float *>(lds.heap);
     int *oval = reinterpret_cast<int *>(okey + kHeapCells);
     Open open;
@@ -160,6 +170,25 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
     uint32_t *seen = a.seen + (size_t)blockIdx.x * (size_t)a.slot_stride;
     uint32_t *near_bits =
         reinterpret_cast<uint32_t *>(query_any_length + (DP8 ? 0 : query_floats(dp)));
+    Helped ahead{slots, -1, 0, 0};
+    if constexpr (WAVES > 1) {
+        const int wave = uni((int)(threadIdx.x / kWave));
+        if (threadIdx.x < Helped::kSlots) Helped::put(slots.job[threadIdx.x], Helped::kIdle);
+        __syncthreads();   // the only barrier
+        if (wave > 0) {
+            Helped::help(slots, lane, [&](int row, int *ids, float *dist) {
+                // its neighbours, by lane, and the distances of those that are not
+                // marked yet: a mark is never taken back, so whatever is new when
+                // the node is popped is among them
+                const int v = lane < deg ? a.adj[(size_t)row * deg + lane] : -1;
+                ids[lane] = v;
+                const bool maybe_new =
+                    v >= 0 && !((Helped::get(near_bits[v >> 5]) >> (v & 31)) & 1u);
+                eval_lanes<DP8, TWO>(a.storage, qv, maybe_new, v, dist, dp, lane);
+            });
+            return;
+        }
+    }
     // after the visited slice: the log of admitted candidates, then the
     // levels of the open list kept in device memory
     ResultLog log;
@@ -171,7 +200,10 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
         int q = 0;
         if (lane == 0) q = atomicAdd(a.work_counter, 1);
         q = uni(q);
-        if (q >= a.batch) break;
+        if (q >= a.batch) {
+            if constexpr (WAVES > 1) ahead.end(lane);
+            break;
+        }
 
         unsigned n_expand = 0, n_adj = 0, n_dist = 0, n_admit = 0;
 #ifdef PA_PHASE_TIMERS
@@ -273,9 +305,69 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
             }
             return before;
         };
-        int v = load_row(open.root_val());
-        uint32_t before = test_and_set(v);
-        for (int step = 0; step < a.max_iter; ++step) {
+        // heap_update, traverse_cpu.cpp:25-39, in adjacency order: the lanes'
+        // keys d and rows id; `value` is what the open list keeps of them
+        auto admit = [&](int d, int id, int value) {
+            unsigned long long todo = __ballot(d < res.worst);
+            unsigned long long admitted = 0;
+            while (todo) {
+                const int j = __builtin_ctzll(todo);
+                const int dj = __builtin_amdgcn_readlane(d, j);
+                const int vj = __builtin_amdgcn_readlane(value, j);
+                open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
+                admitted |= 1ull << j;
+                todo &= (todo - 1) & __ballot(d < res.worst);
+            }
+            if (admitted) {
+                n_admit += __popcll(admitted);
+                log.append(admitted, d, id, lane);
+                if (log.nearly_full()) log.cut(res.worst, lane);
+            }
+        };
+        if constexpr (WAVES > 1) {
+            ahead.begin(lane);
+            for (int i = 0; i < WAVES - 1; ++i) ahead.ask(open.A.v, lane);
+            for (int step = 0; step < a.max_iter; ++step) {
+                const int u = open.root_val();
+                if (u == -1 || open.root_key() >= res.worst) break;
+                typename Helped::Found found;
+                if (u >= 0) found = ahead.find(u & ~Helped::kAsked, lane);
+                int popped_k, popped_v;
+                open.pop(lane, popped_k, popped_v);
+                n_expand += 1;
+                if (u >= 0) {
+                    n_adj += deg;
+                    ahead.take(found, lane);
+                    const int v = found.id;
+                    uint32_t before = 0xffffffffu;
+                    if (v >= 0) before = atomicOr(&near_bits[v >> 5], 1u << (v & 31));
+                    ahead.ask(open.A.v, lane);
+                    open.pop_finish();
+                    const bool fresh = !((before >> (v & 31)) & 1u);
+                    n_dist += __popcll(__ballot(fresh));
+                    const int d = fresh ? list_key(found.dist) : Open::kInf;
+                    // a neighbour that is before all of the list is next
+                    int value = v;
+                    if (__ballot(d < open.root_key()) && ahead.room()) {
+                        const int best = ~wave_max_key(~d);
+                        const int at = __builtin_ctzll(__ballot(d == best));
+                        ahead.give(__builtin_amdgcn_readlane(v, at), lane);
+                        value = lane == at ? v | Helped::kAsked : v;
+                    }
+                    admit(d, v, value);
+                } else {
+                    open.pop_finish();
+                }
+            }
+            ahead.drain(lane);
+        }
+        int v = -1;
+        uint32_t before = 0xffffffffu;
+        if constexpr (WAVES == 1) {
+            v = load_row(open.root_val());
+            before = test_and_set(v);
+        }
+        for (int step = 0; WAVES == 1 && step < a.max_iter; ++step) {
             int uk, u;
             open.pop(lane, uk, u);
             const int likely = open.root_val();
@@ -304,23 +396,7 @@ __global__ __launch_bounds__(kWave) PA_OCCUPANCY(H) void traverse_kernel(Travers
                     open.pop_finish();
                     popped = true;
 
-                    const int d = list_key(lane < n ? cand_key[lane] : INFINITY);
-                    // heap_update, traverse_cpu.cpp:25-39, in adjacency order
-                    unsigned long long todo = __ballot(d < res.worst);
-                    unsigned long long admitted = 0;
-                    while (todo) {
-                        const int j = __builtin_ctzll(todo);
-                        const int dj = __builtin_amdgcn_readlane(d, j);
-                        const int vj = __builtin_amdgcn_readlane(id, j);
-                        open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
-                        admitted |= 1ull << j;
-                        todo &= (todo - 1) & __ballot(d < res.worst);
-                    }
-                    if (admitted) {
-                        n_admit += __popcll(admitted);
-                        log.append(admitted, d, id, lane);
-                        if (log.nearly_full()) log.cut(res.worst, lane);
-                    }
+                    admit(list_key(lane < n ? cand_key[lane] : INFINITY), id, id);
                     PA_TIMER(4);
                 }
             }
@@ -636,41 +712,42 @@ typedef void (*TraverseFn)(TraverseArgs);
 #endif
 constexpr int kMaxWavesPerCu = PA_MAX_WAVES_PER_CU;
 constexpr int kStaticLds = 20 << 10;   // no instance has more static LDS
+constexpr int kHelped = 4;   // wavefronts of a query when there are few queries
 constexpr int64_t kTwoRowsBytes = 160ll << 20;   // see make_plan
 
-template <int H, bool NEAR, bool TWO>
+template <int H, bool NEAR, bool TWO, int WAVES>
 TraverseFn pick_dp(int dp) {
-    if (TWO) return dp == 128 ? traverse_kernel<H, 16, NEAR, true> : nullptr;
+    if (TWO) return dp == 128 ? traverse_kernel<H, 16, NEAR, true, WAVES> : nullptr;
     switch (dp) {
-        case 32: return traverse_kernel<H, 4, NEAR, false>;
-        case 64: return traverse_kernel<H, 8, NEAR, false>;
-        case 128: return NEAR ? nullptr : traverse_kernel<H, 16, false, false>;
-        default: return traverse_kernel<H, 0, NEAR, false>;
+        case 32: return traverse_kernel<H, 4, NEAR, false, WAVES>;
+        case 64: return traverse_kernel<H, 8, NEAR, false, WAVES>;
+        case 128: return NEAR ? nullptr : traverse_kernel<H, 16, false, false, 1>;
+        default: return traverse_kernel<H, 0, NEAR, false, WAVES>;
     }
 }
 
-template <bool NEAR, bool TWO>
+template <bool NEAR, bool TWO, int WAVES = 1>
 TraverseFn pick_kernel(int H, int dp) {
     switch (H) {
-        case 16: return pick_dp<16, NEAR, TWO>(dp);
-        case 32: return pick_dp<32, NEAR, TWO>(dp);
-        case 48: return pick_dp<48, NEAR, TWO>(dp);
-        case 64: return pick_dp<64, NEAR, TWO>(dp);
-        case 96: return pick_dp<96, NEAR, TWO>(dp);
-        case 128: return pick_dp<128, NEAR, TWO>(dp);
-        case 192: return pick_dp<192, NEAR, TWO>(dp);
-        case 256: return pick_dp<256, NEAR, TWO>(dp);
-        case 384: return pick_dp<384, NEAR, TWO>(dp);
-        case 512: return pick_dp<512, NEAR, TWO>(dp);
-        case 1024: return pick_dp<1024, NEAR, TWO>(dp);
-        case 2048: return pick_dp<2048, NEAR, TWO>(dp);
+        case 16: return pick_dp<16, NEAR, TWO, WAVES>(dp);
+        case 32: return pick_dp<32, NEAR, TWO, WAVES>(dp);
+        case 48: return pick_dp<48, NEAR, TWO, WAVES>(dp);
+        case 64: return pick_dp<64, NEAR, TWO, WAVES>(dp);
+        case 96: return pick_dp<96, NEAR, TWO, WAVES>(dp);
+        case 128: return pick_dp<128, NEAR, TWO, WAVES>(dp);
+        case 192: return pick_dp<192, NEAR, TWO, WAVES>(dp);
+        case 256: return pick_dp<256, NEAR, TWO, WAVES>(dp);
+        case 384: return pick_dp<384, NEAR, TWO, WAVES>(dp);
+        case 512: return pick_dp<512, NEAR, TWO, WAVES>(dp);
+        case 1024: return pick_dp<1024, NEAR, TWO, WAVES>(dp);
+        case 2048: return pick_dp<2048, NEAR, TWO, WAVES>(dp);
         default: return nullptr;
     }
 }
 
 // Wavefronts (workgroups of one) of `fn` the current device holds at once, and
 // in *max_lds what LDS it gives one workgroup.
-int residency(TraverseFn fn, int lds_bytes, int64_t *slots, int *max_lds) {
+int residency(TraverseFn fn, int threads, int lds_bytes, int64_t *slots, int *max_lds) {
     struct Known {
         int cus, per_cu, max_lds;
     };
@@ -689,7 +766,7 @@ int residency(TraverseFn fn, int lds_bytes, int64_t *slots, int *max_lds) {
         if (e == hipSuccess)
             e = hipDeviceGetAttribute(&k.max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
         if (e == hipSuccess)
-            e = workgroups_per_cu(reinterpret_cast<const void *>(fn), dev, kWave, lds_bytes,
+            e = workgroups_per_cu(reinterpret_cast<const void *>(fn), dev, threads, lds_bytes,
                                   &k.per_cu);
         if (e != hipSuccess) return (int)e;
         // sizes of NEAR follow the index: a few stay
@@ -703,7 +780,7 @@ int residency(TraverseFn fn, int lds_bytes, int64_t *slots, int *max_lds) {
 }
 
 struct Plan {
-    int H, sort_n, lds_bytes, n_slots, words_per_slot, slot_stride;
+    int H, sort_n, lds_bytes, n_slots, words_per_slot, slot_stride, threads;
     size_t workspace_bytes;
     TraverseFn fn;
     bool near_bits;
@@ -725,11 +802,12 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     p->lds_bytes += PA_EXTRA_LDS;
 #endif
     p->near_bits = false;
+    p->threads = kWave;
     p->fn = dp == 128 ? pick_kernel<false, true>(p->H, dp) : pick_kernel<false, false>(p->H, dp);
     if (!p->fn) return PA_E_EF;
     int64_t slots = 0;
     int max_lds = 0;
-    const int rc = residency(p->fn, p->lds_bytes, &slots, &max_lds);
+    const int rc = residency(p->fn, kWave, p->lds_bytes, &slots, &max_lds);
     if (rc != PA_OK) return rc;
     // 128-float rows: two passes of reads in flight per wavefront, or one and five
     // wavefronts per SIMD instead of three.  Two where the queries all run at
@@ -744,7 +822,7 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     if (dp == 128 && batch > slots - beside) {
         const TraverseFn one = pick_kernel<false, false>(p->H, dp);
         int64_t one_slots = 0;
-        const int one_rc = residency(one, p->lds_bytes, &one_slots, &max_lds);
+        const int one_rc = residency(one, kWave, p->lds_bytes, &one_slots, &max_lds);
         if (one_rc != PA_OK) return one_rc;
         const bool short_round =
             batch <= one_slots - beside && batch <= 4 * slots / 3 - beside;
@@ -785,7 +863,7 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
         const TraverseFn near_fn =
             dp == 128 ? pick_kernel<true, true>(p->H, dp) : pick_kernel<true, false>(p->H, dp);
         int64_t near_slots = 0;
-        const int near_rc = residency(near_fn, (int)near_lds, &near_slots, &max_lds);
+        const int near_rc = residency(near_fn, kWave, (int)near_lds, &near_slots, &max_lds);
         if (near_rc != PA_OK) return near_rc;
         const bool near_fits = batch <= near_slots - beside;
         const bool far_fits = batch <= slots - beside;
@@ -794,6 +872,25 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
                            (batch <= near_slots && 3 * near_slots >= 2 * slots)))) {
             p->fn = near_fn, p->lds_bytes = (int)near_lds;
             p->near_bits = true;
+        }
+        // With three helpers as long as every query, those of launches beside this
+        // one too, has its four wavefronts at once.  Measured, without / with, us:
+        // 250 000 rows of 128 floats, H = 128, one query 298 / 217; H = 192, 37
+        // queries 591 / 468, 512 706 / 559; H = 256, 1024 919 / 735; 500 000 rows, H
+        // = 1024, 37 2762 / 2282, 512 (the most that fit) 3145 / 3136; rows of 64
+        // floats, H = 384, 100 895 / 803; of 40, H = 256, 1000 524 / 449.  An
+        // expansion over rows of 32 floats is list work: H = 256, 128 388 / 370,
+        // 1700 538 / 536, but H = 512, 1000 878 / 893, H = 1024, 700 3325 / 3401.
+        // (Seven helpers: 217, 482, 582, 905 where three take 215, 479, 572, 770.)
+        if (near_fits && (dp > 32 || p->H <= 256)) {
+            const TraverseFn helped_fn = dp == 128 ? pick_kernel<true, true, kHelped>(p->H, dp)
+                                                   : pick_kernel<true, false, kHelped>(p->H, dp);
+            int64_t helped_slots = 0;
+            const int helped_rc = residency(helped_fn, kHelped * kWave, (int)near_lds,
+                                            &helped_slots, &max_lds);
+            if (helped_rc != PA_OK) return helped_rc;
+            if (batch <= helped_slots - beside)
+                p->fn = helped_fn, p->threads = kHelped * kWave;
         }
     }
     return PA_OK;
@@ -940,7 +1037,7 @@ int launch_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
 
     hipStream_t stream = (hipStream_t)stream_;
     reset_work_counter<<<1, 1, 0, stream>>>(a.work_counter);
-    p.fn<<<p.n_slots, kWave, p.lds_bytes, stream>>>(a);
+    p.fn<<<p.n_slots, p.threads, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
 }
 
