@@ -383,30 +383,35 @@ struct OpenList {
     // its own and the new one, and the value that goes with that; a node off the
     // path does the same with the largest key for the new one, which changes
     // nothing (a parent's key is never above its child's).
-    __device__ __forceinline__ static void take(Cell &c, const Cell &up, int key, int moved) {
+    __device__ __forceinline__ static bool take(Cell &c, const Cell &up, int key, int moved) {
         const bool moves = c.k > key;
         c.k = med3(up.k, key, c.k);
         c.v = moves ? moved : c.v;
+        return moves;
     }
-    __device__ __forceinline__ void shift(const Path &w, const Parents &up, int k, int v,
+    // Returns whether the lane has a node that took another entry.
+    __device__ __forceinline__ bool shift(const Path &w, const Parents &up, int k, int v,
                                           int lane) {
         const Spread t = on<true>(w, k, kAboveAll, lane);
         // what a node that changes takes: its parent's value or the new one
         const int toA = up.A.k > k ? up.A.v : v, toB = up.B.k > k ? up.B.v : v;
         const int toC = B.k > k ? B.v : v;
+        bool any = false;
         if (kDepth >= 8) {
             const int toE = C.k > k ? C.v : v;
-            if (kSize == 512) take(J, E, t.J, E.k > k ? E.v : v);
-            take(E, C, t.E, toE);
+            if (kSize == 512) any |= take(J, E, t.J, E.k > k ? E.v : v);
+            any |= take(E, C, t.E, toE);
             if (kLast > 0) {
                 const int toG = D.k > k ? D.v : v;
-                take(F, C, t.F, toE);
-                take(G, D, t.G, toG), take(I, D, t.I, toG);
+                any |= take(F, C, t.F, toE);
+                any |= take(G, D, t.G, toG);
+                any |= take(I, D, t.I, toG);
             }
         }
-        if (kDepth >= 7) take(C, B, t.C, toC), take(D, B, t.D, toC);
-        if (kDepth >= 6) take(B, up.B, t.B, toB);
-        take(A, up.A, t.A, toA);
+        if (kDepth >= 7) any |= take(C, B, t.C, toC), any |= take(D, B, t.D, toC);
+        if (kDepth >= 6) any |= take(B, up.B, t.B, toB);
+        any |= take(A, up.A, t.A, toA);
+        return any;
     }
 
     // Long lists: the path below level 8, in the lane whose subtree it is in.
@@ -493,23 +498,39 @@ struct OpenList {
             shift(w, up, k, v, lane);
         }
     }
+    // The same; returns whether the entry got in.
+    __device__ __forceinline__ bool push(int k, int v, int lane) {
+        if constexpr (kLong) {
+            const Path w = path<true>();
+            const Low low = walk(w, lane, [] {});
+            int leaf = low.bottom ? low.at[kEnd - 8].k : low.at[0].k;
+            if (kOneLast) leaf = 2 * low.j == kSize ? J.k : leaf;
+            if (!__ballot(low.mine && leaf > k)) return false;
+            rise(w, low, k, v, lane);
+            return true;
+        } else {
+            const Parents up = parents(lane);
+            __builtin_amdgcn_sched_barrier(0);
+            return __ballot(shift(path<true>(), up, k, v, lane)) != 0;
+        }
+    }
     // Pushes, in lane order, the entries (k, v) of the lanes in `who`, as one
     // insert after the other would.  An entry not below the leaf's key changes
-    // nothing, so the leaf is looked for again only after an entry that got
-    // in, and everything that stays out is passed over by one comparison of all
-    // lanes.  Entries mostly come in ascending order; then nearly all of them stay
-    // out (the path follows the larger child, not the free cells).
+    // nothing: after one that stayed out the leaf's key is looked for, and all that
+    // are not below it are passed over by one comparison of all lanes.  (In
+    // ascending order most stay out: the path follows the larger child, not the
+    // free cells.)
     __device__ __forceinline__ void push_entries(unsigned long long who, int k, int v, int lane) {
         while (who) {
+            const int j = __builtin_ctzll(who);
+            who &= who - 1;
+            if (push(rl(k, j), rl(v, j), lane)) continue;
             const Path w = path<true>();
             Low low = {};
             if constexpr (kLong) low = walk(w, lane, [] {});
             const unsigned long long in = who & __ballot(k < leaf_key(w, low, lane));
             if (!in) return;
-            const int j = __builtin_ctzll(in);
-            who &= ~1ull << j;
-            if constexpr (kLong) rise(w, low, rl(k, j), rl(v, j), lane);
-            else shift(w, parents(lane), rl(k, j), rl(v, j), lane);
+            who &= ~0ull << __builtin_ctzll(in);   // (those behind it meet another leaf)
         }
     }
 };
