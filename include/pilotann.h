@@ -374,6 +374,25 @@ int pa_graph_reach(unsigned char *mark, int *status, const int64_t *adj, int64_t
                    int deg, int backward, int steps, void *stream);
 
 /*
+ * Reverse edges of the graph builder (faiss' part in the reference), in two
+ * calls.  forward [n * m]: the edges of n nodes, what is not in 0 .. n-1 is none.
+ * An edge i -> j is new to j if row j does not hold i: is_new [n * m] receives 1
+ * for those and 0 for the others, count [n] how many are new to each node.
+ * Then, with end [n] the running sum of count (end[i] includes count[i]): row i of
+ * adj [n * degree] receives the edges of row i of forward in order, cut to degree,
+ * and in the slots that are left the nodes whose edge is new to i, those that have
+ * it at a lower place of their row first, then by number; -1 behind them.
+ * list [n * m]: scratch; count is used up.  n < 2^31; m and degree up to
+ * PA_MAX_NEIGHBORS.  Device pointers; enqueued on `stream`.
+ */
+int pa_graph_count_sources(int32_t *count, unsigned char *is_new, const int64_t *forward,
+                           int64_t n, int m, void *stream);
+int pa_graph_add_reverse(int64_t *adj, uint64_t *list, int32_t *count,
+                         const unsigned char *is_new, const int64_t *end,
+                         const int64_t *forward, int64_t n, int m, int degree,
+                         void *stream);
+
+/*
  * Occlusion pruning of candidate lists, the edge selection of the graph
  * builder (faiss' part in the reference, pilot_ann/utils/graphs.py:15-20,52-56;
  * no entry point of the reference's extension corresponds to it).  For each of

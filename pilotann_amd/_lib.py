@@ -51,6 +51,8 @@ _SIGNATURES = {
     'pa_rows_low': (_int, [_vp, _vp, _i64, _i64, _int, _int, ctypes.c_float,
                            ctypes.c_float, _vp]),
     'pa_graph_reach': (_int, [_vp, _vp, _vp, _i64, _int, _int, _int, _vp]),
+    'pa_graph_count_sources': (_int, [_vp, _vp, _vp, _i64, _int, _vp]),
+    'pa_graph_add_reverse': (_int, [_vp] * 6 + [_i64, _int, _int, _vp]),
     'pa_graph_prune': (_int, [_vp, _vp, _vp, _i64, _int, _int, _int, _vp]),
     'pa_graph_prune_rows': (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _int,
                             _int, _int, ctypes.c_float, _vp]),

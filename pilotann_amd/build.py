@@ -16,7 +16,7 @@ LIB = os.path.join(CSRC, 'libpilotann.so')
 PHASE_LIB = os.path.join(CSRC, 'libpilotann_phase_timers.so')
 
 HIP_SOURCES = ['traverse.hip', 'traverse_wide.hip', 'refine.hip', 'route.hip', 'rotate.hip',
-               'knn.hip', 'pipeline.hip']
+               'knn.hip', 'reverse.hip', 'pipeline.hip']
 CXX_SOURCES = ['host_search.cpp']
 
 HIP_FLAGS = [

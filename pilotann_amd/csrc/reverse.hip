@@ -1,0 +1,161 @@
+// Reverse edges of the graph builder (faiss' part in the reference,
+// pilot_ann/utils/graphs.py:43-77): a row's free slots go to the nodes that point
+// at its node, by the place they have it in, then by their number.
+//
+// What bounds it is launches and random reads (a row of the target for every
+// edge, from cache).  Three kernels and a running sum: count a node's new sources,
+// deal them out to their targets' parts of one list, and a wavefront per node that
+// keeps the smallest of its part.  With sorts of all edges (two argsorts, a
+// membership test by a third sort, selections that wait for the host: some sixty
+// launches) a whole build of 20 011 x 96 took 6.05 ms, now 4.74; of 120 000 x 768
+// 71.0, now 69.6.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "device_common.h"
+#include "pilotann.h"
+
+using namespace pa;
+
+namespace {
+
+constexpr int64_t kMaxGrid = 1 << 22;   // workgroups of a launch: under 2^32 work-items
+
+struct ReverseArgs {
+    const int64_t *forward;   // [n, m]
+    int64_t n, n_edges;
+    int m, degree;
+    int32_t *count;           // [n]: new sources, counted up and then down again
+    const int64_t *end;       // [n]: running sum of `count`
+    unsigned char *is_new;    // [n * m]
+    uint64_t *list;           // [n * m]: place << 32 | source
+    int64_t *adj;             // [n, degree]
+};
+
+__global__ void clear_counts(int32_t *count, int64_t n) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
+        count[i] = 0;
+}
+
+// An edge src -> dst is new to dst if dst's own row does not have src.
+__global__ __launch_bounds__(256) void count_sources(ReverseArgs a) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < a.n_edges; e += step) {
+        const int64_t dst = a.forward[e], src = e / a.m;
+        bool is_new = dst >= 0 && dst < a.n;
+        if (is_new) {
+            const int64_t *row = a.forward + dst * a.m;
+            bool has = false;
+            for (int i = 0; i < a.m; ++i) has |= row[i] == src;
+            is_new = !has;
+        }
+        a.is_new[e] = is_new;
+        if (is_new) atomicAdd(&a.count[dst], 1);
+    }
+}
+
+__global__ __launch_bounds__(256) void deal_sources(ReverseArgs a) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < a.n_edges; e += step) {
+        if (!a.is_new[e]) continue;
+        const int64_t dst = a.forward[e], src = e / a.m;
+        const int left = atomicSub(&a.count[dst], 1);
+        a.list[a.end[dst] - left] = (uint64_t)(e - src * a.m) << 32 | (uint64_t)src;
+    }
+}
+
+__device__ __forceinline__ uint64_t of_lane(uint64_t x, int lane) {
+    const int lo = __builtin_amdgcn_ds_bpermute(lane << 2, (int)x);
+    const int hi = __builtin_amdgcn_ds_bpermute(lane << 2, (int)(x >> 32));
+    return (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
+}
+// Compare-exchange stages over the lanes of a wavefront, smallest first: all of
+// them (first_size 2) or the last merge alone (64, for a bitonic row).
+__device__ __forceinline__ uint64_t sort_lanes(uint64_t x, int first_size, int lane) {
+    for (int size = first_size; size <= kWave; size <<= 1) {
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            const uint64_t y = of_lane(x, lane ^ stride);
+            const bool small = ((lane & stride) == 0) == ((lane & size & (kWave - 1)) == 0);
+            x = (x < y) == small ? x : y;
+        }
+    }
+    return x;
+}
+
+__global__ __launch_bounds__(256) void fill_rows(ReverseArgs a) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int per_block = blockDim.x / kWave;
+    for (int64_t r = (int64_t)blockIdx.x * per_block + threadIdx.x / kWave; r < a.n;
+         r += (int64_t)gridDim.x * per_block) {
+        int64_t *out = a.adj + r * a.degree;
+        const int64_t to = lane < a.m ? a.forward[r * a.m + lane] : -1;
+        const unsigned long long valid = __ballot(to >= 0);
+        const int place = lane_rank(valid);
+        if (to >= 0 && place < a.degree) out[place] = to;
+        const int used = min(a.degree, (int)__popcll(valid));
+        const int64_t first = r > 0 ? a.end[r - 1] : 0, last = a.end[r];
+        // the smallest 64 so far, in order over the lanes
+        uint64_t best = ~0ull;
+        if (used < a.degree) {
+            for (int64_t at = first; at < last; at += kWave) {
+                uint64_t x = at + lane < last ? a.list[at + lane] : ~0ull;
+                if (!__ballot(x < of_lane(best, a.degree - used - 1))) continue;
+                x = sort_lanes(x, 2, lane);
+                if (at == first) {
+                    best = x;
+                    continue;
+                }
+                const uint64_t y = of_lane(x, kWave - 1 - lane);
+                best = sort_lanes(best < y ? best : y, kWave, lane);
+            }
+        }
+        if (lane < a.degree - used)
+            out[used + lane] = best == ~0ull ? -1 : (int64_t)(uint32_t)best;
+    }
+}
+
+unsigned blocks_for(int64_t items, int per_block) {
+    const int64_t blocks = (items + per_block - 1) / per_block;
+    return (unsigned)(blocks < kMaxGrid ? blocks : kMaxGrid);
+}
+
+int check(int64_t n, int m, int degree) {
+    if (n < 0) return PA_E_SHAPE;
+    if (m < 1 || m > PA_MAX_NEIGHBORS || degree < 1 || degree > PA_MAX_NEIGHBORS)
+        return PA_E_NEIGHBORS;
+    return n >= (1ll << 31) ? PA_E_RANGE : PA_OK;
+}
+
+}  // namespace
+
+extern "C" int pa_graph_count_sources(int32_t *count, unsigned char *is_new,
+                                      const int64_t *forward, int64_t n, int m, void *stream_) {
+    const int rc = check(n, m, 1);
+    if (rc != PA_OK || n == 0) return rc;
+    if (!count || !is_new || !forward) return PA_E_NULL;
+    ReverseArgs a = {};
+    a.forward = forward, a.n = n, a.n_edges = n * m, a.m = m;
+    a.count = count, a.is_new = is_new;
+    hipStream_t stream = (hipStream_t)stream_;
+    clear_counts<<<blocks_for(n, 256), 256, 0, stream>>>(count, n);
+    count_sources<<<blocks_for(a.n_edges, 256), 256, 0, stream>>>(a);
+    return (int)hipGetLastError();
+}
+
+extern "C" int pa_graph_add_reverse(int64_t *adj, uint64_t *list, int32_t *count,
+                                    const unsigned char *is_new, const int64_t *end,
+                                    const int64_t *forward, int64_t n, int m, int degree,
+                                    void *stream_) {
+    const int rc = check(n, m, degree);
+    if (rc != PA_OK || n == 0) return rc;
+    if (!adj || !list || !count || !is_new || !end || !forward) return PA_E_NULL;
+    ReverseArgs a;
+    a.forward = forward, a.n = n, a.n_edges = n * m, a.m = m, a.degree = degree;
+    a.count = count, a.end = end, a.is_new = const_cast<unsigned char *>(is_new);
+    a.list = list, a.adj = adj;
+    hipStream_t stream = (hipStream_t)stream_;
+    deal_sources<<<blocks_for(a.n_edges, 256), 256, 0, stream>>>(a);
+    fill_rows<<<blocks_for(n, 256 / kWave), 256, 0, stream>>>(a);
+    return (int)hipGetLastError();
+}

@@ -539,6 +539,29 @@ def graph_reachable(adj: torch.Tensor, sources: torch.Tensor, reverse: bool = Fa
     return mark != 0
 
 
+def graph_add_reverse(forward: torch.Tensor, degree: int):
+    """Rows of ``degree`` slots (``pa_graph_add_reverse``): the edges of
+    ``forward`` ``[n, m]`` (int64 on the device, negative: none), then the nodes
+    that point at the row's node and are not in ``forward``'s row, lowest place
+    first, then lowest number, until the row is full.  ``-1`` pads."""
+    _check(forward, 'forward', 2, torch.int64, True)
+    n, m = forward.shape
+    dev = forward.device
+    adj = torch.empty(n, degree, dtype=torch.long, device=dev)
+    count = torch.empty(n, dtype=torch.int32, device=dev)
+    is_new = torch.empty(n * m, dtype=torch.uint8, device=dev)
+    source = torch.empty(n * m, dtype=torch.long, device=dev)
+    lib = _lib.lib()
+    with torch.cuda.device(dev):
+        _lib.check(lib.pa_graph_count_sources(_ptr(count), _ptr(is_new), _ptr(forward), n, m,
+                                              _stream()), 'pa_graph_count_sources')
+        end = torch.cumsum(count, 0, dtype=torch.long)
+        _lib.check(lib.pa_graph_add_reverse(_ptr(adj), _ptr(source), _ptr(count), _ptr(is_new),
+                                            _ptr(end), _ptr(forward), n, m, int(degree),
+                                            _stream()), 'pa_graph_add_reverse')
+    return adj
+
+
 def graph_prune(pair: torch.Tensor, cand_dist: torch.Tensor, m_keep: int, fill: bool):
     """Occlusion pruning of candidate lists (``pa_graph_prune``): ``pair``
     ``[n, k, k]`` distances between a node's candidates, ``cand_dist``

@@ -266,6 +266,9 @@ def _add_reverse(forward: torch.Tensor, degree: int):
     the row's node and are not in it yet, strongest (lowest forward rank)
     first, until the row is full.  ``-1`` pads."""
     n, m = forward.shape
+    if forward.is_cuda and 0 < m <= 64 and 0 < degree <= 64:
+        from .. import kernels
+        return kernels.graph_add_reverse(forward.contiguous(), degree)
     dev = forward.device
     adj = torch.full((n, degree), -1, dtype=torch.long, device=dev)
     # compact forward edges to the left of each row

@@ -1,0 +1,31 @@
+"""The reverse edges made on the device against those made with torch on the host:
+the same rows, place for place."""
+import pytest
+import torch
+
+from pilotann_amd.utils import graphs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('n,m,degree,edges', [
+    (1, 1, 1, 'any'), (2, 1, 2, 'any'), (65, 64, 64, 'any'), (300, 7, 5, 'any'),
+    (5000, 16, 32, 'any'), (5000, 48, 48, 'any'), (4097, 24, 64, 'holes'),
+    (3000, 8, 40, 'hub'), (3000, 1, 64, 'hub'), (700, 5, 9, 'none'),
+])
+def test_same_rows_as_on_the_host(n, m, degree, edges, device):
+    g = torch.Generator().manual_seed(n + m)
+    forward = torch.stack([torch.randperm(max(n, m), generator=g)[:m] for _ in range(n)])
+    forward[forward >= n] = -1
+    if edges == 'hub':      # nodes that thousands point at, from every place
+        hubs = torch.randint(0, 3, (n,), generator=g)
+        place = torch.randint(0, m, (n,), generator=g)
+        forward[forward < 3] = -1
+        forward[torch.arange(n), place] = hubs
+    if edges == 'holes':
+        forward[torch.rand(n, m, generator=g) < 0.4] = -1
+    if edges == 'none':
+        forward[:] = -1
+    want = graphs._add_reverse(forward, degree)
+    got = graphs._add_reverse(forward.to(device), degree)
+    assert torch.equal(got.cpu(), want)
