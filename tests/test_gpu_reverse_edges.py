@@ -29,3 +29,10 @@ def test_same_rows_as_on_the_host(n, m, degree, edges, device):
     want = graphs._add_reverse(forward, degree)
     got = graphs._add_reverse(forward.to(device), degree)
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize('n', [0, 1, 1000, 1001, 2999, 3000, 10_007])
+def test_ids_reach_the_host_whole(n, device):
+    g = torch.Generator().manual_seed(n)
+    ids = torch.randint(-1, max(n, 1), (n,), generator=g)
+    assert torch.equal(graphs._ids_to_host(ids.to(device), piece=1000), ids)
