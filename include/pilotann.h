@@ -550,7 +550,8 @@ int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
                      void *workspace, size_t workspace_bytes,
                      uint64_t *counters, void *stream);
 
-/* The form that such a launch takes: wavefronts (out), 1 or 4 per query. */
+/* The form that such a launch takes: wavefronts (out), 1 or 4 per query (4 also where
+ * a compute unit has one query at most, which then has eight, seven reading ahead). */
 int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, int d_model,
                    int ef_search, int *wavefronts);
 

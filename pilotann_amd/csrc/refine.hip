@@ -13,7 +13,8 @@
 // a pooled bitmask), kept across the two searches.  Rows are d_model floats; a
 // quad of lanes streams a row sixteen 32-byte groups at a time.  In launches
 // whose queries all run at once three more wavefronts read a query's rows with
-// the first, 32 groups at a time.
+// the first, 32 groups at a time; with a compute unit to a query, seven more read
+// the rows of the nodes it is about to expand.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -95,6 +96,28 @@ __device__ __forceinline__ void eval_rows_from(const float *__restrict__ storage
     }
 }
 
+// The same for the rows of the lanes that `wanted` names, by one wavefront; the
+// distance of lane l's row to dist[l].
+template <int CHUNK>
+__device__ __forceinline__ void eval_lanes_from(const float *__restrict__ storage,
+                                                const float *qv, bool wanted, int id,
+                                                float *dist, int d, int from, int lane) {
+    const LaneRows rows(wanted, id, lane);
+    const int quad = lane >> 2, part = lane & 3;
+    const int groups = d >> 3;
+    const float2 *qrun =
+        reinterpret_cast<const float2 *>(qv) + part * query_run(groups);
+    for (int base = 0; base < rows.n; base += kRowsPerPass) {
+        const int c = base + quad;
+        const bool active = c < rows.n;
+        const int row_id = LaneRows::of(rows.id, c), at = LaneRows::of(rows.from, c);
+        const float *row = active ? storage + (size_t)row_id * (size_t)d : storage;
+        const float s = quad_square_dist_long<CHUNK>(row, qrun, groups, from >> 3,
+                                                     part, active);
+        if (active && part == 0) dist[at] = s;
+    }
+}
+
 // Plain rows -> the interleaved layout (row_pair_slot); one thread per pair.
 __global__ void interleave_rows(const float *__restrict__ src,
                                 float *__restrict__ dst, int64_t n_pairs,
@@ -122,12 +145,14 @@ __global__ void interleave_rows(const float *__restrict__ src,
 typedef Visited<PA_REFINE_SEEN_LOG2, PA_REFINE_SEEN_WAYS> RefineVisited;
 
 constexpr int kHelped = 4;   // wavefronts of a query when there are few queries
+constexpr int kAhead = 8;    // when there are very few
 // blocks of a row read at once
 template <int WAVES>
-constexpr int kRefineChunk = WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
+constexpr int kRefineChunk = WAVES > 4 ? 4 * PA_LONG_CHUNK
+                             : WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
 
 #define PA_REFINE_OCCUPANCY(H, WAVES) \
-    __attribute__((amdgpu_waves_per_eu((H) <= 256 || ((WAVES) > 1 && (H) <= 512) ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+    __attribute__((amdgpu_waves_per_eu((WAVES) > 4 ? 2 : (H) <= 256 || ((WAVES) > 1 && (H) <= 512) ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
 
 // WAVES = 1: the wavefront of a query reads its rows itself.  WAVES = 4: three
 // more wavefronts wait at a barrier and read rows with it.  A search with the
@@ -139,8 +164,17 @@ constexpr int kRefineChunk = WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
 // 512 / 1024 queries: 249 / 416 / 620 us so, 247 / 408 / 735 without a spill at
 // half the queries a compute unit (for which 1024 take two rounds), 269 / 449 /
 // 629 with 8 blocks a trip.
+//
+// WAVES = 8: seven wavefronts read the rows of nodes the search is about to expand
+// (LookAhead), two a node, 32 blocks of a row at a time, and the candidates' rows
+// all together.  87 - 92 % of the nodes popped have been asked for, but a node's rows take
+// longer than a step, so that what bounds it is still half the waits (4000 of 9500 cycles
+// an expansion at one query, H = 32), then the inserts (2400) and the marks (1800).
 template <int H, int WAVES>
 __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void refine_kernel(RefineArgs a) {
+    constexpr bool AHEAD = WAVES == kAhead;
+    using Ahead = LookAhead<AHEAD ? WAVES - 1 : 0, AHEAD ? 2 : 1>;
+    constexpr int kEntries = 0x7fffffff;   // a job: rows of the list in cand_id
     constexpr int S = (H + kWave - 1) / kWave;
     constexpr int kSortN = H <= kWave ? kWave : 1 << (floor_log2(H - 1) + 1);
     constexpr int kHeapCells =
@@ -149,14 +183,63 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
         uint32_t seen_table[RefineVisited::kWords];
         int cand_id[kWave];
         float cand_key[kWave];
-        int job_rows, job_from;  // WAVES > 1: rows to read, from which coordinate
+        // WAVES > 1: rows to read, from which coordinate; AHEAD: on which graph
+        int job_rows, job_from, job_stage;
         int2 heap[kHeapCells];   // open list tail; the sorts reuse it
     };
     __shared__ __align__(16) Lds lds;
     extern __shared__ __align__(16) float qv[];  // the query, query_slot layout
+    __shared__ __align__(16) typename Ahead::Slots slots;   // AHEAD
     const int lane = threadIdx.x & (kWave - 1);
     const int d = a.d;
-    if constexpr (WAVES > 1) {
+    // A node's row of neighbours, by lane.
+    auto neighbours = [&](int stage, int deg, int u) -> int {
+        int v = -1;
+        if (u < 0) return v;
+        if (stage == 0) {
+            const int64_t r = a.sub_mapping[u];
+            if (r >= 0 && lane < deg) {
+                const int w = a.sub_adj[(size_t)r * deg + lane];
+                if (w >= 0) v = a.sub_gid[w];
+            }
+        } else if (lane < deg) {
+            v = a.full_adj[(size_t)u * deg + lane];
+        }
+        return v;
+    };
+    Ahead ahead{slots, -1, 0, 0};
+    if constexpr (AHEAD) {
+        const int wave = uni((int)(threadIdx.x / kWave));
+        if (threadIdx.x < Ahead::kJobs) Ahead::put(slots.job[threadIdx.x], Ahead::kIdle);
+        __syncthreads();   // the only barrier
+        if (wave > 0) {
+            RefineVisited marks;
+            marks.init(lds.seen_table, nullptr, a.n_nodes);
+            Ahead::help(slots, lane, [&](int node, int job, int *ids, float *dist) {
+                int v, from = 0;
+                bool wanted;
+                if (node == kEntries) {
+                    const int n = Ahead::get(lds.job_rows);
+                    from = uni(Ahead::get(lds.job_from));
+                    v = lane < n ? lds.cand_id[lane] : -1;
+                    wanted = lane < n && lane % (WAVES - 1) == job;
+                    dist = lds.cand_key;
+                } else {
+                    // the part's neighbours, and the distances of those that are
+                    // not known to be marked: whatever is new when the node is
+                    // popped is among them
+                    const int stage = uni(Ahead::get(lds.job_stage));
+                    const bool mine = (lane & 1) == job / Ahead::kSlots;
+                    v = neighbours(stage, stage == 0 ? a.sub_deg : a.full_deg, node);
+                    if (mine) ids[lane] = v;
+                    wanted = mine && v >= 0 && !marks.known(v);
+                }
+                eval_lanes_from<kRefineChunk<WAVES>>(a.storage, qv, wanted, v, dist, d, from,
+                                                     lane);
+            });
+            return;
+        }
+    } else if constexpr (WAVES > 1) {
         // a scalar: the two sides of this branch meet at the same barriers,
         // two per job, and one when the queries are used up
         const int wave = uni((int)(threadIdx.x / kWave));
@@ -174,6 +257,14 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
     }
     // distances of the n rows in cand_id over the coordinates [from, d)
     auto eval = [&](int n, int from) {
+        if constexpr (AHEAD) {
+            lds.job_rows = n, lds.job_from = from;
+            ahead.drain(lane);
+            ahead.give_all(kEntries, lane);
+            ahead.drain(lane);
+            Ahead::in_order();
+            return;
+        }
         if constexpr (WAVES > 1) {
             lds.job_rows = n, lds.job_from = from;
             __syncthreads();
@@ -202,7 +293,10 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
         if (lane == 0) q = atomicAdd(a.work_counter, 1);
         q = uni(q);
         if (q >= a.batch) {
-            if constexpr (WAVES > 1) {
+            if constexpr (AHEAD) {
+                ahead.drain(lane);
+                ahead.end(lane);
+            } else if constexpr (WAVES > 1) {
                 lds.job_rows = -1;
                 __syncthreads();
             }
@@ -215,6 +309,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
 #endif
         PA_TIMER_BEGIN();
 
+        if constexpr (AHEAD) ahead.drain(lane);   // of what was asked for in vain
         // empty visited set (it serves both searches), query to LDS
         visited.reset(lane);
         for (int i = lane; i < d; i += kWave)
@@ -239,6 +334,10 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
             const int n_out = stage == 0 ? a.n_buffers : a.k;
 
             PA_TIMER(0);
+            if constexpr (AHEAD) {
+                ahead.drain(lane);
+                lds.job_stage = stage;
+            }
             open.reset(lane);
             // Which node a key of the result list belongs to: beside it in its
             // lane where a lane has one key, else in the log.  Measured with
@@ -283,7 +382,13 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     wave_sync();
                 }
                 if (u >= 0) visited.mark(u);
-                open.push_entries(__ballot(u >= 0), list_key(dist), u, lane);
+                int value = u;
+                if constexpr (AHEAD) {
+                    if (base == 0) ahead.begin(lane);
+                    for (int j = 0; j < 3 && j < max_iter; ++j)
+                        ahead.ask_lowest(list_key(dist), value, lane);
+                }
+                open.push_entries(__ballot(u >= 0), list_key(dist), value, lane);
                 PA_TIMER(2);
             }
 
@@ -295,23 +400,62 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
             // fill the device the wasted requests cost more (10 000 queries,
             // 96 floats, H = 96: 2.02 against 1.94 ms).
             constexpr bool kEarly = WAVES > 1;
-            auto load_row = [&](int u) -> int {
-                int v = -1;
-                if (u < 0) return v;
-                if (stage == 0) {
-                    const int64_t r = a.sub_mapping[u];
-                    if (r >= 0 && lane < deg) {
-                        const int w = a.sub_adj[(size_t)r * deg + lane];
-                        if (w >= 0) v = a.sub_gid[w];
+            auto load_row = [&](int u) -> int { return neighbours(stage, deg, u); };
+            // heap_update, traverse_cpu.cpp:25-39, in adjacency order: the lanes'
+            // keys and nodes; `value` is what the open list keeps of them
+            auto admit = [&](int dk, int id, int value) {
+                unsigned long long todo = __ballot(dk < res.worst);
+                unsigned long long admitted = 0;
+                while (todo) {
+                    const int j = __builtin_ctzll(todo);
+                    const int dj = __builtin_amdgcn_readlane(dk, j);
+                    const int vj = __builtin_amdgcn_readlane(value, j);
+                    if (kBeside) {
+                        const int node = AHEAD ? __builtin_amdgcn_readlane(id, j) : vj;
+                        held = lane == res.holder ? node : held;
                     }
-                } else if (lane < deg) {
-                    v = a.full_adj[(size_t)u * deg + lane];
+                    open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
+                    admitted |= 1ull << j;
+                    todo &= (todo - 1) & __ballot(dk < res.worst);
                 }
-                return v;
+                if (admitted) {
+                    n_admit += __popcll(admitted);
+                    if (!kBeside) {
+                        log.append(admitted, dk, id, lane);
+                        if (log.nearly_full()) log.cut(res.worst, lane);
+                    }
+                }
             };
-            int next = open.root_val();
-            int next_row = load_row(next);
-            for (int step = 0; step < max_iter; ++step) {
+            if constexpr (AHEAD) {
+                for (int step = 0; step < max_iter; ++step) {
+                    const int u = open.root_val();
+                    if (u < 0 || open.root_key() >= res.worst) break;
+                    typename Ahead::Found found = ahead.find(u & ~Ahead::kAsked, lane);
+                    int popped_k, popped_v;
+                    open.pop(lane, popped_k, popped_v);
+                    n_expand0 += stage == 0, n_expand1 += stage != 0;
+                    n_adj += deg;
+                    ahead.ids(found, lane);
+                    const int v = found.id;
+                    if (step + 1 < max_iter) ahead.ask(open.A.v, lane);
+                    const bool fresh = v >= 0 && visited.mark(v);
+                    ahead.take(found, lane);
+                    n_dist += __popcll(__ballot(fresh));
+                    const int dk = fresh ? list_key(found.dist) : OpenList<H>::kInf;
+                    // a neighbour that is before all of the list is next
+                    int value = v;
+                    if (__ballot(dk < open.root_key()) && ahead.room()) {
+                        const int best = ~wave_max_key(~dk);
+                        const int at = __builtin_ctzll(__ballot(dk == best));
+                        ahead.give(__builtin_amdgcn_readlane(v, at), lane);
+                        value = lane == at ? v | Ahead::kAsked : v;
+                    }
+                    admit(dk, v, value);
+                }
+            }
+            int next = -1, next_row = -1;
+            if constexpr (!AHEAD) next = open.root_val(), next_row = load_row(next);
+            for (int step = 0; !AHEAD && step < max_iter; ++step) {
                 int uk, u;
                 open.pop(lane, uk, u);
                 PA_TIMER(3);
@@ -337,25 +481,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                 const int dk = list_key(lane < n ? cand_key[lane] : INFINITY);
                 const int id = lane < n ? cand_id[lane] : -1;
                 wave_sync();
-                // heap_update, traverse_cpu.cpp:25-39, in adjacency order
-                unsigned long long todo = __ballot(dk < res.worst);
-                unsigned long long admitted = 0;
-                while (todo) {
-                    const int j = __builtin_ctzll(todo);
-                    const int dj = __builtin_amdgcn_readlane(dk, j);
-                    const int vj = __builtin_amdgcn_readlane(id, j);
-                    if (kBeside) held = lane == res.holder ? vj : held;
-                    open.insert(dj, vj, lane, [&] { res.insert(dj, lane); });
-                    admitted |= 1ull << j;
-                    todo &= (todo - 1) & __ballot(dk < res.worst);
-                }
-                if (admitted) {
-                    n_admit += __popcll(admitted);
-                    if (!kBeside) {
-                        log.append(admitted, dk, id, lane);
-                        if (log.nearly_full()) log.cut(res.worst, lane);
-                    }
-                }
+                admit(dk, id, id);
                 const int root = open.root_val();
                 if (!kEarly || root != next) next = root, next_row = load_row(root);
                 PA_TIMER(6);
@@ -547,12 +673,24 @@ int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_sear
     // 374 -> 286 us, 37 482 -> 322, 512 642 -> 447; beyond that the wavefronts
     // that only read rows take the place of queries: 1536 910 -> 1100 us; two
     // launches of 1024 at a time, H = 128, 2.12 ms with four, 1.91 with one.
-    p->threads = kHelped * kWave;
-    p->fn = pick_kernel<kHelped>(p->H);
+    // Eight where a compute unit has one query at most, seven of them helpers that
+    // read ahead (H = 32, 768 floats: 1 query 229 us with four wavefronts, 181 with
+    // eight; H = 48, 37 queries 342 / 284, 256 394 / 345; H = 128, 100 696 / 537; H =
+    // 512, 9 1787 / 1781; 96 floats, H = 64, 128 267 / 242).  With half the registers
+    // and two queries a compute unit, rows in three trips instead of two, they
+    // were at 204 and 317 us, and 512 queries at 491 against 466.
+    p->threads = kAhead * kWave;
+    p->fn = pick_kernel<kAhead>(p->H);
     if (!p->fn) return PA_E_EF;
     int slots = 0;
     int rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
     if (rc != PA_OK) return rc;
+    if (batch > slots - beside || n_nodes >= LookAhead<1>::kAsked) {
+        p->threads = kHelped * kWave;
+        p->fn = pick_kernel<kHelped>(p->H);
+        rc = residency(p->fn, p->threads, p->lds_bytes, &slots);
+        if (rc != PA_OK) return rc;
+    }
     if (batch > slots - beside) {
         p->threads = kWave;
         p->fn = pick_kernel<1>(p->H);
@@ -603,7 +741,7 @@ extern "C" int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, in
     Plan p;
     const int rc = make_plan(n_nodes, batch, beside, d_model, ef_search, &p);
     if (rc != PA_OK) return rc;
-    if (wavefronts) *wavefronts = p.threads / kWave;
+    if (wavefronts) *wavefronts = p.threads == kWave ? 1 : kHelped;
     return PA_OK;
 }
 

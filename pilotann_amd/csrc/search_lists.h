@@ -718,6 +718,21 @@ struct Visited {
     __device__ __forceinline__ static bool fresh(int state, uint32_t before, int v) {
         return state == 1 || (state == 2 && !((before >> (v & 31)) & 1u));
     }
+    // Whether the table alone shows that node v (>= 0) is marked (looked up
+    // beside the marking: a mark may be missed, none is seen that is not there).
+    __device__ __forceinline__ bool known(int v) const {
+        if (!small) return false;
+        const uint32_t tag = (uint32_t)v >> LOG2;
+        const uint32_t *w = table + kBucketWords * (v & (kBuckets - 1));
+        bool found = false;
+#pragma unroll
+        for (int i = 0; i < kBucketWords; ++i) {
+            const uint32_t word =
+                __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            found |= (word & 0xffffu) == tag || (word >> 16) == tag;
+        }
+        return found;
+    }
     // marks node v (>= 0); true if it was not marked before
     __device__ __forceinline__ bool mark(int v) {
         uint32_t before = 0;
@@ -782,22 +797,33 @@ __device__ __forceinline__ void eval_rows(const float *__restrict__ storage,
     }
 }
 
+// The lanes that `wanted` names first, in order, then the others.
+struct LaneRows {
+    int n;     // wanted
+    int id;    // lane c: the id of the c-th
+    int from;  // and its lane
+    __device__ __forceinline__ LaneRows(bool wanted, int x, int lane) {
+        const unsigned long long mask = __ballot(wanted);
+        n = __popcll(mask);
+        const int to4 = (wanted ? lane_rank(mask) : n + lane_rank(~mask)) << 2;
+        id = __builtin_amdgcn_ds_permute(to4, x);
+        from = __builtin_amdgcn_ds_permute(to4, lane);
+    }
+    __device__ __forceinline__ static int of(int x, int c) {
+        return __builtin_amdgcn_ds_bpermute(c << 2, x);
+    }
+};
+
 // The same for the rows of lanes that `wanted` names, the distance of lane l's row
 // to dist[l] (LDS).
 template <int DP8, bool TWO>
 __device__ __forceinline__ void eval_lanes(const float *__restrict__ storage, const float *qv,
                                            bool wanted, int id, float *dist, int dp, int lane) {
-    const unsigned long long mask = __ballot(wanted);
-    const int n = __popcll(mask);
-    if (n == 0) return;
-    // the wanted lanes first, in order, then the others: lane c gets row c's id
-    // and the lane that is from
-    const int to4 = (wanted ? lane_rank(mask) : n + lane_rank(~mask)) << 2;
-    const int row_id = __builtin_amdgcn_ds_permute(to4, id);
-    const int from = __builtin_amdgcn_ds_permute(to4, lane);
+    const LaneRows rows(wanted, id, lane);
+    const int n = rows.n, row_id = rows.id, from = rows.from;
     const int quad = lane >> 2, part = lane & 3;
     const float2 *qq = reinterpret_cast<const float2 *>(qv) + part * query_run(dp >> 3);
-    auto of = [](int x, int c) { return __builtin_amdgcn_ds_bpermute(c << 2, x); };
+    auto of = [](int x, int c) { return LaneRows::of(x, c); };
     int base = 0;
     if constexpr (TWO && DP8 > 0 && DP8 % 2 == 0) {
         for (; base + kRowsPerPass < n; base += 2 * kRowsPerPass) {
@@ -840,15 +866,22 @@ __device__ __forceinline__ void eval_lanes(const float *__restrict__ storage, co
 // that claimed it.  LDS operations of a wavefront take effect in order.  A slot
 // that holds a node is always taken and finished, so every wait of the search
 // ends; a helper returns at kExit, which the search gives when all are idle.
-template <int HELPERS>
+//
+// With PARTS = 2 a slot is two jobs, for two helpers: the even lanes' neighbours and
+// the odd lanes'.
+template <int HELPERS, int PARTS = 1>
 struct LookAhead {
     static constexpr int kIdle = -1, kTaken = -2, kExit = -3;   // else: the node to do
+    static constexpr bool kEarlyIds = PARTS == 2;    // ids() is called before take()
+    static constexpr int kUnset = (int)0x80000000;   // a neighbour not there yet
     static constexpr int kSlots = HELPERS > 0 ? 8 : 1;
+    static constexpr int kJobs = kSlots * PARTS;   // of slot s: s, s + kSlots
+    static_assert(PARTS == 1 || PARTS == 2, "see slots_idle()");
     // Set in the open list's value of a node that has been put into a slot.
     static constexpr int kAsked = 1 << 30;
     static constexpr unsigned long long kTop = 0xfe;   // its first seven cells
     struct Slots {
-        int job[kSlots];
+        int job[kJobs];
         int ids[kSlots][HELPERS > 0 ? kWave : 4];
         float dist[kSlots][HELPERS > 0 ? kWave : 4];
     };
@@ -872,30 +905,37 @@ struct LookAhead {
     template <class WORK>
     __device__ __forceinline__ static void help(Slots &slots, int lane, WORK &&work) {
         for (;;) {
-            const int job = get(slots.job[lane & (kSlots - 1)]);
+            const int job = get(slots.job[lane & (kJobs - 1)]);
             if (__ballot(job == kExit)) return;
             const unsigned long long todo = __ballot(job >= 0);
             if (!todo) {
                 __builtin_amdgcn_s_sleep(1);
                 continue;
             }
-            const int slot = __builtin_ctzll(todo) & (kSlots - 1);
-            const int node = __builtin_amdgcn_readlane(job, slot);
+            const int mine = __builtin_ctzll(todo) & (kJobs - 1);
+            const int node = __builtin_amdgcn_readlane(job, mine);
             int was = node;
-            if (lane == 0) was = atomicCAS(&slots.job[slot], node, kTaken);
+            if (lane == 0) was = atomicCAS(&slots.job[mine], node, kTaken);
             if (uni(was) != node) continue;   // another helper was first
             in_order();
-            work(node, slots.ids[slot], slots.dist[slot]);
+            const int slot = mine & (kSlots - 1);
+            work(node, mine, slots.ids[slot], slots.dist[slot]);
             in_order();
-            if (lane == 0) put(slots.job[slot], kIdle);
+            if (lane == 0) put(slots.job[mine], kIdle);
         }
     }
 
-    __device__ __forceinline__ void look(int lane) {
-        idle = __ballot(get(slots.job[lane & (kSlots - 1)]) == kIdle);
+    // (bits 0 .. kSlots - 1 count)
+    __device__ __forceinline__ static unsigned long long slots_idle(int job) {
+        const unsigned long long jobs = __ballot(job == kIdle);
+        return PARTS == 2 ? jobs & jobs >> kSlots : jobs;
     }
+    __device__ __forceinline__ void look(int lane) {
+        idle = slots_idle(get(slots.job[lane & (kJobs - 1)]));
+    }
+    // Nothing is asked for; all slots are idle.
     __device__ __forceinline__ void begin(int lane) {
-        in_order();   // the query and the entries' marks are in LDS
+        in_order();   // what the helpers are to read is in LDS
         node = -1, ring = 0;
         look(lane);
     }
@@ -905,7 +945,9 @@ struct LookAhead {
     __device__ __forceinline__ int give(int what, int lane) {
         const int old = __builtin_amdgcn_readlane(node, ring);
         node = lane == ring ? what : node;
-        if (lane == ring) put(slots.job[lane], what);
+        if (kEarlyIds) put(slots.ids[ring][lane], kUnset);
+        if (PARTS == 1 ? lane == ring : lane < kJobs && (lane & (kSlots - 1)) == ring)
+            put(slots.job[lane], what);
         idle &= ~(1ull << ring);
         ring = (ring + 1) & (kSlots - 1);
         return old;
@@ -921,16 +963,31 @@ struct LookAhead {
         top = lane == at ? top | kAsked : top;
         top = top == (old | kAsked) && old >= 0 ? old : top;
     }
+    // Puts the node whose key is the lowest into a slot, if there is room: the
+    // entries' best are known before the list is made of them.  `value`: by lane, the
+    // node or what is below 0; the one put is flagged in it.
+    __device__ __forceinline__ void ask_lowest(int key, int &value, int lane) {
+        const int best = ~wave_max_key(~((unsigned)value < (unsigned)kAsked ? key : 0x7fffffff));
+        const unsigned long long at = __ballot((unsigned)value < (unsigned)kAsked && key == best);
+        if (!at || !room()) return;
+        const int l = __builtin_ctzll(at);
+        give(__builtin_amdgcn_readlane(value, l), lane);
+        value = lane == l ? value | kAsked : value;
+    }
     // What the slot of the node popped holds: its neighbours (by lane, -1: none)
     // and the distances of those that were not marked yet when it was asked for.
-    // In two parts, with the pop between them: it is read at once, in the hope that
-    // the helper is done (`job`, read before the rest), and again if it was not.
+    // All of it is read at once when the node is known, in the hope that the helper
+    // is done (`job`, read before the rest), so that it travels beside the pop.
+    // Then take() waits for all of it, or, where rows are long and marking takes
+    // time, ids() for the neighbours alone, which are there before their rows are
+    // read, and take() later (short rows: 128 queries, 32 floats, 372 us without ids(),
+    // 401 with it).
     struct Found {
         int slot, job, id;
         float dist;
     };
     __device__ __forceinline__ void read(Found &f, int lane) const {
-        f.job = get(slots.job[lane & (kSlots - 1)]);
+        f.job = get(slots.job[lane & (kJobs - 1)]);
         asm volatile("" ::: "memory");
         f.id = get(slots.ids[f.slot][lane]);
         f.dist = get(slots.dist[f.slot][lane]);
@@ -950,21 +1007,35 @@ struct LookAhead {
         __builtin_amdgcn_sched_barrier(0);
         return f;
     }
+    // Come after find() and, the first that is called, before the next give().
+    __device__ __forceinline__ void ids(Found &f, int lane) {
+        static_assert(kEarlyIds, "the slots' neighbours are unset when they are given");
+        idle = slots_idle(f.job);
+        while (__ballot(f.id == kUnset)) f.id = get(slots.ids[f.slot][lane]);
+    }
     __device__ __forceinline__ void take(Found &f, int lane) {
-        idle = __ballot(f.job == kIdle);
-        while (!((idle >> f.slot) & 1)) {
+        unsigned long long there = slots_idle(f.job);
+        if (!kEarlyIds) idle = there;
+        while (!((there >> f.slot) & 1)) {
             read(f, lane);
-            idle = __ballot(f.job == kIdle);
+            idle = there = slots_idle(f.job);
         }
         in_order();   // read before the slot is used again
     }
     // All slots are idle.
     __device__ __forceinline__ void drain(int lane) {
         do look(lane);
-        while (~idle);
+        while (~idle & ((1ull << kSlots) - 1));
+    }
+    // A job for every helper, 0 .. HELPERS - 1 (all slots are idle), whose results
+    // have a place of their own.
+    __device__ __forceinline__ void give_all(int what, int lane) const {
+        static_assert(HELPERS <= kJobs, "a job for every helper");
+        in_order();
+        if (lane < HELPERS) put(slots.job[lane], what);
     }
     __device__ __forceinline__ void end(int lane) const {
-        if (lane < kSlots) put(slots.job[lane], kExit);
+        if (lane < kJobs) put(slots.job[lane], kExit);
     }
 };
 

@@ -173,10 +173,10 @@ __global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_
     Helped ahead{slots, -1, 0, 0};
     if constexpr (WAVES > 1) {
         const int wave = uni((int)(threadIdx.x / kWave));
-        if (threadIdx.x < Helped::kSlots) Helped::put(slots.job[threadIdx.x], Helped::kIdle);
+        if (threadIdx.x < Helped::kJobs) Helped::put(slots.job[threadIdx.x], Helped::kIdle);
         __syncthreads();   // the only barrier
         if (wave > 0) {
-            Helped::help(slots, lane, [&](int row, int *ids, float *dist) {
+            Helped::help(slots, lane, [&](int row, int, int *ids, float *dist) {
                 // its neighbours, by lane, and the distances of those that are not
                 // marked yet: a mark is never taken back, so whatever is new when
                 // the node is popped is among them
@@ -258,8 +258,15 @@ __global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_
                     }
                 }
             }
-            open.push_entries(__ballot(u >= 0), list_key(d),
-                              row >= 0 ? row : -2 - i, lane);
+            int value = row >= 0 ? row : u >= 0 ? -2 - i : -1;
+            if constexpr (WAVES > 1) {
+                if (base == 0) {
+                    ahead.begin(lane);
+                    for (int j = 0; j < WAVES - 1; ++j)
+                        ahead.ask_lowest(list_key(d), value, lane);
+                }
+            }
+            open.push_entries(__ballot(u >= 0), list_key(d), value, lane);
         }
 
         PA_TIMER(5);
@@ -325,8 +332,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_
             }
         };
         if constexpr (WAVES > 1) {
-            ahead.begin(lane);
-            for (int i = 0; i < WAVES - 1; ++i) ahead.ask(open.A.v, lane);
+            if (a.n_init == 0) ahead.begin(lane);
             for (int step = 0; step < a.max_iter; ++step) {
                 const int u = open.root_val();
                 if (u == -1 || open.root_key() >= res.worst) break;
