@@ -288,10 +288,8 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
     visited.dirty = true;
     visited.clean(a.words_per_slot, lane);
 
-    for (;;) {
-        int q = 0;
-        if (lane == 0) q = atomicAdd(a.work_counter, 1);
-        q = uni(q);
+    for (int turn = 0;;) {
+        const int q = next_query(a.work_counter, turn, a.batch, lane);
         if (q >= a.batch) {
             if constexpr (AHEAD) {
                 ahead.drain(lane);
@@ -778,7 +776,7 @@ extern "C" int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, fl
     a.init_I = init_I, a.init_D = init_D;
     a.sub_adj = sub_adj, a.sub_gid = sub_gid, a.sub_mapping = sub_mapping;
     a.full_adj = full_adj, a.storage = storage, a.query = query;
-    a.work_counter = reinterpret_cast<int *>(workspace);
+    a.work_counter = p.n_slots < batch ? reinterpret_cast<int *>(workspace) : nullptr;
     a.seen = reinterpret_cast<uint32_t *>(
         reinterpret_cast<unsigned char *>(workspace) + kWorkCounterBytes);
     a.counters = reinterpret_cast<unsigned long long *>(counters);
@@ -793,7 +791,7 @@ extern "C" int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, fl
     a.sort_n = p.sort_n;
 
     hipStream_t stream = (hipStream_t)stream_;
-    reset_refine_counter<<<1, 1, 0, stream>>>(a.work_counter);
+    if (a.work_counter) reset_refine_counter<<<1, 1, 0, stream>>>(a.work_counter);
     p.fn<<<p.n_slots, p.threads, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
 }

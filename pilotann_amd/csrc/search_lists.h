@@ -18,6 +18,16 @@ constexpr int kWorkCounterBytes = 256; // head of the workspace
 constexpr int kSeenCacheLog2 = PA_SEEN_LOG2;
 constexpr int kSeenCache = 1 << kSeenCacheLog2;  // LDS words remembering visited rows
 
+// The next query of a workgroup.  Where every query has its workgroup (no
+// `counter`) it is the workgroup's own number, once: no launch that sets a
+// counter, no trip to memory for it.  `turn`: how many this workgroup had.
+__device__ __forceinline__ int next_query(int *counter, int &turn, int batch, int lane) {
+    if (!counter) return turn++ ? batch : (int)blockIdx.x;
+    int q = 0;
+    if (lane == 0) q = atomicAdd(counter, 1);
+    return uni(q);
+}
+
 // ---- open list: heapq.cuh, top of the heap in registers ----------------------
 //
 // The reference's open list is an array heap of 2H cells with the sift rules

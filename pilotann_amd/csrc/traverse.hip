@@ -196,10 +196,8 @@ __global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_
     log.capacity = ResultLog::capacity_for(H);
     open.deep = log.entry + ResultLog::capacity_for(H);
 
-    for (;;) {
-        int q = 0;
-        if (lane == 0) q = atomicAdd(a.work_counter, 1);
-        q = uni(q);
+    for (int turn = 0;;) {
+        const int q = next_query(a.work_counter, turn, a.batch, lane);
         if (q >= a.batch) {
             if constexpr (WAVES > 1) ahead.end(lane);
             break;
@@ -1029,7 +1027,7 @@ int launch_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
     a.adj = adj, a.gid = gid, a.mapping = mapping;
     a.storage = storage, a.query = query;
     a.init_I = init_I, a.init_D = init_D;
-    a.work_counter = reinterpret_cast<int *>(workspace);
+    a.work_counter = p.n_slots < batch ? reinterpret_cast<int *>(workspace) : nullptr;
     a.seen = reinterpret_cast<uint32_t *>(
         reinterpret_cast<unsigned char *>(workspace) + kWorkCounterBytes);
     a.counters = reinterpret_cast<unsigned long long *>(counters);
@@ -1042,7 +1040,7 @@ int launch_traverse(int64_t *out_I, float *out_D, const int32_t *adj,
     a.slot_stride = p.slot_stride;
 
     hipStream_t stream = (hipStream_t)stream_;
-    reset_work_counter<<<1, 1, 0, stream>>>(a.work_counter);
+    if (a.work_counter) reset_work_counter<<<1, 1, 0, stream>>>(a.work_counter);
     p.fn<<<p.n_slots, p.threads, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
 }

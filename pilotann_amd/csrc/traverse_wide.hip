@@ -210,10 +210,8 @@ __global__ __launch_bounds__(kWave) void wide_kernel(WideArgs a) {
     const int deg = a.deg;
     uint32_t *seen = a.seen + (size_t)blockIdx.x * (size_t)a.words_per_slot;
 
-    for (;;) {
-        int q = 0;
-        if (lane == 0) q = atomicAdd(a.work_counter, 1);
-        q = uni(q);
+    for (int turn = 0;;) {
+        const int q = next_query(a.work_counter, turn, a.batch, lane);
         if (q >= a.batch) break;
         unsigned n_expand = 0, n_adj = 0, n_dist = 0, n_admit = 0;
 
@@ -528,7 +526,7 @@ extern "C" int pa_traverse_wide(int64_t *out_I, float *out_D, const int32_t *adj
     a.adj = adj, a.gid = gid, a.mapping = mapping;
     a.storage = storage, a.query = query;
     a.init_I = init_I, a.init_D = init_D;
-    a.work_counter = reinterpret_cast<int *>(workspace);
+    a.work_counter = p.n_slots < batch ? reinterpret_cast<int *>(workspace) : nullptr;
     a.seen = reinterpret_cast<uint32_t *>(
         reinterpret_cast<unsigned char *>(workspace) + kWorkCounterBytes);
     a.counters = reinterpret_cast<unsigned long long *>(counters);
@@ -539,7 +537,7 @@ extern "C" int pa_traverse_wide(int64_t *out_I, float *out_D, const int32_t *adj
     a.words_per_slot = p.words_per_slot;
 
     hipStream_t stream = (hipStream_t)stream_;
-    reset_wide_counter<<<1, 1, 0, stream>>>(a.work_counter);
+    if (a.work_counter) reset_wide_counter<<<1, 1, 0, stream>>>(a.work_counter);
     p.fn<<<p.n_slots, kWave, p.lds_bytes, stream>>>(a);
     return (int)hipGetLastError();
 }
