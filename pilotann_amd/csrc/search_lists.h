@@ -679,21 +679,20 @@ struct Visited {
     uint32_t *bits;   // device memory: one bit per node, zero between queries
     bool small;       // tags fit 16 bits (0xffff marks a free slot)
     bool dirty;       // this lane has set a bit in `bits`
+    bool zeroed;      // uniform: `bits` has been cleared
 
     __device__ __forceinline__ void init(uint32_t *lds_words, uint32_t *slice,
                                          int n_nodes) {
         table = lds_words, bits = slice;
         small = n_nodes <= (0xffff << LOG2);
-        dirty = false;
+        dirty = zeroed = false;
     }
     __device__ __forceinline__ void reset(int lane) {
         for (int i = lane; i < kWords; i += kWave) table[i] = 0xffffffffu;
     }
-    // Marks node v (>= 0).  Returns 0: it was marked before; 1: it was not;
-    // 2: the bitmask was asked, `before` will hold its word as it was (the
-    // caller may look at it later, so that the atomic's round trip overlaps
-    // other work): fresh() tells.
-    __device__ __forceinline__ int probe(int v, uint32_t &before) {
+    // Marks node v (>= 0) in the table.  Returns 0: it was marked before; 1: it
+    // was not; 2: the bitmask has to be asked.
+    __device__ __forceinline__ int probe(int v) {
         if (small) {
             const uint32_t tag = (uint32_t)v >> LOG2;
             uint32_t *w = table + kBucketWords * (v & (kBuckets - 1));
@@ -721,12 +720,7 @@ struct Visited {
                 if (atomicCAS(w + (at >> 1), old, neu) == old) return 1;
             }
         }
-        dirty = true;
-        before = atomicOr(&bits[v >> 5], 1u << (v & 31));
         return 2;
-    }
-    __device__ __forceinline__ static bool fresh(int state, uint32_t before, int v) {
-        return state == 1 || (state == 2 && !((before >> (v & 31)) & 1u));
     }
     // Whether the table alone shows that node v (>= 0) is marked (looked up
     // beside the marking: a mark may be missed, none is seen that is not there).
@@ -743,20 +737,32 @@ struct Visited {
         }
         return found;
     }
-    // marks node v (>= 0); true if it was not marked before
-    __device__ __forceinline__ bool mark(int v) {
-        uint32_t before = 0;
-        const int state = probe(v, before);
-        return fresh(state, before, v);
+    // Marks the lanes' nodes v (negative: none), all lanes together; true in a
+    // lane whose node was not marked before.  The slice of `words` is cleared when
+    // it is asked for the first time.
+    __device__ __forceinline__ bool mark(int v, int words, int lane) {
+        const int state = v >= 0 ? probe(v) : 0;
+        bool is_new = state == 1;
+        if (__ballot(state == 2)) {
+            if (!zeroed) clear(words, lane);
+            zeroed = true;
+            if (state == 2) {
+                dirty = true;
+                is_new = !((atomicOr(&bits[v >> 5], 1u << (v & 31)) >> (v & 31)) & 1u);
+            }
+        }
+        return is_new;
+    }
+    __device__ __forceinline__ void clear(int words, int lane) {
+        for (int w = lane * 4; w < words; w += kWave * 4)
+            *reinterpret_cast<uint4 *>(bits + w) = make_uint4(0, 0, 0, 0);
+        // (only this wavefront touches the slice)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     // after a query: the slice back to zero if any lane touched it
     __device__ __forceinline__ void clean(int words, int lane) {
-        if (__ballot(dirty)) {
-            for (int w = lane * 4; w < words; w += kWave * 4)
-                *reinterpret_cast<uint4 *>(bits + w) = make_uint4(0, 0, 0, 0);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            dirty = false;
-        }
+        if (__ballot(dirty)) clear(words, lane);
+        dirty = false;
     }
 };
 
