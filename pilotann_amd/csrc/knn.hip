@@ -495,17 +495,31 @@ __global__ __launch_bounds__(kWave * kRankWaves) void merge_kernel(
     for (int seg = 1; seg < n_seg; ++seg) {
         const size_t at = (size_t)seg * m + row;
         const int cnt = uni(count[at]);
-        for (int base = 0; base < cnt; base += kWave) {
-            const int i = base + lane;
-            const float x = i < cnt ? score[at * kCap + i] : INFINITY;
-            const bool in = i < cnt && x < limit;
-            const unsigned long long mask = __ballot(in);
-            if (in) {
-                my_score[n + lane_rank(mask)] = x;
-                my_id[n + lane_rank(mask)] = id[at * kCap + i];
+        // up to 256 entries of the segment's list in one trip (64 at a time, and their
+        // ids behind the comparison: 1024 rows of 4 lists 36 us, now 25; 8192 of 8
+        // lists 104, now 74)
+        constexpr int kAtOnce = KEEP < 256 ? KEEP / kWave : 4;
+        for (int base = 0; base < cnt; base += kAtOnce * kWave) {
+            float x[kAtOnce];
+            int32_t node[kAtOnce];
+#pragma unroll
+            for (int r = 0; r < kAtOnce; ++r) {
+                const int i = base + r * kWave + lane;
+                x[r] = i < cnt ? score[at * kCap + i] : INFINITY;
+                node[r] = i < cnt ? id[at * kCap + i] : -1;
             }
-            n += __popcll(mask);
-            if (n > kCap - kWave) cut();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < kAtOnce; ++r) {
+                const bool in = base + r * kWave + lane < cnt && x[r] < limit;
+                const unsigned long long mask = __ballot(in);
+                if (in) {
+                    my_score[n + lane_rank(mask)] = x[r];
+                    my_id[n + lane_rank(mask)] = node[r];
+                }
+                n += __popcll(mask);
+                if (n > kCap - kWave) cut();
+            }
         }
     }
     if (n > KEEP) cut();
@@ -534,6 +548,27 @@ __device__ __forceinline__ float team_square_dist(const floatx4 *mine, const flo
 #pragma unroll
     for (int step = 8; step >= 1; step >>= 1) sum += __shfl_xor(sum, step, 16);
     return sum;
+}
+
+// The same for two rows, whose loads are in flight together.
+__device__ __forceinline__ void team_square_dists(const floatx4 *mine, const floatx4 *row0,
+                                                  const floatx4 *row1, int d4, int place,
+                                                  float &sum0, float &sum1) {
+    sum0 = sum1 = 0.f;
+    for (int i = place; i < d4; i += 16) {
+        const floatx4 x = row0[i], z = row1[i], y = mine[i];
+        const float e0 = x[0] - y[0], e1 = x[1] - y[1], e2 = x[2] - y[2], e3 = x[3] - y[3];
+        const float f0 = z[0] - y[0], f1 = z[1] - y[1], f2 = z[2] - y[2], f3 = z[3] - y[3];
+        sum0 = fmaf(e0, e0, sum0), sum1 = fmaf(f0, f0, sum1);
+        sum0 = fmaf(e1, e1, sum0), sum1 = fmaf(f1, f1, sum1);
+        sum0 = fmaf(e2, e2, sum0), sum1 = fmaf(f2, f2, sum1);
+        sum0 = fmaf(e3, e3, sum0), sum1 = fmaf(f3, f3, sum1);
+    }
+#pragma unroll
+    for (int step = 8; step >= 1; step >>= 1) {
+        sum0 += __shfl_xor(sum0, step, 16);
+        sum1 += __shfl_xor(sum1, step, 16);
+    }
 }
 
 // Exact squared distances from query row first + q to its candidates.  A
@@ -575,7 +610,7 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rerank_kernel(
 // (36 passes of two exchanges a lane) hides behind other wavefronts' reads,
 // where ranking in steps of torch (ids widened, top-k, gather, masks) wrote and
 // read the table several times.
-template <int KEEP>
+template <int KEEP, bool TWO>
 __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     const float *__restrict__ rows, const float *__restrict__ cand_score,
     const int32_t *__restrict__ cand_id, const int32_t *__restrict__ count,
@@ -595,21 +630,52 @@ __global__ __launch_bounds__(kWave * kRankWaves) void rank_kernel(
     if (q >= m) return;
     const floatx4 *src = reinterpret_cast<const floatx4 *>(rows + (size_t)(first + q) * d);
     for (int i = lane; i < d4; i += kWave) mine[i] = src[i];
-    for (int i = lane; i < KEEP; i += kWave) entry[i] = ~0ull;
-    wave_sync();
     const int32_t *ids = cand_id + (size_t)q * kCap;
     const int cnt = min(KEEP, uni(count[q]));
+    // the list, an id a lane and 64 of them a register; what an entry holds below
+    // its distance
+    int32_t held[KEEP / kWave];
+#pragma unroll
+    for (int r = 0; r < KEEP / kWave; ++r) {
+        const int j = r * kWave + lane;
+        held[r] = j < cnt ? ids[j] : -1;
+        const unsigned score =
+            merged && j < cnt ? ordered(cand_score[(size_t)q * kCap + j]) : 0u;
+        entry[j] = j < cnt ? (score & ~kPlaces) | (unsigned)j : ~0ull;
+    }
+    wave_sync();
     const int team = lane >> 4, place = lane & 15;
-    for (int j0 = 0; j0 < cnt; j0 += 4) {
-        const int j = j0 + team;
-        const int32_t id = j < cnt ? ids[j] : -1;
-        const bool ok = id >= 0 && id < n && id != first + q;
-        const float sum = team_square_dist(
-            mine, reinterpret_cast<const floatx4 *>(rows + (ok ? (size_t)id * d : 0)), d4, place, ok);
-        if (place == 0 && j < cnt) {
-            const unsigned score = merged ? ordered(cand_score[(size_t)q * kCap + j]) : 0u;
-            entry[j] = ((unsigned long long)__float_as_uint(ok ? sum : INFINITY) << 32) |
-                       (score & ~kPlaces) | (unsigned)j;
+    unsigned *high = reinterpret_cast<unsigned *>(entry) + 1;
+#pragma unroll
+    for (int r = 0; r < KEEP / kWave; ++r) {
+        const int here = min(kWave, cnt - r * kWave);
+        for (int j0 = 0; !TWO && j0 < here; j0 += 4) {
+            const int at = r * kWave + j0 + team;
+            const int32_t id = __shfl(held[r], j0 + team);
+            const bool ok = id >= 0 && id < n && id != first + q;
+            const float sum = team_square_dist(
+                mine, reinterpret_cast<const floatx4 *>(rows + (ok ? (size_t)id * d : 0)), d4,
+                place, ok);
+            if (place == 0 && at < cnt) high[2 * at] = __float_as_uint(ok ? sum : INFINITY);
+        }
+#pragma unroll 1
+        for (int j0 = 0; TWO && j0 < here; j0 += 8) {
+            // two candidates a team, their rows requested together
+            const int j = j0 + team;
+            const int32_t id0 = __shfl(held[r], j), id1 = __shfl(held[r], j + 4);
+            const bool ok0 = id0 >= 0 && id0 < n && id0 != first + q;
+            const bool ok1 = id1 >= 0 && id1 < n && id1 != first + q;
+            const floatx4 *row0 =
+                reinterpret_cast<const floatx4 *>(rows + (ok0 ? (size_t)id0 * d : 0));
+            const floatx4 *row1 =
+                reinterpret_cast<const floatx4 *>(rows + (ok1 ? (size_t)id1 * d : 0));
+            float sum0, sum1;
+            team_square_dists(mine, row0, row1, d4, place, sum0, sum1);
+            if (place == 0) {
+                const int at = r * kWave + j;
+                if (at < cnt) high[2 * at] = __float_as_uint(ok0 ? sum0 : INFINITY);
+                if (at + 4 < cnt) high[2 * at + 8] = __float_as_uint(ok1 ? sum1 : INFINITY);
+            }
         }
     }
     wave_sync();
@@ -1084,14 +1150,22 @@ extern "C" int pa_knn_rank(int64_t *out_id, float *out_dist, float *cand_score,
     hipStream_t stream = (hipStream_t)stream_;
     const unsigned blocks = (unsigned)((m + kRankWaves - 1) / kRankWaves);
     const unsigned lds = (unsigned)(kRankWaves * (d * sizeof(float) + keep * 8));
+    // Two candidates a team at a time where few rows are ranked, which is a chain of
+    // trips to memory, or rows are short; else one, whose rows stay in L2.  Kernel
+    // alone, one / two, us, 96 floats: 1024 rows 62 / 42, 8192 123 / 84; 768 floats: 1024
+    // 178 / 118, 4096 296 / 189, 8192 378 / 485, 54 464 4855 / 5473; builds of 150 000
+    // x 256 37.7 (one from 8192 rows on) / 38.5 ms.
+    const bool two = m <= 4096 || d <= 128;
 #define PA_RANK(KEEP_)                                                                        \
     {                                                                                         \
         if (n_seg > 1)                                                                        \
             merge_kernel<KEEP_><<<blocks, kWave * kRankWaves, 0, stream>>>(                   \
                 cand_score, cand_id, cand_count, m, n_seg);                                   \
-        rank_kernel<KEEP_><<<blocks, kWave * kRankWaves, lds, stream>>>(                      \
-            rows, cand_score, cand_id, cand_count, out_id, out_dist, m, first, n, d, k,       \
-            hide_inf, n_seg > 1);                                                             \
+        (two ? rank_kernel<KEEP_, true> : rank_kernel<KEEP_, false>)                          \
+            <<<blocks, kWave * kRankWaves, lds, stream>>>(rows, cand_score, cand_id,          \
+                                                          cand_count, out_id, out_dist, m,    \
+                                                          first, n, d, k, hide_inf,           \
+                                                          n_seg > 1);                         \
     }
     switch (keep) {
         case 64: PA_RANK(64) break;
