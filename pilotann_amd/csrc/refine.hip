@@ -231,8 +231,9 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
                     const int stage = uni(Ahead::get(lds.job_stage));
                     const bool mine = (lane & 1) == job / Ahead::kSlots;
                     v = neighbours(stage, stage == 0 ? a.sub_deg : a.full_deg, node);
-                    if (mine) ids[lane] = v;
-                    wanted = mine && v >= 0 && !marks.known(v);
+                    wanted = Ahead::look_then_show(
+                        v, mine, [&](int u) { return marks.known(u); },
+                        [] { Ahead::in_order(); }, [&](int u) { Ahead::put(ids[lane], u); });
                 }
                 eval_lanes_from<kRefineChunk<WAVES>>(a.storage, qv, wanted, v, dist, d, from,
                                                      lane);

@@ -941,6 +941,24 @@ struct LookAhead {
         }
     }
 
+    // What a helper does before it reads rows, in this order: look which neighbours
+    // are marked, have the answers, and only then show the search their numbers.
+    // The search marks what ids() gives it at once, before it takes the distances: a
+    // helper that looked after that would take the node's own marks for older ones
+    // and leave distances out that the search is about to use.  `v`: the lane's
+    // neighbour, -1 for none; `mine`: it is of this helper's part.  Returns whether the
+    // lane's row is to be read.  (Of functions, so that a test can stand between them.)
+    template <class MARKED, class ANSWERED, class SHOW>
+    __host__ __device__ __forceinline__ static bool look_then_show(int v, bool mine,
+                                                                   const MARKED &marked,
+                                                                   const ANSWERED &answered,
+                                                                   const SHOW &show) {
+        const bool wanted = mine && v >= 0 && !marked(v);
+        answered();
+        if (mine) show(v);
+        return wanted;
+    }
+
     // (bits 0 .. kSlots - 1 count)
     __device__ __forceinline__ static unsigned long long slots_idle(int job) {
         const unsigned long long jobs = __ballot(job == kIdle);
