@@ -634,7 +634,8 @@ struct Plan {
 #endif
 constexpr int kMaxWavesPerCu = PA_REFINE_MAX_WAVES;
 
-// Workgroups of `fn` the current device holds at once.
+// Workgroups of `fn` the current device holds at once (none where one does not fit a
+// compute unit's LDS).
 int residency(RefineFn fn, int threads, int lds_bytes, int *slots) {
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -651,7 +652,6 @@ int residency(RefineFn fn, int threads, int lds_bytes, int *slots) {
             e = workgroups_per_cu(reinterpret_cast<const void *>(fn), dev, threads, lds_bytes,
                                   &per_cu);
         if (e != hipSuccess) return (int)e;
-        if (per_cu < 1) per_cu = 1;
         if (per_cu > kMaxWavesPerCu) per_cu = kMaxWavesPerCu;
         it = known.emplace(key, per_cu * cus).first;
     }
@@ -681,6 +681,8 @@ int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_sear
     // 512, 9 1787 / 1781; 96 floats, H = 64, 128 267 / 242).  With half the registers
     // and two queries a compute unit, rows in three trips instead of two, they
     // were at 204 and 317 us, and 512 queries at 491 against 466.
+    // (Their slots are 4 KB of LDS: of the longest rows a query fits beside them in the
+    // other forms alone, and has no workgroup here.)
     p->threads = kAhead * kWave;
     p->fn = pick_kernel<kAhead>(p->H);
     if (!p->fn) return PA_E_EF;
@@ -700,7 +702,7 @@ int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_sear
         if (rc != PA_OK) return rc;
     }
     if (slots > batch) slots = (int)batch;
-    if (slots < 1) slots = 1;
+    if (slots < 1) slots = 1;   // (no query, or rows that fit no form: the launch says so)
     p->n_slots = slots;
     p->words_per_slot = round_up((n_nodes + 31) / 32, kSlotAlignWords);
     // a slot: the visited slice, then the log of admitted candidates (lists of
