@@ -90,9 +90,10 @@ __global__ __launch_bounds__(256) void fill_rows(ReverseArgs a) {
          r += (int64_t)gridDim.x * per_block) {
         int64_t *out = a.adj + r * a.degree;
         const int64_t to = lane < a.m ? a.forward[r * a.m + lane] : -1;
-        const unsigned long long valid = __ballot(to >= 0);
+        const bool edge = to >= 0 && to < a.n;
+        const unsigned long long valid = __ballot(edge);
         const int place = lane_rank(valid);
-        if (to >= 0 && place < a.degree) out[place] = to;
+        if (edge && place < a.degree) out[place] = to;
         const int used = min(a.degree, (int)__popcll(valid));
         const int64_t first = r > 0 ? a.end[r - 1] : 0, last = a.end[r];
         // the smallest 64 so far, in order over the lanes

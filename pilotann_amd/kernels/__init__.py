@@ -541,8 +541,8 @@ def graph_reachable(adj: torch.Tensor, sources: torch.Tensor, reverse: bool = Fa
 
 def graph_add_reverse(forward: torch.Tensor, degree: int):
     """Rows of ``degree`` slots (``pa_graph_add_reverse``): the edges of
-    ``forward`` ``[n, m]`` (int64 on the device, negative: none), then the nodes
-    that point at the row's node and are not in ``forward``'s row, lowest place
+    ``forward`` ``[n, m]`` (int64 on the device; what is not in ``0 .. n - 1`` is
+    none), then the nodes that point at the row's node and are not in ``forward``'s row, lowest place
     first, then lowest number, until the row is full.  ``-1`` pads."""
     _check(forward, 'forward', 2, torch.int64, True)
     n, m = forward.shape

@@ -3,6 +3,7 @@ the same rows, place for place."""
 import pytest
 import torch
 
+from pilotann_amd import kernels
 from pilotann_amd.utils import graphs
 
 pytestmark = pytest.mark.gpu
@@ -28,6 +29,18 @@ def test_same_rows_as_on_the_host(n, m, degree, edges, device):
         forward[:] = -1
     want = graphs._add_reverse(forward, degree)
     got = graphs._add_reverse(forward.to(device), degree)
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize('n,m,degree', [(1, 1, 1), (65, 9, 12), (3000, 48, 48), (3000, 64, 20)])
+def test_a_number_beyond_the_nodes_is_no_edge(n, m, degree, device):
+    g = torch.Generator().manual_seed(n + m)
+    forward = torch.randint(-1, n, (n, m), generator=g)
+    none = torch.rand(n, m, generator=g) < 0.3
+    beyond = torch.tensor([n, n + 1, (1 << 31) - 1, 1 << 31, 1 << 40])
+    beyond = beyond[torch.randint(5, (n, m), generator=g)]
+    got = kernels.graph_add_reverse(torch.where(none, beyond, forward).to(device), degree)
+    want = graphs._add_reverse(forward.masked_fill(none, -1), degree)
     assert torch.equal(got.cpu(), want)
 
 
