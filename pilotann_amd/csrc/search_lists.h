@@ -980,6 +980,9 @@ struct LookAhead {
         const int old = __builtin_amdgcn_readlane(node, ring);
         node = lane == ring ? what : node;
         if (kEarlyIds) put(slots.ids[ring][lane], kUnset);
+        // (not the other way round, also not by the compiler: a helper's neighbours would
+        // be unset again, and ids() would wait for them for ever)
+        asm volatile("" ::: "memory");
         if (PARTS == 1 ? lane == ring : lane < kJobs && (lane & (kSlots - 1)) == ring)
             put(slots.job[lane], what);
         idle &= ~(1ull << ring);
@@ -1060,6 +1063,7 @@ struct LookAhead {
     __device__ __forceinline__ void drain(int lane) {
         do look(lane);
         while (~idle & ((1ull << kSlots) - 1));
+        asm volatile("" ::: "memory");   // (what helpers read is not changed before)
     }
     // A job for every helper, 0 .. HELPERS - 1 (all slots are idle), whose results
     // have a place of their own.
