@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from pilotann_amd import utils
+from pilotann_amd.utils import graphs
 
 
 def test_graph_format_and_quality():
@@ -228,3 +229,30 @@ def test_insertion_order_makes_the_graph_navigable_across_clusters():
     # same seed, same graph
     again = utils.graph_init(x, 'nsw', deg, connect=False, seed=3)[1]
     assert torch.equal(again, indices)
+
+
+@pytest.mark.parametrize('batch,wrong', [(0, 1024), (1, 2048), (1, -2), (2, 2500)])
+def test_a_candidate_beyond_its_batch_is_seen(batch, wrong, monkeypatch):
+    """Each batch of the table ranks the rows up to its own end: another number in
+    it raises, also one that later batches may hold."""
+    x = torch.randn(2500, 8, generator=torch.Generator().manual_seed(1))
+    real, calls = graphs._knn_rows_host, []
+
+    def planted(*args):
+        ids, dist = real(*args)
+        if len(calls) == batch:
+            ids[3, 2] = wrong
+        calls.append(args[1:4])
+        return ids, dist
+
+    graphs.insertion_order_candidates(x, 6)
+    monkeypatch.setattr(graphs, '_knn_rows_host', planted)
+    with pytest.raises(AssertionError):
+        graphs.insertion_order_candidates(x, 6)
+    assert calls == [(0, 1024, 1024), (1024, 2048, 2048), (2048, 2500, 2500)]
+
+
+def test_no_candidates_asked_for():
+    for n in (0, 1, 1500):
+        ids, dist = graphs.insertion_order_candidates(torch.randn(n, 8), 0)
+        assert ids.shape == dist.shape == (n, 0)
