@@ -91,10 +91,14 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 // sizes within 1 % (64-float rows at H = 256, 103 registers: four 2.24, five 2.27
 // ms, so no floor there).  H = 512 and 1024 with two passes need 172 - 183 and are
 // held to three wavefronts (168, up to 17 spilled), which LDS then allows.
+// Rows of a length without a kernel of its own need 133 - 137 at H = 384 and 512 and
+// 175 at H = 2048: held to four wavefronts and to three (up to 8 spilled), without
+// which, 75 000 rows of 40 floats, 10 000 queries, H = 384 took 3.73 ms, now 3.23; 512
+// 5.20 / 4.48; 2048 28.0 / 25.3; 300 000 rows of 96 floats 5.01 / 4.66, 7.12 / 6.65, 36.2 / 34.0.
 #ifdef PA_WAVES_PER_EU
 #define PA_OCCUPANCY(H, WAVES) __attribute__((amdgpu_waves_per_eu(PA_WAVES_PER_EU, PA_WAVES_PER_EU)))
 #else
-#define PA_OCCUPANCY(H, WAVES) __attribute__((amdgpu_waves_per_eu((WAVES) > 1 && (H) <= 512 ? 4 : (H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 512 ? 3 : (H) <= 1024 ? (TWO ? 3 : 2) : 1, 8)))
+#define PA_OCCUPANCY(H, WAVES) __attribute__((amdgpu_waves_per_eu((WAVES) > 1 && (H) <= 512 ? 4 : (H) <= 256 ? (TWO ? 3 : DP8 == 16 ? 5 : 4) : (H) <= 512 ? (DP8 == 0 ? 4 : 3) : (H) <= 1024 ? (TWO ? 3 : 2) : DP8 == 0 ? 3 : 1, 8)))
 #endif
 
 // The longest open list (4096 cells) keeps level 11 in the wavefront's region of
