@@ -164,6 +164,11 @@ int pa_traverse_beside(int64_t *out_I, float *out_D, const int32_t *adj,
 int pa_traverse_form(int64_t n_storage, int64_t batch, int64_t beside, int dp,
                      int ef_total, int *near_bits);
 
+/* How many wavefronts (out) a query of such a launch has: 1, or 4 (three that read
+ * ahead of it; with near_bits only). */
+int pa_traverse_wavefronts(int64_t n_storage, int64_t batch, int64_t beside, int dp,
+                           int ef_total, int *wavefronts);
+
 /*
  * pa_traverse for callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops and harnesses that forbid it).  No counterpart
@@ -550,10 +555,16 @@ int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
                      void *workspace, size_t workspace_bytes,
                      uint64_t *counters, void *stream);
 
-/* The form that such a launch takes: wavefronts (out), 1 or 4 per query (4 also where
- * a compute unit has one query at most, which then has eight, seven reading ahead). */
+/* The form that such a launch takes: wavefronts (out) is 1 where a query's wavefront
+ * reads its rows itself and 4 where others read them, with it or ahead of it. */
 int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, int d_model,
                    int ef_search, int *wavefronts);
+
+/* How many wavefronts (out) a query of such a launch has: 1, 4 (three that read rows
+ * with it) or 8 (seven that read ahead of it, where a compute unit has one query at
+ * most). */
+int pa_refine_wavefronts(int64_t n_nodes, int64_t batch, int64_t beside, int d_model,
+                         int ef_search, int *wavefronts);
 
 #ifdef __cplusplus
 }

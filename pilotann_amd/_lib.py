@@ -27,6 +27,7 @@ _SIGNATURES = {
     'pa_traverse_beside': (_int, [_vp] * 9 + [_i64] * 4 + [_int] * 5 +
                            [_vp, _sz, _vp, _vp]),
     'pa_traverse_form': (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)]),
+    'pa_traverse_wavefronts': (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)]),
     'pa_traverse_static': (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                   _i64, _i64, _i64, _int, _int, _int, _int,
                                   _int, _vp, _vp]),
@@ -69,6 +70,7 @@ _SIGNATURES = {
     'pa_refine_beside': (_int, [_vp] * 12 + [_i64, _i64, _i64] + [_int] * 8 +
                          [_vp, _sz, _vp, _vp]),
     'pa_refine_form': (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)]),
+    'pa_refine_wavefronts': (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)]),
     'pa_pipeline': (_int, [_vp] * 15 + [_i64, _i64, _i64] + [_int] * 7 + [_vp]),
 }
 

@@ -749,6 +749,15 @@ extern "C" int pa_refine_form(int64_t n_nodes, int64_t batch, int64_t beside, in
     return PA_OK;
 }
 
+extern "C" int pa_refine_wavefronts(int64_t n_nodes, int64_t batch, int64_t beside,
+                                    int d_model, int ef_search, int *wavefronts) {
+    Plan p;
+    const int rc = make_plan(n_nodes, batch, beside, d_model, ef_search, &p);
+    if (rc != PA_OK) return rc;
+    if (wavefronts) *wavefronts = p.threads / kWave;
+    return PA_OK;
+}
+
 extern "C" int pa_refine_beside(int64_t *out_I, float *out_D, int64_t *buf_I, float *buf_D,
                                 const int64_t *init_I, float *init_D, const int32_t *sub_adj,
                                 const int32_t *sub_gid, const int64_t *sub_mapping,

@@ -985,6 +985,15 @@ extern "C" int pa_traverse_form(int64_t n_storage, int64_t batch, int64_t beside
     return PA_OK;
 }
 
+extern "C" int pa_traverse_wavefronts(int64_t n_storage, int64_t batch, int64_t beside, int dp,
+                                      int ef_total, int *wavefronts) {
+    Plan p;
+    const int rc = make_plan(n_storage, batch, beside, dp, ef_total, &p);
+    if (rc != PA_OK) return rc;
+    if (wavefronts) *wavefronts = p.threads / kWave;
+    return PA_OK;
+}
+
 namespace {
 
 // Checks and launch shared by pa_traverse and pa_traverse_static.  With

@@ -101,6 +101,26 @@ def test_both_forms(ef, dp, graph, device):
     assert near == far
 
 
+def wavefronts(n_storage, batch, beside, dp, ef_total):
+    form = ctypes.c_int(-1)
+    _lib.check(_lib.lib().pa_traverse_wavefronts(n_storage, batch, beside, dp, ef_total,
+                                                 ctypes.byref(form)), 'pa_traverse_wavefronts')
+    return form.value
+
+
+@pytest.mark.parametrize('dp', [32, 40, 64, 72, 128])
+@pytest.mark.parametrize('ef', [3, 8, 12, 16, 24, 32, 48, 64, 96, 128, 256, 512])
+def test_bits_in_lds_without_helpers(ef, dp, graph, device):
+    """Launches too large for wavefronts that read ahead, whose bits are in LDS still."""
+    print('no helpers', ef, dp, flush=True)
+    B = graph.query.size(0)
+    beside = next(b for b in range(0, 8192, 64)
+                  if wavefronts(graph.n_rows, B, b, dp, 4 * ef) == 1)
+    assert near_bits(graph.n_rows, B, beside, dp, 4 * ef) == 1
+    few, many = graph.check(dp, ef, device, [0, beside])
+    assert few == many
+
+
 def slots(n_storage, batch, dp, ef_total):
     n = ctypes.c_int(-1)
     _lib.check(_lib.lib().pa_traverse_plan(n_storage, batch, dp, ef_total, ctypes.byref(n),

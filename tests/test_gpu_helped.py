@@ -1,12 +1,14 @@
 """Searches whose wavefront has helpers that read rows ahead of it, against the
 oracle and, bit for bit and counter for counter, against the form without."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from common import Problem, assert_same_search
-from pilotann_amd import kernels
+from pilotann_amd import _lib, kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -14,7 +16,7 @@ pytestmark = pytest.mark.gpu
 # every storage form (registers, LDS, device memory); one, a few, many queries
 CASES = [
     (8, 1, 4, 1, 1),
-    (8, 8, 4, 2, 1024),   # (a workgroup that is done early takes a second query)
+    (8, 8, 4, 2, 1024),   # (as many as run at once: four workgroups a compute unit)
     (32, 32, 16, 32, 65),
     (40, 17, 24, 64, 128),
     (64, 64, 48, 0, 3),
@@ -24,6 +26,13 @@ CASES = [
     (128, 48, 250, 16, 9),
     (64, 32, 512, 32, 5),
 ]
+
+
+def wavefronts(n_storage, batch, beside, dp, ef_total):
+    form = ctypes.c_int(-1)
+    _lib.check(_lib.lib().pa_traverse_wavefronts(n_storage, batch, beside, dp, ef_total,
+                                                 ctypes.byref(form)), 'pa_traverse_wavefronts')
+    return form.value
 
 
 @pytest.mark.parametrize('dp,deg,ef,n_init,n_query', CASES)
@@ -38,6 +47,8 @@ def test_same_as_without_helpers(dp, deg, ef, n_init, n_query, device):
                                 p.mapping.to(device), p.nodelist.numel(), deg)
     rows = kernels.prepare_rows(p.x[p.nodelist].contiguous().to(device))
     query, dI, dD = p.query.to(device), I.to(device), D.to(device)
+    assert [wavefronts(p.nodelist.numel(), n_query, beside, dp, 4 * ef)
+            for beside in (0, 1 << 40)] == [4, 1]
     results = []
     for beside in (0, 1 << 40):
         out_I = torch.empty(n_query, 4, ef, dtype=torch.long, device=device)
@@ -53,4 +64,3 @@ def test_same_as_without_helpers(dp, deg, ef, n_init, n_query, device):
                         p.sub_indptr.numpy(), p.sub_indices.numpy(), p.x.numpy(),
                         p.query.numpy(), 4 * ef)
     assert_same_search(results[0][0].numpy(), results[0][1].numpy(), ref_I, ref_D)
-

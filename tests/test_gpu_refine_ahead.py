@@ -1,15 +1,24 @@
 """The refine's three forms (eight, four and one wavefront a query) on the random cases
 of the sweep: the same in every bit.  Cases with more candidates than a wavefront has
-lanes, with and without coordinates to complete, one query and more than one a slot."""
+lanes, with and without coordinates to complete, one query and some dozens."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from pilotann_amd import kernels
+from pilotann_amd import _lib, kernels
 from test_gpu_refine_fuzz import make_case
 
 pytestmark = pytest.mark.gpu
+
+
+def wavefronts(c, beside):
+    form = ctypes.c_int(-1)
+    _lib.check(_lib.lib().pa_refine_wavefronts(c['n'], c['B'], beside, c['d'], c['ef_search'],
+                                               ctypes.byref(form)), 'pa_refine_wavefronts')
+    return form.value
 
 
 @pytest.mark.parametrize('seed', range(24))
@@ -26,8 +35,10 @@ def test_three_forms_agree(seed, device):
                                       c['full_indices'].to(device), c['deg_full'])
     rows = kernels.PreparedRows(c['x'].to(device))
     query = c['query'].to(device)
+    besides = [next(b for b in range(0, 1 << 13, 16) if wavefronts(c, b) == form)
+               for form in (8, 4, 1)]
     results = []
-    for beside in (0, 300, 1 << 40):
+    for beside in besides:
         init_I, init_D = c['cand'].to(device), cand_D.clone()
         buf_I = torch.empty(c['B'], c['n_buffers'], dtype=torch.long, device=device)
         buf_D = torch.empty(c['B'], c['n_buffers'], device=device)
