@@ -152,7 +152,7 @@ constexpr int kRefineChunk = WAVES > 4 ? 4 * PA_LONG_CHUNK
                              : WAVES > 1 ? 2 * PA_LONG_CHUNK : PA_LONG_CHUNK;
 
 #define PA_REFINE_OCCUPANCY(H, WAVES) \
-    __attribute__((amdgpu_waves_per_eu((WAVES) > 4 ? 2 : (H) <= 256 || ((WAVES) > 1 && (H) <= 512) ? 4 : (H) <= 384 ? 3 : (H) <= 1024 ? 2 : 1, 8)))
+    __attribute__((amdgpu_waves_per_eu((WAVES) > 4 ? 2 : (H) <= 256 || ((WAVES) > 1 && (H) <= 512) ? 4 : (H) <= 384 || ((WAVES) > 1 && (H) <= 1024) ? 3 : (H) <= 1024 ? 2 : 1, 8)))
 
 // WAVES = 1: the wavefront of a query reads its rows itself.  WAVES = 4: three
 // more wavefronts wait at a barrier and read rows with it.  A search with the
@@ -160,10 +160,12 @@ constexpr int kRefineChunk = WAVES > 4 ? 4 * PA_LONG_CHUNK
 // 22 rows an expansion are two passes of 16, each of six trips to memory at 8
 // blocks a trip; with four wavefronts they are one pass of three trips at 16
 // blocks.  Up to H = 512 that is a few registers more than the 128 that four
-// wavefronts a SIMD have (14 - 27 spilled).  Measured at H = 32, 768 floats, 1 /
+// wavefronts a SIMD have (12 - 42 spilled).  Measured at H = 32, 768 floats, 1 /
 // 512 / 1024 queries: 249 / 416 / 620 us so, 247 / 408 / 735 without a spill at
 // half the queries a compute unit (for which 1024 take two rounds), 269 / 449 /
-// 629 with 8 blocks a trip.
+// 629 with 8 blocks a trip.  Lists of 2048 cells are held to three wavefronts a SIMD,
+// 768 queries at once: 600 / 760 of 768 floats 7.04 / 7.18 ms, where the two that they
+// took by themselves leave those batches to one wavefront a query (9.40 / 9.52).
 //
 // WAVES = 8: seven wavefronts read the rows of nodes the search is about to expand
 // (LookAhead), two a node, 32 blocks of a row at a time, and the candidates' rows

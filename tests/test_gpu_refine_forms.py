@@ -48,3 +48,12 @@ def test_forms_agree(seed, device):
         results.append([t.cpu().numpy() for t in (out_I, out_D, buf_I, buf_D, init_D, counters)])
     for few, many in zip(*results):
         assert np.array_equal(few, many, equal_nan=few.dtype == np.float32)
+
+
+@pytest.mark.parametrize('ef_search,batch', [(16, 1024), (64, 1024), (512, 1024), (513, 768),
+                                             (1024, 768), (1025, 512), (2048, 512)])
+def test_batches_that_have_four_wavefronts(ef_search, batch, device):
+    """The registers of each size of the lists leave room for so many queries at once."""
+    for d in (96, 768):
+        case = dict(n=1_000_000, B=batch, d=d, ef_search=ef_search)
+        assert wavefronts(case, 0) == 4
