@@ -284,12 +284,13 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
     int *cand_id = lds.cand_id;
     float *cand_key = lds.cand_key;
     uint32_t *seen = a.seen + (size_t)blockIdx.x * (size_t)a.slot_stride;
-    RefineVisited visited;   // (its slice is put back to zero after a query that used it)
+    RefineVisited visited;
     visited.init(lds.seen_table, seen, a.n_nodes);
     // The slice is cleared when it is first asked, which most queries never do (a
     // million nodes are 125 KB: one query 170 -> 164 us, 2500 of 768 floats 1321 ->
     // 1287), but in launches of more queries than workgroups at once: 10 000
-    // queries 5181 us so, 5266 the other way.
+    // queries 5181 us so, 5266 the other way.  There it is put back to zero after a
+    // query that used it; a workgroup's only query leaves it as it is.
     if (a.work_counter) {
         visited.clear(a.words_per_slot, lane);
         visited.zeroed = true;
@@ -586,7 +587,7 @@ __global__ __launch_bounds__(kWave *WAVES) PA_REFINE_OCCUPANCY(H, WAVES) void re
             PA_TIMER(7);
         }
 
-        visited.clean(a.words_per_slot, lane);
+        if (a.work_counter) visited.clean(a.words_per_slot, lane);
 
         if (a.counters && lane == 0) {
             atomicAdd(&a.counters[0], (unsigned long long)n_expand0);
