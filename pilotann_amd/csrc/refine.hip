@@ -161,9 +161,8 @@ constexpr int kRefineChunk = WAVES > 4 ? 4 * PA_LONG_CHUNK
 // blocks a trip; with four wavefronts they are one pass of three trips at 16
 // blocks.  Up to H = 512 that is a few registers more than the 128 that four
 // wavefronts a SIMD have (12 - 42 spilled).  Measured at H = 32, 768 floats, 1 /
-// 512 / 1024 queries: 249 / 416 / 620 us so, 247 / 408 / 735 without a spill at
-// half the queries a compute unit (for which 1024 take two rounds), 269 / 449 /
-// 629 with 8 blocks a trip.  Lists of 2048 cells are held to three wavefronts a SIMD,
+// 512 / 1000 queries: 230 / 393 / 594 us so, 226 / 376 / 774 at three wavefronts a SIMD
+// (for which 1000 take two rounds), 248 / 422 / 594 with 8 blocks a trip.  Lists of 2048 cells are held to three wavefronts a SIMD,
 // 768 queries at once: 600 / 760 of 768 floats 7.04 / 7.18 ms, where the two that they
 // took by themselves leave those batches to one wavefront a query (9.40 / 9.52).
 //
@@ -674,16 +673,17 @@ int make_plan(int64_t n_nodes, int64_t batch, int64_t beside, int d, int ef_sear
     while (p->sort_n < p->H) p->sort_n <<= 1;
     p->lds_bytes = query_floats(d) * 4;
     // Four wavefronts per query as long as every query, those of launches beside
-    // this one too, has its workgroup at once (1024 queries at H <= 512).  Measured on 1M x 768, H = 32: 1 query
-    // 374 -> 286 us, 37 482 -> 322, 512 642 -> 447; beyond that the wavefronts
-    // that only read rows take the place of queries: 1536 910 -> 1100 us; two
-    // launches of 1024 at a time, H = 128, 2.12 ms with four, 1.91 with one.
+    // this one too, has its workgroup at once (1024 queries at H <= 512).  Measured on
+    // 1M x 768, one / four, us: H = 32, one query 342 / 230 (the median of 60), 37 431 / 263,
+    // 512 587 / 393; H = 512, 1000 3574 / 2949; beyond that the wavefronts that only read rows
+    // take the place of queries: H = 32, 1500 854 / 990, H = 512 3860 / 5216; 96 floats, H = 64
+    // 419 / 678; two launches of 1250 at a time, H = 128, 2976 / 3604 (of 1000, which would
+    // be two full rounds, 2747 / 2205).
     // Eight where a compute unit has one query at most, seven of them helpers that
-    // read ahead (H = 32, 768 floats: 1 query 229 us with four wavefronts, 181 with
-    // eight; H = 48, 37 queries 342 / 284, 256 394 / 345; H = 128, 100 696 / 537; H =
-    // 512, 9 1787 / 1781; 96 floats, H = 64, 128 267 / 242).  With half the registers
-    // and two queries a compute unit, rows in three trips instead of two, they
-    // were at 204 and 317 us, and 512 queries at 491 against 466.
+    // read ahead.  Four / eight: H = 32, 768 floats, one query 230 / 182, 37 263 / 218, 256
+    // 320 / 283; H = 128, 37 621 / 490; H = 512, 37 1981 / 1908; 96 floats, H = 64, 256 299 /
+    // 265.  With half the registers and two queries a compute unit, rows in three trips
+    // instead of two, they were at 204 us for one query of H = 32 and 512 at 491 against 466.
     // (Their slots are 4 KB of LDS: of the longest rows a query fits beside them in the
     // other forms alone, and has no workgroup here.)
     p->threads = kAhead * kWave;

@@ -58,8 +58,8 @@ __device__ __forceinline__ int next_query(int *counter, int &turn, int batch, in
 // a level) with levels 8 and on in LDS: lists of 64 cells 416 / 537 -> 204 / 288,
 // of 256 584 / 602 -> 236 / 332, of 512 695 / 669 -> 296 / 388, of 2048 860 / 911 ->
 // 541 / 745.  In the searches: 100 000 rows of 32 floats, H = 256, 128 queries 495
-// -> 405 us; a million rows, 250 000 of 128 floats, H = 128, one query 302 -> 253
-// us; 10 000 queries, rows of 64 floats, H = 256 2.60 -> 2.26 ms; H = 1024,
+// -> 405 us; a million rows, 250 000 of 128 floats, H = 128, one query 334 -> 262
+// us (the median of 60); 10 000 queries, rows of 64 floats, H = 256 2.60 -> 2.26 ms; H = 1024,
 // 500 000 rows of 128 floats 19.7 -> 17.7 ms.
 __device__ __forceinline__ int float_to_key(float x) {
     const int b = __float_as_int(x);

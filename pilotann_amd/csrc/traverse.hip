@@ -83,10 +83,10 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 // instance has to be squeezed (the largest heaps are bounded by their LDS
 // anyway), and the allocator's own count decides the residency above it: 8 for
 // the smallest instances, 3 for 128-float rows with two passes of loads in flight
-// (TWO), which take 64 registers.  Measured for those over a million rows, three
-// wavefronts (153 registers) against four (128, 22 spilled): one query, H =
-// 128, 524 -> 507 us, 5000 1.63 -> 1.51 ms, 10 000 2.80 -> 2.67 ms.  With one pass,
-// which is for launches that fill the device, five (96, up to 15 spilled) against
+// (TWO), which take 64 registers.  Measured for those on 250 000 rows of a million, four
+// wavefronts (128 registers) / three (155 - 168), ms: H = 128, 1500 queries 0.72 / 0.64, 3000
+// 1.01 / 0.93, 10 000 2.88 / 2.61; H = 256, 1500 1.58 / 1.11, 10 000 5.79 / 4.66.  With one pass,
+// which is for launches that fill the device, five (96, up to 17 spilled) against
 // four (103 - 115): 500 000 rows, H = 256, 10 000 queries 3.22 -> 3.10 ms, the other
 // sizes within 1 % (64-float rows at H = 256, 103 registers: four 2.24, five 2.27
 // ms, so no floor there).  H = 512 and 1024 with two passes need 172 - 183 and are
@@ -103,12 +103,12 @@ __global__ void reset_work_counter(int *counter) { *counter = 0; }
 
 // The longest open list (4096 cells) keeps level 11 in the wavefront's region of
 // device memory instead of LDS (search_lists.h): first level kept there, 0 = the
-// whole list in registers and LDS.  Measured, with one LDS level more, on 10 000 queries over 500 000 rows of 128 floats: lists of 4096 cells run in
-// 50.0 instead of 69.7 ms with level 11 on in device memory (7 instead of 4
-// wavefronts per compute unit) and in 60.4 ms with level 10 on; lists of 2048
-// cells take 23.1 ms with level 10 on in device memory against 23.4 ms
-// without (11 instead of 8 wavefronts, each as much slower) and 29.6 ms with
-// level 9 on, so they stay in LDS.
+// whole list in registers and LDS.  Measured on 250 000 rows of 128 floats, 10 000
+// queries: lists of 4096 cells run in 22.2 ms so (10 wavefronts a compute unit, one pass of
+// rows), in 26.0 with all of it in LDS (5) and in 24.0 with level 10 there too; 3000
+// queries 8.9, 9.1 and 7.4.  (Where all have room with the list in LDS, it is the faster:
+// 1000 queries 4.33 / 3.32.)  Lists of 2048 cells: 8.9 ms in LDS, 11.0 with level 10 in
+// device memory.
 constexpr int deep_from(int H) { return H == 2048 ? 11 : 0; }
 
 // NEAR: the visited bits of a query are in LDS (behind the query where that is
@@ -133,8 +133,11 @@ __global__ __launch_bounds__(kWave *WAVES) PA_OCCUPANCY(H, WAVES) void traverse_
     // cells of the final sort: all of them, and those sorted in LDS at once
     constexpr int kSortAll = H <= kWave ? kWave : 1 << (floor_log2(H - 1) + 1);
     constexpr int kSortLds = kSortAll > 1024 ? 1024 : kSortAll;
-    // (NEAR: room for the levels from 8 on, and distances of their own: the size
-    // for which its lines in make_plan were measured)
+    // NEAR's lines in make_plan stand for room for the levels from 8 on and distances
+    // of their own.  2 KB of it are idle at H = 512 and more: without them the same
+    // times where the form stays the same, and where one more workgroup fits (250 000
+    // rows, H = 512, 1000 queries, which then have helpers) rows of 40 floats 1.97 -> 1.69 ms,
+    // of 64 1.51 -> 1.41, of 96 1.41 -> 1.28, of 128 1.26 -> 1.28.
     constexpr int kNearCells = !NEAR ? 0 : H == 2048 ? 1792 : 2 * H > 254 ? 2 * H - 254 : 0;
     constexpr int kListCells = Open::kLdsCells > kNearCells ? Open::kLdsCells : kNearCells;
     constexpr int kHeapCells = kListCells > kSortLds ? kListCells : kSortLds;
@@ -821,12 +824,14 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     // wavefronts per SIMD instead of three.  Two where the queries all run at
     // once; beyond that one, if it still has them all at once and two would leave
     // most of a second round empty, where the rows do not stay in cache, or
-    // with lists of 4096 cells (eight instead of nine wavefronts).  Measured,
-    // two passes / one, ms: 250 000 rows, H = 128, 3500 queries 1.31 / 1.24, 5000
-    // 1.49 / 1.55, 10 000 2.65 / 2.72, 40 000 9.40 / 9.70; 350 000 rows, H = 192, 5000
-    // queries 1.94 / 1.81, 40 000 10.8 / 10.0; 500 000 rows, H = 256, 5000 2.25 / 1.96,
-    // 10 000 3.70 / 3.23, 40 000 12.7 / 10.3; 250 000 rows, H = 2048, 10 000 42.0 /
-    // 37.2.  One query, one pass: 10 % slower and more.
+    // with lists of 4096 cells (ten instead of eight wavefronts).  Measured, two passes /
+    // one, ms.  250 000 rows of a million of 768 floats: H = 128, 3500 queries 1.20 / 1.10,
+    // 10 000 2.59 / 2.68, 40 000 9.60 / 9.66; H = 256, 6000 2.95 / 3.07, 40 000 17.1 / 17.4;
+    // H = 512, 10 000 10.5 / 10.8.  Rows of a mixture in 128 dimensions, which share more of
+    // their neighbours: 350 000, H = 192, 5000 1.60 / 1.41, 40 000 9.39 / 8.48; 500 000, H =
+    // 256, 10 000 3.61 / 3.16, 40 000 12.1 / 9.85; 250 000, H = 2048, 10 000 23.7 / 21.8; but one
+    // is the better on fewer of these too from H = 128 on: 75 000, H = 256, 10 000 2.42 / 2.16;
+    // 250 000, H = 128 1.78 / 1.75, H = 256 2.84 / 2.60 (H = 64 1.35 / 1.39).
     if (dp == 128 && batch > slots - beside) {
         const TraverseFn one = pick_kernel<false, false>(p->H, dp);
         int64_t one_slots = 0;
@@ -835,7 +840,7 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
         const bool short_round =
             batch <= one_slots - beside && batch <= 4 * slots / 3 - beside;
         // (where LDS holds no more of them than of the other form, as with lists
-        // of 2048 cells, two: 500 000 rows, 40 000 queries 72.2 / 74.2)
+        // of 2048 cells, two: 500 000 rows, 40 000 queries 37.8 / 38.0)
         if (one_slots > slots &&
             (short_round || n_storage * 512 > kTwoRowsBytes || p->H > 1024))
             p->fn = one, slots = one_slots;
@@ -853,19 +858,18 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
     // this one too, still has its wavefront at once: a test there is one LDS
     // operation where it was a table look-up and a trip to L2 or beyond for the
     // atomic.  (One word of table: a build for tests of the paths behind it.)
-    // Measured with 250 000 rows (31 KB, 1024 queries fit): 128-float rows, H =
-    // 128, one query 502 -> 478 us, 37 565 -> 520, 1024 710 -> 640; 64-float
-    // rows, H = 384, 37 queries 1.04 -> 0.99 ms; 500 000 rows, H = 1024, 512
-    // queries 3.88 -> 3.63 ms.
-    // Where only the other form has all queries at once, that one (whole
-    // searches in two halves; 100 000 rows of 64 floats, H = 512, 2 x 1500
-    // queries 4.94 with near bits, 4.03 ms without; 75 000 rows of 40 floats, H
-    // = 128, 2 x 2000 1.83 and 1.69 ms).  Where neither has, near bits if they
-    // take no query's place, or up to a third of them and each launch runs at
-    // once (the latter, H = 256, 2 x 2500 queries, 2816 at a time against 4096:
-    // 3.41 and 3.53 ms; the former, 2 x 2000, 2048 against 3584: 5.63 and 5.56;
-    // 6250 rows of 64 floats, H = 1024, 2 x 2500, 2304 at a time in both: 9.9
-    // and 10.5 ms).
+    // Measured without helpers on 250 000 rows (31 KB, 1024 queries fit), far / near, us:
+    // 128 floats, H = 128, one query 221 / 205, 37 382 / 378, 1024 516 / 493; H = 192, 512 686 /
+    // 610; 64 floats, H = 384, 37 929 / 885; 40 floats, H = 256, 1000 1373 / 1256; 500 000 rows
+    // of 128, H = 1024, 512 2416 / 2182.
+    // Where only the other form has all queries at once, that one (whole searches in
+    // two halves, far / near, ms: 100 000 rows of 64 floats, H = 512, 2 x 1500 2.16 / 2.34,
+    // 2 x 2000 2.27 / 2.74; 75 000 of 40, H = 128, 2 x 2000 0.83 / 0.95; but 100 000 of 128, H =
+    // 64, 2 x 2000 0.64 / 0.60).  Where neither has, near bits if they take no query's
+    // place (20 000 rows, 10 000 queries: 128 floats, H = 64 0.86 / 0.74, H = 512 3.54 / 3.35; 32
+    // floats, H = 256 1.84 / 1.72), or up to a third of them and each launch runs at once
+    // (2 x 2500: 50 000 rows of 40 floats, H = 256 1.66 / 1.53; 75 000 of 128, H = 256 1.66 /
+    // 1.52; at the end of it the other form is the better: 75 000 of 64, H = 256 1.42 / 1.55).
     const int64_t near_lds = p->lds_bytes + (int64_t)p->words_per_slot * 4;
     if (kSeenCacheLog2 > 0 && near_lds + kStaticLds <= max_lds) {
         const TraverseFn near_fn =
@@ -883,13 +887,17 @@ int make_plan(int64_t n_storage, int64_t batch, int64_t beside, int dp, int ef_t
         }
         // With three helpers as long as every query, those of launches beside this
         // one too, has its four wavefronts at once.  Measured, without / with, us:
-        // 250 000 rows of 128 floats, H = 128, one query 298 / 217; H = 192, 37
-        // queries 591 / 468, 512 706 / 559; H = 256, 1024 919 / 735; 500 000 rows, H
-        // = 1024, 37 2762 / 2282, 512 (the most that fit) 3145 / 3136; rows of 64
-        // floats, H = 384, 100 895 / 803; of 40, H = 256, 1000 524 / 449.  An
-        // expansion over rows of 32 floats is list work: H = 256, 128 388 / 370,
-        // 1700 538 / 536, but H = 512, 1000 878 / 893, H = 1024, 700 3325 / 3401.
-        // (Seven helpers: 217, 482, 582, 905 where three take 215, 479, 572, 770.)
+        // 250 000 rows of a million of 768 floats, dp = 128, H = 128, one query 262 / 201
+        // (the median of 60), 37 418 / 333, 1024 510 / 419; H = 192, 37 592 / 459; H = 256, 512
+        // 820 / 650, 1024 843 / 754; H = 1024, 37 3198 / 2552, 512 (the most that fit) 3348 /
+        // 2765; rows of 64 floats, H = 384, 100 1121 / 1033; of 40, H = 256, 1000 1256 / 946.
+        // (Seven helpers, H = 128, one query: the same; H = 256, 1024: 905 where three
+        // take 770.)  An expansion over rows of 32 floats is list work, and in lists
+        // of 768 cells and more how much of it depends on the rows: 25 000 of 100 000 in 64
+        // clusters, H = 384, 1000 660 / 776, H = 512 852 / 996, H = 1024 1748 / 2010; 250 000 of a
+        // wider mixture, H = 384, 500 1539 / 1348, H = 1024, 700 3043 / 2627.  Up to H = 256
+        // helpers are the faster on both (128 on the first 388 / 370, 1000 on the second
+        // 965 / 830).
         if (near_fits && (dp > 32 || p->H <= 256)) {
             const TraverseFn helped_fn = dp == 128 ? pick_kernel<true, true, kHelped>(p->H, dp)
                                                    : pick_kernel<true, false, kHelped>(p->H, dp);
