@@ -114,7 +114,7 @@ def test_refine_top_100_matches_oracle(index, device):
 
 
 def test_longest_lists_when_wavefronts_take_a_second_query(index, device):
-    """More queries than a launch has wavefronts (9 per compute unit with the
+    """More queries than a launch has wavefronts (10 per compute unit with the
     lists of 4096 cells), so that a wavefront starts a query on the log whose
     head the last query's two-part sort has rewritten: the 48 queries 60 times
     over, every copy equal to the oracle's answer for its query."""
