@@ -179,7 +179,7 @@ def insertion_order_candidates(x: torch.Tensor, pool: int, first: int = 1024):
     ids = torch.empty(n, pool, dtype=torch.long, device=x.device)
     dist = torch.empty(n, pool, dtype=torch.float32, device=x.device)
     lo, hi = 0, min(n, first)
-    ends, his = [], []      # a batch's lowest and highest id, and what it is below
+    batches = []
     while lo < n:
         # at most 2^21 rows a pass: the candidate lists of a pass are
         # 8 * pa_knn_list_capacity(keep) bytes a row
@@ -193,16 +193,19 @@ def insertion_order_candidates(x: torch.Tensor, pool: int, first: int = 1024):
                 if x.is_cuda:
                     torch.cuda.synchronize(x.device)
                 progress(f'neighbour table: {b} of {n} rows')
-        if __debug__ and pool:
-            ends += torch.aminmax(ids[lo:hi])
-            his.append(hi)
+        batches.append((lo, hi))
         lo, hi = hi, min(n, 2 * hi)
-    if __debug__ and ends:
+    if __debug__ and n and pool:
         # a kernel that left a place unwritten must raise here, not fault in a
         # later gather, and so must one that looked beyond the rows of its batch
-        # (one look at the answers of all: each is a wait for the device)
-        for (low, high), hi in zip(torch.stack(ends).view(-1, 2).tolist(), his):
-            assert -1 <= low and high < hi
+        # (one look at the answers for all: each is a wait for the device; by rows
+        # first, so that a batch is one small launch: 20 011 rows 65 us, each
+        # batch's ids by themselves 93)
+        low, high = torch.aminmax(ids, dim=1)
+        ends = [low.amin()] + [high[a:b].amax() for a, b in batches]
+        low, *highs = torch.stack(ends).tolist()
+        assert low >= -1
+        assert all(high < hi for high, (_, hi) in zip(highs, batches))
     return ids, dist
 
 
